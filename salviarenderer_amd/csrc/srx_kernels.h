@@ -110,7 +110,12 @@ void launch_batch_check(const batch_job* jobs, uint32_t njobs, uint32_t capacity
 void launch_batch_counts(const batch_job* jobs, uint32_t njobs, uint32_t* out, hipStream_t s);
 int vis_mode(const draw_params& P);
 
-hipError_t upload_ewa_table(const float* table256, hipStream_t s);
+// The anisotropic weights: each source that samples holds its own copy.
+hipError_t upload_ewa_table_raster(const float* table256, hipStream_t s);
+hipError_t upload_ewa_table_vis(const float* table256, hipStream_t s);
+
+// stats[slot] += sum(partial[0..n))
+void launch_reduce_partials(const unsigned long long* partial, uint32_t n, unsigned long long* stats, int slot, hipStream_t s);
 
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 // The vertex launch of a single draw; it also zeroes the draw's counters and ntiles words of tiles.

@@ -12,31 +12,16 @@
 //   sort            by GPU tile: a counting sort (order-independent draws) or a stable 8-bit LSD
 //                   radix sort -> per-tile lists in primitive order (the reference's per-tile
 //                   std::sort, rasterizer.cpp:947-994)
-//   raster_kernel   one workgroup per GPU tile, one thread per 2x2 quad; walks its tile's list in
+//   raster_kernel   (srx_raster.hip) one workgroup per GPU tile, one thread per 2x2 quad; walks its tile's list in
 //                   order and evaluates the reference's 64->16->4->sample decision chain per quad
 //                   (rasterizer.cpp:298-773), early/late depth-stencil, pixel shader and blending
 //                   (framebuffer.cpp).  Opaque early-Z draws defer the pixel shader to one pass over
 //                   the final per-sample winners.
-#include "srx_kernels.h"
-#include "srx_sampler.h"
-#include "srx_shade_common.h"
-#include "srx_sasl_exec.h"
-
-#include <type_traits>
+//   vis_kernel      (srx_vis.hip) the same decisions for opaque early-Z draws, whose result does not
+//                   depend on primitive order, fused with their shading
+#include "srx_kernel_common.h"
 
 namespace srx {
-
-__constant__ float c_ewa[256];
-
-enum { VS_PASSTHROUGH_COLOR = 1, VS_WVP_NORMAL_UV = 2, VS_WVP_COLOR = 3, VS_WVP_COLOR_LIGHT = 4, VS_COLORIZED = 5,
-       VS_MESH = 6, VS_SSM_DRAW = 7, VS_CUP = 8, VS_BOX = 9 };
-enum { PS_GOURAUD = 1, PS_LAMBERT_TEX = 2, PS_TEX_CPP = 3, PS_CONSTANT = 4, PS_SHADOW_PCF = 5, PS_COLORIZED = 6,
-       PS_MESH = 7, PS_SSM = 8, PS_CUP = 9, PS_BOX = 10 };
-enum { BLEND_OFF = 0, BLEND_ON = 1, BLEND_DISABLED = 2 };
-enum { TOPO_TRIANGLE_LIST = 2, TOPO_TRIANGLE_STRIP = 4 };
-enum { FMT_RGBA32F = 2, FMT_RGBA32I = 4, FMT_RGB32F = 6, FMT_RG32F = 16, FMT_R32F = 41 };
-enum { CULL_NONE = 0, CULL_FRONT = 1, CULL_BACK = 2 };
-enum { SOP_KEEP = 1, SOP_ZERO, SOP_REPLACE, SOP_INCR_SAT, SOP_DECR_SAT, SOP_INVERT, SOP_INCR_WRAP, SOP_DECR_WRAP };
 
 template <int NA>
 struct vtx {
@@ -303,11 +288,6 @@ struct tri_setup {
 };
 
 // compute_triangle_info (rasterizer.cpp:864-945) + compute_derivative_n (shader.cpp:414-450)
-// Register selects of whole vertices, one float at a time: a conditional over vertex lvalues
-// would select addresses and push the vertices into scratch memory.
-__device__ __forceinline__ float4 sel4(bool c, float4 a, float4 b) {
-  return make_float4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
-}
 template <int NA>
 __device__ __forceinline__ vtx<NA> vsel(bool c, const vtx<NA>& a, const vtx<NA>& b) {
   vtx<NA> o;
@@ -660,30 +640,6 @@ __device__ __forceinline__ void write_tri_attr(float4* a, const tri_setup<NA>& t
   for (int k = 0; k < 3 * (NA + 1); ++k) a[k] = w[k];
 }
 
-__device__ __forceinline__ void read_tri_rec(const float4* rec, float* e, float* bb) {
-  float4 a = rec[0], b = rec[1], c = rec[2], d = rec[3];
-  e[0] = a.x; e[1] = a.y; e[2] = a.z; e[3] = a.w; e[4] = b.x; e[5] = b.y; e[6] = b.z; e[7] = b.w; e[8] = c.x;
-  bb[0] = c.y; bb[1] = c.z; bb[2] = c.w; bb[3] = d.x;
-}
-
-// Sums v over the workgroup and stores the total in partial[blockIdx.x] (no global atomics: many
-// same-address device-scope atomics from every XCD serialise badly).  All threads must call it.
-__device__ __forceinline__ void block_partial(unsigned long long* __restrict__ partial, unsigned long long v) {
-  __shared__ unsigned long long wsum[16];
-  unsigned long long s = v;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  const int wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) wsum[wave] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (int w = 0; w < nw; ++w) t += wsum[w];
-    partial[blockIdx.x] = t;
-  }
-}
-
 // Sum of v over the workgroup, returned to thread 0.  All threads must call it.
 __device__ __forceinline__ uint32_t block_sum_u32(uint32_t v) {
   __shared__ uint32_t wsum[16];
@@ -1003,15 +959,6 @@ __global__ void clip_kernel(draw_params P, const float4* __restrict__ vbuf, floa
 // off: exclusive scan of the per-triangle record counts; a triangle owns [off[id], off[id+1]).
 // One thread per primitive, over its (at most 3) clipped triangles in fan order.  Records beyond
 // `capacity` are dropped; the host compares the total with it and emits again.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  int lane = __lane_id();
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    uint32_t t = __shfl_up(v, off, 64);
-    if (lane >= off) v += t;
-  }
-  return v;
-}
 
 // Records of one clipped triangle emitted by a whole wave: lanes take the triangle's 64x64 tiles in
 // for_each_gtile's order, count each tile's GPU tiles with the same tests, and write at their
@@ -1895,62 +1842,6 @@ void launch_tile_order(const draw_params& P, const draw_buffers& B, uint32_t* or
   hipLaunchKernelGGL(tile_class_order_kernel, dim3((T + 255) / 256), dim3(256), 0, s, B.tstart, B.tend, T, B.counters, order);
 }
 
-// records per workgroup beyond which a tile of a depth-only draw is split
-constexpr uint32_t VIS_PART = 256;
-
-// Work table of the order-independent visibility kernel for draws without shading (depth-only
-// passes), whose time is the longest tile's: a GPU tile with more than VIS_PART records is split
-// into parts of at most VIS_PART records, each a workgroup of the first launch that leaves its
-// partial per-sample keys in `partial`; the second launch merges a split tile's parts (a minimum,
-// so the order of the parts is immaterial) and finishes it.  (Draws that shade keep whole tiles:
-// their shading fills the GPU while the long tiles run.)  Entries follow `order`, heaviest first.
-//   entries[i] = (tile, part, parts, first partial slot)   i < counts[0]
-//   merges[i]  = (tile, parts, first partial slot, 0)      i < counts[1]
-__global__ void __launch_bounds__(1024) vis_table_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
-                                                         const uint32_t* __restrict__ order, uint32_t T,
-                                                         uint4* __restrict__ entries, uint4* __restrict__ merges,
-                                                         uint32_t* __restrict__ counts) {
-  __shared__ uint32_t wtot[3][16];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t per = (T + 1023) / 1024, p0 = tid * per, p1 = min(T, p0 + per);
-  uint32_t c[3] = {0, 0, 0};  // blocks, partial slots, merges in this thread's segment of `order`
-  for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = order[p], n = te[t] - ts[t];
-    const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
-    c[0] += parts;
-    if (parts > 1) { c[1] += parts; c[2] += 1; }
-  }
-  uint32_t incl[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    incl[k] = wave_incl_scan(c[k]);
-    if (lane == 63) wtot[k][wave] = incl[k];
-  }
-  __syncthreads();
-  uint32_t base[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    uint32_t before = 0, total = 0;
-    for (uint32_t w = 0; w < 16; ++w) {
-      if (w < wave) before += wtot[k][w];
-      total += wtot[k][w];
-    }
-    base[k] = before + incl[k] - c[k];
-    if (tid == 0) counts[k == 0 ? 0 : (k == 1 ? 2 : 1)] = total;
-  }
-  uint32_t b = base[0], sl = base[1], m = base[2];
-  for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = order[p], n = te[t] - ts[t];
-    const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
-    for (uint32_t k = 0; k < parts; ++k) entries[b + k] = make_uint4(t, k, parts, sl);
-    b += parts;
-    if (parts > 1) {
-      merges[m++] = make_uint4(t, parts, sl, 0u);
-      sl += parts;
-    }
-  }
-}
-
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s) {
   if (n) hipLaunchKernelGGL(fill_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
 }
@@ -1967,1391 +1858,9 @@ void launch_tile_ranges(const draw_params& P, const draw_buffers& B, int which, 
   hipLaunchKernelGGL(tile_range_kernel, dim3((n + 255) / 256), dim3(256), 0, s, B.keys[which], n, T, B.tstart, B.tend);
 }
 
-// ============================================================== pixel shaders
-__device__ __forceinline__ void normalize3(float x, float y, float z, float& ox, float& oy, float& oz) {
-  float t = 0.0f;
-  t += x * x;
-  t += y * y;
-  t += z * z;
-  float len = sqrtf(t);
-  if (equal_eps(len, 0.0f)) len = 1.0f;
-  float inv = 1.0f / len;
-  ox = x * inv;
-  oy = y * inv;
-  oz = z * inv;
-}
-
-// 3x3 percentage-closer shadow lookup of one pixel (attr0 colour, attr1 light clip position): the
-// tap layout of StandardShadowMap.cpp:86-106, each tap a tex2dlod at lod 0, lit when the light-space
-// depth minus the bias does not exceed it.
-__device__ __forceinline__ float4 shadow_pcf(const draw_params& P, const ps_samplers* __restrict__ SM, float4 a, float4 l) {
-  const float lx = l.x / l.w, ly = l.y / l.w, lz = l.z / l.w;
-  const float cu = (lx + 1.0f) * 0.5f, cv = 1.0f - (ly + 1.0f) * 0.5f;
-  const float o = P.ps_consts[2];
-  int count = 0;
-  if (P.has_sampler[0]) {
-    for (int ty = -1; ty <= 1; ++ty)
-      for (int tx = -1; tx <= 1; ++tx) {
-        const float u = cu + static_cast<float>(tx) * o, v = cv + static_cast<float>(ty) * o;
-        const float4 t = sample_lod0(SM->s[0], u, v);
-        if (lz - P.ps_consts[1] <= t.x) ++count;
-      }
-  }
-  const float lit = static_cast<float>(count) / 9.0f;
-  const float k = P.ps_consts[0] + (1.0f - P.ps_consts[0]) * lit;
-  return make_float4(a.x * k, a.y * k, a.z * k, a.w);
-}
-
-// cpp_pixel_shader::tex2d(s, reg) (cpp_pixel_shader.cpp:13-31): one LOD per quad from the register's
-// p1 - p0 and p2 - p0 (calc_lod_2d, sampler.cpp:834-852), then sample_2d_lod at pixel pi
-template <int NA>
-__device__ __forceinline__ float4 tex2d_cpp(const sampler_desc_dev& sp, const quad_lazy<NA>& q, int reg, int pi) {
-  const float4 u0 = q.reg(reg, 0, q.inv_w(0), 2), u1 = q.reg(reg, 1, q.inv_w(1), 2), u2 = q.reg(reg, 2, q.inv_w(2), 2);
-  const float dxu = u1.x - u0.x, dxv = u1.y - u0.y;
-  const float dyu = u2.x - u0.x, dyv = u2.y - u0.y;
-  const float lod = (sp.mip_filter == FILTER_ANISO && sp.max_aniso > 1) ? calc_aniso(sp, dxu, dxv, dyu, dyv, 0.0f).lod
-                                                                        : calc_lod(sp, dxu, dxv, dyu, dyv, 0.0f);
-  const float4 uv = q.reg(reg, pi, q.inv_w(pi), 2);
-  return sample_impl(sp, uv.x, uv.y, lod, nullptr);
-}
-// eflib vector helpers on .xyz (vector_generic.h:110-118, math.cpp:39-41,85-87)
-__device__ __forceinline__ float dot3(float4 a, float4 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ float length3(float4 a) {
-  float t = 0.0f;
-  t += a.x * a.x;
-  t += a.y * a.y;
-  t += a.z * a.z;
-  return sqrtf(t);
-}
-__device__ __forceinline__ float4 normalize3v(float4 v) {
-  float x, y, z;
-  normalize3(v.x, v.y, v.z, x, y, z);
-  return make_float4(x, y, z, 0.0f);
-}
-__device__ __forceinline__ float4 reflect3(float4 i, float4 n) {
-  const float k = 2.0f * dot3(i, n);
-  return make_float4(i.x - n.x * k, i.y - n.y * k, i.z - n.z * k, 0.0f);
-}
-
-// ColorizedTriangle.cpp:55-92: three lights, attr0 normal, attr1..3 light vectors
-template <int NA>
-__device__ __forceinline__ float4 ps_colorized(const quad_lazy<NA>& q, int pi) {
-  const float iw = q.inv_w(pi);
-  const float4 n = q.reg(1, pi, iw, 3);
-  float4 ld[3];
-  float inv[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    ld[i] = q.reg(2 + i, pi, iw, 3);
-    inv[i] = 1.0f / length3(ld[i]);
-  }
-  const float4 nn = normalize3v(n);
-  float refl[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) refl[i] = dot3(nn, make_float4(ld[i].x * inv[i], ld[i].y * inv[i], ld[i].z * inv[i], 0.0f));
-  const float c[3][3] = {{0.7f, 0.1f, 0.3f}, {0.1f, 0.3f, 0.7f}, {0.3f, 0.7f, 0.1f}};
-  float o[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    float a = ((c[0][k] * refl[0]) * inv[0]) * inv[0];
-    float b = ((c[1][k] * refl[1]) * inv[1]) * inv[1];
-    float d = ((c[2][k] * refl[2]) * inv[2]) * inv[2];
-    o[k] = std_clamp((a + b) + d, 0.0f, 1.0f);
-  }
-  return make_float4(o[0], o[1], o[2], 1.0f);
-}
-
-// ComplexMesh.cpp:227-246
-template <int NA>
-__device__ __forceinline__ float4 ps_mesh(const quad_lazy<NA>& q, int pi) {
-  const float iw = q.inv_w(pi);
-  const float4 l = normalize3v(q.reg(1, pi, iw, 3)), e = normalize3v(q.reg(2, pi, iw, 3)), n = normalize3v(q.reg(3, pi, iw, 3));
-  const float n_dot_l = dot3(n, l);
-  const float4 h = normalize3v(make_float4(l.x + e.x, l.y + e.y, l.z + e.z, 0.0f));
-  const float spec = 3.5f * powf(std_max(dot3(h, n), 0.0f), 5.0f);  // (roughness + 2) / 2 with roughness 5
-  const float clr = n_dot_l * (0.8f + spec * 0.4f);
-  return make_float4(clr, clr, clr, 1.0f);
-}
-
-// StandardShadowMap.cpp:62-142 (exponential shadow map, esm_constant 25000, 3x3 Gaussian weights)
-template <int NA>
-__device__ __forceinline__ float4 ps_ssm(const draw_params& P, const ps_samplers* __restrict__ SM, const quad_lazy<NA>& q,
-                                         int pi) {
-  const float iw = q.inv_w(pi);
-  float occlusion = 0.0f;
-  if (P.has_sampler[0]) {
-    const float4 l4 = q.reg(5, pi, iw);
-    const float lx = l4.x / l4.w, ly = l4.y / l4.w, lz = l4.z / l4.w;
-    const float cx = (lx + 1.0f) * 0.5f, cy = 1.0f - (ly + 1.0f) * 0.5f;
-    const float o = 1 / 512.0f;
-    const float ox[9] = {-o, 0.0f, +o, -o, 0.0f, +o, -o, 0.0f, +o};
-    const float oy[9] = {-o, -o, -o, 0.0f, 0.0f, 0.0f, +o, +o, +o};
-    const float gw[9] = {0.027681f, 0.111014f, 0.027681f, 0.111014f, 0.445213f, 0.111014f, 0.027681f, 0.111014f, 0.027681f};
-    float sd[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) sd[i] = sample_lod0(SM->s[0], cx + ox[i], cy + oy[i]).x;
-    const float esm = 25000.0f;
-    float occ = 0.0f;
-#pragma unroll
-    for (int i = 1; i < 9; ++i) occ += gw[i] * expf(esm * (sd[i] - sd[0]));
-    occ += gw[0];
-    occ = logf(occ);
-    occ += esm * sd[0];
-    occlusion = std_clamp(expf(occ - esm * lz), 0.0f, 1.0f);
-  }
-  float4 tex = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-  if (P.has_sampler[1]) tex = tex2d_cpp(SM->s[1], q, 1, pi);
-  const float4 n = normalize3v(q.reg(2, pi, iw, 3)), ld = normalize3v(q.reg(3, pi, iw, 3)), ed = normalize3v(q.reg(4, pi, iw, 3));
-  const float idiff = std_clamp(dot3(ld, n), 0.0f, 1.0f);
-  const float4 r = reflect3(ld, n);
-  const float ispec = std_clamp(dot3(make_float4(-r.x, -r.y, -r.z, 0.0f), ed), 0.0f, 1.0f);
-  // pow(float, int) promotes to double (C++11 <cmath>), then the vec4 product rounds it to float
-  const float p = static_cast<float>(pow(static_cast<double>(ispec), static_cast<double>(__float_as_int(P.ps_consts[12]))));
-  const float* amb = P.ps_consts;
-  const float* dif = P.ps_consts + 4;
-  const float* spc = P.ps_consts + 8;
-  float4 out;
-  out.x = tex.x * (amb[0] + (dif[0] * idiff + spc[0] * p) * occlusion);
-  out.y = tex.y * (amb[1] + (dif[1] * idiff + spc[1] * p) * occlusion);
-  out.z = tex.z * (amb[2] + (dif[2] * idiff + spc[2] * p) * occlusion);
-  out.w = 1.0f;
-  return out;
-}
-
-// StencilMirror.cpp:66-110
-template <int NA>
-__device__ __forceinline__ float4 ps_cup(const draw_params& P, const ps_samplers* __restrict__ SM, const quad_lazy<NA>& q,
-                                         int pi) {
-  const float iw = q.inv_w(pi);
-  float4 tex = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-  if (P.has_sampler[0]) tex = tex2d_cpp(SM->s[0], q, 1, pi);
-  const float4 n = normalize3v(q.reg(2, pi, iw, 3)), ld = normalize3v(q.reg(3, pi, iw, 3)), ed = normalize3v(q.reg(4, pi, iw, 3));
-  const float idiff = std_clamp(dot3(ld, n), 0.0f, 1.0f);
-  const float ispec = std_clamp(dot3(reflect3(ld, n), ed), 0.0f, 1.0f);
-  const float* amb = P.ps_consts;
-  const float* dif = P.ps_consts + 4;
-  const float* spc = P.ps_consts + 8;
-  float4 out;
-  out.x = tex.x * ((amb[0] + dif[0] * idiff) + spc[0] * ispec);
-  out.y = tex.y * ((amb[1] + dif[1] * idiff) + spc[1] * ispec);
-  out.z = tex.z * ((amb[2] + dif[2] * idiff) + spc[2] * ispec);
-  out.w = 1.0f;
-  return out;
-}
-
-// Pixel shader (cpp_pixel_shader::execute, cpp_pixel_shader.cpp:62-74) colour of quad pixel pi
-// only; the other three pixels supply derivatives.  The sample shaders never discard.
-template <int NA>
-__device__ __forceinline__ float4 run_ps_pixel(const draw_params& P, const ps_samplers* __restrict__ SM,
-                                               const quad_lazy<NA>& q, int pi) {
-  switch (P.ps_id) {
-  case PS_GOURAUD:
-    return q.reg(1, pi, q.inv_w(pi));
-  case PS_CONSTANT:
-    return make_float4(P.ps_consts[0], P.ps_consts[1], P.ps_consts[2], P.ps_consts[3]);
-  case PS_LAMBERT_TEX:
-    if constexpr (NA >= 2) {
-      // SASL tex2D: ddx per row (p1-p0, p3-p2), ddy per column (p2-p0, p3-p1)
-      // (sasl/src/codegen/cgs_simd.cpp:275-312), then sample_2d_grad (sampler_api.cpp:13-18);
-      // uv at pi and its row and column neighbours
-      const int pr = pi ^ 1, pc = pi ^ 2;
-      const float iw = q.inv_w(pi), iwr = q.inv_w(pr), iwc = q.inv_w(pc);
-      const float4 uv = q.reg(2, pi, iw, 2), uvr = q.reg(2, pr, iwr, 2), uvc = q.reg(2, pc, iwc, 2);
-      const bool col1 = (pi & 1) != 0, row1 = (pi & 2) != 0;
-      // row: (left, right) = col1 ? (neighbour, pi) : (pi, neighbour); column likewise
-      const float4 r0 = sel4(col1, uvr, uv), r1 = sel4(col1, uv, uvr);
-      const float4 c0 = sel4(row1, uvc, uv), c1 = sel4(row1, uv, uvc);
-      const float dxu = r1.x - r0.x, dxv = r1.y - r0.y;
-      const float dyu = c1.x - c0.x, dyv = c1.y - c0.y;
-      const float4 nrm = q.reg(1, pi, iw, 3);
-      float4 t = make_float4(0, 0, 0, 0);
-      if (P.has_sampler[0]) {
-        const sampler_desc_dev& sp = SM->s[0];
-        t = sp.fast_aniso ? sample_2d_grad_fast(sp, uv.x, uv.y, dxu, dxv, dyu, dyv, 0.0f)
-                          : sample_2d_grad(sp, uv.x, uv.y, dxu, dxv, dyu, dyv, 0.0f);
-      }
-      float nx, ny, nz;
-      normalize3(nrm.x, nrm.y, nrm.z, nx, ny, nz);
-      float d = nx * P.ps_consts[0] + ny * P.ps_consts[1] + nz * P.ps_consts[2];
-      float k = std_clamp(d, 0.0f, 1.0f);
-      return make_float4(t.x * k, t.y * k, t.z * k, 1.0f);
-    }
-    return make_float4(0, 0, 0, 0);
-  case PS_TEX_CPP: {
-    // AnisotropicFilter / TextureAndBlending ps_plane: tex2d(s0, attr0) with alpha 1
-    if (!P.has_sampler[0]) return make_float4(0, 0, 0, 1.0f);
-    float4 t = tex2d_cpp(SM->s[0], q, 1, pi);
-    t.w = 1.0f;
-    return t;
-  }
-  case PS_COLORIZED:
-    if constexpr (NA >= 4) return ps_colorized(q, pi);
-    return make_float4(0, 0, 0, 0);
-  case PS_MESH:
-    if constexpr (NA >= 3) return ps_mesh(q, pi);
-    return make_float4(0, 0, 0, 0);
-  case PS_SSM:
-    if constexpr (NA >= 5) return ps_ssm(P, SM, q, pi);
-    return make_float4(0, 0, 0, 0);
-  case PS_CUP:
-    if constexpr (NA >= 4) return ps_cup(P, SM, q, pi);
-    return make_float4(0, 0, 0, 0);
-  case PS_BOX: {  // TextureAndBlending.cpp:96-114
-    if constexpr (NA >= 2) {
-      if (!P.has_sampler[0]) return make_float4(1.0f, 1.0f, 1.0f, 0.5f);
-      float4 t = tex2d_cpp(SM->s[0], q, 2, pi);
-      t.w = 0.5f;
-      return t;
-    }
-    return make_float4(0, 0, 0, 0);
-  }
-  case PS_SHADOW_PCF:
-    if constexpr (NA >= 2) {
-      const float iw = q.inv_w(pi);
-      return shadow_pcf(P, SM, q.reg(1, pi, iw), q.reg(2, pi, iw));
-    }
-    return make_float4(0, 0, 0, 0);
-  default:
-    return make_float4(0, 0, 0, 0);
-  }
-}
-
-// ============================================================== raster
-struct prim_lds {
-  float e[9];
-  float bb[4];     // relative to the 64x64 tile origin
-  float ev1[3];    // stage-16 rejection value, already offset by the 64x64 tile origin
-  float s1x[3], s1y[3], ra1[3];
-  float ev2[3], s2x[3], s2y[3], ra2[3];
-  float zx, zy, z0, dzx, dzy;
-  float aa[4];
-  uint32_t idf;    // triangle id << 1 | tile-level accept
-  uint32_t r16;    // bit k: 16x16 region k of the GPU tile rejected; bit 16+k: accepted
-  uint32_t front;
-};
-
-__device__ __forceinline__ bool cmpf(int f, float a, float b) {
-  switch (f) {
-  case 0: return false;
-  case 1: return a < b;
-  case 2: return a == b;
-  case 3: return a <= b;
-  case 4: return a > b;
-  case 5: return a != b;
-  case 6: return a >= b;
-  default: return true;
-  }
-}
-__device__ __forceinline__ bool cmpu(int f, uint32_t a, uint32_t b) {
-  switch (f) {
-  case 0: return false;
-  case 1: return a < b;
-  case 2: return a == b;
-  case 3: return a <= b;
-  case 4: return a > b;
-  case 5: return a != b;
-  case 6: return a >= b;
-  default: return true;
-  }
-}
-// framebuffer.cpp:136-166
-__device__ __forceinline__ uint32_t stencil_op(int op, uint32_t ref, uint32_t cur) {
-  switch (op) {
-  case SOP_ZERO: return 0;
-  case SOP_REPLACE: return ref;
-  case SOP_INCR_SAT: return min(0xFFu, cur + 1);
-  case SOP_DECR_SAT: return cur - 1;  // std::max<uint32_t>(0, cur - 1) never clamps
-  case SOP_INVERT: return ~cur;
-  case SOP_INCR_WRAP: return (cur + 1) & 0xFF;
-  case SOP_DECR_WRAP: return (cur - 1 + 256) & 0xFF;
-  default: return cur;
-  }
-}
-
-
-__device__ __forceinline__ void blend_store(const draw_params& P, int x, int y, int smp, float4 src) {
-  if (!P.color.data) return;
-  uint8_t* a = sample_addr(P.color, x, y, smp);
-  if (P.blend_id == BLEND_OFF) {
-    store_texel(P.color.pf, a, src);
-  } else if (P.blend_id == BLEND_ON) {
-    store_texel(P.color.pf, a, lerp4(load_texel(P.color.pf, a), src, src.w));
-  }
-}
-
-
-// Pixel shader and backend for one triangle on a 2x2 quad: `pm` holds the samples to store, bits
-// 4i..4i+S-1 for pixel i.  Interpolants are formed per pixel where read (quad_lazy), so only one
-// pixel's registers are live at a time; the colour of each pixel is the quad shader's.
-template <int NA, int S, bool SASL = false>
-__device__ __forceinline__ void shade_store(const draw_params& P, const ps_samplers* __restrict__ SM,
-                                         const float4* __restrict__ tri_attr, uint32_t id, int px0, int py0, uint32_t pm) {
-  attr_setup<NA> at;
-  load_attr<NA>(P, tri_attr, id, at);
-  const quad_lazy<NA> q(at, P, px0, py0);
-  if constexpr (SASL) {
-    // pixel_shader_unit::update + execute (shader_unit.cpp:106-176) on the whole quad: input i is
-    // attribute inputs[i].attr of each pixel, the program runs the four pixels together
-    const sasl_program* __restrict__ prog = P.sasl;
-    sasl_regs R;
-    const uint32_t nregs = prog->nregs;
-    for (uint32_t r = 0; r < nregs; ++r)
-      for (int px = 0; px < 4; ++px) R.r[r][px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const uint32_t nin = prog->ninputs;
-    for (int px = 0; px < 4; ++px) {
-      const float iw = q.inv_w(px);
-      for (uint32_t k = 0; k < nin; ++k) {
-        const sasl_input inp = prog->inputs[k];
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int a = 0; a < NA; ++a)
-          if (a == inp.attr) v = q.reg(a + 1, px, iw);
-        R.r[inp.reg][px] = make_float4(v.x, inp.ncomp > 1 ? v.y : 0.0f, inp.ncomp > 2 ? v.z : 0.0f, inp.ncomp > 3 ? v.w : 0.0f);
-      }
-    }
-    sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
-      if (!P.has_sampler[slot]) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      const sampler_desc_dev& sp = SM->s[slot];
-      return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                           : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
-    });
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t m = (pm >> (4 * i)) & 15u;
-      if (!m) continue;
-      const float4 c = sasl_color0(prog, R, i);
-      for (int s = 0; s < S; ++s)
-        if (m & (1u << s)) blend_store(P, px0 + (i & 1), py0 + (i >> 1), s, c);
-    }
-    return;
-  }
-#pragma unroll 1
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t m = (pm >> (4 * i)) & 15u;
-    if (!m) continue;
-    const float4 c = run_ps_pixel<NA>(P, SM, q, i);
-    for (int s = 0; s < S; ++s)
-      if (m & (1u << s)) blend_store(P, px0 + (i & 1), py0 + (i >> 1), s, c);
-  }
-}
-
-// One workgroup per GPU tile, one thread per 2x2 quad.  VIS: opaque early-Z draws -- record for every
-// sample the last triangle that passed (the colour it ends with) into `vis`; the pixel shader runs
-// later in shade_kernel.  Otherwise every quad runs the pixel shader and the backend in primitive order.
-template <int NA, int S, bool VIS, bool SASL = false>
-__global__ void __launch_bounds__(256) raster_kernel(draw_params P, const ps_samplers* __restrict__ SM,
-                                                      const uint32_t* __restrict__ order, const uint32_t* __restrict__ vals,
-                                                      const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
-                                                      const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
-                                                      uint32_t* __restrict__ vis, unsigned long long* __restrict__ partial) {
-  extern __shared__ prim_lds lds[];
-  const int G = P.gt, QW = G / 2;
-  const int gtile = order[blockIdx.x];
-  const int gx = gtile % P.gtiles_x, gy = gtile / P.gtiles_x;
-  const int tid = threadIdx.x, nthreads = blockDim.x;
-  const int qx = tid % QW, qy = tid / QW;
-  const int px0 = gx * G + qx * 2, py0 = gy * G + qy * 2;  // quad origin
-  const int t64x = (gx * G) & ~(TILE - 1), t64y = (gy * G) & ~(TILE - 1);
-  const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
-  // pixel i of the quad: (px0 + (i & 1), py0 + (i >> 1))
-  bool pin[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) pin[i] = (px0 + (i & 1)) < tw && (py0 + (i >> 1)) < th;
-
-  // depth/stencil of the quad's samples, held in registers for the whole tile
-  // VIS draws have stencil off, so only depth is kept (and written back)
-  float depth[4][S];
-  uint32_t stencil[4][VIS ? 1 : S];
-  uint32_t winner[4][VIS ? S : 1];
-  const bool has_ds = P.ds.data != nullptr;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      depth[i][s] = 0.0f;
-      if constexpr (!VIS) stencil[i][s] = 0;
-      if constexpr (VIS) winner[i][s] = NO_WINNER;
-      if (has_ds && pin[i]) {
-        if constexpr (VIS) {
-          depth[i][s] = *reinterpret_cast<const float*>(sample_addr(P.ds, px0 + (i & 1), py0 + (i >> 1), s));
-        } else {
-          float2 d = *reinterpret_cast<const float2*>(sample_addr(P.ds, px0 + (i & 1), py0 + (i >> 1), s));
-          depth[i][s] = d.x;
-          stencil[i][s] = __float_as_uint(d.y);
-        }
-      }
-    }
-  if constexpr (!VIS) {
-    // Stencil changes only where the stencil test passes, so a tile none of whose samples passes it
-    // now can never pass it during this draw: nothing in the tile changes (exact early-out, taken
-    // only when no statistics are counted).
-    if (P.stencil_enable && !P.count_stats) {
-      int can = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-          if (pin[i]) {
-            const uint32_t os = stencil[i][s] & P.read_mask;
-            can |= cmpu(P.st_func[0], P.stencil_ref, os) || cmpu(P.st_func[1], P.stencil_ref, os);
-          }
-      if (!__syncthreads_or(can)) return;
-    }
-  }
-  const bool any_in = pin[0];
-  unsigned long long ps_inv = 0, be_pix = 0;
-  const uint32_t full_px = (S == 1) ? 1u : (S == 2 ? 3u : 15u);
-
-  const uint32_t t0 = tstart[gtile], t1 = tend[gtile];
-  // 16x16, 4x4 regions of this quad inside its 64x64 tile
-  const int rx64 = px0 - t64x, ry64 = py0 - t64y;
-  const int ix16 = rx64 >> 4, iy16 = ry64 >> 4;
-  const int r16k = ((py0 - gy * G) >> 4) * (G / 16) + ((px0 - gx * G) >> 4);
-  const int R16x = t64x + ix16 * 16, R16y = t64y + iy16 * 16;
-  const int ix4 = (px0 - R16x) >> 2, iy4 = (py0 - R16y) >> 2;
-  const int Bx = R16x + ix4 * 4, By = R16y + iy4 * 4;
-
-  for (uint32_t base = t0; base < t1; base += nthreads) {
-    uint32_t nb = min(static_cast<uint32_t>(nthreads), t1 - base);
-    if (tid < static_cast<int>(nb)) {
-      prim_lds& L = lds[tid];
-      uint32_t rec = vals[base + tid];
-      uint32_t id = rec >> 1;
-      const float4* tr = tri_rec + tri_slot(P, id) * 5;
-      float e[9], bb[4];
-      read_tri_rec(tr, e, bb);
-      float4 d3 = tr[3], d4 = tr[4];
-      for (int k = 0; k < 9; ++k) L.e[k] = e[k];
-      const float tvx = static_cast<float>(t64x), tvy = static_cast<float>(t64y);
-      L.bb[0] = bb[0] - tvx;
-      L.bb[1] = bb[1] - tvx;
-      L.bb[2] = bb[2] - tvy;
-      L.bb[3] = bb[3] - tvy;
-      // per-stage constants (rasterize_triangle, rasterizer.cpp:662-675, 704-710)
-      for (int k = 0; k < 3; ++k) {
-        float ex = e[k * 3], ey = e[k * 3 + 1], ez = e[k * 3 + 2];
-        bool mx = ex > 0, my = ey > 0;
-        float sx = TILE * ex, sy = TILE * ey;
-        float ra = -fabsf(sx) - fabsf(sy);
-        float part = static_cast<float>(mx * TILE) * ex + static_cast<float>(my * TILE) * ey;
-        sx *= 0.25f; sy *= 0.25f; ra *= 0.25f; part *= 0.25f;
-        float ev = ez - part;
-        L.s1x[k] = sx; L.s1y[k] = sy; L.ra1[k] = ra;
-        L.ev1[k] = ev - ((tvx * ex) + (tvy * ey));
-        sx *= 0.25f; sy *= 0.25f; ra *= 0.25f; part *= 0.25f;
-        L.s2x[k] = sx; L.s2y[k] = sy; L.ra2[k] = ra;
-        L.ev2[k] = ez - part;
-      }
-      L.zx = d3.y;
-      L.zy = d3.z;
-      L.z0 = d3.w;
-      L.dzx = d4.x;
-      L.dzy = d4.y;
-      L.front = d4.z != 0.0f;
-      for (int s = 0; s < 4; ++s) L.aa[s] = (S > 1 && s < S) ? (P.sp[s][0] - 0.5f) * d4.x + (P.sp[s][1] - 0.5f) * d4.y : 0.0f;
-      L.idf = rec;
-      // stage-16 decision for each 16x16 region of the GPU tile (subdivide_tile, SSE order)
-      uint32_t bits = 0;
-      int nreg = G / 16;
-      for (int ry = 0; ry < nreg; ++ry)
-        for (int rx = 0; rx < nreg; ++rx) {
-          int jx = ((gx * G - t64x) >> 4) + rx, jy = ((gy * G - t64y) >> 4) + ry;
-          bool rej = false, nacc = false;
-          for (int k = 0; k < 3; ++k) {
-            float r = (L.s1x[k] * static_cast<float>(jx)) + (L.s1y[k] * static_cast<float>(jy));
-            float a = r + L.ra1[k];
-            rej |= r < L.ev1[k];
-            nacc |= a < L.ev1[k];
-          }
-          int mxr = jx * 16, myr = jy * 16;
-          rej |= L.bb[0] >= static_cast<float>(mxr + 16);
-          rej |= L.bb[1] < static_cast<float>(mxr);
-          rej |= L.bb[2] >= static_cast<float>(myr + 16);
-          rej |= L.bb[3] < static_cast<float>(myr);
-          int k = ry * nreg + rx;
-          if (rej) bits |= 1u << k;
-          else if (!nacc) bits |= 1u << (16 + k);
-        }
-      L.r16 = bits;
-    }
-    __syncthreads();
-    if (any_in) {
-      for (uint32_t j = 0; j < nb; ++j) {
-        const prim_lds& L = lds[j];
-        uint32_t cov[4];
-        if (L.idf & 1) {
-          cov[0] = cov[1] = cov[2] = cov[3] = full_px;
-        } else {
-          uint32_t bits = L.r16;
-          if (bits & (1u << r16k)) continue;
-          if (bits & (1u << (16 + r16k))) {
-            cov[0] = cov[1] = cov[2] = cov[3] = full_px;
-          } else {
-            // stage 4: child (ix4, iy4) of the 16x16 region at (R16x, R16y)
-            bool rej = false, nacc = false;
-            const float lf = static_cast<float>(R16x), tf = static_cast<float>(R16y);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              float ev = L.ev2[k] - ((lf * L.e[k * 3]) + (tf * L.e[k * 3 + 1]));
-              float r = (L.s2x[k] * static_cast<float>(ix4)) + (L.s2y[k] * static_cast<float>(iy4));
-              float a = r + L.ra2[k];
-              rej |= r < ev;
-              nacc |= a < ev;
-            }
-            int mxr = ix16 * 16 + ix4 * 4, myr = iy16 * 16 + iy4 * 4;
-            rej |= L.bb[0] >= static_cast<float>(mxr + 4);
-            rej |= L.bb[1] < static_cast<float>(mxr);
-            rej |= L.bb[2] >= static_cast<float>(myr + 4);
-            rej |= L.bb[3] < static_cast<float>(myr);
-            if (rej) continue;
-            if (!nacc) {
-              cov[0] = cov[1] = cov[2] = cov[3] = full_px;
-            } else {
-              // pixel level: draw_partial_tile on the 4x4 block at (Bx, By)
-              float evp[3];
-              const float bl = static_cast<float>(Bx), bt = static_cast<float>(By);
-#pragma unroll
-              for (int k = 0; k < 3; ++k) evp[k] = L.e[k * 3 + 2] - ((bl * L.e[k * 3]) + (bt * L.e[k * 3 + 1]));
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                uint32_t m = 0;
-                const float fx = static_cast<float>(px0 + (i & 1) - Bx), fy = static_cast<float>(py0 + (i >> 1) - By);
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                  float mx = P.sp[s][0] + fx, my = P.sp[s][1] + fy;
-                  bool r = false;
-#pragma unroll
-                  for (int k = 0; k < 3; ++k) r |= ((mx * L.e[k * 3]) + (my * L.e[k * 3 + 1])) < evp[k];
-                  if (!r) m |= 1u << s;
-                }
-                cov[i] = m;
-              }
-            }
-          }
-        }
-        // pixels outside the render target are never drawn
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (!pin[i]) cov[i] = 0;
-        if ((cov[0] | cov[1] | cov[2] | cov[3]) == 0) continue;
-        // depth of the quad's pixels (step_2d_unproj_pos_quad, z lane)
-        const float dx = (0.5f + static_cast<float>(px0)) - L.zx;
-        const float dy = (0.5f + static_cast<float>(py0)) - L.zy;
-        float z[4];
-        z[0] = L.z0 + ((L.dzx * dx) + (L.dzy * dy));
-        z[1] = z[0] + L.dzx;
-        z[2] = z[0] + L.dzy;
-        z[3] = z[1] + L.dzy;
-        const uint32_t id = L.idf >> 1;
-        if (P.early_z) {
-          // early_z_test (framebuffer.cpp:522-614): depth written at test time
-          uint32_t tested[4] = {0, 0, 0, 0};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-              if (!(cov[i] & (1u << s))) continue;
-              float nd = (S > 1) ? (L.aa[s] + z[i]) : z[i];
-              float od = P.read_depth ? depth[i][s] : 0.0f;
-              bool pass = P.depth_enable ? cmpf(P.depth_func, nd, od) : true;
-              if (pass) {
-                if (P.write_depth) depth[i][s] = nd;
-                tested[i] |= 1u << s;
-              }
-            }
-          if ((tested[0] | tested[1] | tested[2] | tested[3]) == 0) continue;
-          ps_inv += 4;
-          be_pix += 4;
-          if constexpr (VIS) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-              for (int s = 0; s < S; ++s)
-                if (tested[i] & (1u << s)) winner[i][s] = id;
-          } else {
-            shade_store<NA, S, SASL>(P, SM, tri_attr, id, px0, py0,
-                                     tested[0] | (tested[1] << 4) | (tested[2] << 8) | (tested[3] << 12));
-          }
-        } else if constexpr (!VIS) {
-          // late depth/stencil (render_sample, framebuffer.cpp:445-479); writes only when both pass.
-          // The tests of a sample depend only on that sample's depth/stencil, not on the colour, so
-          // they run first and the pixel shader (side-effect free) runs only when some sample passes.
-          ps_inv += 4;
-          be_pix += 4;
-          const int face = L.front ? 0 : 1;
-          uint32_t passed[4] = {0, 0, 0, 0};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-              if (!(cov[i] & (1u << s))) continue;
-              float nd = (S > 1) ? (z[i] + L.aa[s]) : z[i];
-              float od = P.read_depth ? depth[i][s] : 0.0f;
-              uint32_t os = P.stencil_enable ? (stencil[i][s] & P.read_mask) : 0u;
-              bool dp = has_ds ? (P.depth_enable ? cmpf(P.depth_func, nd, od) : true) : true;
-              bool sp = P.stencil_enable ? cmpu(P.st_func[face], P.stencil_ref, os) : true;
-              if (dp && sp) passed[i] |= 1u << s;
-            }
-          if ((passed[0] | passed[1] | passed[2] | passed[3]) == 0) continue;
-          shade_store<NA, S, SASL>(P, SM, tri_attr, id, px0, py0,
-                                   passed[0] | (passed[1] << 4) | (passed[2] << 8) | (passed[3] << 12));
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-              if (!(passed[i] & (1u << s))) continue;
-              float nd = (S > 1) ? (z[i] + L.aa[s]) : z[i];
-              uint32_t os = P.stencil_enable ? (stencil[i][s] & P.read_mask) : 0u;
-              uint32_t ns = P.stencil_enable ? stencil_op(P.st_pass_op[face], P.stencil_ref, os) : 0u;
-              if (P.write_depth) depth[i][s] = nd;
-              if (P.stencil_enable) stencil[i][s] = ns & P.write_mask;
-            }
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  if constexpr (VIS) {
-    // winners for the shading pass, laid out like the colour target's samples
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (pin[i]) {
-        size_t base = (static_cast<size_t>(py0 + (i >> 1)) * tw + (px0 + (i & 1))) * S;
-#pragma unroll
-        for (int s = 0; s < S; ++s) vis[base + s] = winner[i][s];
-      }
-    if (has_ds && P.write_depth) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (pin[i])
-#pragma unroll
-          for (int s = 0; s < S; ++s)
-            *reinterpret_cast<float*>(sample_addr(P.ds, px0 + (i & 1), py0 + (i >> 1), s)) = depth[i][s];
-    }
-  } else if (has_ds && (P.write_depth || P.stencil_enable)) {
-    // write back depth/stencil
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (pin[i])
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-          *reinterpret_cast<float2*>(sample_addr(P.ds, px0 + (i & 1), py0 + (i >> 1), s)) =
-              make_float2(depth[i][s], __uint_as_float(stencil[i][s]));
-  }
-  // ps_invocations and backend_input_pixels advance together (+4 per shaded quad: the sample shaders
-  // never discard), so one partial carries both
-  (void)be_pix;
-  if (P.count_stats) block_partial(partial, ps_inv);  // uniform over the launch
-}
-
-// ---------------------------------------------------------------- order-independent visibility
-// For an opaque early-Z draw with blending off, the reference's sequential early-Z test (depth written
-// at test time, framebuffer.cpp:522-614) leaves in every sample the result of a running reduction:
-//   LESS/GREATER (+write): the first triangle reaching the extreme depth wins;
-//   LESS_EQUAL/GREATER_EQUAL (+write): the last triangle reaching the extreme depth wins;
-//   ALWAYS, depth off, EQUAL, or any function without depth write: among the triangles that pass
-//   against the initial depth, the last one wins.
-// Each of these is a minimum over a 64-bit key (ordered depth, primitive order), so lanes can
-// rasterise different triangles of a tile at once and merge with LDS atomic-min.
-enum { VIS_LESS = 0, VIS_LEQUAL = 1, VIS_GREATER = 2, VIS_GEQUAL = 3, VIS_LATEST = 4, VIS_NONE = 5 };
-
-__device__ __forceinline__ uint32_t ord_depth(float z) {
-  uint32_t u = __float_as_uint(z + 0.0f);  // -0 compares equal to +0
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
-__device__ __forceinline__ unsigned long long initial_key(int mode, float d0) {
-  if (mode == VIS_LATEST || mode == VIS_NONE) return 0xFFFFFFFFull;
-  if (d0 != d0) return 0ull;  // a NaN depth lets nothing pass
-  uint32_t zk = ord_depth(d0);
-  if (mode == VIS_GREATER || mode == VIS_GEQUAL) zk = ~zk;
-  uint32_t lo = (mode == VIS_LESS || mode == VIS_GREATER) ? 0u : 0xFFFFFFFFu;
-  return (static_cast<unsigned long long>(zk) << 32) | lo;
-}
-
-__device__ __forceinline__ uint32_t key_winner(int mode, unsigned long long k) {
-  uint32_t lo = static_cast<uint32_t>(k);
-  if (mode == VIS_LESS || mode == VIS_GREATER) return lo == 0u ? NO_WINNER : lo - 1u;
-  return lo == 0xFFFFFFFFu ? NO_WINNER : 0xFFFFFFFEu - lo;
-}
-
-// Depth the reference's early-Z test wrote for winner w of sample smp of pixel (px, py).
-template <int S>
-__device__ __forceinline__ float winner_depth(const draw_params& P, int mode, unsigned long long key, uint32_t w,
-                                              const float4* __restrict__ tri_rec, int px, int py, int smp) {
-  if (mode != VIS_LATEST) {
-    // depth modes carry the winning sample depth in the key; only +-0 is ambiguous there
-    uint32_t zk = static_cast<uint32_t>(key >> 32);
-    if (mode == VIS_GREATER || mode == VIS_GEQUAL) zk = ~zk;
-    const uint32_t u = (zk & 0x80000000u) ? (zk & 0x7FFFFFFFu) : ~zk;
-    if (u != 0u) return __uint_as_float(u);
-  }
-  // the winner's depth at this sample, as its quad computed it
-  const float4* tr = tri_rec + tri_slot(P, w) * 5;
-  const float4 d3 = tr[3], d4 = tr[4];
-  const int qx0 = px & ~1, qy0 = py & ~1;
-  const float dx = (0.5f + static_cast<float>(qx0)) - d3.y;
-  const float dy = (0.5f + static_cast<float>(qy0)) - d3.z;
-  float z00 = d3.w + ((d4.x * dx) + (d4.y * dy));
-  float zp;
-  if ((px & 1) == 0 && (py & 1) == 0) zp = z00;
-  else if ((py & 1) == 0) zp = z00 + d4.x;
-  else if ((px & 1) == 0) zp = z00 + d4.y;
-  else zp = (z00 + d4.x) + d4.y;
-  float nd = zp;
-  if (S > 1) nd = ((P.sp[smp][0] - 0.5f) * d4.x + (P.sp[smp][1] - 0.5f) * d4.y) + zp;
-  return nd;
-}
-
-// cmpf as a truth table over the comparison's outcome: bit 0 less, 1 equal, 2 greater, 3 unordered.
-__device__ __forceinline__ uint32_t cmpf_table(int f) {
-  // nibble f: never, less, equal, less_equal, greater, not_equal, greater_equal, always
-  return (f >= 0 && f < 8) ? (0xF6D43210u >> (4 * f)) & 0xFu : 0xFu;
-}
-__device__ __forceinline__ bool cmpf_by_table(uint32_t table, float a, float b) {
-  const uint32_t o = (a < b) ? 0u : (a == b) ? 1u : (a > b) ? 2u : 3u;
-  return ((table >> o) & 1u) != 0u;
-}
-
-// Phase 1c of vis_body over the chunk's work list: items [0, np) are (record, 4x4 block) pairs the
-// rasteriser tests sample by sample (draw_partial_tile, rasterizer.cpp:298-439), items [np, nt)
-// blocks it accepts whole (draw_full_tile, :285-296).  A partial item tests, pixel by pixel, only
-// the pixels a conservative bound leaves (see below), each sample with the reference's expression
-// ((sx + fx) * ex) + ((sy + fy) * ey) < e_value, and every covered sample's key goes to the LDS
-// atomic-min.  Depth per sample is the quad chain of
-// step_2d_unproj_pos_quad (p00 = v0 + (ddx*dx + ddy*dy), +ddx to the right, +ddy below) plus the
-// sample offset term of rasterize_triangle (rasterizer.cpp:678-687).
-// Keys: DEPTH (the LESS, LEQUAL, GREATER, GEQUAL modes with depth writes) = the sample depth's
-// order-preserving bits (complemented when the greater depth wins) over the record's order term,
-// and a NaN depth passes nothing; otherwise (VIS_LATEST) the sample passes against the target's
-// initial depth (always without a depth test) and the key is the order term alone.  The per-sample
-// predicates are combined with bitwise operators so that each sample costs one masked atomic and
-// no branch.
-template <int S, int GT, bool DEPTH>
-__device__ __forceinline__ void vis_items(const draw_params& P, int mode, const float4* __restrict__ recs,
-                                          const uint16_t* __restrict__ work, uint32_t np, uint32_t nt,
-                                          unsigned long long* __restrict__ keys, const float* __restrict__ d0s,
-                                          int ox, int oy, int tw, int th, int tid, int NT) {
-  constexpr int NBS = GT / 4;
-  const uint32_t flip = (mode == VIS_GREATER || mode == VIS_GEQUAL) ? 0xFFFFFFFFu : 0u;
-  const bool later_wins = mode == VIS_LEQUAL || mode == VIS_GEQUAL || mode == VIS_LATEST;
-  const uint32_t table = P.depth_enable ? cmpf_table(P.depth_func) : 0xFu;
-  const bool read_depth = P.read_depth != 0;
-  // extreme sample positions inside a pixel
-  float spx_lo = P.sp[0][0], spx_hi = P.sp[0][0], spy_lo = P.sp[0][1], spy_hi = P.sp[0][1];
-#pragma unroll
-  for (int s = 1; s < S; ++s) {
-    spx_lo = fminf(spx_lo, P.sp[s][0]);
-    spx_hi = fmaxf(spx_hi, P.sp[s][0]);
-    spy_lo = fminf(spy_lo, P.sp[s][1]);
-    spy_hi = fmaxf(spy_hi, P.sp[s][1]);
-  }
-  for (uint32_t wi = tid; wi < nt; wi += NT) {
-    const uint32_t wk = work[wi];
-    const int j = static_cast<int>(wk >> 7), b = static_cast<int>((wk >> 1) & 63u);
-    const float4 r0 = recs[j * 4 + 0], r1 = recs[j * 4 + 1], r2 = recs[j * 4 + 2], r3 = recs[j * 4 + 3];
-    const float e[9] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x};
-    const float z0 = r2.y, zx = r2.z, zy = r2.w, dzx = r3.x, dzy = r3.y;
-    const uint32_t id = __float_as_uint(r3.z);
-    const uint32_t lo = later_wins ? 0xFFFFFFFEu - id : id + 1u;
-    const bool full = wi >= np;
-    float aa[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) aa[s] = (S > 1) ? (P.sp[s][0] - 0.5f) * dzx + (P.sp[s][1] - 0.5f) * dzy : 0.0f;
-    const int bc = b % NBS, br = b / NBS;
-    const int Bx = ox + bc * 4, By = oy + br * 4;
-    const int lbase = (br * 4 * GT + bc * 4) * S;  // the block's first sample in `keys`
-    const int bw = min(4, tw - Bx), bh = min(4, th - By);  // columns and rows inside the target
-    // depth at the top-left pixel of each 2x2 quad of the block
-    float zq[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float dx = (0.5f + static_cast<float>(Bx + (q & 1) * 2)) - zx;
-      const float dy = (0.5f + static_cast<float>(By + (q >> 1) * 2)) - zy;
-      zq[q] = z0 + ((dzx * dx) + (dzy * dy));
-    }
-    float evp[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      evp[k] = e[k * 3 + 2] - ((static_cast<float>(Bx) * e[k * 3]) + (static_cast<float>(By) * e[k * 3 + 1]));
-    if (!full) {
-      // Pixels that may hold a covered sample.  Float rounding is monotonic, so an edge's value at
-      // any sample of a pixel is at most its value at the pixel's extreme sample column and row
-      // for that edge's signs, computed with the same operations; a pixel whose extreme value
-      // fails an edge has no sample that passes it.  Only the remaining pixels are tested sample
-      // by sample.
-      uint32_t M = 0;
-      {
-        float cx[3][4], cy[3][4];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const float sx = e[k * 3] >= 0.0f ? spx_hi : spx_lo, sy = e[k * 3 + 1] >= 0.0f ? spy_hi : spy_lo;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            cx[k][c] = (sx + static_cast<float>(c)) * e[k * 3];
-            cy[k][c] = (sy + static_cast<float>(c)) * e[k * 3 + 1];
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const bool maybe = !((cx[0][c] + cy[0][r]) < evp[0]) & !((cx[1][c] + cy[1][r]) < evp[1]) &
-                               !((cx[2][c] + cy[2][r]) < evp[2]) & (c < bw) & (r < bh);
-            if (maybe) M |= 1u << (r * 4 + c);
-          }
-      }
-      while (M) {
-        const int px = __builtin_ctz(M);
-        M &= M - 1u;
-        const int r = px >> 2, c = px & 3;
-        const int q = ((r >> 1) << 1) | (c >> 1);
-        float z = (q & 2) ? ((q & 1) ? zq[3] : zq[2]) : ((q & 1) ? zq[1] : zq[0]);
-        z = (c & 1) ? z + dzx : z;
-        z = (r & 1) ? z + dzy : z;
-        const float fx = static_cast<float>(c), fy = static_cast<float>(r);
-        const int lp = lbase + (r * GT + c) * S;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const float mx = P.sp[s][0] + fx, my = P.sp[s][1] + fy;
-          const bool covered = !(((mx * e[0]) + (my * e[1])) < evp[0]) & !(((mx * e[3]) + (my * e[4])) < evp[1]) &
-                               !(((mx * e[6]) + (my * e[7])) < evp[2]);
-          const float nd = (S > 1) ? (aa[s] + z) : z;
-          unsigned long long k;
-          bool pass;
-          if (DEPTH) {
-            const uint32_t u = __float_as_uint(nd + 0.0f);  // -0 orders as +0
-            const uint32_t ord = u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
-            k = (static_cast<unsigned long long>(ord ^ flip) << 32) | lo;
-            pass = nd == nd;
-          } else {
-            k = lo;
-            pass = cmpf_by_table(table, nd, read_depth ? d0s[lp + s] : 0.0f);
-          }
-          if (covered & pass) atomicMin(&keys[lp + s], k);
-        }
-      }
-      continue;
-    }
-    // a block the rasteriser accepts whole: every sample inside the target
-    float zp[16];  // pixel depths (row r, column c at [r * 4 + c]) by the quad chain
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int p0 = (q >> 1) * 8 + (q & 1) * 2;
-      zp[p0] = zq[q];
-      zp[p0 + 1] = zq[q] + dzx;
-      zp[p0 + 4] = zq[q] + dzy;
-      zp[p0 + 5] = zp[p0 + 1] + dzy;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const float nd = (S > 1) ? (aa[s] + zp[r * 4 + c]) : zp[r * 4 + c];
-          const int li = lbase + (r * GT + c) * S + s;
-          unsigned long long k;
-          bool pass;
-          if (DEPTH) {
-            const uint32_t u = __float_as_uint(nd + 0.0f);
-            const uint32_t ord = u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
-            k = (static_cast<unsigned long long>(ord ^ flip) << 32) | lo;
-            pass = nd == nd;
-          } else {
-            k = lo;
-            pass = cmpf_by_table(table, nd, read_depth ? d0s[li] : 0.0f);
-          }
-          if (pass & (c < bw) & (r < bh)) atomicMin(&keys[li], k);
-        }
-  }
-}
-
-// One 16x16 GPU tile per workgroup, in three phases:
-//  1. one triangle per lane: coverage with the reference's decision chain, LDS atomic-min of the
-//     (ordered depth, primitive order) key of every covered sample;
-//  2. one pixel per lane: winners -> depth/stencil target, and one shading item per distinct winner
-//     (pixel, winner, sample mask) appended to an LDS list;
-//  3. (SHADE) one item per lane: the winner's quad interpolants at the pixel's quad (the values the
-//     reference's last passing draw_quad/draw_full_quad computed), the pixel shader for that pixel,
-//     and the colour stored to the item's samples.  Items are spread evenly over the lanes however
-//     many triangles share a pixel.
-#ifndef SRX_VIS_THREADS
-#define SRX_VIS_THREADS 256
-#endif
-// LDS shared by phase 1 (a chunk of NT records + their (record, block) work list) and phase 3
-// (shading items), for GT x GT GPU tiles
-__host__ __device__ constexpr int vis_union_bytes(int nt, int s, bool shade, int gt = 16) {
-  return (nt * 64 + nt * (gt / 4) * (gt / 4) * 2) > (shade ? gt * gt * s * 8 : 0) ? (nt * 64 + nt * (gt / 4) * (gt / 4) * 2)
-                                                                                   : gt * gt * s * 8;
-}
-// Static LDS of vis_body besides the union (keys, initial depths).
-__host__ __device__ constexpr int vis_static_bytes(int s, int gt) { return gt * gt * s * 12 + 256; }
-// NTC > 0: NTC lanes per workgroup, static LDS.  NTC == 0: blockDim.x lanes (64, 128 or 256) with
-// the phase-1/3 union in dynamic LDS of vis_union_bytes(blockDim.x, S, SHADE, GT) bytes.
-// GT: GPU tile side, 8, 16 or 32 pixels: a quarter of a 16x16 stage-16 region, one region, or 2x2
-// regions of the reference's 64x64 tile; the 4x4 blocks are the reference's stage-4 blocks either way.
-template <int NA, int S, bool SHADE, int NTC, int GT>
-__device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pass, const uint32_t* __restrict__ order,
-                                         const uint4* __restrict__ entries, const uint4* __restrict__ merges,
-                                         const uint32_t* __restrict__ counts, unsigned long long* __restrict__ partial,
-                                         const uint32_t* __restrict__ vals, const uint32_t* __restrict__ tstart,
-                                         const uint32_t* __restrict__ tend, const float4* __restrict__ tri_rec,
-                                         const float4* __restrict__ tri_attr, const ps_samplers* __restrict__ SM,
-                                         uint32_t bx, uint32_t* __restrict__ wout = nullptr) {
-  static_assert(GT == 8 || GT == 16 || GT == 32, "GPU tile side");
-  constexpr int PX = GT * GT;       // pixels per GPU tile
-  constexpr int NBS = GT / 4;       // 4x4 blocks per side
-  constexpr int RPS = GT > 16 ? GT / 16 : 1;  // stage-16 regions per side
-  using bmask_t = typename std::conditional<(GT > 16), unsigned long long, uint32_t>::type;
-  const int NT = NTC > 0 ? NTC : static_cast<int>(blockDim.x);
-  constexpr int UNION_BYTES = NTC > 0 ? vis_union_bytes(NTC, S, SHADE, GT) : 16;
-  __shared__ unsigned long long keys[PX * S];
-  __shared__ float d0s[PX * S];
-  __shared__ __align__(16) unsigned char lds_static[UNION_BYTES];
-  extern __shared__ __align__(16) unsigned char lds_dynamic[];
-  unsigned char* const lds_union = NTC > 0 ? lds_static : lds_dynamic;
-  __shared__ uint32_t wsum[4];
-  __shared__ uint32_t hiz[NBS * NBS];
-  __shared__ uint32_t nitems;
-  float4* recs = reinterpret_cast<float4*>(lds_union);                           // [NT][4]
-  uint16_t* work = reinterpret_cast<uint16_t*>(lds_union + NT * 64);             // [NT * NBS^2]
-  uint2* items = reinterpret_cast<uint2*>(lds_union);                            // [PX * S]
-  // pass 0: one tile, or one part of a split tile; pass 1: merge and finish a split tile
-  int gtile;
-  uint32_t part = 0, parts = 1, slot = 0;
-  if (entries == nullptr) {  // whole tiles in `order`
-    gtile = static_cast<int>(order[bx]);
-  } else if (pass == 0) {
-    if (bx >= counts[0]) return;
-    const uint4 en = entries[bx];
-    gtile = static_cast<int>(en.x);
-    part = en.y;
-    parts = en.z;
-    slot = en.w + en.y;
-  } else {
-    if (bx >= counts[1]) return;
-    const uint4 mg = merges[bx];
-    gtile = static_cast<int>(mg.x);
-    parts = mg.y;
-    slot = mg.z;
-  }
-  const int gx = gtile % P.gtiles_x, gy = gtile / P.gtiles_x;
-  const int ox = gx * GT, oy = gy * GT;
-  const int t64x = ox & ~(TILE - 1), t64y = oy & ~(TILE - 1);
-  const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
-  const int tid = threadIdx.x;
-  const bool has_ds = P.ds.data != nullptr;
-  if (tid == 0) nitems = 0;
-  if (pass == 1) {
-    // the parts' keys, each started from the target's depth: their minimum is the tile's result
-    const unsigned long long* src = partial + static_cast<size_t>(slot) * (PX * S);
-    for (int i = tid; i < PX * S; i += NT) {
-      unsigned long long k = src[i];
-      for (uint32_t q = 1; q < parts; ++q) {
-        const unsigned long long kq = src[static_cast<size_t>(q) * (PX * S) + i];
-        k = kq < k ? kq : k;
-      }
-      keys[i] = k;
-    }
-  } else {
-    for (int i = tid; i < PX * S; i += NT) {
-      int px = ox + ((i / S) % GT), py = oy + ((i / S) / GT), smp = i % S;
-      float d0 = 0.0f;
-      bool blocked = false;
-      if (has_ds && px < tw && py < th) {
-        const float2 ds = P.clear_ds ? make_float2(P.clear_depth, __uint_as_float(P.clear_stencil))
-                                     : *reinterpret_cast<const float2*>(sample_addr(P.ds, px, py, smp));
-        d0 = ds.x;
-        if (P.vis_stencil) {
-          // framebuffer.cpp:445-479 (both faces share the function here); a failing sample takes
-          // no colour and no depth
-          const uint32_t os = __float_as_uint(ds.y) & P.read_mask;
-          blocked = !cmpu(P.st_func[1], P.stencil_ref, os);
-        }
-      }
-      d0s[i] = d0;
-      // a blocked sample's key is below every candidate's and decodes as no winner
-      keys[i] = blocked ? ((mode == VIS_LEQUAL || mode == VIS_GEQUAL) ? 0xFFFFFFFFull : 0ull) : initial_key(mode, d0);
-    }
-  }
-  // this workgroup's records: the whole tile, or one part of it (none when merging)
-  const uint32_t tr0 = tstart[gtile], tr1 = tend[gtile];
-  const uint32_t t0 = pass == 1 ? tr1 : min(tr1, tr0 + part * VIS_PART);
-  const uint32_t t1 = (pass == 1 || entries == nullptr) ? tr1 : min(tr1, t0 + VIS_PART);
-  const int jx0 = (ox - t64x) >> 4, jy0 = (oy - t64y) >> 4;  // first stage-16 region of the tile
-  // an 8x8 tile covers blocks [qx, qx+2) x [qy, qy+2) of its region; larger tiles whole regions
-  const int qx = GT < 16 ? ((ox - t64x) & 15) >> 2 : 0, qy = GT < 16 ? ((oy - t64y) & 15) >> 2 : 0;
-  constexpr int CW = GT < 16 ? GT / 4 : 4;  // block columns (rows) of a region inside the tile
-  const float tvx = static_cast<float>(t64x), tvy = static_cast<float>(t64y);
-  // Depth culling from the second chunk on: hiz[b] is the largest key depth word of 4x4 block b's
-  // samples after the previous chunks.  Keys only decrease, so a record whose smallest possible
-  // depth word over the block exceeds it cannot win any sample there and skips the block.
-  const bool depth_keys = mode == VIS_LESS || mode == VIS_LEQUAL || mode == VIS_GREATER || mode == VIS_GEQUAL;
-  const bool far_is_min = mode == VIS_GREATER || mode == VIS_GEQUAL;
-  for (uint32_t c0 = t0; c0 < t1; c0 += NT) {
-    __syncthreads();  // the previous chunk's work list is consumed (and the keys are initialised)
-    const bool hiz_on = depth_keys && c0 > t0;
-    if (hiz_on) {
-      // 16 consecutive lanes take one block's 16 pixels
-      for (int u = tid; u < PX; u += NT) {
-        const int b = u >> 4, q = u & 15;
-        const int pl = ((b / NBS) * 4 + (q >> 2)) * GT + (b % NBS) * 4 + (q & 3);
-        uint32_t m = 0;
-#pragma unroll
-        for (int smp = 0; smp < S; ++smp) m = max(m, static_cast<uint32_t>(keys[pl * S + smp] >> 32));
-        m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 1, 64)));
-        m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 2, 64)));
-        m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 4, 64)));
-        m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 8, 64)));
-        if (q == 0) hiz[b] = m;
-      }
-      __syncthreads();
-    }
-    // phase 1a: one record per lane -> the 4x4 blocks of this GPU tile it reaches (full or partial)
-    bmask_t bm = 0, fm = 0;
-    const uint32_t ri = c0 + tid;
-    if (ri < t1) {
-      const uint32_t rec = vals[ri];
-      const uint32_t id = rec >> 1;
-      const float4* tr = tri_rec + tri_slot(P, id) * 5;
-      float e[9], bb[4];
-      read_tri_rec(tr, e, bb);
-      const float4 d3 = tr[3], d4 = tr[4];
-      const float bx0 = bb[0] - tvx, bx1 = bb[1] - tvx, by0 = bb[2] - tvy, by1 = bb[3] - tvy;
-      // per-stage constants (rasterize_triangle, rasterizer.cpp:662-675, 704-710)
-      float s1x[3], s1y[3], ra1[3], ev1[3], s2x[3], s2y[3], ra2[3], ev2[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        float ex = e[k * 3], ey = e[k * 3 + 1], ez = e[k * 3 + 2];
-        bool mx = ex > 0, my = ey > 0;
-        float sx = TILE * ex, sy = TILE * ey;
-        float ra = -fabsf(sx) - fabsf(sy);
-        float part = static_cast<float>(mx * TILE) * ex + static_cast<float>(my * TILE) * ey;
-        sx *= 0.25f; sy *= 0.25f; ra *= 0.25f; part *= 0.25f;
-        s1x[k] = sx; s1y[k] = sy; ra1[k] = ra;
-        ev1[k] = (ez - part) - ((tvx * ex) + (tvy * ey));
-        sx *= 0.25f; sy *= 0.25f; ra *= 0.25f; part *= 0.25f;
-        s2x[k] = sx; s2y[k] = sy; ra2[k] = ra;
-        ev2[k] = ez - part;
-      }
-      const bool rec_full = (rec & 1) != 0;  // the record covers its whole 64x64 tile
-#pragma unroll
-      for (int rr = 0; rr < RPS * RPS; ++rr) {
-        const int jx = jx0 + rr % RPS, jy = jy0 + rr / RPS;
-        bool region_full = rec_full;
-        bool keep = true;
-        if (!region_full) {
-          // stage 16 (subdivide_tile on the 64x64 tile)
-          bool rej = false, nacc = false;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            float r = (s1x[k] * static_cast<float>(jx)) + (s1y[k] * static_cast<float>(jy));
-            float a = r + ra1[k];
-            rej |= r < ev1[k];
-            nacc |= a < ev1[k];
-          }
-          rej |= bx0 >= static_cast<float>(jx * 16 + 16);
-          rej |= bx1 < static_cast<float>(jx * 16);
-          rej |= by0 >= static_cast<float>(jy * 16 + 16);
-          rej |= by1 < static_cast<float>(jy * 16);
-          keep = !rej;
-          region_full = !nacc;
-        }
-        if (!keep) continue;
-        const int rox = t64x + jx * 16, roy = t64y + jy * 16;  // the region's origin
-        float ev2q[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          ev2q[k] = ev2[k] - ((static_cast<float>(rox) * e[k * 3]) + (static_cast<float>(roy) * e[k * 3 + 1]));
-        // candidate 4x4 blocks of the region inside this tile: all of them for an accepted region,
-        // else those the stage-4 bounding-box test keeps (bx0 < mxr + 4 and bx1 >= mxr, the same
-        // comparisons on the same floats)
-        uint32_t cols = 0, rows = 0;
-#pragma unroll
-        for (int cc = 0; cc < CW; ++cc) {
-          const int cx = qx + cc, cy = qy + cc;
-          const int mxr = jx * 16 + cx * 4, myr = jy * 16 + cy * 4;
-          if (region_full || !(bx0 >= static_cast<float>(mxr + 4) || bx1 < static_cast<float>(mxr))) cols |= 0x1111u << cx;
-          if (region_full || !(by0 >= static_cast<float>(myr + 4) || by1 < static_cast<float>(myr))) rows |= 0xFu << (cy * 4);
-          if (rox + cx * 4 >= tw) cols &= ~(0x1111u << cx);  // blocks outside the target
-          if (roy + cy * 4 >= th) rows &= ~(0xFu << (cy * 4));
-        }
-        uint32_t blocks = cols & rows;
-        while (blocks) {
-          const int b16 = __builtin_ctz(blocks);
-          blocks &= blocks - 1;
-          const int ix4 = b16 & 3, iy4 = b16 >> 2;
-          bool block_full = region_full;
-          if (!block_full) {
-            // stage 4 (subdivide_tile on the 16x16 region); the bounding-box half was applied above
-            bool rej = false, nacc = false;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              float r = (s2x[k] * static_cast<float>(ix4)) + (s2y[k] * static_cast<float>(iy4));
-              float a = r + ra2[k];
-              rej |= r < ev2q[k];
-              nacc |= a < ev2q[k];
-            }
-            if (rej) continue;
-            block_full = !nacc;
-          }
-          // the block's index in this tile
-          const int b = ((rr / RPS) * 4 + iy4 - qy) * NBS + (rr % RPS) * 4 + ix4 - qx;
-          if (hiz_on) {
-            // the depth plane's extreme over the block's sample positions [Bx, Bx+4) x [By, By+4),
-            // widened by far more than the rounding of the per-sample evaluation
-            const float z0 = d3.w, zx = d3.y, zy = d3.z, dzx = d4.x, dzy = d4.y;
-            const float ax = static_cast<float>(rox + ix4 * 4) - zx, ay = static_cast<float>(roy + iy4 * 4) - zy;
-            const float tx0 = dzx * ax, tx1 = dzx * (ax + 4.0f), ty0 = dzy * ay, ty1 = dzy * (ay + 4.0f);
-            const float margin = (fabsf(z0) + fmaxf(fabsf(tx0), fabsf(tx1)) + fmaxf(fabsf(ty0), fabsf(ty1))) * 1.52587890625e-05f;
-            const float zext = far_is_min ? (z0 + fmaxf(tx0, tx1) + fmaxf(ty0, ty1)) + margin
-                                          : (z0 + fminf(tx0, tx1) + fminf(ty0, ty1)) - margin;
-            if (fabsf(zext) < 3.0e38f) {  // finite: planes with inf/nan terms are never culled
-              const uint32_t zk = far_is_min ? ~ord_depth(zext) : ord_depth(zext);
-              if (zk > hiz[b]) continue;
-            }
-          }
-          bm |= static_cast<bmask_t>(1) << b;
-          if (block_full) fm |= static_cast<bmask_t>(1) << b;
-        }
-      }
-      float4* rs = recs + tid * 4;
-      rs[0] = make_float4(e[0], e[1], e[2], e[3]);
-      rs[1] = make_float4(e[4], e[5], e[6], e[7]);
-      rs[2] = make_float4(e[8], d3.w, d3.y, d3.z);          // z0, zx, zy
-      rs[3] = make_float4(d4.x, d4.y, __uint_as_float(id), 0.0f);  // dzx, dzy, id
-    }
-    // phase 1b: work list of (record, block) pairs spread evenly over the lanes: blocks tested
-    // sample by sample first, then blocks accepted whole, so each wave runs one kind
-    const bmask_t pm = bm & ~fm;
-    const uint32_t np = GT > 16 ? static_cast<uint32_t>(__popcll(static_cast<unsigned long long>(pm))) : __popc(static_cast<uint32_t>(pm));
-    const uint32_t nf = GT > 16 ? static_cast<uint32_t>(__popcll(static_cast<unsigned long long>(fm))) : __popc(static_cast<uint32_t>(fm));
-    const uint32_t cnt = np | (nf << 16);  // both sums stay below 2^16 (NT * NBS^2 <= 16384)
-    const uint32_t incl = wave_incl_scan(cnt);
-    if ((tid & 63) == 63) wsum[tid >> 6] = incl;
-    __syncthreads();
-    uint32_t off = incl - cnt, total = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (w >= NT / 64) break;
-      if (w < (tid >> 6)) off += wsum[w];
-      total += wsum[w];
-    }
-    const uint32_t total_p = total & 0xFFFFu, total_all = total_p + (total >> 16);
-    uint32_t off_p = off & 0xFFFFu, off_f = total_p + (off >> 16);
-    bmask_t pr = pm, fr = fm;
-    while (pr) {
-      const uint32_t b = static_cast<uint32_t>(__builtin_ctzll(static_cast<unsigned long long>(pr)));
-      pr &= pr - 1;
-      work[off_p++] = static_cast<uint16_t>((tid << 7) | (b << 1));
-    }
-    while (fr) {
-      const uint32_t b = static_cast<uint32_t>(__builtin_ctzll(static_cast<unsigned long long>(fr)));
-      fr &= fr - 1;
-      work[off_f++] = static_cast<uint16_t>((tid << 7) | (b << 1) | 1u);
-    }
-    __syncthreads();
-    // phase 1c: one (record, block) item per lane: coverage, depth and the key atomic-min
-    if (depth_keys)
-      vis_items<S, GT, true>(P, mode, recs, work, total_p, total_all, keys, d0s, ox, oy, tw, th, tid, NT);
-    else if (mode == VIS_LATEST)
-      vis_items<S, GT, false>(P, mode, recs, work, total_p, total_all, keys, d0s, ox, oy, tw, th, tid, NT);
-  }
-  __syncthreads();
-  if (pass == 0 && parts > 1) {  // one part of a split tile: leave the partial keys for the merge
-    unsigned long long* dst = partial + static_cast<size_t>(slot) * (PX * S);
-    for (int i = tid; i < PX * S; i += NT) dst[i] = keys[i];
-    return;
-  }
-  // phase 2: winners -> depth, shading items
-  for (int p = tid; p < PX; p += NT) {
-    const int px = ox + (p % GT), py = oy + (p / GT);
-    if (px >= tw || py >= th) continue;
-    uint32_t w[S];
-    uint32_t left = 0;
-#pragma unroll
-    for (int smp = 0; smp < S; ++smp) {
-      const unsigned long long key = keys[p * S + smp];
-      w[smp] = key_winner(mode, key);
-      const bool won = w[smp] != NO_WINNER;
-      if (won) left |= 1u << smp;
-      if (has_ds && P.clear_ds) {
-        // a cleared target: every sample is written, the stencil keeps its clear value
-        const float d = (won && P.write_depth) ? winner_depth<S>(P, mode, key, w[smp], tri_rec, px, py, smp) : P.clear_depth;
-        *reinterpret_cast<float2*>(sample_addr(P.ds, px, py, smp)) = make_float2(d, __uint_as_float(P.clear_stencil));
-      } else if (won && has_ds && P.write_depth) {
-        *reinterpret_cast<float*>(sample_addr(P.ds, px, py, smp)) =
-            winner_depth<S>(P, mode, key, w[smp], tri_rec, px, py, smp);
-      }
-      if (SHADE && !won && P.clear_color) {
-        const float4 cc = make_float4(P.clear_rgba[0], P.clear_rgba[1], P.clear_rgba[2], P.clear_rgba[3]);
-        store_texel(P.color.pf, sample_addr(P.color, px, py, smp), cc);
-      }
-      // winners for a separate shading pass (SASL pixel shaders), laid out like the colour samples
-      if (!SHADE && wout) wout[(static_cast<size_t>(py) * tw + px) * S + smp] = w[smp];
-    }
-    if (SHADE) {
-#pragma unroll
-      for (int it = 0; it < S; ++it) {
-        if (!left) break;
-        const int s0 = __builtin_ctz(left);
-        uint32_t cur = w[0];
-#pragma unroll
-        for (int smp = 1; smp < S; ++smp)
-          if (smp == s0) cur = w[smp];
-        uint32_t m = 0;
-#pragma unroll
-        for (int smp = 0; smp < S; ++smp)
-          if (w[smp] == cur) m |= 1u << smp;
-        left &= ~m;
-        items[atomicAdd(&nitems, 1u)] = make_uint2(cur, static_cast<uint32_t>(p) | (m << 12));
-      }
-    }
-  }
-  if (!SHADE) return;
-  __syncthreads();
-  // phase 3: shading items
-  const uint32_t n = nitems;
-  for (uint32_t j = tid; j < n; j += NT) {
-    const uint2 item = items[j];
-    const uint32_t cur = item.x, p = item.y & 4095u, m = item.y >> 12;
-    if (cur >= 3u * P.prim_count) continue;  // every winner id is below 3 * prim_count
-    const int px = ox + static_cast<int>(p % GT), py = oy + static_cast<int>(p / GT);
-    const int pi = (px & 1) | ((py & 1) << 1);
-    attr_setup<NA> at;
-    load_attr<NA>(P, tri_attr, cur, at);
-    const quad_lazy<NA> q(at, P, px & ~1, py & ~1);
-    const float4 c = run_ps_pixel<NA>(P, SM, q, pi);
-#pragma unroll
-    for (int smp = 0; smp < S; ++smp)
-      if (m & (1u << smp)) store_texel(P.color.pf, sample_addr(P.color, px, py, smp), c);
-  }
-}
-template <int NA, int S, bool SHADE>
-__global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, int pass,
-                                                   const uint32_t* __restrict__ order,
-                                                   const uint4* __restrict__ entries, const uint4* __restrict__ merges,
-                                                   const uint32_t* __restrict__ counts,
-                                                   unsigned long long* __restrict__ partial,
-                                                   const uint32_t* __restrict__ vals,
-                                                   const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
-                                                   const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
-                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
-  vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, pass, order, entries, merges, counts, partial, vals, tstart, tend,
-                                              tri_rec, tri_attr, SM, blockIdx.x, wout);
-}
-
-
-// Deferred pixel shading of an opaque early-Z draw: one thread per pixel (16x16 pixels per
-// workgroup).  For each distinct winning triangle of the pixel's samples, the thread evaluates that
-// triangle's quad interpolants (the values the reference's last passing draw_quad/draw_full_quad
-// computed for this quad), runs the pixel shader for its own pixel and writes the winning samples.
-template <int NA, int S>
-__global__ void __launch_bounds__(256) shade_kernel(draw_params P, const ps_samplers* __restrict__ SM,
-                                                     const float4* __restrict__ tri_attr, const uint32_t* __restrict__ vis) {
-  const int x = blockIdx.x * 16 + (threadIdx.x & 15), y = blockIdx.y * 16 + (threadIdx.x >> 4);
-  const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
-  if (x >= tw || y >= th) return;
-  const int px0 = x & ~1, py0 = y & ~1;
-  const int pi = (x & 1) | ((y & 1) << 1);  // position in the quad
-  const size_t base = (static_cast<size_t>(y) * tw + x) * S;
-  uint32_t w[S];
-#pragma unroll
-  for (int s = 0; s < S; ++s) w[s] = vis[base + s];
-#pragma unroll
-  for (int it = 0; it < S; ++it) {
-    uint32_t cur = NO_WINNER;
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-      if (cur == NO_WINNER) cur = w[s];
-    if (cur >= 3u * P.prim_count) break;  // NO_WINNER (every id is below 3 * prim_count)
-    attr_setup<NA> at;
-    load_attr<NA>(P, tri_attr, cur, at);
-    const quad_lazy<NA> q(at, P, px0, py0);
-    const float4 c = run_ps_pixel<NA>(P, SM, q, pi);
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-      if (w[s] == cur) {
-        store_texel(P.color.pf, sample_addr(P.color, x, y, s), c);
-        w[s] = NO_WINNER;
-      }
-  }
-}
-
-// Deferred SASL shading of an opaque early-Z draw: one thread per 2x2 quad of a 16x16 GPU tile
-// (the tiles the visibility pass wrote).  For each distinct winning triangle among the quad's samples
-// the program runs once on the whole quad (pixel_shader_unit::execute, shader_unit.cpp:147-176) and
-// the samples that triangle won take their pixel's colour: a SASL pixel's colour depends only on the
-// triangle and the quad, so this equals shading every early-Z pass in order.
-template <int NA, int S>
-__global__ void __launch_bounds__(64) sasl_shade_kernel(draw_params P, const ps_samplers* __restrict__ SM,
-                                                        const float4* __restrict__ tri_attr, const uint32_t* __restrict__ vis) {
-  const int px0 = blockIdx.x * 16 + (threadIdx.x & 7) * 2, py0 = blockIdx.y * 16 + (threadIdx.x >> 3) * 2;
-  const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
-  if (px0 >= tw || py0 >= th) return;
-  uint32_t w[4][S];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int x = px0 + (i & 1), y = py0 + (i >> 1);
-    const bool in = x < tw && y < th;
-#pragma unroll
-    for (int s = 0; s < S; ++s) w[i][s] = in ? vis[(static_cast<size_t>(y) * tw + x) * S + s] : NO_WINNER;
-  }
-  const sasl_program* __restrict__ prog = P.sasl;
-  for (int it = 0; it < 4 * S; ++it) {
-    uint32_t cur = NO_WINNER;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int s = 0; s < S; ++s)
-        if (cur == NO_WINNER) cur = w[i][s];
-    if (cur >= 3u * P.prim_count) break;  // NO_WINNER (every id is below 3 * prim_count)
-    attr_setup<NA> at;
-    load_attr<NA>(P, tri_attr, cur, at);
-    const quad_lazy<NA> q(at, P, px0, py0);
-    sasl_regs R;
-    const uint32_t nregs = prog->nregs, nin = prog->ninputs;
-    for (uint32_t r = 0; r < nregs; ++r)
-      for (int px = 0; px < 4; ++px) R.r[r][px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int px = 0; px < 4; ++px) {
-      const float iw = q.inv_w(px);
-      for (uint32_t k = 0; k < nin; ++k) {
-        const sasl_input inp = prog->inputs[k];
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int a = 0; a < NA; ++a)
-          if (a == inp.attr) v = q.reg(a + 1, px, iw);
-        R.r[inp.reg][px] = make_float4(v.x, inp.ncomp > 1 ? v.y : 0.0f, inp.ncomp > 2 ? v.z : 0.0f, inp.ncomp > 3 ? v.w : 0.0f);
-      }
-    }
-    sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
-      if (!P.has_sampler[slot]) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      const sampler_desc_dev& sp = SM->s[slot];
-      return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                           : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
-    });
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bool any = false;
-#pragma unroll
-      for (int s = 0; s < S; ++s) any |= w[i][s] == cur;
-      if (!any) continue;
-      const float4 c = sasl_color0(prog, R, i);
-      const int x = px0 + (i & 1), y = py0 + (i >> 1);
-#pragma unroll
-      for (int s = 0; s < S; ++s)
-        if (w[i][s] == cur) {
-          store_texel(P.color.pf, sample_addr(P.color, x, y, s), c);
-          w[i][s] = NO_WINNER;
-        }
-    }
-  }
-}
-
 // ============================================================== host launchers
-hipError_t upload_ewa_table(const float* table256, hipStream_t s) {
-  return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_ewa), table256, 256 * sizeof(float), 0, hipMemcpyHostToDevice, s);
+void launch_reduce_partials(const unsigned long long* partial, uint32_t n, unsigned long long* stats, int slot, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, partial, n, stats, slot);
 }
 
 void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t* tiles, size_t ntiles, hipStream_t s) {
@@ -3359,22 +1868,6 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
   hipLaunchKernelGGL(vs_kernel, dim3((n + 255) / 256), dim3(256), 0, s, P, vbuf, counters, tiles,
                      static_cast<uint32_t>(ntiles));
 }
-
-// Kernels are instantiated per attribute count: the vertex and setup buffers are strided by it.
-#define SRX_NA_DISPATCH(NAV, CALL) \
-  switch (NAV) {                   \
-  case 1: CALL(1); break;          \
-  case 2: CALL(2); break;          \
-  case 3: CALL(3); break;          \
-  case 4: CALL(4); break;          \
-  default: CALL(5); break;         \
-  }
-// Batched draws are refused above two attributes when they are recorded (batch_max_attrs).
-#define SRX_NA_DISPATCH_BATCH(NAV, CALL) \
-  switch (NAV) {                         \
-  case 1: CALL(1); break;                \
-  default: CALL(2); break;               \
-  }
 
 void launch_setup(const draw_params& P, const draw_buffers& B, hipStream_t s) {
   if (P.prim_count == 0) return;
@@ -3385,7 +1878,7 @@ void launch_setup(const draw_params& P, const draw_buffers& B, hipStream_t s) {
   SRX_NA_DISPATCH(P.nattr, SRX_SETUP)
 #undef SRX_SETUP
   if (P.count_stats)
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, B.partial, grid.x, B.stats, static_cast<int>(ST_CPRIMITIVES));
+    launch_reduce_partials(B.partial, grid.x, B.stats, ST_CPRIMITIVES, s);
 }
 
 void launch_clip(const draw_params& P, const draw_buffers& B, hipStream_t s) {
@@ -3403,188 +1896,6 @@ void launch_emit(const draw_params& P, const draw_buffers& B, uint32_t capacity,
   if (!n) return;
   hipLaunchKernelGGL(emit_kernel, dim3((n + 255) / 256), dim3(256), 0, s, P, B.tri_rec, B.cnt, B.bsum, B.pairs,
                      capacity, B.keys[0], B.vals[0]);
-}
-
-void launch_raster(const draw_params& P, const draw_buffers& B, int which, hipStream_t s) {
-  uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-  if (!T) return;
-  int threads = (P.gt / 2) * (P.gt / 2);
-  size_t lds = sizeof(prim_lds) * threads;
-  bool vis = P.early_z && (P.blend_id == BLEND_OFF || P.blend_id == BLEND_DISABLED);
-  const bool sasl = !vis && sasl_shades(P);  // in-order shading by the SASL program
-#define SRX_RASTER_S(NA, S)                                                                                          \
-  do {                                                                                                               \
-    if (vis)                                                                                                         \
-      hipLaunchKernelGGL((raster_kernel<NA, S, true>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order, B.vals[which], \
-                         B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                                 \
-    else if (sasl)                                                                                                   \
-      hipLaunchKernelGGL((raster_kernel<NA, S, false, true>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order, \
-                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                  \
-    else                                                                                                             \
-      hipLaunchKernelGGL((raster_kernel<NA, S, false>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order,      \
-                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                  \
-  } while (0)
-#define SRX_RASTER(NA)                     \
-  switch (P.samples) {                     \
-  case 1: SRX_RASTER_S(NA, 1); break;      \
-  case 2: SRX_RASTER_S(NA, 2); break;      \
-  default: SRX_RASTER_S(NA, 4); break;     \
-  }
-  SRX_NA_DISPATCH(P.nattr, SRX_RASTER)
-#undef SRX_RASTER
-#undef SRX_RASTER_S
-  if (P.count_stats) {
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, B.partial, T, B.stats, static_cast<int>(ST_PS_INVOCATIONS));
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, B.partial, T, B.stats, static_cast<int>(ST_BACKEND_PIXELS));
-  }
-}
-
-// Visibility mode of an opaque early-Z draw for vis_kernel, or -1 when only the in-order kernel
-// reproduces the reference (NOT_EQUAL with depth writes).
-int vis_mode(const draw_params& P) {
-  if (P.vis_stencil && !(P.depth_enable && P.write_depth && (P.depth_func == 1 || P.depth_func == 3 ||
-                                                            P.depth_func == 4 || P.depth_func == 6)))
-    return -1;  // a stencil mask is expressed through the depth keys only
-  if (!P.depth_enable) return VIS_LATEST;
-  if (P.depth_func == 0) return VIS_NONE;
-  if (!P.write_depth) return VIS_LATEST;
-  switch (P.depth_func) {
-  case 1: return VIS_LESS;
-  case 3: return VIS_LEQUAL;
-  case 4: return VIS_GREATER;
-  case 6: return VIS_GEQUAL;
-  case 2:
-  case 7: return VIS_LATEST;  // EQUAL keeps the depth it compares against; ALWAYS ignores it
-  default: return -1;
-  }
-}
-
-void vis_table_bounds(uint32_t T, uint32_t records, uint32_t* entries, uint32_t* merges, uint32_t* slots) {
-  const uint32_t chunks = (records + VIS_PART - 1) / VIS_PART;
-  *entries = T + chunks;            // sum over tiles of max(1, ceil(n / VIS_PART))
-  *merges = records / (VIS_PART + 1) + 1;  // tiles with more than VIS_PART records
-  *slots = 2 * chunks + 1;          // parts of split tiles: ceil(n / VIS_PART) <= 2n / VIS_PART
-}
-
-bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, hipStream_t s) {
-  int mode = vis_mode(P);
-  // a SASL pixel shader runs in its own pass (launch_shade) over the winners this pass writes
-  uint32_t* const wout = sasl_shades(P) ? B.vis : nullptr;
-  if (wout) shade = false;
-  uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-  if (mode < 0 || P.gt != 16) return false;
-  if (!T) return true;
-  uint32_t ne = T, nm = 0, nsl;
-  if (!shade) {
-    vis_table_bounds(T, records, &ne, &nm, &nsl);
-    hipLaunchKernelGGL(vis_table_kernel, dim3(1), dim3(1024), 0, s, B.tstart, B.tend, B.order, T, B.vis_entries,
-                       B.vis_merges, B.vis_counts);
-  }
-  const uint4* entries = shade ? nullptr : B.vis_entries;
-#define SRX_VIS_LAUNCH(NA, S, SH)                                                                                 \
-  for (int pass = 0; pass < (SH ? 1 : 2); ++pass)                                                                 \
-    hipLaunchKernelGGL((vis_kernel<NA, S, SH>), dim3(pass == 0 ? ne : nm), dim3(SRX_VIS_THREADS), 0, s, P, mode, pass, \
-                       B.order, entries, B.vis_merges, B.vis_counts, B.vis_partial, B.vals[which], B.tstart,      \
-                       B.tend, B.tri_rec, B.tri_attr, B.samplers, wout)
-#define SRX_VIS_SHADE(NA)                   \
-  switch (P.samples) {                      \
-  case 1: SRX_VIS_LAUNCH(NA, 1, true); break; \
-  case 2: SRX_VIS_LAUNCH(NA, 2, true); break; \
-  default: SRX_VIS_LAUNCH(NA, 4, true); break; \
-  }
-  if (shade) {
-    SRX_NA_DISPATCH(P.nattr, SRX_VIS_SHADE)
-  } else {
-    switch (P.samples) {
-    case 1: SRX_VIS_LAUNCH(1, 1, false); break;
-    case 2: SRX_VIS_LAUNCH(1, 2, false); break;
-    default: SRX_VIS_LAUNCH(1, 4, false); break;
-    }
-  }
-#undef SRX_VIS_SHADE
-#undef SRX_VIS_LAUNCH
-  return true;
-}
-
-bool vis_applicable(const draw_params& P) { return vis_mode(P) >= 0 && P.gt == 16; }
-
-// One thread per quad: pixel_shader_unit::update/execute on caller-supplied inputs (the quad
-// evaluation behind srx_ps_execute_quads).  in: [quad][pixel][input] float4, out: [quad][pixel][output].
-__global__ void __launch_bounds__(64) sasl_quads_kernel(const sasl_program* __restrict__ prog,
-                                                        const ps_samplers* __restrict__ SM, uint32_t has_mask,
-                                                        const float4* __restrict__ in, float4* __restrict__ out,
-                                                        uint32_t nquads) {
-  const uint32_t qi = blockIdx.x * blockDim.x + threadIdx.x;
-  if (qi >= nquads) return;
-  const uint32_t nin = prog->ninputs, nout = prog->noutputs, nregs = prog->nregs;
-  sasl_regs R;
-  for (uint32_t r = 0; r < nregs; ++r)
-    for (int px = 0; px < 4; ++px) R.r[r][px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int px = 0; px < 4; ++px)
-    for (uint32_t k = 0; k < nin; ++k) {
-      const sasl_input inp = prog->inputs[k];
-      const float4 v = in[(static_cast<size_t>(qi) * 4 + px) * nin + k];
-      R.r[inp.reg][px] = make_float4(v.x, inp.ncomp > 1 ? v.y : 0.0f, inp.ncomp > 2 ? v.z : 0.0f, inp.ncomp > 3 ? v.w : 0.0f);
-    }
-  sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
-    if (!((has_mask >> slot) & 1u)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const sampler_desc_dev& sp = SM->s[slot];
-    return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                         : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
-  });
-  for (int px = 0; px < 4; ++px)
-    for (uint32_t o = 0; o < nout; ++o) {
-      const float4 v = R.r[prog->outputs[o].reg][px];
-      const int nc = prog->outputs[o].ncomp;
-      out[(static_cast<size_t>(qi) * 4 + px) * nout + o] =
-          make_float4(v.x, nc > 1 ? v.y : 0.0f, nc > 2 ? v.z : 0.0f, nc > 3 ? v.w : 0.0f);
-    }
-}
-
-void launch_sasl_quads(const sasl_program* prog, const ps_samplers* SM, uint32_t has_mask, const float4* in, float4* out,
-                       uint32_t nquads, hipStream_t s) {
-  if (!nquads) return;
-  hipLaunchKernelGGL(sasl_quads_kernel, dim3((nquads + 63) / 64), dim3(64), 0, s, prog, SM, has_mask, in, out, nquads);
-}
-
-bool sasl_shades(const draw_params& P) {
-  return P.ps_id == PS_SASL && P.color.data != nullptr && P.blend_id != BLEND_DISABLED;
-}
-
-bool needs_shading(const draw_params& P) {
-  return (P.early_z || P.vis_stencil) && P.blend_id == BLEND_OFF && P.color.data != nullptr;
-}
-
-// Covers exactly the 16x16 GPU tiles vis_kernel wrote: pixels of the target beyond the viewport's
-// 64x64 tile grid hold no winners of this draw.
-void launch_shade(const draw_params& P, const draw_buffers& B, hipStream_t s) {
-  if (P.gtiles_x <= 0 || P.gtiles_y <= 0) return;
-  dim3 grid(P.gtiles_x, P.gtiles_y);
-  if (P.ps_id == PS_SASL) {
-#define SRX_SASL_SHADE_S(NA, S) \
-  hipLaunchKernelGGL((sasl_shade_kernel<NA, S>), grid, dim3(64), 0, s, P, B.samplers, B.tri_attr, B.vis)
-#define SRX_SASL_SHADE(NA)                    \
-  switch (P.samples) {                        \
-  case 1: SRX_SASL_SHADE_S(NA, 1); break;     \
-  case 2: SRX_SASL_SHADE_S(NA, 2); break;     \
-  default: SRX_SASL_SHADE_S(NA, 4); break;    \
-  }
-    SRX_NA_DISPATCH(P.nattr, SRX_SASL_SHADE)
-#undef SRX_SASL_SHADE
-#undef SRX_SASL_SHADE_S
-    return;
-  }
-#define SRX_SHADE_S(NA, S) \
-  hipLaunchKernelGGL((shade_kernel<NA, S>), grid, dim3(256), 0, s, P, B.samplers, B.tri_attr, B.vis)
-#define SRX_SHADE(NA)                    \
-  switch (P.samples) {                   \
-  case 1: SRX_SHADE_S(NA, 1); break;     \
-  case 2: SRX_SHADE_S(NA, 2); break;     \
-  default: SRX_SHADE_S(NA, 4); break;    \
-  }
-  SRX_NA_DISPATCH(P.nattr, SRX_SHADE)
-#undef SRX_SHADE
-#undef SRX_SHADE_S
 }
 
 // ============================================================== clears, resolve, mip generation
@@ -3684,13 +1995,6 @@ __global__ void mip_kernel(surface_desc src, surface_desc dst, int filter) {
 // parameters and buffers.  Record counts are read on the device (from the batch-wide scan of the
 // per-triangle counts), clamped to the capacities the batch was prepared with, so a replay whose
 // geometry changed stays in bounds and reports the overflow through the status word.
-__device__ __forceinline__ uint32_t stage_job(const stage_map& m, uint32_t& local, uint32_t& blocks) {
-  const uint32_t j = m.job[blockIdx.x];
-  const uint2 r = m.range[j];
-  local = blockIdx.x - r.x;
-  blocks = r.y;
-  return j;
-}
 
 __global__ void batch_reset_kernel(uint32_t* __restrict__ counters, uint32_t n, uint32_t* __restrict__ cnt_tail,
                                    uint32_t* __restrict__ hist_tail, uint32_t* __restrict__ status) {
@@ -3802,14 +2106,6 @@ __global__ void __launch_bounds__(1024) tile_order_batch_kernel(const batch_job*
   tile_order_body(J.B.tstart, J.B.tend, J.tiles, const_cast<uint32_t*>(J.B.order));
 }
 
-template <int NA, int S, bool SHADE, int GT>
-__global__ void __launch_bounds__(256, 4) vis_batch_kernel(const batch_job* __restrict__ jobs, stage_map m) {
-  uint32_t lb, nb;
-  const batch_job& J = jobs[stage_job(m, lb, nb)];
-  vis_body<NA, S, SHADE, 0, GT>(J.P, J.vis_mode, 0, J.B.order, nullptr, nullptr, nullptr, nullptr, J.B.vals[1], J.B.tstart,
-                            J.B.tend, J.B.tri_rec, J.B.tri_attr, J.B.samplers, lb);
-}
-
 // status bit 0: a job's records exceeded the capacity it was prepared with; bit 1: clip overflow
 __global__ void batch_check_kernel(const batch_job* __restrict__ jobs, uint32_t njobs, uint32_t capacity, uint32_t items,
                                    uint32_t* __restrict__ status) {
@@ -3886,55 +2182,6 @@ void launch_range_batch(const batch_job* jobs, stage_map m, uint32_t blocks, hip
 }
 void launch_tile_order_batch(const batch_job* jobs, uint32_t njobs, hipStream_t s) {
   if (njobs) hipLaunchKernelGGL(tile_order_batch_kernel, dim3(njobs), dim3(1024), 0, s, jobs);
-}
-// GPU tiles of 8 and 32 pixels are built for single-sample draws; every variant must fit 64 KB of LDS.
-bool vis_batch_supported(int samples, bool shade, int threads, int gt) {
-  if (!(threads == 64 || threads == 128 || threads == 256)) return false;
-  if (gt != 16 && !(gt == 8 || gt == 32)) return false;
-  if (gt != 16 && samples != 1) return false;
-  return vis_static_bytes(samples, gt) + vis_union_bytes(threads, samples, shade, gt) <= 65536;
-}
-bool launch_vis_batch(int na, int samples, bool shade, int threads, int gt, const batch_job* jobs, stage_map m,
-                      uint32_t blocks, hipStream_t s) {
-  if (!vis_batch_supported(samples, shade, threads, gt)) return false;
-  if (!blocks) return true;
-  const size_t lds = static_cast<size_t>(vis_union_bytes(threads, samples, shade, gt));
-#define SRX_VIS_B(NA, S, SH, GT) \
-  hipLaunchKernelGGL((vis_batch_kernel<NA, S, SH, GT>), dim3(blocks), dim3(threads), lds, s, jobs, m)
-#define SRX_VIS_BS(NA)                       \
-  switch (samples) {                         \
-  case 1: SRX_VIS_B(NA, 1, true, 16); break; \
-  case 2: SRX_VIS_B(NA, 2, true, 16); break; \
-  default: SRX_VIS_B(NA, 4, true, 16); break; \
-  }
-#define SRX_VIS_B8(NA) SRX_VIS_B(NA, 1, true, 8)
-#define SRX_VIS_B32(NA) SRX_VIS_B(NA, 1, true, 32)
-  if (gt == 8) {
-    if (shade) {
-      SRX_NA_DISPATCH_BATCH(na, SRX_VIS_B8)
-    } else {
-      SRX_VIS_B(1, 1, false, 8);
-    }
-  } else if (gt == 32) {
-    if (shade) {
-      SRX_NA_DISPATCH_BATCH(na, SRX_VIS_B32)
-    } else {
-      SRX_VIS_B(1, 1, false, 32);
-    }
-  } else if (shade) {
-    SRX_NA_DISPATCH_BATCH(na, SRX_VIS_BS)
-  } else {
-    switch (samples) {
-    case 1: SRX_VIS_B(1, 1, false, 16); break;
-    case 2: SRX_VIS_B(1, 2, false, 16); break;
-    default: SRX_VIS_B(1, 4, false, 16); break;
-    }
-  }
-#undef SRX_VIS_B32
-#undef SRX_VIS_B8
-#undef SRX_VIS_BS
-#undef SRX_VIS_B
-  return true;
 }
 void launch_batch_check(const batch_job* jobs, uint32_t njobs, uint32_t capacity, int pt, uint32_t* status, hipStream_t s) {
   if (njobs)

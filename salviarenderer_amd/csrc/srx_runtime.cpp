@@ -637,7 +637,8 @@ int32_t srx_create_renderer(uint32_t kind, srx_renderer* out) {
   std::call_once(g_ewa_once, [] {
     float t[256];
     make_ewa(t);
-    hipError_t e = upload_ewa_table(t, nullptr);
+    hipError_t e = upload_ewa_table_raster(t, nullptr);
+    if (e == hipSuccess) e = upload_ewa_table_vis(t, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) g_ewa_status = hip_fail(e, "EWA table upload");
   });

@@ -11,7 +11,11 @@ enum { ADDR_WRAP = 0, ADDR_MIRROR = 1, ADDR_CLAMP = 2, ADDR_BORDER = 3 };
 enum { FILTER_POINT = 0, FILTER_LINEAR = 1, FILTER_ANISO = 2 };
 enum { MIP_LO = 0, MIP_MI = 1, MIP_HI = 2 };
 
-extern __constant__ float c_ewa[256];
+#ifdef __HIPCC_RTC__
+extern __constant__ float c_ewa[256];  // defined by the program that includes this
+#else
+static __constant__ float c_ewa[256];  // one per source that samples
+#endif
 
 struct coord2 {
   int x0, y0, x1, y1;
