@@ -14,7 +14,8 @@ CSRC = os.path.join(PKG, "csrc")
 OUT_DIR = os.path.join(PKG, "lib")
 OUT = os.path.join(OUT_DIR, "libsrx_hip.so")
 SOURCES = ["srx_runtime.cpp", "srx_batch.cpp", "srx_server.cpp", "srx_sasl.cpp", "srx_sasl_jit.cpp", "srx_noalloc.hip",
-           "srx_kernels.hip", "srx_raster.hip", "srx_vis.hip"]
+           "srx_kernels.hip", "srx_raster.hip", "srx_inorder.hip",
+           "srx_vis.hip"]
 # device headers the SASL shading kernels compiled at run time include (embedded in the library)
 JIT_HEADERS = ["srx_device.h", "srx_sampler.h", "srx_sasl_program.h", "srx_shade_common.h", "srx_sasl_exec.h"]
 JIT_GEN = os.path.join(OUT_DIR, "srx_jit_sources.gen.h")

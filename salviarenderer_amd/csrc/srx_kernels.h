@@ -112,6 +112,7 @@ int vis_mode(const draw_params& P);
 
 // The anisotropic weights: each source that samples holds its own copy.
 hipError_t upload_ewa_table_raster(const float* table256, hipStream_t s);
+hipError_t upload_ewa_table_inorder(const float* table256, hipStream_t s);
 hipError_t upload_ewa_table_vis(const float* table256, hipStream_t s);
 
 // stats[slot] += sum(partial[0..n))
@@ -147,6 +148,11 @@ uint32_t bucket_hist_size(uint32_t T, uint32_t n);
 bool vis_applicable(const draw_params& P);
 void launch_tile_ranges(const draw_params& P, const draw_buffers& B, int which, uint32_t n, hipStream_t s);
 void launch_raster(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
+// In-order rasterisation, shading and blending with one pixel per lane: every in-order draw with 16x16
+// GPU tiles, except under a statistics query and with a SASL pixel shader (launch_raster takes those).
+bool inorder_applicable(const draw_params& P);
+bool inorder_takes_color_clear(const draw_params& P);
+void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
 // Order-independent visibility for opaque early-Z draws without statistics; false if not applicable.
 // Order-independent visibility (and, with shade, the deferred pixel shader) of an opaque early-Z
 // draw; false when the draw needs the in-order kernel.

@@ -391,18 +391,19 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   // the counters are final after the clip launch: their read-back overlaps the emission
   HIPCHK(hipEventRecord(r->ev_counted, s));
   launch_emit(P, B, capacity, s);
-  // A target's pending full clear is applied by the order-independent visibility pass as it writes
-  // the target, when that pass covers the whole target (it then reads nothing back); the others run
+  // A target's pending full clear is applied by the visibility or in-order pass as it writes the
+  // target, when that pass covers the whole target (it then reads nothing back); the others run
   // here, while the record count travels to the host.
-  const bool will_vis = vis_tables && vis_applicable(P);
+  const bool will_vis = vis_tables && vis_applicable(P), will_inorder = !will_vis && inorder_applicable(P);
   surface_obj* const ct0 = r->st.color_targets.empty() ? nullptr : r->st.color_targets[0].get();
   surface_obj* const dst = r->st.ds_target.get();
   auto covers = [&](const surface_obj* o) {
     return o && P.target_w == static_cast<float>(o->w) && P.target_h == static_cast<float>(o->h) &&
            P.gtiles_x * P.gt >= o->w && P.gtiles_y * P.gt >= o->h;
   };
-  const bool eat_color = will_vis && needs_shading(P) && P.ps_id != PS_SASL && ct0 && ct0->pend.kind == 1 && covers(ct0);
-  const bool eat_ds = will_vis && dst && dst->pend.kind == 2 && dst->pend.flags == (SRX_CLEAR_DEPTH | SRX_CLEAR_STENCIL) &&
+  const bool writes_color = will_vis ? needs_shading(P) && P.ps_id != PS_SASL : will_inorder && inorder_takes_color_clear(P);
+  const bool eat_color = writes_color && ct0 && ct0->pend.kind == 1 && covers(ct0);
+  const bool eat_ds = (will_vis || will_inorder) && dst && dst->pend.kind == 2 && dst->pend.flags == (SRX_CLEAR_DEPTH | SRX_CLEAR_STENCIL) &&
                       covers(dst);
   for (auto& ct : r->st.color_targets)
     if (!(eat_color && ct.get() == ct0)) RCHK(run_pending_clear(ct.get(), s));
@@ -490,7 +491,10 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     RCHK(run_pending_clear(dst, s, true));
   }
   const bool fused = vis_tables && launch_vis(P, B, which, needs_shading(P), total, s);
-  if (!fused) launch_raster(P, B, which, s);
+  if (!fused) {
+    if (inorder_applicable(P)) launch_inorder(P, B, which, s);
+    else launch_raster(P, B, which, s);
+  }
   mark(5);
   // the in-order kernel defers shading (to shade_kernel) only for early-Z draws
   // deferred shading: the in-order kernel's early-Z winners, or a SASL shader over vis_kernel's winners
@@ -638,6 +642,7 @@ int32_t srx_create_renderer(uint32_t kind, srx_renderer* out) {
     float t[256];
     make_ewa(t);
     hipError_t e = upload_ewa_table_raster(t, nullptr);
+    if (e == hipSuccess) e = upload_ewa_table_inorder(t, nullptr);
     if (e == hipSuccess) e = upload_ewa_table_vis(t, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) g_ewa_status = hip_fail(e, "EWA table upload");
