@@ -60,14 +60,16 @@ template <int NA, int S>
 __global__ void __launch_bounds__(256) inorder_kernel(draw_params P, const ps_samplers* __restrict__ SM,
                                                       const uint32_t* __restrict__ order, const uint32_t* __restrict__ vals,
                                                       const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
-                                                      const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr) {
+                                                      const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
+                                                      const uint32_t* __restrict__ counters, uint32_t cap) {
+  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
   __shared__ float4 recs[IO_CHUNK * 4];            // edges, depth plane, id << 1 | front
   __shared__ unsigned long long cov[IO_CHUNK][16];  // covered samples of a record's block, 4 bits a pixel
   __shared__ unsigned long long pmask[256];         // records with a covered sample in the pixel (partial blocks)
   __shared__ unsigned long long fmask[16];          // records that cover the block whole
   __shared__ uint16_t work[IO_CHUNK * 16];
   __shared__ uint32_t nwork;
-  const int gtile = order[blockIdx.x];
+  const int gtile = static_cast<int>(scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x));
   const uint32_t t0 = tstart[gtile], t1 = tend[gtile];
   if (t0 == t1 && !P.clear_ds && !P.clear_color) return;
   const int tid = threadIdx.x;
@@ -324,7 +326,7 @@ void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipS
   if (!T) return;
 #define SRX_INORDER_S(NA, S)                                                                                            \
   hipLaunchKernelGGL((inorder_kernel<NA, S>), dim3(T), dim3(256), 0, s, P, B.samplers, B.order, B.vals[which], B.tstart, \
-                     B.tend, B.tri_rec, B.tri_attr)
+                     B.tend, B.tri_rec, B.tri_attr, B.counters, B.list_cap)
 #define SRX_INORDER(NA)                  \
   switch (P.samples) {                   \
   case 1: SRX_INORDER_S(NA, 1); break;   \

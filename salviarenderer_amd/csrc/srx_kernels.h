@@ -15,10 +15,32 @@ enum stat_slot {
   ST_PS_INVOCATIONS, ST_BACKEND_PIXELS, ST_COUNT
 };
 // Setup counters
-// CT_WIDE: triangles whose records the clip launch counts by wave (their ids in wide_list)
-// CT_CLASS: GPU tiles per record-count class (16 slots), CT_CURSOR: their placement cursors
-enum counter_slot { CT_CLIP_PRIMS = 0, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_TOTAL, CT_WIDE, CT_CLASS, CT_CURSOR = CT_CLASS + 16,
-                    CT_CLIP_DONE = CT_CURSOR + 16, CT_COUNT };
+// CT_TOTAL: records emitted (single draws); CT_WIDE: primitives on wide_list, left to the clip launch.
+// The two are added to as one 64-bit word.
+// CT_CURSOR: records given to the tiles' lists; CT_CLASS: GPU tiles per record-count class.
+constexpr int TILE_CLASSES = 16;
+enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_CLASS,
+                    CT_COUNT = CT_CLASS + TILE_CLASSES };
+static_assert(CT_TOTAL % 2 == 0 && CT_WIDE == CT_TOTAL + 1, "one aligned 64-bit word");
+
+// Where a tile's record count lies in tile_count: atomics to words of one cache line are served one after
+// another (330k of them on 1,024 adjacent words take 95 us, on words spread over 32 KB 14 us), and
+// neighbouring tiles are counted at the same time, so they lie at least 64 bytes apart.
+constexpr uint32_t TILE_SLOT_ROWS = 512;
+__host__ __device__ inline uint32_t tile_slot_shift(uint32_t T) {  // log2 of the words per row
+  uint32_t w = 4;
+  while ((TILE_SLOT_ROWS << w) < T) ++w;
+  return w;
+}
+__host__ __device__ inline uint32_t tile_slot(uint32_t t, uint32_t shift) {
+  return ((t % TILE_SLOT_ROWS) << shift) + t / TILE_SLOT_ROWS;
+}
+__host__ __device__ inline uint32_t slot_tile(uint32_t s, uint32_t shift) {
+  return (s & ((1u << shift) - 1u)) * TILE_SLOT_ROWS + (s >> shift);
+}
+__host__ __device__ inline uint32_t tile_slots(uint32_t T) {
+  return (T < TILE_SLOT_ROWS ? T : TILE_SLOT_ROWS) << tile_slot_shift(T);
+}
 
 // Per-draw device buffers (owned by the renderer, grown on demand).
 struct draw_buffers {
@@ -27,28 +49,28 @@ struct draw_buffers {
   float4* tri_attr;    // 3*prims * 3*(nattr+1): v0, ddx, ddy of every register
   uint32_t* vis;       // target w*h*samples: winning triangle per sample (opaque early-Z draws)
   const ps_samplers* samplers;  // device copy of the bound samplers
-  uint32_t* cnt;       // 3*prims: GPU-tile records per clipped triangle (batches: then its exclusive scan)
-  uint32_t* bsum;      // single draws: records of each 256-primitive block's triangles (null in batches)
-  uint4* pairs;        // single draws, per primitive: fan triangle 0's first four (tile << 1 | full)
-                       // records as setup found them, x = 0xFFFFFFFF when not kept (null in batches)
+  uint32_t* cnt;       // batches, 3*prims: GPU-tile records per clipped triangle, then their exclusive scan
   uint8_t* clip_flag;  // prims
   int32_t* clip_slot;  // prims
   float4* clip_verts;  // clip_capacity * 5 * (nattr+1), screen space
   uint32_t* clip_hdr;  // clip_capacity
   uint32_t clip_capacity;
-  uint32_t* wide_list; // prims: triangles over many 64x64 tiles, counted by the clip launch
-  uint32_t* keys[2];   // records: GPU tile id
-  uint32_t* vals[2];   // records: triangle id << 1 | tile-level accept
-  const uint32_t* order;  // GPU tiles, most records first (workgroup launch order)
+  uint32_t* wide_list; // prims: triangles whose records the clip launch emits (batches: counts)
+  uint32_t* keys[2];   // [0] records: GPU tile id; [1] single draws: the record's rank in its tile
+  uint32_t* vals[2];   // records: triangle id << 1 | tile-level accept; [0] as emitted, [1] by tile
+                       // (single draws that need primitive order: sorted back into [0])
+  uint32_t list_cap;      // records the tiles' lists are formed for; with more the raster passes return at once
+  const uint32_t* order;  // workgroup launch order of the GPU tiles, heaviest record-count class first: single
+                          // draws, the tiles of class k at order[k * tiles], counters[CT_CLASS + k] of them
+                          // (scheduled_tile); batches, the tiles one after another
   uint4* vis_entries;     // visibility work table (vis_table_bounds)
   uint4* vis_merges;
   uint32_t* vis_counts;   // entries, merges, partial slots
   unsigned long long* vis_partial;  // partial per-sample keys of split tiles
   uint32_t* tstart;    // GPU tiles
-  uint32_t* tile_count;  // 2 * GPU tiles: records per tile, then the scatter's per-tile cursors
+  uint32_t* tile_count;  // tile_slots(T) words: records per tile, at tile_slot (zero before the setup launch)
   uint32_t* tend;
-  uint32_t* hist;      // radix histogram 256 * blocks
-  uint32_t* scan_tmp;  // scan partial sums
+  uint32_t* hist;      // batches: bucket histogram
   uint32_t* counters;  // CT_COUNT
   unsigned long long* stats;    // ST_COUNT
   unsigned long long* partial;  // per-workgroup statistics partials (>= max(setup blocks, GPU tiles))
@@ -121,32 +143,20 @@ void launch_reduce_partials(const unsigned long long* partial, uint32_t n, unsig
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 // The vertex launch of a single draw; it also zeroes the draw's counters and ntiles words of tiles.
 void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t* tiles, size_t ntiles, hipStream_t s);
-void launch_setup(const draw_params& P, const draw_buffers& B, hipStream_t s);
-void launch_clip(const draw_params& P, const draw_buffers& B, hipStream_t s);
+// Setup and clipping of a single draw, which emit its records (those beyond `capacity` are counted and
+// dropped) and count them per tile.
+void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
+void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
+// The tiles' record lists from the emitted records: ranges in tstart/tend, the tiles by record-count
+// class in `order` (TILE_CLASSES * tiles words), lists in vals[1], or in primitive order in vals[0]
+// (`sorted`).  Sized for `cap` records; the count is read from B.counters[CT_TOTAL] on the device.
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, hipStream_t s);
 // In-place exclusive scan of n u32; writes the total to *total_dev.  tmp holds >= scan_tmp_size(n).
 size_t scan_tmp_size(uint32_t n);
 void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* total_dev, hipStream_t s);
-void launch_emit(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
-// Stable LSD radix sort of (keys, vals) by the low `bits` bits of keys; returns the buffer index
-// (0 or 1) that holds the result.
-int launch_sort(const draw_buffers& B, uint32_t n, int bits, hipStream_t s);
-// Sorts the GPU tiles by record count, heaviest first, into O.vals[result]; O supplies keys/vals
-// scratch (>= tiles each) and shares hist/scan_tmp with B.
-// GPU tile scheduling order, heaviest record-count class first.  `counted`: the bucket sort's range
-// pass has already counted the tiles per class.
-void launch_tile_order(const draw_params& P, const draw_buffers& B, uint32_t* order, bool counted, hipStream_t s);
-// One-pass (unstable within a tile) bucket sort of the n emitted records by GPU tile into vals[1],
-// with the tile ranges; false when the tile count exceeds its LDS histogram (then radix-sort).
-// Counting sort of the records by GPU tile (order-independent draws) into vals[1] with the tile ranges
-// in tstart/tend, sized for `cap` records; the kernels read the record count from
-// B.counters[CT_TOTAL] (at most cap are sorted).  B.tile_count must be zero.  With `order`, the
-// tiles' scheduling order (as launch_tile_order writes it) is written too.
-bool bucket_sort_applicable(const draw_params& P);
-bool launch_bucket_sort(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s);
-uint32_t bucket_hist_size(uint32_t T, uint32_t n);
 // Whether launch_vis will take the draw (its visibility mode exists and the tiles are 16x16).
 bool vis_applicable(const draw_params& P);
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, int which, uint32_t n, hipStream_t s);
+// The raster passes read the record count on the device and do nothing when it exceeds B.list_cap.
 void launch_raster(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
 // In-order rasterisation, shading and blending with one pixel per lane: every in-order draw with 16x16
 // GPU tiles, except under a statistics query and with a SASL pixel shader (launch_raster takes those).

@@ -4,14 +4,13 @@
 //   vs_kernel       vertex fetch + vertex shader, one thread per vertex    (stream_assembler.cpp,
 //                   default_vertex_cache.cpp: the shader runs once per vertex instead of per cache miss)
 //   setup_kernel    index fetch, near/far trivial accept, cull, winding, viewport transform and
-//                   triangle setup, one thread per primitive                (clipper.cpp, rasterizer.cpp:864-945)
-//   clip_kernel     Sutherland-Hodgman near/far clipping for the few primitives that need it; the
-//                   draw's record total from setup's per-block totals
-//   emit_kernel     per-triangle GPU-tile records written in clipped-primitive order (offsets from
-//                   the per-block totals and a workgroup scan)
-//   sort            by GPU tile: a counting sort (order-independent draws) or a stable 8-bit LSD
-//                   radix sort -> per-tile lists in primitive order (the reference's per-tile
-//                   std::sort, rasterizer.cpp:947-994)
+//                   triangle setup, one thread per primitive; emits the (GPU tile, triangle) records of
+//                   triangles on few tiles                                  (clipper.cpp, rasterizer.cpp:864-945)
+//   clip_kernel     Sutherland-Hodgman near/far clipping for the few primitives that need it; emits the
+//                   records of the clipped triangles and of those on many tiles
+//   tile_ranges     tile ranges and scheduling order from the record counts per tile
+//   tile_scatter    records to their tiles' lists; in-order draws then sort each list (tile_sort), so it
+//                   is in primitive order (the reference's per-tile std::sort, rasterizer.cpp:947-994)
 //   raster_kernel   (srx_raster.hip) one workgroup per GPU tile, one thread per 2x2 quad; walks its tile's list in
 //                   order and evaluates the reference's 64->16->4->sample decision chain per quad
 //                   (rasterizer.cpp:298-773), early/late depth-stencil, pixel shader and blending
@@ -67,14 +66,6 @@ __device__ __forceinline__ float4 fetch_elem(const input_elem_dev& e, uint32_t v
   case FMT_RGB32F: return make_float4(f[0], f[1], f[2], e.default_w);
   default: return make_float4(f[0], f[1], f[2], f[3]);
   }
-}
-
-// a[i] for i < n, else 0, loaded without a branch (the index is clamped): guarded loads in an
-// unrolled loop would each sit in a branch of its own and wait for its data before the next issues.
-// n must be at least 1.
-__device__ __forceinline__ uint32_t load_or_zero(const uint32_t* __restrict__ a, uint32_t i, uint32_t n) {
-  const uint32_t x = a[min(i, n - 1u)];
-  return i < n ? x : 0u;
 }
 
 // Coalesced stores of a wave's per-lane blocks of W float4 (lane i's block at dst + i*W): the lanes
@@ -422,14 +413,7 @@ struct tri_bin {
   bool mx[3], my[3];
   float r2a[3], s1x[3], s1y[3];
 };
-__device__ __forceinline__ void bin_setup(const draw_params& P, const float* e, const float* bb, tri_bin& t) {
-  const int tx = P.tiles_x, ty = P.tiles_y;
-  t.sx = min(fast_floori(std_max(0.0f, bb[0]) / TILE), tx);
-  t.sy = min(fast_floori(std_max(0.0f, bb[2]) / TILE), ty);
-  t.ex = min(fast_ceili(std_max(0.0f, bb[1]) / TILE) + 1, tx);
-  t.ey = min(fast_ceili(std_max(0.0f, bb[3]) / TILE) + 1, ty);
-  t.small = (t.sx + 1 == t.ex) && (t.sy + 1 == t.ey);
-  t.regions = (t.ex - t.sx) * (t.ey - t.sy) <= REGION_TEST_TILES;
+__device__ __forceinline__ void bin_edges(const float* e, tri_bin& t) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float ex = e[k * 3 + 0], ey = e[k * 3 + 1];
@@ -442,6 +426,16 @@ __device__ __forceinline__ void bin_setup(const draw_params& P, const float* e, 
     t.s1x[k] = stx;
     t.s1y[k] = sty;
   }
+}
+__device__ __forceinline__ void bin_setup(const draw_params& P, const float* e, const float* bb, tri_bin& t) {
+  const int tx = P.tiles_x, ty = P.tiles_y;
+  t.sx = min(fast_floori(std_max(0.0f, bb[0]) / TILE), tx);
+  t.sy = min(fast_floori(std_max(0.0f, bb[2]) / TILE), ty);
+  t.ex = min(fast_ceili(std_max(0.0f, bb[1]) / TILE) + 1, tx);
+  t.ey = min(fast_ceili(std_max(0.0f, bb[3]) / TILE) + 1, ty);
+  t.small = (t.sx + 1 == t.ex) && (t.sy + 1 == t.ey);
+  t.regions = (t.ex - t.sx) * (t.ey - t.sy) <= REGION_TEST_TILES;
+  bin_edges(e, t);
 }
 // The GPU tiles of 64x64 tile (x, y) that get a record, bit j * sub + i for GPU tile (i, j) of it
 // (row-major, the order records are written in); full: the tile is fully accepted.
@@ -577,16 +571,12 @@ __device__ __forceinline__ uint32_t count_gtiles(const draw_params& P, const flo
   return n;
 }
 
-// count_gtiles that also keeps the first four GPU tiles for_each_gtile visits, packed as
-// tile << 1 | full (setup's pairs, which spare the emission the walk of triangles with at most four
-// records).
-constexpr uint32_t NO_PAIRS = 0xFFFFFFFFu;  // no tile is that large
-__device__ __forceinline__ uint32_t count_gtiles_pairs(const draw_params& P, const float* e, const float* bb, uint4& k) {
-  tri_bin t;
-  bin_setup(P, e, bb, t);
+// The same for a triangle whose walk has been set up, keeping the first four GPU tiles for_each_gtile
+// visits, packed as tile << 1 | full.
+__device__ __forceinline__ uint32_t count_gtiles_pairs(const draw_params& P, const float* e, const float* bb,
+                                                       const tri_bin& t, uint32_t (&k)[4]) {
   const int sub = TILE / P.gt;
   uint32_t n = 0;
-  k = make_uint4(NO_PAIRS, NO_PAIRS, NO_PAIRS, NO_PAIRS);
   for (int y = t.sy; y < t.ey; ++y)
     for (int x = t.sx; x < t.ex; ++x) {
       bool full;
@@ -596,10 +586,10 @@ __device__ __forceinline__ uint32_t count_gtiles_pairs(const draw_params& P, con
         const int b = __builtin_ctzll(m);
         const uint32_t g = static_cast<uint32_t>((y * sub + b / sub) * P.gtiles_x + x * sub + b % sub);
         const uint32_t v = (g << 1) | (full ? 1u : 0u);
-        if (i == 0) k.x = v;
-        else if (i == 1) k.y = v;
-        else if (i == 2) k.z = v;
-        else k.w = v;
+        if (i == 0) k[0] = v;
+        else if (i == 1) k[1] = v;
+        else if (i == 2) k[2] = v;
+        else k[3] = v;
       }
       n += c;
     }
@@ -668,94 +658,211 @@ __global__ void __launch_bounds__(256) reduce_partials_kernel(const unsigned lon
 }
 
 // ============================================================== setup (fast path)
+// Primitive p of the draw: near/far trivial accept, cull, winding, viewport transform, triangle setup.
+// Sets the clip flag; returns whether the primitive gave a set-up triangle.
 template <int NA>
-__device__ __forceinline__ void setup_body(const draw_params& P, const float4* __restrict__ vbuf, float4* __restrict__ tri_rec,
-                                           float4* __restrict__ tri_attr, uint32_t* __restrict__ cnt,
-                                           uint8_t* __restrict__ clip_flag, uint32_t* __restrict__ counters,
-                                           uint32_t* __restrict__ wide_list, unsigned long long* __restrict__ partial,
-                                           uint32_t* __restrict__ bsum, uint4* __restrict__ pairs, uint32_t bx) {
-  uint32_t p = bx * blockDim.x + threadIdx.x;
+__device__ __forceinline__ bool setup_primitive(const draw_params& P, const float4* __restrict__ vbuf, uint32_t p,
+                                                uint8_t* __restrict__ clip_flag, uint32_t* __restrict__ counters,
+                                                unsigned long long& cprims, tri_setup<NA>& t) {
+  vtx<NA> v[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) load_vertex<NA>(P, vbuf, fetch_index(P, p, i), v[i]);
+  // near (0,0,1,0) and far (0,0,-1,1) planes (clipper.cpp:21-27,104-120)
+  const float4 pn = make_float4(0.0f, 0.0f, 1.0f, 0.0f), pf = make_float4(0.0f, 0.0f, -1.0f, 1.0f);
+  bool in = true;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) in &= !(dot4(pn, v[i].r[0]) < 0);
+  if (in)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) in &= !(dot4(pf, v[i].r[0]) < 0);
+  clip_flag[p] = in ? 0 : 1;
+  if (!in) {
+    atomicAdd(&counters[CT_CLIP_PRIMS], 1u);
+    return false;
+  }
+  const bool front = compute_front(v[0].r[0], v[1].r[0], v[2].r[0]);
+  if (cull_fn(P, front ? 1.0f : -1.0f)) return false;
+  cprims = 1;
+  // winding normalisation (clipper.cpp:59-65) by selects
+  vtx<NA> o[3] = {v[0], vsel<NA>(front, v[1], v[2]), vsel<NA>(front, v[2], v[1])};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) viewport_project<NA>(o[i], P);
+  triangle_info<NA>(o[0], o[1], o[2], t);
+  return t.valid;
+}
+// The fan-0 slots of the wave's 64 consecutive primitives (first of the block: bx * 256) are
+// consecutive: the set-up triangles' words are stored coalesced.
+template <int NA>
+__device__ __forceinline__ void store_setup(const float4 (&rec)[5], const float4 (&attr)[3 * (NA + 1)], bool have,
+                                            float4* __restrict__ tri_rec, float4* __restrict__ tri_attr, uint32_t bx,
+                                            float4* stage) {
+  const uint64_t mask = __ballot(have);
+  if (!mask) return;
+  const size_t p0 = static_cast<size_t>(bx) * 256 + (threadIdx.x & ~63u);
+  float4* ws = stage + (threadIdx.x >> 6) * WAVE_STAGE;
+  wave_store_blocks<5>(tri_rec + p0 * 5, rec, mask, ws);
+  wave_store_blocks<3 * (NA + 1)>(tri_attr + p0 * 3 * (NA + 1), attr, mask, ws);
+}
+
+// Batches: counts each triangle's records (emitted at offsets from a scan of the counts).
+template <int NA>
+__device__ __forceinline__ void setup_count_body(const draw_params& P, const draw_buffers& B, uint32_t bx) {
+  __shared__ float4 stage[4 * WAVE_STAGE];
+  const uint32_t p = bx * 256 + threadIdx.x;
   unsigned long long cprims = 0;
   float4 rec[5], attr[3 * (NA + 1)];  // this lane's setup words, stored by the whole wave below
   bool have = false;
-  uint32_t c0 = 0;  // records of fan triangle 0 counted here
-  uint4 kp = make_uint4(NO_PAIRS, NO_PAIRS, NO_PAIRS, NO_PAIRS);  // its first four (tile, full) pairs
   if (p < P.prim_count) {
-    cnt[3 * p + 1] = 0;
-    cnt[3 * p + 2] = 0;
-    vtx<NA> v[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) load_vertex<NA>(P, vbuf, fetch_index(P, p, i), v[i]);
-    // near (0,0,1,0) and far (0,0,-1,1) planes (clipper.cpp:21-27,104-120)
-    const float4 pn = make_float4(0.0f, 0.0f, 1.0f, 0.0f), pf = make_float4(0.0f, 0.0f, -1.0f, 1.0f);
-    bool in = true;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) in &= !(dot4(pn, v[i].r[0]) < 0);
-    if (in)
-#pragma unroll
-      for (int i = 0; i < 3; ++i) in &= !(dot4(pf, v[i].r[0]) < 0);
-    clip_flag[p] = in ? 0 : 1;
-    if (!in) {
-      atomicAdd(&counters[CT_CLIP_PRIMS], 1u);
-    } else {
-      bool front = compute_front(v[0].r[0], v[1].r[0], v[2].r[0]);
-      if (!cull_fn(P, front ? 1.0f : -1.0f)) {
-        cprims = 1;
-        // winding normalisation (clipper.cpp:59-65) by selects
-        vtx<NA> o[3] = {v[0], vsel<NA>(front, v[1], v[2]), vsel<NA>(front, v[2], v[1])};
-#pragma unroll
-        for (int i = 0; i < 3; ++i) viewport_project<NA>(o[i], P);
-        tri_setup<NA> t;
-        triangle_info<NA>(o[0], o[1], o[2], t);
-        if (t.valid) {
-          have = true;
-          tri_rec_words<NA>(t, rec);
-          tri_attr_words<NA>(t, attr);
-          float e[9], bb[4];
-          for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j) e[i * 3 + j] = t.e[i][j];
-          for (int i = 0; i < 4; ++i) bb[i] = t.bb[i];
-          if (bin_span(P, bb) > COUNT_WIDE)
-            wide_list[atomicAdd(&counters[CT_WIDE], 1u)] = p;  // counted in the clip launch
-          else if (pairs)
-            c0 = count_gtiles_pairs(P, e, bb, kp);
-          else
-            c0 = count_gtiles(P, e, bb);
+    uint32_t c0 = 0;  // records of fan triangle 0
+    tri_setup<NA> t;
+    have = setup_primitive<NA>(P, B.vbuf, p, B.clip_flag, B.counters, cprims, t);
+    if (have) {
+      tri_rec_words<NA>(t, rec);
+      tri_attr_words<NA>(t, attr);
+      float e[9], bb[4];
+      for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 3; ++j) e[i * 3 + j] = t.e[i][j];
+      for (int i = 0; i < 4; ++i) bb[i] = t.bb[i];
+      if (bin_span(P, bb) > COUNT_WIDE)
+        B.wide_list[atomicAdd(&B.counters[CT_WIDE], 1u)] = p;  // counted in the clip launch
+      else
+        c0 = count_gtiles(P, e, bb);
+    }
+    B.cnt[3 * p] = c0;
+    B.cnt[3 * p + 1] = 0;
+    B.cnt[3 * p + 2] = 0;
+  }
+  store_setup<NA>(rec, attr, have, B.tri_rec, B.tri_attr, bx, stage);
+}
+
+// ---------------------------------------------------------------- records of single draws
+// A record is (GPU tile, triangle id << 1 | full, rank among the tile's records).  Records are emitted
+// as triangles are set up, at positions taken from the draw's cursor (counters[CT_TOTAL]) a workgroup
+// at a time, in no particular order: the rank comes from the tile's count, so the tiles' lists need no
+// counting pass afterwards, and draws that need primitive order sort each tile's list.  Records
+// beyond `capacity` are counted and dropped (the host compares the total with it and repeats).
+//
+// A triangle is emitted by the lane that set it up when its box lies on at most four GPU tiles and nine
+// 64x64 tiles (a box inside one 64x64 tile spans four of them, see bin_setup); any other goes to the
+// wide list, whose (triangle, 64x64 tile) pairs the clip launch spreads over all lanes.  Walking up to
+// 32 64x64 tiles in one lane, and emitting long lists by the lane's wave one triangle after another,
+// took 117 + 72 + 342 us of a 2,000-triangle draw at 512x512, which leaves 32 waves to do it; setup now
+// takes 7 and the clip launch 31 us there.  What bounds the clip launch is the tiles' counts: 330k
+// device atomics take 14 us however they are spread.
+constexpr int SMALL_SPAN = 9;
+__device__ __forceinline__ void put_record(const draw_buffers& B, uint32_t capacity, uint32_t pos, uint32_t tile,
+                                           uint32_t val, uint32_t rank) {
+  if (pos < capacity) {
+    B.keys[0][pos] = tile;
+    B.vals[0][pos] = val;
+    B.keys[1][pos] = rank;
+  }
+}
+
+// Ranks of one record per lane (of lanes with `valid`) in their tiles.  Lanes on the same tile are
+// matched in the wave and their tile's count is taken with one atomic: consecutive triangles lie on the
+// same few tiles, where an atomic per record serialises (590k records: 400 us).  Lanes still unmatched
+// after RANK_ROUNDS tiles take their own (scattered triangles: their atomics do not meet).
+constexpr int RANK_ROUNDS = 16;
+__device__ __forceinline__ uint32_t take_ranks(const draw_buffers& B, uint32_t slot_shift, uint32_t tile, bool valid) {
+  const int lane = __lane_id();
+  int leader = lane;
+  uint32_t rank = 0, n = 1;
+  bool open = valid;
+  for (int it = 0; it < RANK_ROUNDS; ++it) {
+    const uint64_t left = __ballot(open);
+    if (!left) break;
+    const int first = __builtin_ctzll(left);
+    const uint32_t t0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tile), first));
+    const bool same = open && tile == t0;
+    const uint64_t m = __ballot(same);
+    if (same) {
+      leader = first;
+      rank = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+      n = static_cast<uint32_t>(__popcll(m));
+      open = false;
+    }
+  }
+  uint32_t old = 0;
+  if (valid && leader == lane) old = atomicAdd(&B.tile_count[tile_slot(tile, slot_shift)], n);
+  return static_cast<uint32_t>(__shfl(static_cast<int>(old), leader, 64)) + rank;
+}
+
+// One workgroup: 256 primitives.
+template <int NA>
+__global__ void __launch_bounds__(256) setup_kernel(draw_params P, draw_buffers B, uint32_t capacity, uint32_t slot_shift) {
+  __shared__ float4 stage[4 * WAVE_STAGE];
+  __shared__ uint32_t wtot[4], s_base, s_wide;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, bx = blockIdx.x;
+  const uint32_t p = bx * 256 + tid;
+  unsigned long long cprims = 0;
+  uint32_t c = 0;     // records this lane emits (its triangle's, when it is small)
+  bool wide = false;  // left to the clip launch
+  uint32_t kp[4] = {0, 0, 0, 0};
+  {
+    float4 rec[5], attr[3 * (NA + 1)];
+    bool have = false;
+    if (p < P.prim_count) {
+      tri_setup<NA> t;
+      have = setup_primitive<NA>(P, B.vbuf, p, B.clip_flag, B.counters, cprims, t);
+      if (have) {
+        tri_rec_words<NA>(t, rec);
+        tri_attr_words<NA>(t, attr);
+        float e[9], bb[4];
+        for (int i = 0; i < 3; ++i)
+          for (int j = 0; j < 3; ++j) e[i * 3 + j] = t.e[i][j];
+        for (int i = 0; i < 4; ++i) bb[i] = t.bb[i];
+        tri_bin w;
+        bin_setup(P, e, bb, w);
+        if (w.ex > w.sx && w.ey > w.sy) {
+          const float inv = 1.0f / static_cast<float>(P.gt);
+          const float gw = floorf(bb[1] * inv) - floorf(bb[0] * inv) + 1.0f, gh = floorf(bb[3] * inv) - floorf(bb[2] * inv) + 1.0f;
+          wide = !(gw * gh <= 4.0f) || (w.ex - w.sx) * (w.ey - w.sy) > SMALL_SPAN;
+          if (!wide) {
+            c = count_gtiles_pairs(P, e, bb, w, kp);
+            if (c > 4) {  // the corner tests accept tiles beyond the box of a triangle far below a pixel
+              wide = true;
+              c = 0;
+            }
+          }
         }
       }
     }
-    cnt[3 * p] = c0;
-    if (pairs) {
-      if (c0 > 4u) kp.x = NO_PAIRS;
-      pairs[p] = kp;
-    }
+    store_setup<NA>(rec, attr, have, B.tri_rec, B.tri_attr, bx, stage);
   }
-  // The fan-0 slots of the wave's 64 consecutive primitives are consecutive: store the set-up
-  // triangles' words coalesced (blockDim.x is 256).
-  {
-    __shared__ float4 stage[4 * WAVE_STAGE];
-    const uint64_t mask = __ballot(have);
-    if (mask) {
-      const size_t p0 = static_cast<size_t>(bx) * blockDim.x + (threadIdx.x & ~63u);
-      float4* ws = stage + (threadIdx.x >> 6) * WAVE_STAGE;
-      wave_store_blocks<5>(tri_rec + p0 * 5, rec, mask, ws);
-      wave_store_blocks<3 * (NA + 1)>(tri_attr + p0 * 3 * (NA + 1), attr, mask, ws);
-    }
+  const uint32_t incl = wave_incl_scan(c | (wide ? 0x10000u : 0u));
+  if (lane == 63) wtot[wave] = incl;
+  __syncthreads();  // the staging area is stored
+  uint32_t before = 0, total = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    if (w < wave) before += wtot[w];
+    total += wtot[w];
   }
-  if (bsum) {  // uniform over the launch: the block's total; the clip launch adds the counts it makes
-    const uint32_t t = block_sum_u32(c0);
-    if (threadIdx.x == 0) bsum[bx] = t;
+  const uint32_t off = before + incl - (c | (wide ? 0x10000u : 0u));
+  const uint32_t nrec = total & 0xFFFFu;
+  if (tid == 0 && total) {
+    // the record cursor and the wide list's length are one 64-bit word
+    const unsigned long long old =
+        atomicAdd(reinterpret_cast<unsigned long long*>(B.counters + CT_TOTAL),
+                  static_cast<unsigned long long>(nrec) | (static_cast<unsigned long long>(total >> 16) << 32));
+    s_base = static_cast<uint32_t>(old);
+    s_wide = static_cast<uint32_t>(old >> 32);
   }
-  if (P.count_stats) block_partial(partial, cprims);  // uniform over the launch
-}
-template <int NA>
-__global__ void __launch_bounds__(256) setup_kernel(draw_params P, const float4* __restrict__ vbuf, float4* __restrict__ tri_rec,
-                                                     float4* __restrict__ tri_attr,
-                                                     uint32_t* __restrict__ cnt, uint8_t* __restrict__ clip_flag,
-                                                     uint32_t* __restrict__ counters, uint32_t* __restrict__ wide_list,
-                                                     unsigned long long* __restrict__ partial, uint32_t* __restrict__ bsum,
-                                                     uint4* __restrict__ pairs) {
-  setup_body<NA>(P, vbuf, tri_rec, tri_attr, cnt, clip_flag, counters, wide_list, partial, bsum, pairs, blockIdx.x);
+  uint32_t rank[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    rank[i] = 0;
+    if (__ballot(i < c)) rank[i] = take_ranks(B, slot_shift, kp[i] >> 1, i < c);
+  }
+  __syncthreads();
+  if (nrec) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i)
+      if (i < c) put_record(B, capacity, s_base + (off & 0xFFFFu) + i, kp[i] >> 1, (3 * p) << 1 | (kp[i] & 1u), rank[i]);
+  }
+  if (wide && s_wide + (off >> 16) < P.prim_count) B.wide_list[s_wide + (off >> 16)] = p;
+  if (P.count_stats) block_partial(B.partial, cprims);  // uniform over the launch
 }
 
 // ============================================================== clipping (slow path)
@@ -845,27 +952,18 @@ __device__ uint32_t clip_primitive(const draw_params& P, uint32_t p, const float
   return fans;
 }
 
-// Clipping launch: a bounded grid strides over the primitives setup flagged (none, usually).  With
-// `bsum` (single draws) the counts it makes are added to their 256-primitive block's total.
+// Batches: the clip launch counts the records of the triangles it clips and of those on the wide list.
 template <int NA>
-__device__ __forceinline__ void clip_work(const draw_params& P, const float4* __restrict__ vbuf, float4* __restrict__ tri_rec,
-                                          float4* __restrict__ tri_attr, uint32_t* __restrict__ cnt,
-                                          const uint8_t* __restrict__ clip_flag, int32_t* __restrict__ clip_slot,
-                                          float4* __restrict__ clip_verts, uint32_t* __restrict__ clip_hdr, uint32_t capacity,
-                                          uint32_t* __restrict__ counters, unsigned long long* __restrict__ stats,
-                                          const uint32_t* __restrict__ wide_list, uint32_t* __restrict__ bsum,
-                                          uint32_t nclip, uint32_t nwide, uint32_t bx, uint32_t gx) {
+__device__ __forceinline__ void clip_count_body(const draw_params& P, const draw_buffers& B, uint32_t bx, uint32_t gx) {
+  const uint32_t nclip = B.counters[CT_CLIP_PRIMS], nwide = B.counters[CT_WIDE];
   // triangles over many 64x64 tiles: one wave counts each one's records
   const uint32_t wave = (bx * blockDim.x + threadIdx.x) >> 6, waves = (gx * blockDim.x) >> 6;
   for (uint32_t w = wave; w < nwide; w += waves) {
-    const uint32_t p = wide_list[w];
+    const uint32_t p = B.wide_list[w];
     float e[9], bb[4];
-    read_tri_rec(tri_rec + static_cast<size_t>(p) * 5, e, bb);  // fan 0 of primitive p
+    read_tri_rec(B.tri_rec + static_cast<size_t>(p) * 5, e, bb);  // fan 0 of primitive p
     const uint32_t n = count_gtiles_wave(P, e, bb);
-    if (__lane_id() == 0) {
-      cnt[3 * p] = n;
-      if (bsum) atomicAdd(&bsum[p / 256], n);
-    }
+    if (__lane_id() == 0) B.cnt[3 * p] = n;
   }
   if (nclip == 0) return;
   // lanes clip the flagged primitives among the wave's 64; the wave then counts the records of the
@@ -874,8 +972,9 @@ __device__ __forceinline__ void clip_work(const draw_params& P, const float4* __
   for (uint32_t b = wave * 64; b < P.prim_count; b += waves * 64) {
     const uint32_t p = b + static_cast<uint32_t>(lane);
     uint32_t fans = 0;  // bit k: fan triangle 3p + k was set up
-    if (p < P.prim_count && clip_flag[p])
-      fans = clip_primitive<NA>(P, p, vbuf, tri_rec, tri_attr, clip_slot, clip_verts, clip_hdr, capacity, counters, stats);
+    if (p < P.prim_count && B.clip_flag[p])
+      fans = clip_primitive<NA>(P, p, B.vbuf, B.tri_rec, B.tri_attr, B.clip_slot, B.clip_verts, B.clip_hdr, B.clip_capacity,
+                                B.counters, B.stats);
     __threadfence();  // the fans' records are read back by every lane of the wave
     for (unsigned long long m = __ballot(fans != 0); m; m &= m - 1) {
       const int src = __builtin_ctzll(m);
@@ -885,85 +984,169 @@ __device__ __forceinline__ void clip_work(const draw_params& P, const float4* __
         if (!(fs & (1u << k))) continue;
         const uint32_t id = 3 * ps + k;
         float e[9], bb[4];
-        read_tri_rec(tri_rec + tri_slot(P, id) * 5, e, bb);
+        read_tri_rec(B.tri_rec + tri_slot(P, id) * 5, e, bb);
         const uint32_t n = count_gtiles_wave(P, e, bb);
-        if (lane == 0) {
-          cnt[id] = n;
-          if (bsum) atomicAdd(&bsum[ps / 256], n);
-        }
+        if (lane == 0) B.cnt[id] = n;
       }
     }
   }
 }
 
-// counters[CT_TOTAL] = the sum of the block totals (every thread of the workgroup calls it).
-__device__ __forceinline__ void record_total(const draw_params& P, const uint32_t* __restrict__ bsum,
-                                             uint32_t* __restrict__ counters) {
-  const uint32_t nb = (P.prim_count + 255) / 256;
-  uint32_t t = 0;
-  for (uint32_t i0 = 0; i0 < nb; i0 += 8 * blockDim.x) {
-    uint32_t v[8];
+// The workgroup emits the records of its lanes' triangles (`has`: lane's triangle `id`, set up in
+// B.tri_rec): their (triangle, 64x64 tile) pairs are numbered consecutively and taken one per lane, so
+// a triangle over the whole target and a hundred small ones fill the lanes alike.  The records of
+// WIDE_STEP pairs per lane then take their positions together and are listed in LDS, so that consecutive
+// lanes write consecutive records and no lane waits for another's longer list.  Every thread of the
+// workgroup calls it.
+constexpr uint32_t WIDE_STEP = 4;
+constexpr uint32_t WIDE_LIST = 4096;  // records listed at a time
+struct wide_lds {
+  uint16_t list[WIDE_LIST];  // pair << 4 | GPU tile of the pair's 64x64 tile
+  float4 tri[256 * 4];  // edges, bounding box, first 64x64 tile and columns, id
+  uint2 pair[256 * WIDE_STEP];  // a pair's first GPU tile; GPU tile mask | full << 16 | owner lane << 17
+  uint32_t pre[256];  // pairs of the lanes up to and including this one
+  uint32_t wsum[4], base;
+};
+__device__ __forceinline__ void emit_wide(const draw_params& P, const draw_buffers& B, uint32_t capacity,
+                                          uint32_t slot_shift, bool has, uint32_t id, wide_lds& L) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t R = 0;
+  if (has) {
+    float e[9], bb[4];
+    read_tri_rec(B.tri_rec + tri_slot(P, id) * 5, e, bb);
+    tri_bin t;
+    bin_setup(P, e, bb, t);
+    if (t.ex > t.sx && t.ey > t.sy) R = static_cast<uint32_t>((t.ex - t.sx) * (t.ey - t.sy));
+    L.tri[tid * 4] = make_float4(e[0], e[1], e[2], e[3]);
+    L.tri[tid * 4 + 1] = make_float4(e[4], e[5], e[6], e[7]);
+    L.tri[tid * 4 + 2] = make_float4(e[8], bb[0], bb[1], bb[2]);
+    // at most 129 64x64 tiles a side (targets are at most 8192 wide)
+    L.tri[tid * 4 + 3] = make_float4(bb[3], __uint_as_float(static_cast<uint32_t>(t.sx) | (static_cast<uint32_t>(t.sy) << 10) |
+                                                            (static_cast<uint32_t>(t.ex - t.sx) << 20)),
+                                     __uint_as_float(id), __uint_as_float((t.small ? 1u : 0u) | (t.regions ? 2u : 0u)));
+  }
+  const uint32_t incl = wave_incl_scan(R);
+  if (lane == 63) L.wsum[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0, total = 0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t i = i0 + k * blockDim.x + threadIdx.x;
-      const uint32_t x = __hip_atomic_load(bsum + min(i, nb - 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      v[k] = i < nb ? x : 0u;  // no branch per load (see load_or_zero)
+  for (uint32_t w = 0; w < 4; ++w) {
+    if (w < wave) before += L.wsum[w];
+    total += L.wsum[w];
+  }
+  L.pre[tid] = before + incl;
+  __syncthreads();
+  const int sub = TILE / P.gt;
+  for (uint32_t q0 = 0; q0 < total; q0 += 256 * WIDE_STEP) {
+    uint32_t n = 0;  // records of this lane's pairs
+#pragma unroll 1
+    for (uint32_t u = 0; u < WIDE_STEP; ++u) {
+      const uint32_t q = q0 + u * 256 + tid;
+      uint2 pr = make_uint2(0, 0);
+      if (q < total) {
+        uint32_t o = 0;  // the first lane with q < pre[o]
+#pragma unroll
+        for (uint32_t step = 128; step; step >>= 1)
+          if (L.pre[o + step - 1] <= q) o += step;
+        const uint32_t local = q - (o ? L.pre[o - 1] : 0u);
+        const float4 a = L.tri[o * 4], b = L.tri[o * 4 + 1], c = L.tri[o * 4 + 2], d = L.tri[o * 4 + 3];
+        const float e[9] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x}, bb[4] = {c.y, c.z, c.w, d.x};
+        const uint32_t box = __float_as_uint(d.y), flags = __float_as_uint(d.w);
+        const uint32_t w = box >> 20;
+        tri_bin t;
+        t.small = (flags & 1u) != 0;
+        t.regions = (flags & 2u) != 0;
+        bin_edges(e, t);
+        const int x = static_cast<int>((box & 1023u) + local % w), y = static_cast<int>(((box >> 10) & 1023u) + local / w);
+        bool full;
+        const uint32_t m = static_cast<uint32_t>(tile_gmask(P, e, bb, t, x, y, full));  // GPU tiles of 16 or 32 pixels
+        n += __popc(m);
+        pr = make_uint2(static_cast<uint32_t>(y * sub * P.gtiles_x + x * sub), m | (full ? 0x10000u : 0u) | (o << 17));
+      }
+      L.pair[u * 256 + tid] = pr;
     }
+    const uint32_t in = wave_incl_scan(n);
+    if (lane == 63) L.wsum[wave] = in;
+    __syncthreads();
+    uint32_t pos = in - n, all = 0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) t += v[k];
+    for (uint32_t w = 0; w < 4; ++w) {
+      if (w < wave) pos += L.wsum[w];
+      all += L.wsum[w];
+    }
+    if (tid == 0 && all) L.base = atomicAdd(&B.counters[CT_TOTAL], all);
+    __syncthreads();
+    const uint32_t base = L.base;
+    for (uint32_t w0 = 0; w0 < all; w0 += WIDE_LIST) {
+      uint32_t at = pos - w0;  // this lane's next entry of the window (wraps below it)
+#pragma unroll 1
+      for (uint32_t u = 0; u < WIDE_STEP; ++u)
+        for (uint32_t m = L.pair[u * 256 + tid].y & 0xFFFFu; m; m &= m - 1, ++at)
+          if (at < WIDE_LIST) L.list[at] = static_cast<uint16_t>(((u * 256 + tid) << 4) | static_cast<uint32_t>(__builtin_ctz(m)));
+      __syncthreads();
+      const uint32_t nw = min(all - w0, WIDE_LIST);
+      for (uint32_t r0 = 0; r0 < nw; r0 += 1024) {
+        uint32_t tile[4], val[4], rank[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {  // four ranks in flight
+          const uint32_t r = r0 + i * 256 + tid;
+          const uint32_t en = L.list[min(r, nw - 1)];
+          const uint2 pr = L.pair[en >> 4];
+          const int b = static_cast<int>(en & 15u);
+          tile[i] = pr.x + static_cast<uint32_t>((b / sub) * P.gtiles_x + b % sub);
+          val[i] = (__float_as_uint(L.tri[(pr.y >> 17) * 4 + 3].z) << 1) | ((pr.y >> 16) & 1u);
+          rank[i] = r < nw ? atomicAdd(&B.tile_count[tile_slot(tile[i], slot_shift)], 1u) : 0u;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+          const uint32_t r = r0 + i * 256 + tid;
+          if (r < nw) put_record(B, capacity, base + w0 + r, tile[i], val[i], rank[i]);
+        }
+      }
+      __syncthreads();
+    }
+    __syncthreads();  // the sums, the base and the pairs are used again
   }
-  t = block_sum_u32(t);
-  if (threadIdx.x == 0) counters[CT_TOTAL] = t;
 }
 
+// Single draws: emits the records of the wide list's triangles, then clips the flagged primitives and
+// emits theirs.  A draw with neither returns at once.
 template <int NA>
-__device__ __forceinline__ void clip_body(const draw_params& P, const float4* __restrict__ vbuf, float4* __restrict__ tri_rec,
-                                          float4* __restrict__ tri_attr, uint32_t* __restrict__ cnt,
-                                          const uint8_t* __restrict__ clip_flag, int32_t* __restrict__ clip_slot,
-                                          float4* __restrict__ clip_verts, uint32_t* __restrict__ clip_hdr, uint32_t capacity,
-                                          uint32_t* __restrict__ counters, unsigned long long* __restrict__ stats,
-                                          const uint32_t* __restrict__ wide_list, uint32_t* __restrict__ bsum, uint32_t bx,
-                                          uint32_t gx) {
-  const uint32_t nclip = counters[CT_CLIP_PRIMS], nwide = counters[CT_WIDE];
-  const bool flagged = nclip != 0 || nwide != 0;  // uniform over the launch
-  if (flagged)
-    clip_work<NA>(P, vbuf, tri_rec, tri_attr, cnt, clip_flag, clip_slot, clip_verts, clip_hdr, capacity, counters, stats,
-                  wide_list, bsum, nclip, nwide, bx, gx);
-  if (!bsum) return;
-  // single draws: the record total, once every workgroup's counts are in the block totals (the last
-  // workgroup to finish sums them; with nothing flagged, setup's totals are final and workgroup 0 does)
-  if (flagged) {
-    __shared__ uint32_t s_last;
-    __threadfence();
+__global__ void __launch_bounds__(256) clip_kernel(draw_params P, draw_buffers B, uint32_t capacity, uint32_t slot_shift) {
+  __shared__ wide_lds L;
+  const uint32_t nclip = B.counters[CT_CLIP_PRIMS], nwide = min(B.counters[CT_WIDE], P.prim_count);
+  const uint32_t tid = threadIdx.x;
+  const uint32_t per = min(max((nwide + gridDim.x - 1) / gridDim.x, 1u), 256u);  // triangles per workgroup and turn
+  for (uint32_t g = blockIdx.x * per; g < nwide; g += gridDim.x * per) {
+    const bool has = tid < min(per, nwide - g);
+    emit_wide(P, B, capacity, slot_shift, has, has ? 3 * B.wide_list[g + tid] : 0u, L);
     __syncthreads();
-    if (threadIdx.x == 0) s_last = atomicAdd(&counters[CT_CLIP_DONE], 1u) == gx - 1 ? 1u : 0u;
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
-  } else if (bx != 0) {
-    return;
   }
-  record_total(P, bsum, counters);
-}
-template <int NA>
-__global__ void clip_kernel(draw_params P, const float4* __restrict__ vbuf, float4* __restrict__ tri_rec,
-                            float4* __restrict__ tri_attr, uint32_t* __restrict__ cnt, const uint8_t* __restrict__ clip_flag, int32_t* __restrict__ clip_slot,
-                            float4* __restrict__ clip_verts, uint32_t* __restrict__ clip_hdr, uint32_t capacity,
-                            uint32_t* __restrict__ counters, unsigned long long* __restrict__ stats,
-                            const uint32_t* __restrict__ wide_list, uint32_t* __restrict__ bsum) {
-  clip_body<NA>(P, vbuf, tri_rec, tri_attr, cnt, clip_flag, clip_slot, clip_verts, clip_hdr, capacity, counters, stats,
-                wide_list, bsum, blockIdx.x, gridDim.x);
+  if (nclip == 0) return;
+  for (uint32_t b = blockIdx.x * 256; b < P.prim_count; b += gridDim.x * 256) {
+    const uint32_t p = b + tid;
+    uint32_t fans = 0;  // bit k: fan triangle 3p + k was set up
+    if (p < P.prim_count && B.clip_flag[p])
+      fans = clip_primitive<NA>(P, p, B.vbuf, B.tri_rec, B.tri_attr, B.clip_slot, B.clip_verts, B.clip_hdr, B.clip_capacity,
+                                B.counters, B.stats);
+    for (uint32_t k = 0; k < 3; ++k) {
+      const bool has = ((fans >> k) & 1u) != 0;
+      if (!__syncthreads_or(has)) continue;
+      emit_wide(P, B, capacity, slot_shift, has, 3 * p + k, L);
+      __syncthreads();
+    }
+  }
 }
 
-// ============================================================== record emission
+// ============================================================== record emission (batches)
 // off: exclusive scan of the per-triangle record counts; a triangle owns [off[id], off[id+1]).
 // One thread per primitive, over its (at most 3) clipped triangles in fan order.  Records beyond
-// `capacity` are dropped; the host compares the total with it and emits again.
+// `capacity` are dropped; the batch's status word reports them.
 
 // Records of one clipped triangle emitted by a whole wave: lanes take the triangle's 64x64 tiles in
 // for_each_gtile's order, count each tile's GPU tiles with the same tests, and write at their
 // wave-scanned offsets -- for triangles that reach many tiles, which one lane would walk serially.
-__device__ __forceinline__ void emit_wide(const draw_params& P, const float4* __restrict__ tri_rec, uint32_t id,
+__device__ __forceinline__ void emit_wave(const draw_params& P, const float4* __restrict__ tri_rec, uint32_t id,
                                           uint32_t first, uint32_t next, uint32_t capacity,
                                           uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   const int lane = __lane_id();
@@ -1005,10 +1188,8 @@ constexpr uint32_t EMIT_WIDE = 64;
 
 // Records of primitive p's fan triangles: triangle 3p+k owns [o[k], o[k+1]).  Every lane of the wave
 // calls it (p >= prim_count: nothing of its own).
-// pr: setup's first four (tile << 1 | full) pairs of fan triangle 0, pr.x == NO_PAIRS when it kept
-// none (then, and for the other fan triangles, the tiles are walked again).
 __device__ __forceinline__ void emit_records(const draw_params& P, const float4* __restrict__ tri_rec, uint32_t p,
-                                             const uint32_t (&o)[4], uint4 pr, uint32_t capacity,
+                                             const uint32_t (&o)[4], uint32_t capacity,
                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   uint32_t wide = 0;  // fan triangles left to the wave
   if (p < P.prim_count) {
@@ -1018,16 +1199,6 @@ __device__ __forceinline__ void emit_records(const draw_params& P, const float4*
       const uint32_t id = id3 + k;
       const uint32_t first = o[k], next = o[k + 1];
       if (next == first) continue;
-      if (k == 0 && pr.x != NO_PAIRS) {  // at most four records, as setup's walk found them
-        const uint32_t v[4] = {pr.x, pr.y, pr.z, pr.w};
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i)
-          if (first + i < next && first + i < capacity) {
-            keys[first + i] = v[i] >> 1;
-            vals[first + i] = (id << 1) | (v[i] & 1u);
-          }
-        continue;
-      }
       if (next - first > EMIT_WIDE) {
         wide |= 1u << k;
         continue;
@@ -1060,7 +1231,7 @@ __device__ __forceinline__ void emit_records(const draw_params& P, const float4*
       if (!(ws & (1u << k))) continue;
       const uint32_t first = static_cast<uint32_t>(__shfl(static_cast<int>(o[k]), src, 64));
       const uint32_t next = static_cast<uint32_t>(__shfl(static_cast<int>(o[k + 1]), src, 64));
-      emit_wide(P, tri_rec, 3 * ps + k, first, next, capacity, keys, vals);
+      emit_wave(P, tri_rec, 3 * ps + k, first, next, capacity, keys, vals);
     }
   }
 }
@@ -1079,56 +1250,8 @@ __device__ __forceinline__ void emit_body(const draw_params& P, const float4* __
     o[2] = off[id3 + 2];
     o[3] = (id3 + 3 < n) ? off[id3 + 3] : *total;
   }
-  emit_records(P, tri_rec, p, o, make_uint4(NO_PAIRS, NO_PAIRS, NO_PAIRS, NO_PAIRS), capacity, keys, vals);
+  emit_records(P, tri_rec, p, o, capacity, keys, vals);
 }
-// Single draws: the offsets come from the counts of the workgroup's 256 primitives (a workgroup
-// scan) and the totals of the blocks before it, which setup and the clip launch left in `bsum`, so
-// no scan of the counts runs: triangle id's first record is the sum of the counts of the triangles
-// before it, as an exclusive scan of the counts gives it.
-__global__ void __launch_bounds__(256) emit_kernel(draw_params P, const float4* __restrict__ tri_rec,
-                                                   const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ bsum,
-                                                   const uint4* __restrict__ pairs, uint32_t capacity,
-                                                   uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  __shared__ uint32_t wtot[4], wbefore[4];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t p = blockIdx.x * 256 + tid;
-  uint32_t c[3] = {0, 0, 0};
-  uint4 pr = make_uint4(NO_PAIRS, NO_PAIRS, NO_PAIRS, NO_PAIRS);
-  if (p < P.prim_count) {
-    c[0] = cnt[3 * p];
-    c[1] = cnt[3 * p + 1];
-    c[2] = cnt[3 * p + 2];
-    pr = pairs[p];
-  }
-  uint32_t before = 0;  // records of the blocks before this one
-  for (uint32_t i0 = 0; i0 < blockIdx.x; i0 += 4 * 256) {
-    uint32_t v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t i = i0 + k * 256 + tid;
-      v[k] = load_or_zero(bsum, i, blockIdx.x);
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) before += v[k];
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) before += static_cast<uint32_t>(__shfl_xor(static_cast<int>(before), off, 64));
-  const uint32_t t = c[0] + c[1] + c[2];
-  const uint32_t incl = wave_incl_scan(t);
-  if (lane == 63) {
-    wtot[wave] = incl;
-    wbefore[wave] = before;
-  }
-  __syncthreads();
-  uint32_t o[4];
-  o[0] = wbefore[0] + wbefore[1] + wbefore[2] + wbefore[3] + incl - t;
-  for (uint32_t w = 0; w < wave; ++w) o[0] += wtot[w];
-  o[1] = o[0] + c[0];
-  o[2] = o[1] + c[1];
-  o[3] = o[2] + c[2];
-  emit_records(P, tri_rec, p, o, pr, capacity, keys, vals);
-}
-
 __global__ void fill_u32_kernel(uint32_t* p, uint32_t n, uint32_t v) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1234,103 +1357,10 @@ void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* 
   scan_rec(data, n, tmp, total_dev, s);
 }
 
-// ============================================================== radix sort (stable LSD, 8-bit digits)
-constexpr int SORT_BLOCK = 4096;  // 256 threads x 16 items
-
-__global__ void __launch_bounds__(256) radix_hist_kernel(const uint32_t* __restrict__ keys, uint32_t n, int shift,
-                                                          uint32_t nblocks, uint32_t* __restrict__ hist) {
-  __shared__ uint32_t cnt[256];
-  cnt[threadIdx.x] = 0;
-  __syncthreads();
-  uint32_t b0 = blockIdx.x * SORT_BLOCK;
-  uint32_t end = min(n, b0 + SORT_BLOCK);
-  for (uint32_t i = b0 + threadIdx.x; i < end; i += 256) atomicAdd(&cnt[(keys[i] >> shift) & 255u], 1u);
-  __syncthreads();
-  hist[threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
-}
-
-// Each wave ranks its 1024 consecutive items in 16 rounds of 64; a lane finds the lanes sharing its
-// digit with eight ballots (one per digit bit), so ranks follow input order (stability) at a cost
-// independent of how many digits a round holds.
-__global__ void __launch_bounds__(256) radix_scatter_kernel(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                             uint32_t n, int shift, uint32_t nblocks,
-                                                             const uint32_t* __restrict__ hist_scanned,
-                                                             uint32_t* __restrict__ kout, uint32_t* __restrict__ vout) {
-  __shared__ uint32_t wcnt[4][256];
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int i = threadIdx.x; i < 4 * 256; i += 256) (&wcnt[0][0])[i] = 0;
-  __syncthreads();
-  uint32_t base = blockIdx.x * SORT_BLOCK + wave * 1024;
-  uint32_t rank[16], key[16], val[16];
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    uint32_t i = base + r * 64 + lane;
-    bool valid = i < n;
-    key[r] = valid ? kin[i] : 0u;
-    val[r] = valid ? vin[i] : 0u;
-    uint32_t d = (key[r] >> shift) & 255u;
-    // m: the valid lanes holding this lane's digit, from one ballot per digit bit
-    uint64_t m = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = ((d >> b) & 1u) != 0;
-      const uint64_t bal = __ballot(bit);
-      m &= bit ? bal : ~bal;
-    }
-    const uint32_t before = valid ? wcnt[wave][d] : 0u;
-    rank[r] = before + static_cast<uint32_t>(__popcll(m & lt));
-    __builtin_amdgcn_wave_barrier();
-    if (valid && (m & lt) == 0) wcnt[wave][d] = before + static_cast<uint32_t>(__popcll(m));  // lowest lane of the digit
-    __builtin_amdgcn_wave_barrier();
-  }
-  __syncthreads();
-  {
-    uint32_t d = threadIdx.x, s = 0;
-    for (int w = 0; w < 4; ++w) {
-      uint32_t c = wcnt[w][d];
-      wcnt[w][d] = s;
-      s += c;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    uint32_t i = base + r * 64 + lane;
-    if (i < n) {
-      uint32_t d = (key[r] >> shift) & 255u;
-      uint32_t pos = hist_scanned[d * nblocks + blockIdx.x] + wcnt[wave][d] + rank[r];
-      if (pos < n) {
-        kout[pos] = key[r];
-        vout[pos] = val[r];
-      }
-    }
-  }
-}
-
-int launch_sort(const draw_buffers& B, uint32_t n, int bits, hipStream_t s) {
-  int cur = 0;
-  if (n == 0) return cur;
-  uint32_t nblocks = (n + SORT_BLOCK - 1) / SORT_BLOCK;
-  for (int shift = 0; shift < bits; shift += 8) {
-    hipLaunchKernelGGL(radix_hist_kernel, dim3(nblocks), dim3(256), 0, s, B.keys[cur], n, shift, nblocks, B.hist);
-    launch_exclusive_scan(B.hist, 256 * nblocks, B.scan_tmp, nullptr, s);
-    hipLaunchKernelGGL(radix_scatter_kernel, dim3(nblocks), dim3(256), 0, s, B.keys[cur], B.vals[cur], n, shift, nblocks,
-                       B.hist, B.keys[cur ^ 1], B.vals[cur ^ 1]);
-    cur ^= 1;
-  }
-  return cur;
-}
-
-// [ts, te) of every GPU tile in the sorted records.  With T > 0 the thread at the last record of a
-// tile (or before the first record) also writes the empty ranges of the tiles up to the next
-// record's tile, so every tile is written exactly once without a separate clear (dense records).
 // ---------------------------------------------------------------- one-pass bucket sort by GPU tile
-// For the order-independent path the order of a tile's records is immaterial, so one counting pass
-// replaces the stable radix passes: per-workgroup tile histograms in LDS, one scan of the
-// tile-major histogram, and a scatter whose in-workgroup ranks come from LDS atomics.
-constexpr int BUCKET_PER_THREAD = 16;
-constexpr int BUCKET_ITEMS = 256 * BUCKET_PER_THREAD;  // records per workgroup
+// Batches: the order of a tile's records is immaterial, so one counting pass bins them: per-workgroup
+// tile histograms in LDS, one scan of the tile-major histogram, and a scatter whose in-workgroup
+// ranks come from LDS atomics.
 constexpr uint32_t BUCKET_MAX_TILES = 8192;
 
 // PT records per thread: 256 * PT records per workgroup (the batched path tunes PT)
@@ -1442,345 +1472,161 @@ __device__ __forceinline__ void bucket_range_body(const uint32_t* __restrict__ h
   te[t] = (t + 1 < T) ? hist_scanned[(t + 1) * nblocks] : end;
 }
 
-uint32_t bucket_hist_size(uint32_t T, uint32_t n) {
-  return T * std::max<uint32_t>((n + BUCKET_ITEMS - 1) / BUCKET_ITEMS, 1);
-}
-
-// Counting sort of one draw's records by GPU tile (order-independent draws): the order within a tile
-// is immaterial, so each workgroup of BUCKET_ITEMS records counts its tiles in LDS, noting the
-// tiles it touches, and adds the counts of those tiles to the per-tile totals; one workgroup turns
-// the totals into tile ranges; the scatter counts again, reserves its range in each touched tile
-// with one atomic and places its records at the LDS ranks.  tile_count and tile_cursor are zero
-// at the start of the draw.
-// Counts the workgroup's records of tiles [r0, r0 + tn) in LDS (rank[j]: the record's rank among the
-// workgroup's records of its tile) and lists the tiles it touches (relative to r0).
-__device__ __forceinline__ void tile_count_lds(const uint32_t (&k)[BUCKET_PER_THREAD], uint32_t (&rank)[BUCKET_PER_THREAD],
-                                               uint32_t r0, uint32_t tn, uint32_t* cnt, uint16_t* touched,
-                                               uint32_t* ntouched) {
-  for (uint32_t d = threadIdx.x; d < tn; d += 256) cnt[d] = 0;
-  if (threadIdx.x == 0) *ntouched = 0;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < BUCKET_PER_THREAD; ++j)
-    if (k[j] - r0 < tn) {  // also skips the 0xFFFFFFFF padding
-      rank[j] = atomicAdd(&cnt[k[j] - r0], 1u);
-      if (rank[j] == 0) touched[atomicAdd(ntouched, 1u)] = static_cast<uint16_t>(k[j] - r0);
-    }
-  __syncthreads();
-}
-__device__ __forceinline__ void tile_load_keys(const uint32_t* __restrict__ keys, uint32_t n, uint32_t b0,
-                                               uint32_t (&k)[BUCKET_PER_THREAD]) {
-#pragma unroll
-  for (int j = 0; j < BUCKET_PER_THREAD; ++j) {
-    const uint32_t i = b0 + j * 256 + threadIdx.x;
-    k[j] = i < n ? keys[i] : 0xFFFFFFFFu;
-  }
-}
-__global__ void __launch_bounds__(256) tile_count_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ count,
-                                                         uint32_t cap, uint32_t T, uint32_t* __restrict__ tile_count) {
-  __shared__ uint32_t cnt[BUCKET_MAX_TILES];
-  __shared__ uint16_t touched[BUCKET_ITEMS];
-  __shared__ uint32_t ntouched;
-  const uint32_t n = min(*count, cap);
-  const uint32_t b0 = blockIdx.x * BUCKET_ITEMS;
-  if (b0 >= n) return;
-  uint32_t k[BUCKET_PER_THREAD], rank[BUCKET_PER_THREAD];
-  tile_load_keys(keys, n, b0, k);
-  for (uint32_t r0 = 0; r0 < T; r0 += BUCKET_MAX_TILES) {
-    const uint32_t tn = min(T - r0, BUCKET_MAX_TILES);
-    if (r0) __syncthreads();  // the previous range's touched tiles are consumed
-    tile_count_lds(k, rank, r0, tn, cnt, touched, &ntouched);
-    for (uint32_t i = threadIdx.x; i < ntouched; i += 256) {
-      const uint32_t t = touched[i];
-      atomicAdd(&tile_count[r0 + t], cnt[t]);
-    }
-  }
-}
-// counters[key] += the number of valid lanes with this lane's key (< 16), one LDS atomic per distinct
-// key; returns the counter's old value plus the lane's rank among them.  Lanes with equal keys are
-// matched by four ballots, one per key bit.  All lanes of the wave call it.
-__device__ __forceinline__ uint32_t wave_counted_add16(uint32_t* counters, uint32_t key, bool valid) {
+// ---------------------------------------------------------------- tile ranges of single draws
+// Each tile's range of the lists and its place in the scheduling order, both from cursors a wave takes
+// its share of at once: neither the ranges nor the tiles of a class need an order, so no workgroup
+// waits for another's counts.  (A scan over all counts took 12 us whatever the number of tiles.)
+__global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __restrict__ tile_count, uint32_t T, uint32_t N,
+                                                          uint32_t shift, uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
+                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ order) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   const int lane = __lane_id();
+  const uint32_t t = slot_tile(i, shift);
+  const bool valid = i < N && t < T;
+  const uint32_t n = valid ? tile_count[i] : 0u;
+  const uint32_t incl = wave_incl_scan(n);
+  const uint32_t all = static_cast<uint32_t>(__shfl(static_cast<int>(incl), 63, 64));
+  uint32_t base = 0;
+  if (lane == 0 && all) base = atomicAdd(&counters[CT_CURSOR], all);
+  // lanes of the same class, matched by one ballot per class bit
+  const uint32_t c = tile_class(n);
   uint64_t m = __ballot(valid);
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    const bool bit = ((key >> b) & 1u) != 0;
+    const bool bit = ((c >> b) & 1u) != 0;
     const uint64_t bal = __ballot(bit);
     m &= bit ? bal : ~bal;
   }
-  const uint64_t lt = (1ull << lane) - 1ull;
-  uint32_t old = 0;
-  if (valid && (m & lt) == 0) old = atomicAdd(&counters[key], static_cast<uint32_t>(__popcll(m)));
   const int leader = valid ? __builtin_ctzll(m) : lane;
-  old = static_cast<uint32_t>(__shfl(static_cast<int>(old), leader, 64));
-  return old + static_cast<uint32_t>(__popcll(m & lt));
-}
-
-// One workgroup: tile ranges from the totals (exclusive prefix, BUCKET_MAX_TILES tiles per step), the
-// tiles per record-count class, and, when `order` is given, the tiles' scheduling order: tiles of
-// class c after every tile of the classes before c, within a class in the atomics' order (tiles are
-// independent, so the order never changes a pixel).
-__global__ void __launch_bounds__(1024) tile_prefix_kernel(const uint32_t* __restrict__ tile_count, uint32_t T,
-                                                          uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
-                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ order) {
-  constexpr int PER = BUCKET_MAX_TILES / 1024;
-  __shared__ uint32_t wsum[16];
-  __shared__ uint32_t classes[16];
-  const uint32_t tid = threadIdx.x;
-  if (tid < 16) classes[tid] = 0;
-  uint32_t carry = 0;  // records of the tiles before this step
-  for (uint32_t base = 0; base < T; base += BUCKET_MAX_TILES) {
-    const uint32_t t0 = base + tid * PER;
-    uint32_t c[PER], sum = 0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      c[i] = load_or_zero(tile_count, t0 + i, T);
-      sum += c[i];
-    }
-    const uint32_t incl = wave_incl_scan(sum);
-    if (base) __syncthreads();  // the previous step's wave sums are read
-    if ((tid & 63) == 63) wsum[tid >> 6] = incl;
-    __syncthreads();
-    uint32_t run = carry + incl - sum, step = 0;
-    for (uint32_t w = 0; w < 16; ++w) {
-      if (w < (tid >> 6)) run += wsum[w];
-      step += wsum[w];
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      if (t0 + i < T) {
-        ts[t0 + i] = run;
-        te[t0 + i] = run + c[i];
-      }
-      run += c[i];
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) (void)wave_counted_add16(classes, tile_class(c[i]), t0 + i < T);
-    carry += step;
-  }
-  __syncthreads();
-  if (tid < 16) counters[CT_CLASS + tid] = classes[tid];
-  if (!order) return;
-  // classes[] becomes each class's next position
-  if (tid == 0) {
-    uint32_t b = 0;
-    for (int k = 0; k < 16; ++k) {
-      const uint32_t n = classes[k];
-      classes[k] = b;
-      b += n;
-    }
-  }
-  __syncthreads();
-  for (uint32_t base = 0; base < T; base += BUCKET_MAX_TILES) {
-    const uint32_t t0 = base + tid * PER;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const bool valid = t0 + i < T;
-      const uint32_t pos = wave_counted_add16(classes, tile_class(load_or_zero(tile_count, t0 + i, T)), valid);
-      if (valid) order[pos] = t0 + i;
-    }
+  uint32_t old = 0;
+  if (valid && leader == lane) old = atomicAdd(&counters[CT_CLASS + c], static_cast<uint32_t>(__popcll(m)));
+  const uint32_t at = static_cast<uint32_t>(__shfl(static_cast<int>(old), leader, 64)) +
+                      static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+  base = static_cast<uint32_t>(__shfl(static_cast<int>(base), 0, 64));
+  if (valid) {
+    ts[t] = base + incl - n;
+    te[t] = base + incl;
+    order[static_cast<size_t>(c) * T + at] = t;
   }
 }
-// The same for targets of at most PREFIX_MAX_TILES tiles, one workgroup per PREFIX_TILES tiles and
-// no communication between them: every workgroup reads all T tile totals (8 per thread at 1080p),
-// from which it takes the records of the tiles before its own, the tiles of each record-count class
-// in the whole target and before its own tiles, and writes its tiles' ranges and scheduling
-// positions.  The order is class by class (heaviest first), by tile within a class.
-constexpr uint32_t PREFIX_TILES = 1024;
-constexpr uint32_t PREFIX_MAX_TILES = 65536;
-__global__ void __launch_bounds__(1024) tile_prefix_par_kernel(const uint32_t* __restrict__ tile_count, uint32_t T,
-                                                              uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
-                                                              uint32_t* __restrict__ counters, uint32_t* __restrict__ order) {
-  __shared__ uint32_t w_all[16][16], w_before[16][16], w_mine[16][16];  // [wave][class]
-  __shared__ uint32_t w_rec[16], w_scan[16], c_base[16], s_start[16], s_pos[16][16];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, bx = blockIdx.x;
-  const uint32_t nj = (T + PREFIX_TILES - 1) / PREFIX_TILES;  // at most 64
-  // this lane's tiles per class, one 8-bit field per class (classes 0-7 in [0], 8-15 in [1]): all of
-  // them, and those before the workgroup's
-  unsigned long long all[2] = {0, 0}, before[2] = {0, 0};
-  uint32_t rec_before = 0, mine = 0;
-  for (uint32_t j0 = 0; j0 < nj; j0 += 8) {
-    uint32_t v[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const uint32_t i = (j0 + q) * PREFIX_TILES + tid;
-      v[q] = load_or_zero(tile_count, i, T);
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const uint32_t j = j0 + q;  // uniform
-      if (j >= nj) break;
-      const bool valid = j * PREFIX_TILES + tid < T;
-      const uint32_t c = tile_class(v[q]);
-      if (j < bx) rec_before += v[q];
-      if (j == bx) mine = v[q];
-      const unsigned long long one = valid ? 1ull << (8 * (c & 7)) : 0ull;
-      all[c >> 3] += one;
-      if (j < bx) before[c >> 3] += one;
-    }
-  }
-  const uint32_t t = bx * PREFIX_TILES + tid;
-  const bool mine_valid = t < T;
-  const uint32_t cm = tile_class(mine);
-  // rank among the wave's own tiles of the same class (four ballots, one per class bit)
-  uint64_t m = __ballot(mine_valid);
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const bool bit = ((cm >> b) & 1u) != 0;
-    const uint64_t bal = __ballot(bit);
-    m &= bit ? bal : ~bal;
-  }
-  const uint32_t rank = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
-  unsigned long long mine_f[2] = {0, 0};
-  mine_f[cm >> 3] = mine_valid ? 1ull << (8 * (cm & 7)) : 0ull;
-  // the wave's per-class sums: the 8-bit fields widened to 16 bits (4 classes per word, at most
-  // 64 lanes x 64 chunks per class), added over the wave
-  unsigned long long wa[4], wb[4], wm[4];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const unsigned long long lo = 0x00FF00FF00FF00FFull;
-    wa[2 * h] = all[h] & lo;
-    wa[2 * h + 1] = (all[h] >> 8) & lo;
-    wb[2 * h] = before[h] & lo;
-    wb[2 * h + 1] = (before[h] >> 8) & lo;
-    wm[2 * h] = mine_f[h] & lo;
-    wm[2 * h + 1] = (mine_f[h] >> 8) & lo;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      wa[w] += __shfl_xor(wa[w], off, 64);
-      wb[w] += __shfl_xor(wb[w], off, 64);
-      wm[w] += __shfl_xor(wm[w], off, 64);
-    }
-  // class k = 8h + 2f + e lives in word 2h + e, 16-bit field f (fields of a word: classes of one parity)
-  auto field = [](const unsigned long long (&w)[4], uint32_t k) -> uint32_t {
-    const bool h = (k >> 3) != 0, e = (k & 1) != 0;
-    const unsigned long long x = h ? (e ? w[3] : w[2]) : (e ? w[1] : w[0]);  // selects, no indexing
-    return static_cast<uint32_t>((x >> (16 * ((k & 7) >> 1))) & 0xFFFFull);
-  };
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) rec_before += static_cast<uint32_t>(__shfl_xor(static_cast<int>(rec_before), off, 64));
-  const uint32_t incl = wave_incl_scan(mine);
-  if (lane < 16) {
-    w_all[wave][lane] = field(wa, lane);
-    w_before[wave][lane] = field(wb, lane);
-    w_mine[wave][lane] = field(wm, lane);
-  }
-  if (lane == 0) w_rec[wave] = rec_before;
-  if (lane == 63) w_scan[wave] = incl;
-  __syncthreads();
-  // Per-wave and per-class bases, each a fixed-length sum over the 16 waves (unrolled, the loads
-  // issued together):
-  //   c_base[k]     tiles of classes < k in the target + tiles of class k before the workgroup's
-  //   s_start[w]    records of the tiles before the workgroup's + of waves < w's tiles
-  //   s_pos[w][k]   c_base[k] + this workgroup's class-k tiles in waves < w
-  if (tid < 64) {
-    const uint32_t k = tid & 15;
-    uint32_t tot = 0, bef = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      tot += w_all[w][k];
-      bef += w_before[w][k];
-    }
-    uint32_t below = tot;  // inclusive scan over the 16 classes, then exclusive
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-      const uint32_t y = static_cast<uint32_t>(__shfl_up(static_cast<int>(below), off, 16));
-      if (k >= static_cast<uint32_t>(off)) below += y;
-    }
-    below -= tot;
-    if (tid < 16) {
-      c_base[k] = below + bef;
-      if (bx == 0) counters[CT_CLASS + k] = tot;
-    }
-  } else if (tid < 80) {
-    const uint32_t w = tid - 64;
-    uint32_t rec = 0, pre = 0;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      rec += w_rec[v];
-      pre += static_cast<uint32_t>(v) < w ? w_scan[v] : 0u;
-    }
-    s_start[w] = rec + pre;
-  }
-  __syncthreads();
-  if (tid < 256) {
-    const uint32_t w = tid >> 4, k = tid & 15;
-    uint32_t pre = 0;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) pre += static_cast<uint32_t>(v) < w ? w_mine[v][k] : 0u;
-    s_pos[w][k] = c_base[k] + pre;
-  }
-  __syncthreads();
-  if (mine_valid) {
-    const uint32_t start = s_start[wave] + incl - mine;
-    ts[t] = start;
-    te[t] = start + mine;
-    order[s_pos[wave][cm] + rank] = t;
-  }
-}
+// The records to their tiles' lists: position = first record of the tile + rank in the tile.
+constexpr uint32_t SCATTER_PER_THREAD = 4;
 __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                           const uint32_t* __restrict__ count, uint32_t cap, uint32_t T,
-                                                           const uint32_t* __restrict__ ts, uint32_t* __restrict__ tile_cursor,
+                                                           const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ count,
+                                                           uint32_t cap, const uint32_t* __restrict__ ts,
                                                            uint32_t* __restrict__ vout) {
-  __shared__ uint32_t cnt[BUCKET_MAX_TILES];
-  __shared__ uint16_t touched[BUCKET_ITEMS];
-  __shared__ uint32_t ntouched;
   const uint32_t n = min(*count, cap);
-  const uint32_t b0 = blockIdx.x * BUCKET_ITEMS;
+  const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
   if (b0 >= n) return;
-  uint32_t k[BUCKET_PER_THREAD], rank[BUCKET_PER_THREAD];
-  tile_load_keys(keys, n, b0, k);
-  for (uint32_t r0 = 0; r0 < T; r0 += BUCKET_MAX_TILES) {
-    const uint32_t tn = min(T - r0, BUCKET_MAX_TILES);
-    if (r0) __syncthreads();  // the previous range's positions are consumed
-    tile_count_lds(k, rank, r0, tn, cnt, touched, &ntouched);
-    // this workgroup's range in each touched tile; cnt[t] becomes its first position
-    for (uint32_t i = threadIdx.x; i < ntouched; i += 256) {
-      const uint32_t t = touched[i];
-      cnt[t] = ts[r0 + t] + atomicAdd(&tile_cursor[r0 + t], cnt[t]);
+  uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
+#pragma unroll
+  for (uint32_t j = 0; j < SCATTER_PER_THREAD; ++j) {  // clamped indices: no branch per load
+    const uint32_t i = min(b0 + j * 256 + threadIdx.x, n - 1);
+    k[j] = keys[i];
+    v[j] = vals[i];
+    r[j] = ranks[i];
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < SCATTER_PER_THREAD; ++j) {
+    const uint32_t pos = ts[k[j]] + r[j];
+    if (b0 + j * 256 + threadIdx.x < n && pos < cap) vout[pos] = v[j];  // beyond cap: the draw is emitted again
+  }
+}
+
+// Each tile's list in ascending order (primitive order: a triangle is on a tile once), from `in` to
+// `out`, one workgroup per tile.  Lists of up to SORT_LDS records are sorted in LDS; a longer one is
+// taken in windows of consecutive values that hold at most SORT_LDS records each, found by a histogram
+// of its values that is narrowed until its first bucket fits.  Sorting the lists costs in-order draws a
+// pass over their records; two stable radix passes over all records (by tile) took 50 us of a
+// 32k-triangle draw at 1280x720.
+constexpr uint32_t SORT_LDS = 2048;
+__device__ __forceinline__ void sort_lds(uint32_t* a, uint32_t n) {
+  uint32_t m = 2;
+  while (m < n) m <<= 1;  // uniform
+  for (uint32_t i = n + threadIdx.x; i < m; i += 256) a[i] = 0xFFFFFFFFu;
+  for (uint32_t k = 2; k <= m; k <<= 1)
+    for (uint32_t j = k >> 1; j; j >>= 1) {
+      __syncthreads();
+      for (uint32_t t = threadIdx.x; t < m / 2; t += 256) {
+        const uint32_t i = ((t & ~(j - 1)) << 1) | (t & (j - 1));  // bit j clear
+        const uint32_t x = a[i], y = a[i + j];
+        if ((x > y) == ((i & k) == 0)) {
+          a[i] = y;
+          a[i + j] = x;
+        }
+      }
+    }
+  __syncthreads();
+}
+__global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
+                                                        const uint32_t* __restrict__ order, const uint32_t* __restrict__ counters,
+                                                        uint32_t cap, const uint32_t* __restrict__ in,
+                                                        uint32_t* __restrict__ out) {
+  __shared__ uint32_t a[SORT_LDS];
+  __shared__ uint32_t hist[256];
+  __shared__ uint32_t s_n, s_below, s_k;
+  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
+  const uint32_t t = scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x), t0 = ts[t], n = te[t] - t0, tid = threadIdx.x;
+  if (n <= SORT_LDS) {
+    if (n == 0) return;
+    for (uint32_t i = tid; i < n; i += 256) a[i] = in[t0 + i];
+    if (n > 1) sort_lds(a, n);
+    for (uint32_t i = tid; i < n; i += 256) out[t0 + i] = a[i];
+    return;
+  }
+  uint64_t lo = 0, hi = 1ull << 32;  // values in [lo, hi) are looked at; those below lo are written
+  uint32_t done = 0;
+  while (done < n) {
+    uint32_t shift = 0;  // at most 256 buckets of 1 << shift values
+    while (((hi - lo - 1) >> shift) > 255) ++shift;
+    hist[tid] = 0;
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += 256) {
+      const uint64_t v = in[t0 + i];
+      if (v >= lo && v < hi) atomicAdd(&hist[(v - lo) >> shift], 1u);
     }
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < BUCKET_PER_THREAD; ++j)
-      if (k[j] - r0 < tn) vout[cnt[k[j] - r0] + rank[j]] = vals[b0 + j * 256 + threadIdx.x];
+    if (tid == 0) {  // the leading buckets that fit together
+      uint32_t k = 0, sum = 0;
+      while (k < 256 && sum + hist[k] <= SORT_LDS) sum += hist[k++];
+      s_k = k;
+      s_below = sum;
+    }
+    __syncthreads();
+    const uint32_t k = s_k, m = s_below;
+    if (k == 0) {  // the first bucket alone is too long: look into it
+      if (shift == 0) return;  // not reached: a value is in a list once
+      hi = lo + (1ull << shift);
+      __syncthreads();
+      continue;
+    }
+    const uint64_t end = min(hi, lo + (static_cast<uint64_t>(k) << shift));
+    for (uint32_t i = tid; i < n; i += 256) {
+      const uint64_t v = in[t0 + i];
+      if (v >= lo && v < end) a[atomicAdd(&s_n, 1u)] = static_cast<uint32_t>(v);
+    }
+    __syncthreads();
+    if (m > 1) sort_lds(a, m);
+    for (uint32_t i = tid; i < m; i += 256) out[t0 + done + i] = a[i];
+    __syncthreads();
+    done += m;
+    lo = end;
+    hi = 1ull << 32;
   }
 }
 
-bool bucket_sort_applicable(const draw_params& P) { return P.gtiles_x > 0 && P.gtiles_y > 0; }
-bool launch_bucket_sort(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s) {
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-  if (!bucket_sort_applicable(P)) return false;
-  const uint32_t* count = B.counters + CT_TOTAL;
-  const uint32_t nblocks = std::max<uint32_t>((cap + BUCKET_ITEMS - 1) / BUCKET_ITEMS, 1);
-  hipLaunchKernelGGL(tile_count_kernel, dim3(nblocks), dim3(256), 0, s, B.keys[0], count, cap, T, B.tile_count);
-  if (order && T <= PREFIX_MAX_TILES)
-    hipLaunchKernelGGL(tile_prefix_par_kernel, dim3((T + PREFIX_TILES - 1) / PREFIX_TILES), dim3(1024), 0, s, B.tile_count, T,
-                       B.tstart, B.tend, B.counters, order);
-  else
-    hipLaunchKernelGGL(tile_prefix_kernel, dim3(1), dim3(1024), 0, s, B.tile_count, T, B.tstart, B.tend, B.counters, order);
-  hipLaunchKernelGGL(tile_scatter_kernel, dim3(nblocks), dim3(256), 0, s, B.keys[0], B.vals[0], count, cap, T, B.tstart,
-                     B.tile_count + T, B.vals[1]);
-  return true;
-}
-
-__global__ void tile_range_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t T, uint32_t* __restrict__ ts,
-                                  uint32_t* __restrict__ te) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  // T == 0: the ranges were cleared beforehand, only the non-empty tiles are written
-  uint32_t k = keys[i];
-  if (i == 0 && T) {
-    for (uint32_t t = 0; t < k; ++t) ts[t] = te[t] = 0;
-  }
-  if (i == 0 || keys[i - 1] != k) ts[k] = i;
-  if (i == n - 1 || keys[i + 1] != k) {
-    te[k] = i + 1;
-    const uint32_t next = !T ? k + 1 : ((i == n - 1) ? T : keys[i + 1]);
-    for (uint32_t t = k + 1; t < next; ++t) ts[t] = te[t] = i + 1;
-  }
+  if (!T) return;
+  const uint32_t N = tile_slots(T), shift = tile_slot_shift(T);
+  hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
+                     B.counters, order);
+  const uint32_t per = 256 * SCATTER_PER_THREAD;
+  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max<uint32_t>(cap, 1) + per - 1) / per), dim3(256), 0, s, B.keys[0],
+                     B.vals[0], B.keys[1], B.counters + CT_TOTAL, cap, B.tstart, B.vals[1]);
+  if (sorted) hipLaunchKernelGGL(tile_sort_kernel, dim3(T), dim3(256), 0, s, B.tstart, B.tend, order,
+                                 B.counters, cap, B.vals[1], B.vals[0]);
 }
 
 // Scheduling order of the GPU tiles, heaviest first so that the longest tiles start early.  Tiles
@@ -1819,46 +1665,10 @@ __global__ void __launch_bounds__(1024) tile_order_kernel(const uint32_t* __rest
   tile_order_body(ts, te, T, order);
 }
 
-__global__ void tile_class_count_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te, uint32_t T,
-                                        uint32_t* __restrict__ counters) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < T) (void)wave_counted_add(counters + CT_CLASS, tile_class(te[t] - ts[t]));
-}
-// Tiles of class c take the positions after every tile of the classes before c; within a class the
-// order is the atomics' (tiles are independent, so the order never changes a pixel).
-__global__ void tile_class_order_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te, uint32_t T,
-                                        uint32_t* __restrict__ counters, uint32_t* __restrict__ order) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T) return;
-  const uint32_t c = tile_class(te[t] - ts[t]);
-  uint32_t base = 0;
-  for (uint32_t k = 0; k < c; ++k) base += counters[CT_CLASS + k];
-  order[base + wave_counted_add(counters + CT_CURSOR, c)] = t;
-}
-void launch_tile_order(const draw_params& P, const draw_buffers& B, uint32_t* order, bool counted, hipStream_t s) {
-  const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-  if (!T) return;
-  if (!counted) hipLaunchKernelGGL(tile_class_count_kernel, dim3((T + 255) / 256), dim3(256), 0, s, B.tstart, B.tend, T, B.counters);
-  hipLaunchKernelGGL(tile_class_order_kernel, dim3((T + 255) / 256), dim3(256), 0, s, B.tstart, B.tend, T, B.counters, order);
-}
-
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s) {
   if (n) hipLaunchKernelGGL(fill_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
 }
 
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, int which, uint32_t n, hipStream_t s) {
-  uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-  if (!T) return;
-  if (n < 4 * T) {  // sparse records: clear every range first, so no thread walks a long empty run
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((T + 255) / 256), dim3(256), 0, s, B.tstart, T, 0u);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((T + 255) / 256), dim3(256), 0, s, B.tend, T, 0u);
-    if (n) hipLaunchKernelGGL(tile_range_kernel, dim3((n + 255) / 256), dim3(256), 0, s, B.keys[which], n, 0u, B.tstart, B.tend);
-    return;
-  }
-  hipLaunchKernelGGL(tile_range_kernel, dim3((n + 255) / 256), dim3(256), 0, s, B.keys[which], n, T, B.tstart, B.tend);
-}
-
-// ============================================================== host launchers
 void launch_reduce_partials(const unsigned long long* partial, uint32_t n, unsigned long long* stats, int slot, hipStream_t s) {
   hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(256), 0, s, partial, n, stats, slot);
 }
@@ -1869,33 +1679,25 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
                      static_cast<uint32_t>(ntiles));
 }
 
-void launch_setup(const draw_params& P, const draw_buffers& B, hipStream_t s) {
+void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s) {
   if (P.prim_count == 0) return;
   dim3 grid((P.prim_count + 255) / 256);
-#define SRX_SETUP(NA) \
-  hipLaunchKernelGGL(setup_kernel<NA>, grid, dim3(256), 0, s, P, B.vbuf, B.tri_rec, B.tri_attr, B.cnt, B.clip_flag, B.counters, \
-                     B.wide_list, B.partial, B.bsum, B.pairs)
+  const uint32_t shift = tile_slot_shift(static_cast<uint32_t>(P.gtiles_x * P.gtiles_y));
+#define SRX_SETUP(NA) hipLaunchKernelGGL(setup_kernel<NA>, grid, dim3(256), 0, s, P, B, capacity, shift)
   SRX_NA_DISPATCH(P.nattr, SRX_SETUP)
 #undef SRX_SETUP
-  if (P.count_stats)
-    launch_reduce_partials(B.partial, grid.x, B.stats, ST_CPRIMITIVES, s);
+  if (P.count_stats) launch_reduce_partials(B.partial, grid.x, B.stats, ST_CPRIMITIVES, s);
 }
 
-void launch_clip(const draw_params& P, const draw_buffers& B, hipStream_t s) {
+// Workgroups of the clip launch: enough to fill the GPU four deep when every triangle is on the wide
+// list, few enough that a draw with none (they return at once) loses nothing measurable.
+void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s) {
   if (P.prim_count == 0) return;
-  dim3 grid(std::min<uint32_t>((P.prim_count + 255) / 256, 256));  // up to 1024 waves in 256-lane workgroups
-#define SRX_CLIP(NA)                                                                                                     \
-  hipLaunchKernelGGL(clip_kernel<NA>, grid, dim3(256), 0, s, P, B.vbuf, B.tri_rec, B.tri_attr, B.cnt, B.clip_flag, B.clip_slot, \
-                     B.clip_verts, B.clip_hdr, B.clip_capacity, B.counters, B.stats, B.wide_list, B.bsum)
+  dim3 grid(std::min<uint32_t>((P.prim_count + 3) / 4, 1024));
+  const uint32_t shift = tile_slot_shift(static_cast<uint32_t>(P.gtiles_x * P.gtiles_y));
+#define SRX_CLIP(NA) hipLaunchKernelGGL(clip_kernel<NA>, grid, dim3(256), 0, s, P, B, capacity, shift)
   SRX_NA_DISPATCH(P.nattr, SRX_CLIP)
 #undef SRX_CLIP
-}
-
-void launch_emit(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s) {
-  const uint32_t n = P.prim_count;
-  if (!n) return;
-  hipLaunchKernelGGL(emit_kernel, dim3((n + 255) / 256), dim3(256), 0, s, P, B.tri_rec, B.cnt, B.bsum, B.pairs,
-                     capacity, B.keys[0], B.vals[0]);
 }
 
 // ============================================================== clears, resolve, mip generation
@@ -2045,16 +1847,14 @@ template <int NA>
 __global__ void __launch_bounds__(256) setup_batch_kernel(const batch_job* __restrict__ jobs, stage_map m) {
   uint32_t lb, nb;
   const batch_job& J = jobs[stage_job(m, lb, nb)];
-  setup_body<NA>(J.P, J.B.vbuf, J.B.tri_rec, J.B.tri_attr, J.B.cnt, J.B.clip_flag, J.B.counters, J.B.wide_list, J.B.partial,
-                 nullptr, nullptr, lb);
+  setup_count_body<NA>(J.P, J.B, lb);
 }
 
 template <int NA>
 __global__ void clip_batch_kernel(const batch_job* __restrict__ jobs, stage_map m) {
   uint32_t lb, nb;
   const batch_job& J = jobs[stage_job(m, lb, nb)];
-  clip_body<NA>(J.P, J.B.vbuf, J.B.tri_rec, J.B.tri_attr, J.B.cnt, J.B.clip_flag, J.B.clip_slot, J.B.clip_verts,
-                J.B.clip_hdr, J.B.clip_capacity, J.B.counters, J.B.stats, J.B.wide_list, nullptr, lb, nb);
+  clip_count_body<NA>(J.P, J.B, lb, nb);
 }
 
 // The job's counts are followed by the next job's first scanned count (or the batch total): the

@@ -86,10 +86,15 @@ __global__ void __launch_bounds__(256) raster_kernel(draw_params P, const ps_sam
                                                       const uint32_t* __restrict__ order, const uint32_t* __restrict__ vals,
                                                       const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
                                                       const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
-                                                      uint32_t* __restrict__ vis, unsigned long long* __restrict__ partial) {
+                                                      uint32_t* __restrict__ vis, unsigned long long* __restrict__ partial,
+                                                      const uint32_t* __restrict__ counters, uint32_t cap) {
+  if (counters[CT_TOTAL] > cap) {  // records were dropped: the draw is emitted again
+    if (P.count_stats) block_partial(partial, 0ull);
+    return;
+  }
   extern __shared__ prim_lds lds[];
   const int G = P.gt, QW = G / 2;
-  const int gtile = order[blockIdx.x];
+  const int gtile = static_cast<int>(scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x));
   const int gx = gtile % P.gtiles_x, gy = gtile / P.gtiles_x;
   const int tid = threadIdx.x, nthreads = blockDim.x;
   const int qx = tid % QW, qy = tid / QW;
@@ -506,13 +511,13 @@ void launch_raster(const draw_params& P, const draw_buffers& B, int which, hipSt
   do {                                                                                                               \
     if (vis)                                                                                                         \
       hipLaunchKernelGGL((raster_kernel<NA, S, true>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order, B.vals[which], \
-                         B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                                 \
+                         B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial, B.counters, B.list_cap);                                 \
     else if (sasl)                                                                                                   \
       hipLaunchKernelGGL((raster_kernel<NA, S, false, true>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order, \
-                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                  \
+                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial, B.counters, B.list_cap);                  \
     else                                                                                                             \
       hipLaunchKernelGGL((raster_kernel<NA, S, false>), dim3(T), dim3(threads), lds, s, P, B.samplers, B.order,      \
-                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial);                  \
+                         B.vals[which], B.tstart, B.tend, B.tri_rec, B.tri_attr, B.vis, B.partial, B.counters, B.list_cap);                  \
   } while (0)
 #define SRX_RASTER(NA)                     \
   switch (P.samples) {                     \

@@ -226,16 +226,12 @@ struct draw_scratch {
 
 static size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-// Bytes the record-sized buffers take for `records` binned records (keys/values twice, the sort
-// histogram and its scan space, the tile order and the visibility work table), in take() order.
-static size_t record_scratch_bytes(uint32_t P3, uint32_t T, int samples, bool vis_tables, uint64_t records) {
+// Bytes the record-sized buffers take for `records` binned records (keys, values and ranks as emitted,
+// values by tile, and the visibility work table), in take() order.
+static size_t record_scratch_bytes(uint32_t T, int samples, bool vis_tables, uint64_t records) {
   const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(records, 0xFFFFFFFFu));
   const size_t rn = std::max<uint32_t>(n, 1);
-  const uint32_t nblocks = (std::max(n, T) + 4095) / 4096;
-  const size_t hist_n = std::max<size_t>(static_cast<size_t>(256) * std::max<uint32_t>(nblocks, 1), bucket_hist_size(T, n));
-  size_t b = 2 * align256(rn * 4) + 2 * align256(rn * 4) + align256(hist_n * 4) +
-             align256(std::max(scan_tmp_size(P3), scan_tmp_size(static_cast<uint32_t>(hist_n))) * 4) +
-             align256(std::max<uint32_t>(T, 1) * 4);
+  size_t b = 4 * align256(rn * 4);
   if (vis_tables) {
     uint32_t ne, nm, nsl;
     vis_table_bounds(T, n, &ne, &nm, &nsl);
@@ -292,17 +288,16 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     }
     P.sasl = prog_d;
   }
-  RCHK(X.take(r->cnt, P3, B.cnt));
   RCHK(X.take(r->clip_flag, primcnt, B.clip_flag));
   RCHK(X.take(r->clip_slot, primcnt, B.clip_slot));
   RCHK(X.take(r->wide, primcnt, B.wide_list));
-  RCHK(X.take(r->bsum, (static_cast<size_t>(primcnt) + 255) / 256, B.bsum));
-  RCHK(X.take(r->pairs, primcnt, B.pairs));
-  RCHK(X.take(r->scan_tmp, scan_tmp_size(P3), B.scan_tmp));
-  RCHK(X.take(r->partial, std::max<size_t>(T, (primcnt + 255) / 256) + 1, B.partial));
+  RCHK(X.take(r->partial, std::max<size_t>(T, (primcnt + 255) / 256) + ST_COUNT, B.partial));
   RCHK(X.take(r->tstart, std::max<uint32_t>(T, 1), B.tstart));
   RCHK(X.take(r->tend, std::max<uint32_t>(T, 1), B.tend));
-  RCHK(X.take(r->tile_count, 2 * static_cast<size_t>(std::max<uint32_t>(T, 1)), B.tile_count));
+  RCHK(X.take(r->tile_count, std::max<uint32_t>(tile_slots(T), 1), B.tile_count));
+  uint32_t* order = nullptr;
+  RCHK(X.take(r->order, static_cast<size_t>(TILE_CLASSES) * std::max<uint32_t>(T, 1), order));
+  B.order = order;
   // clipping capacity for every primitive, so no read-back decides whether clipping runs
   RCHK(X.take(r->clip_verts, static_cast<size_t>(primcnt) * 5 * (nout + 1), B.clip_verts));
   RCHK(X.take(r->clip_hdr, primcnt, B.clip_hdr));
@@ -313,38 +308,37 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   // statistics queries need the in-order walk (ps_invocations counts early-Z passes as they happen)
   const bool counting = P.count_stats != 0;
   const bool vis_tables = vis_pass && !counting;
-  // Records are emitted before their count is read back, so the read-back overlaps the emission.
-  // Allocating draws emit into a grow-only buffer sized from the previous draw and repeat the
-  // emission when it was too small; a fixed region gets the largest record capacity whose
-  // record-sized buffers all fit, and a draw with more records is refused.
-  uint32_t capacity, sort_cap;  // records the buffer holds; records the early sort is sized for
+  // The tiles' lists are formed before the record count is read back.  Allocating draws emit into
+  // grow-only buffers sized from the previous draws and repeat the emission when they were too small; a
+  // fixed region gets the largest record capacity whose record-sized buffers all fit, and a draw with
+  // more records is refused.
+  uint32_t capacity, sized;  // records the buffers hold; records the lists are formed for
+  auto take_records = [&](uint32_t n) -> int32_t {
+    RCHK(X.take(r->keys0, n, B.keys[0]));
+    RCHK(X.take(r->vals0, n, B.vals[0]));
+    RCHK(X.take(r->keys1, n, B.keys[1]));
+    return X.take(r->vals1, n, B.vals[1]);
+  };
   if (!fixed) {
     uint32_t recent = 0;
     for (uint32_t v : r->recent_records) recent = std::max(recent, v);
     const uint64_t want = std::max<uint64_t>(std::max<uint64_t>(recent + static_cast<uint64_t>(recent) / 4, static_cast<uint64_t>(P3) + T),
                                              1u << 16);
-    const uint32_t guess = static_cast<uint32_t>(std::min<uint64_t>(want, 0xFFFFFFF0u));
-    if (r->keys0.cap < guess) {
-      RCHK(ensure(r, r->keys0, guess));
-      RCHK(ensure(r, r->vals0, guess));
-    }
-    B.keys[0] = r->keys0.p;
-    B.vals[0] = r->vals0.p;
-    capacity = static_cast<uint32_t>(std::min<size_t>(r->keys0.cap, r->vals0.cap));
-    sort_cap = std::min(capacity, guess);
+    sized = static_cast<uint32_t>(std::min<uint64_t>(want, 0xFFFFFFF0u));
+    RCHK(take_records(sized));
+    const size_t held = std::min(std::min(r->keys0.cap, r->vals0.cap), std::min(r->keys1.cap, r->vals1.cap));
+    capacity = static_cast<uint32_t>(std::min<size_t>(held, 0xFFFFFFF0u));
   } else {
     const size_t room = fixed->bytes - std::min(fixed->bytes, align256(X.used));
     uint64_t lo = 0, hi = 0xFFFFFFFEu;  // largest capacity whose buffers fit
     while (lo < hi) {
       const uint64_t mid = (lo + hi + 1) / 2;
-      if (record_scratch_bytes(P3, T, samples, vis_tables, mid) <= room) lo = mid;
+      if (record_scratch_bytes(T, samples, vis_tables, mid) <= room) lo = mid;
       else hi = mid - 1;
     }
     if (lo == 0) return fail(SRX_OUT_OF_MEMORY, "the draw's scratch exceeds the no-allocation region");
-    capacity = static_cast<uint32_t>(lo);
-    sort_cap = capacity;
-    RCHK(X.take(r->keys0, capacity, B.keys[0]));
-    RCHK(X.take(r->vals0, capacity, B.vals[0]));
+    capacity = sized = static_cast<uint32_t>(lo);
+    RCHK(take_records(capacity));
   }
 
   bool prof = r->profiling() && !fixed;  // event creation may allocate: no-allocation draws are not profiled
@@ -379,18 +373,15 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     }
   }
   mark(0);
-  launch_vs(P, B.vbuf, B.counters, B.tile_count, 2 * static_cast<size_t>(T), s);
+  launch_vs(P, B.vbuf, B.counters, B.tile_count, tile_slots(T), s);
   mark(1);
-  // setup leaves each 256-primitive block's record total in bsum; the clip launch (which returns at
-  // once on the device when setup flagged no primitive) adds the counts it makes and writes the
-  // draw's total, from which the emission takes every triangle's first record: no scan runs
-  launch_setup(P, B, s);
-  launch_clip(P, B, s);
+  // setup and the clip launch emit the draw's records and count them per tile
+  launch_setup(P, B, capacity, s);
+  launch_clip(P, B, capacity, s);
   mark(2);
   mark(3);
-  // the counters are final after the clip launch: their read-back overlaps the emission
+  // the counters are final after the clip launch: their read-back overlaps the tiles' lists
   HIPCHK(hipEventRecord(r->ev_counted, s));
-  launch_emit(P, B, capacity, s);
   // A target's pending full clear is applied by the visibility or in-order pass as it writes the
   // target, when that pass covers the whole target (it then reads nothing back); the others run
   // here, while the record count travels to the host.
@@ -410,92 +401,66 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   if (!eat_ds) RCHK(run_pending_clear(dst, s));
   RCHK(start_counter_read(r));
   const bool order_free = vis_tables && vis_applicable(P);  // tile lists need no primitive order
-  // record-sized buffers of the sort, for `sized` records
-  uint32_t sized = 0;
-  auto take_sort_buffers = [&](uint32_t n) -> int32_t {
-    sized = n;
-    const uint32_t nblocks = (std::max(n, T) + 4095) / 4096;
-    const size_t hist_n = std::max<size_t>(static_cast<size_t>(256) * std::max<uint32_t>(nblocks, 1), bucket_hist_size(T, n));
-    RCHK(X.take(r->keys1, std::max<uint32_t>(n, 1), B.keys[1]));
-    RCHK(X.take(r->vals1, std::max<uint32_t>(n, 1), B.vals[1]));
-    RCHK(X.take(r->hist, hist_n, B.hist));
-    RCHK(X.take(r->scan_tmp, std::max(scan_tmp_size(P3), scan_tmp_size(static_cast<uint32_t>(hist_n))), B.scan_tmp));
+  if (eat_color) {
+    P.clear_color = 1;
+    for (int k = 0; k < 4; ++k) P.clear_rgba[k] = (&ct0->pend.color.x)[k];
+  }
+  if (eat_ds) {
+    P.clear_ds = 1;
+    P.clear_depth = dst->pend.depth;
+    P.clear_stencil = dst->pend.stencil;
+  }
+  // The lists and the raster pass are queued for the buffers' expected size before the count reaches the
+  // host, so the GPU never waits for it; with more records the raster pass returns at once and both are
+  // queued again.
+  const int which = order_free ? 1 : 0;
+  bool fused = false;
+  auto raster = [&]() -> int32_t {
+    if (vis_tables) {
+      uint32_t ne, nm, nsl;
+      vis_table_bounds(T, sized, &ne, &nm, &nsl);
+      RCHK(X.take(r->vis_entries, ne, B.vis_entries));
+      RCHK(X.take(r->vis_merges, nm, B.vis_merges));
+      RCHK(X.take(r->vis_counts, 4, B.vis_counts));
+      RCHK(X.take(r->vis_partial, static_cast<size_t>(nsl) * 256 * samples, B.vis_partial));
+    }
+    B.list_cap = sized;
+    launch_tile_lists(P, B, sized, order, !order_free, s);
+    mark(4);
+    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, s);
+    if (!fused) {
+      if (inorder_applicable(P)) launch_inorder(P, B, which, s);
+      else launch_raster(P, B, which, s);
+    }
+    mark(5);
     return SRX_OK;
   };
-  uint32_t* order = nullptr;
-  // Order-free draws sort their records before the count reaches the host: the sort is sized for the
-  // record buffer's capacity and reads the count on the device, and only a count beyond the
-  // capacity makes the draw emit and sort again.
-  bool bucketed = false, early = false;
-  if (order_free && bucket_sort_applicable(P)) {
-    early = true;
-    RCHK(take_sort_buffers(sort_cap));
-    RCHK(X.take(r->order, std::max<uint32_t>(T, 1), order));
-    bucketed = launch_bucket_sort(P, B, sort_cap, order, s);
-  }
+  RCHK(raster());
   uint32_t ctr[CT_COUNT];
   RCHK(finish_counter_read(r, ctr));
   if (ctr[CT_CLIP_OVERFLOW]) return fail(SRX_OUT_OF_MEMORY, "clip buffer overflow");
   const uint32_t total = ctr[CT_TOTAL];
   if (fixed && total > capacity)
     return fail(SRX_OUT_OF_MEMORY, "the draw's binned records exceed the no-allocation region");
-  if (!fixed) {
-    r->recent_records[r->recent_next++ % 8] = total;
-    if (total > capacity) {
-      RCHK(ensure(r, r->keys0, total));
-      RCHK(ensure(r, r->vals0, total));
-      B.keys[0] = r->keys0.p;
-      B.vals[0] = r->vals0.p;
-      launch_emit(P, B, total, s);
+  if (!fixed) r->recent_records[r->recent_next++ % 8] = total;
+  if (total > sized) {
+    if (total > capacity) {  // emit again into larger buffers, counting no statistics a second time
+      RCHK(take_records(total));
+      launch_fill_u32(B.counters, CT_COUNT, 0u, s);
+      launch_fill_u32(B.tile_count, tile_slots(T), 0u, s);
+      draw_params Pe = P;
+      draw_buffers Be = B;
+      Pe.count_stats = 0;
+      Be.stats = B.partial;
+      launch_setup(Pe, Be, total, s);
+      launch_clip(Pe, Be, total, s);
     }
+    sized = total;
+    launch_fill_u32(B.counters + CT_CURSOR, CT_COUNT - CT_CURSOR, 0u, s);
+    RCHK(raster());
   }
-  if (total > sort_cap) bucketed = false;  // the early sort saw only part of the records
-  int which = 1;
-  if (!bucketed || !order) {
-    // the early sort's tile counts and classes are counted again below
-    if (early) {
-      launch_fill_u32(B.counters + CT_CLASS, CT_COUNT - CT_CLASS, 0u, s);
-      launch_fill_u32(B.tile_count, 2 * T, 0u, s);
-    }
-    // sized for the capacity on a fixed region (the layout the capacity was chosen for), else for the count
-    RCHK(take_sort_buffers(fixed ? capacity : total));
-    RCHK(X.take(r->order, std::max<uint32_t>(T, 1), order));
-    bucketed = order_free && launch_bucket_sort(P, B, std::max<uint32_t>(total, 1), order, s);
-    if (!bucketed) {
-      int bits = 1;
-      while ((1u << bits) < T) ++bits;
-      which = launch_sort(B, total, bits, s);
-      launch_tile_ranges(P, B, which, total, s);
-      launch_tile_order(P, B, order, false, s);
-    }
-  }
-  B.order = order;
-  mark(4);
-  if (vis_tables) {
-    uint32_t ne, nm, nsl;
-    vis_table_bounds(T, sized, &ne, &nm, &nsl);
-    RCHK(X.take(r->vis_entries, ne, B.vis_entries));
-    RCHK(X.take(r->vis_merges, nm, B.vis_merges));
-    RCHK(X.take(r->vis_counts, 4, B.vis_counts));
-    RCHK(X.take(r->vis_partial, static_cast<size_t>(nsl) * 256 * samples, B.vis_partial));
-  }
-  if (eat_color) {
-    P.clear_color = 1;
-    for (int k = 0; k < 4; ++k) P.clear_rgba[k] = (&ct0->pend.color.x)[k];
-    RCHK(run_pending_clear(ct0, s, true));
-  }
-  if (eat_ds) {
-    P.clear_ds = 1;
-    P.clear_depth = dst->pend.depth;
-    P.clear_stencil = dst->pend.stencil;
-    RCHK(run_pending_clear(dst, s, true));
-  }
-  const bool fused = vis_tables && launch_vis(P, B, which, needs_shading(P), total, s);
-  if (!fused) {
-    if (inorder_applicable(P)) launch_inorder(P, B, which, s);
-    else launch_raster(P, B, which, s);
-  }
-  mark(5);
+  if (eat_color) RCHK(run_pending_clear(ct0, s, true));
+  if (eat_ds) RCHK(run_pending_clear(dst, s, true));
   // the in-order kernel defers shading (to shade_kernel) only for early-Z draws
   // deferred shading: the in-order kernel's early-Z winners, or a SASL shader over vis_kernel's winners
   if (vis_pass && needs_shading(P) && ((!fused && P.early_z) || (fused && P.ps_id == PS_SASL))) {
@@ -521,8 +486,9 @@ renderer_obj::~renderer_obj() {
   fr(vbuf); fr(tri_rec); fr(tri_attr); fr(clip_verts); fr(samplers_d); fr(vis);
   if (samplers_h) (void)hipHostFree(samplers_h);
   if (sasl_h) (void)hipHostFree(sasl_h);
-  if (sasl_d) (void)hipFree(sasl_d); fr(cnt); fr(keys0); fr(keys1); fr(vals0); fr(vals1);
-  fr(tstart); fr(tend); fr(hist); fr(scan_tmp); fr(clip_hdr); fr(counters); fr(clip_flag); fr(clip_slot); fr(partial); fr(order); fr(tile_count); fr(wide); fr(bsum); fr(pairs); fr(vis_entries); fr(vis_merges); fr(vis_counts); fr(vis_partial);
+  if (sasl_d) (void)hipFree(sasl_d);
+  fr(keys0); fr(keys1); fr(vals0); fr(vals1);
+  fr(tstart); fr(tend); fr(clip_hdr); fr(counters); fr(clip_flag); fr(clip_slot); fr(partial); fr(order); fr(tile_count); fr(wide); fr(vis_entries); fr(vis_merges); fr(vis_counts); fr(vis_partial);
   if (stats_d) (void)hipFree(stats_d);
   if (pinned) (void)hipHostFree(pinned);
   if (map_host) (void)hipHostFree(map_host);

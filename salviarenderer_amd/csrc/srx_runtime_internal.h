@@ -382,12 +382,10 @@ struct renderer_obj : object {
   sasl_program* sasl_h = nullptr;
   sasl_program sasl_last{};
   bool sasl_valid = false;
-  dev_array<uint32_t> cnt, keys0, keys1, vals0, vals1, tstart, tend, hist, scan_tmp, clip_hdr, counters, vis;
+  dev_array<uint32_t> keys0, keys1, vals0, vals1, tstart, tend, clip_hdr, counters, vis;
   dev_array<uint32_t> order;  // GPU tile scheduling order
-  dev_array<uint32_t> tile_count;  // per-tile record counts and cursors of the counting sort
-  dev_array<uint32_t> wide;   // triangles counted by wave
-  dev_array<uint32_t> bsum;   // records per 256-primitive block
-  dev_array<uint4> pairs;     // setup's first four records of each primitive
+  dev_array<uint32_t> tile_count;  // records per tile
+  dev_array<uint32_t> wide;   // triangles whose records the clip launch emits
   dev_array<uint4> vis_entries, vis_merges;  // visibility work table
   dev_array<uint32_t> vis_counts;
   dev_array<unsigned long long> vis_partial;
@@ -397,7 +395,7 @@ struct renderer_obj : object {
   unsigned long long* stats_d = nullptr;
   uint32_t* pinned = nullptr;  // host staging for counter read-back (CT_COUNT words)
   std::vector<ref<surface_obj>> pending;  // surfaces holding a pending clear issued here
-  // the counters are read back on `side` (default priority) while the main stream emits records
+  // the counters are read back on `side` (default priority) while the main stream forms the tile lists
   hipStream_t side = nullptr;
   hipEvent_t ev_counted = nullptr, ev_read = nullptr;
   // binned records of the last draws; their maximum sizes the next draw's record buffer, so that
@@ -466,13 +464,13 @@ inline int gpu_tile_size() {
 // main stream), on the side stream, so that work queued after ev_counted overlaps it.
 inline int32_t start_counter_read(renderer_obj* r) {
   HIPCHK(hipStreamWaitEvent(r->side, r->ev_counted, 0));
-  HIPCHK(hipMemcpyAsync(r->pinned, r->counters.p, CT_CLASS * sizeof(uint32_t), hipMemcpyDeviceToHost, r->side));
+  HIPCHK(hipMemcpyAsync(r->pinned, r->counters.p, CT_COUNT * sizeof(uint32_t), hipMemcpyDeviceToHost, r->side));
   HIPCHK(hipEventRecord(r->ev_read, r->side));
   return SRX_OK;
 }
 inline int32_t finish_counter_read(renderer_obj* r, uint32_t* out) {
   HIPCHK(hipEventSynchronize(r->ev_read));
-  for (int i = 0; i < CT_COUNT; ++i) out[i] = i < CT_CLASS ? r->pinned[i] : 0u;
+  for (int i = 0; i < CT_COUNT; ++i) out[i] = r->pinned[i];
   return SRX_OK;
 }
 

@@ -24,13 +24,18 @@ constexpr uint32_t VIS_PART = 256;
 __global__ void __launch_bounds__(1024) vis_table_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
                                                          const uint32_t* __restrict__ order, uint32_t T,
                                                          uint4* __restrict__ entries, uint4* __restrict__ merges,
-                                                         uint32_t* __restrict__ counts) {
+                                                         uint32_t* __restrict__ counts, const uint32_t* __restrict__ counters,
+                                                         uint32_t cap) {
+  if (counters[CT_TOTAL] > cap) {  // records were dropped: the draw is emitted again
+    if (threadIdx.x < 3) counts[threadIdx.x] = 0;
+    return;
+  }
   __shared__ uint32_t wtot[3][16];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t per = (T + 1023) / 1024, p0 = tid * per, p1 = min(T, p0 + per);
   uint32_t c[3] = {0, 0, 0};  // blocks, partial slots, merges in this thread's segment of `order`
   for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = order[p], n = te[t] - ts[t];
+    const uint32_t t = scheduled_tile(order, counters + CT_CLASS, T, p), n = te[t] - ts[t];
     const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
     c[0] += parts;
     if (parts > 1) { c[1] += parts; c[2] += 1; }
@@ -55,7 +60,7 @@ __global__ void __launch_bounds__(1024) vis_table_kernel(const uint32_t* __restr
   }
   uint32_t b = base[0], sl = base[1], m = base[2];
   for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = order[p], n = te[t] - ts[t];
+    const uint32_t t = scheduled_tile(order, counters + CT_CLASS, T, p), n = te[t] - ts[t];
     const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
     for (uint32_t k = 0; k < parts; ++k) entries[b + k] = make_uint4(t, k, parts, sl);
     b += parts;
@@ -320,7 +325,8 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
                                          const uint32_t* __restrict__ vals, const uint32_t* __restrict__ tstart,
                                          const uint32_t* __restrict__ tend, const float4* __restrict__ tri_rec,
                                          const float4* __restrict__ tri_attr, const ps_samplers* __restrict__ SM,
-                                         uint32_t bx, uint32_t* __restrict__ wout = nullptr) {
+                                         uint32_t bx, uint32_t* __restrict__ wout = nullptr,
+                                         const uint32_t* __restrict__ classes = nullptr) {
   static_assert(GT == 8 || GT == 16 || GT == 32, "GPU tile side");
   constexpr int PX = GT * GT;       // pixels per GPU tile
   constexpr int NBS = GT / 4;       // 4x4 blocks per side
@@ -343,7 +349,8 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
   int gtile;
   uint32_t part = 0, parts = 1, slot = 0;
   if (entries == nullptr) {  // whole tiles in `order`
-    gtile = static_cast<int>(order[bx]);
+    gtile = static_cast<int>(classes ? scheduled_tile(order, classes, static_cast<uint32_t>(P.gtiles_x * P.gtiles_y), bx)
+                                     : order[bx]);
   } else if (pass == 0) {
     if (bx >= counts[0]) return;
     const uint4 en = entries[bx];
@@ -659,9 +666,11 @@ __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, 
                                                    const uint32_t* __restrict__ vals,
                                                    const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
                                                    const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
-                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
+                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout,
+                                                   const uint32_t* __restrict__ counters, uint32_t cap) {
+  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
   vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, pass, order, entries, merges, counts, partial, vals, tstart, tend,
-                                              tri_rec, tri_attr, SM, blockIdx.x, wout);
+                                              tri_rec, tri_attr, SM, blockIdx.x, wout, counters + CT_CLASS);
 }
 
 
@@ -713,14 +722,14 @@ bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool sha
   if (!shade) {
     vis_table_bounds(T, records, &ne, &nm, &nsl);
     hipLaunchKernelGGL(vis_table_kernel, dim3(1), dim3(1024), 0, s, B.tstart, B.tend, B.order, T, B.vis_entries,
-                       B.vis_merges, B.vis_counts);
+                       B.vis_merges, B.vis_counts, B.counters, B.list_cap);
   }
   const uint4* entries = shade ? nullptr : B.vis_entries;
 #define SRX_VIS_LAUNCH(NA, S, SH)                                                                                 \
   for (int pass = 0; pass < (SH ? 1 : 2); ++pass)                                                                 \
     hipLaunchKernelGGL((vis_kernel<NA, S, SH>), dim3(pass == 0 ? ne : nm), dim3(SRX_VIS_THREADS), 0, s, P, mode, pass, \
                        B.order, entries, B.vis_merges, B.vis_counts, B.vis_partial, B.vals[which], B.tstart,      \
-                       B.tend, B.tri_rec, B.tri_attr, B.samplers, wout)
+                       B.tend, B.tri_rec, B.tri_attr, B.samplers, wout, B.counters, B.list_cap)
 #define SRX_VIS_SHADE(NA)                   \
   switch (P.samples) {                      \
   case 1: SRX_VIS_LAUNCH(NA, 1, true); break; \

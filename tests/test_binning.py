@@ -1,0 +1,65 @@
+"""Binning of single draws at the sizes where it can go wrong, on the HIP library against the oracle, byte
+for byte: primitive counts around the 256 of a workgroup, triangles from far below a pixel to beyond
+the target in one draw (emitted by the lane that set them up or spread over the workgroup), record
+lists that fill a tile's LDS sort or need several windows of it, and first draws whose records
+outgrow the buffers."""
+import numpy as np
+import pytest
+
+from salviarenderer_amd import api as A
+
+from helpers import Target, draw_colored, screen_to_clip
+
+
+def mixed(n, w, h, seed):
+    """n triangles with centres over (and beyond) the target and sizes log-uniform from 0.01 pixels to twice it."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-0.1, 1.1, (n, 1, 2)) * (w, h)
+    xy = c + rng.normal(0, 1, (n, 3, 2)) * np.exp(rng.uniform(np.log(0.01), np.log(2.0 * max(w, h)), (n, 1, 1)))
+    x, y = screen_to_clip(xy[..., 0], xy[..., 1], w, h)
+    pos = np.stack([x, y, rng.uniform(0.05, 0.95, (n, 3)), np.ones((n, 3))], -1).reshape(-1, 4)
+    return pos, rng.uniform(0, 1, (3 * n, 4))
+
+
+def render(lib, tris, w, h, samples, blend, draws=1):
+    r = lib.renderer()
+    t = Target(r, w, h, samples)
+    t.clear((0.1, 0.2, 0.3, 0.4))
+    keep = [draw_colored(r, *tris, blend=blend) for _ in range(draws)]
+    out = t.color.read().copy(), t.ds.read().copy()
+    del keep
+    return out
+
+
+def same(hip_lib, cpu_lib, *args, **kw):
+    h, c = render(hip_lib, *args, **kw), render(cpu_lib, *args, **kw)
+    assert np.array_equal(h[1], c[1]) and np.array_equal(h[0], c[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
+@pytest.mark.parametrize("n", [1, 3, 255, 256, 257, 1025])
+def test_mixed_sizes(hip_lib, cpu_lib, n, blend):
+    for w, h, samples in ((333, 130, 1), (64, 64, 2), (1030, 517, 4)):
+        same(hip_lib, cpu_lib, mixed(n, w, h, 50 + n), w, h, samples, blend)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 7000])
+def test_long_lists(hip_lib, cpu_lib, n):
+    """Every triangle lies on the same few tiles."""
+    rng = np.random.default_rng(n)
+    pos = np.concatenate([rng.uniform(-1.5, 1.5, (3 * n, 2)), rng.uniform(0.05, 0.95, (3 * n, 1)), np.ones((3 * n, 1))], 1)
+    for blend in (A.BLEND_OFF, A.BLEND_ON):
+        same(hip_lib, cpu_lib, (pos, rng.uniform(0, 1, (3 * n, 4))), 20, 18, 1, blend)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
+def test_records_outgrow_the_buffers(hip_lib, cpu_lib, blend):
+    """The first draw of a renderer emits more records than its buffers hold and is repeated; the second fits."""
+    rng = np.random.default_rng(3)
+    n = 700
+    pos = np.concatenate([rng.uniform(-1, 1, (3 * n, 2)), rng.uniform(0.05, 0.95, (3 * n, 1)), np.ones((3 * n, 1))], 1)
+    for draws in (1, 2):
+        same(hip_lib, cpu_lib, (pos, rng.uniform(0, 1, (3 * n, 4))), 512, 512, 1, blend, draws=draws)
