@@ -17,9 +17,11 @@ enum stat_slot {
 // Setup counters
 // CT_TOTAL: records emitted (single draws); CT_WIDE: primitives on wide_list, left to the clip launch.
 // The two are added to as one 64-bit word.
-// CT_CURSOR: records given to the tiles' lists; CT_CLASS: GPU tiles per record-count class.
+// CT_CURSOR: records given to the tiles' lists; CT_PARTS, CT_MERGES: parts of split tiles and split tiles;
+// CT_CLASS: GPU tiles per record-count class.
 constexpr int TILE_CLASSES = 16;
-enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_CLASS,
+enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_PARTS, CT_MERGES,
+                    CT_CLASS,
                     CT_COUNT = CT_CLASS + TILE_CLASSES };
 static_assert(CT_TOTAL % 2 == 0 && CT_WIDE == CT_TOTAL + 1, "one aligned 64-bit word");
 
@@ -42,6 +44,11 @@ __host__ __device__ inline uint32_t tile_slots(uint32_t T) {
   return (T < TILE_SLOT_ROWS ? T : TILE_SLOT_ROWS) << tile_slot_shift(T);
 }
 
+// What the host needs to know of a single draw, written by the device into pinned host memory: seq last.
+struct draw_mail {
+  uint32_t seq, total, merges, clip_overflow;
+};
+
 // Per-draw device buffers (owned by the renderer, grown on demand).
 struct draw_buffers {
   float4* vbuf;        // (nverts+1) * (nattr+1) clip-space vertex-shader outputs
@@ -63,10 +70,13 @@ struct draw_buffers {
   const uint32_t* order;  // workgroup launch order of the GPU tiles, heaviest record-count class first: single
                           // draws, the tiles of class k at order[k * tiles], counters[CT_CLASS + k] of them
                           // (scheduled_tile); batches, the tiles one after another
-  uint4* vis_entries;     // visibility work table (vis_table_bounds)
+  // Tiles of more than vis_part records are split into parts, each a workgroup of the visibility pass whose
+  // per-sample keys a second launch merges: parts (tile, part, parts, 0) at their slot of vis_partial,
+  // and (tile, parts, first slot, 0) per split tile (vis_split_bounds; vis_part 0: no tile is split)
+  uint4* vis_parts;
   uint4* vis_merges;
-  uint32_t* vis_counts;   // entries, merges, partial slots
-  unsigned long long* vis_partial;  // partial per-sample keys of split tiles
+  unsigned long long* vis_partial;  // the parts' keys
+  uint32_t vis_part;
   uint32_t* tstart;    // GPU tiles
   uint32_t* tile_count;  // tile_slots(T) words: records per tile, at tile_slot (zero before the setup launch)
   uint32_t* tend;
@@ -147,10 +157,14 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
 // dropped) and count them per tile.
 void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
-// The tiles' record lists from the emitted records: ranges in tstart/tend, the tiles by record-count
-// class in `order` (TILE_CLASSES * tiles words), lists in vals[1], or in primitive order in vals[0]
-// (`sorted`).  Sized for `cap` records; the count is read from B.counters[CT_TOTAL] on the device.
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, hipStream_t s);
+// The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, the tiles by
+// record-count class in B.order (TILE_CLASSES * tiles words), and with B.vis_part the parts of split
+// tiles (when the count is within `cap`).  Lists: vals[1], or in primitive order vals[0] (`sorted`),
+// sized for `cap` records; the count is read from B.counters[CT_TOTAL] on the device.  The lists' launch
+// writes the draw's mail with sequence number `seq` (targets without GPU tiles: nothing is launched).
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s);
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, bool sorted, draw_mail* mail, uint32_t seq,
+                       hipStream_t s);
 // In-place exclusive scan of n u32; writes the total to *total_dev.  tmp holds >= scan_tmp_size(n).
 size_t scan_tmp_size(uint32_t n);
 void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* total_dev, hipStream_t s);
@@ -163,13 +177,16 @@ void launch_raster(const draw_params& P, const draw_buffers& B, int which, hipSt
 bool inorder_applicable(const draw_params& P);
 bool inorder_takes_color_clear(const draw_params& P);
 void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
-// Order-independent visibility for opaque early-Z draws without statistics; false if not applicable.
-// Order-independent visibility (and, with shade, the deferred pixel shader) of an opaque early-Z
-// draw; false when the draw needs the in-order kernel.
-bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, hipStream_t s);
-// Upper bounds of the visibility work table for T GPU tiles and `records` binned records: entries
-// (first launch), merges (second launch) and partial-key slots (256 * samples keys each).
-void vis_table_bounds(uint32_t T, uint32_t records, uint32_t* entries, uint32_t* merges, uint32_t* slots);
+// Order-independent visibility (and, with shade, the deferred pixel shader) of an opaque early-Z draw,
+// laid out for `records` records; false when the draw needs the in-order kernel.  merges > 0: finishes
+// that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles.
+bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
+                hipStream_t s);
+// Records per part of a split tile for a visibility pass over `prims` primitives and `records` expected
+// records (0: no tile can be split), and upper bounds of the parts and split tiles for at most `records`
+// records (a part takes 256 * samples keys of vis_partial).
+uint32_t vis_part_size(uint32_t prims, uint32_t records);
+void vis_split_bounds(uint32_t part, uint32_t records, uint32_t* parts, uint32_t* merges);
 bool needs_shading(const draw_params& P);
 // A SASL pixel shader whose colour is written: such draws run the in-order raster kernel.
 bool sasl_shades(const draw_params& P);

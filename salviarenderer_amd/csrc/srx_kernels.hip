@@ -1478,7 +1478,9 @@ __device__ __forceinline__ void bucket_range_body(const uint32_t* __restrict__ h
 // waits for another's counts.  (A scan over all counts took 12 us whatever the number of tiles.)
 __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __restrict__ tile_count, uint32_t T, uint32_t N,
                                                           uint32_t shift, uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
-                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ order) {
+                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ order,
+                                                          uint32_t part, uint4* __restrict__ parts, uint4* __restrict__ merges,
+                                                          uint32_t cap) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   const int lane = __lane_id();
   const uint32_t t = slot_tile(i, shift);
@@ -1507,15 +1509,28 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     ts[t] = base + incl - n;
     te[t] = base + incl;
     order[static_cast<size_t>(c) * T + at] = t;
+    if (part && n > part && counters[CT_TOTAL] <= cap) {  // with more records the tables' bounds do not hold
+      const uint32_t np = (n + part - 1) / part;
+      const uint32_t e = atomicAdd(&counters[CT_PARTS], np);
+      merges[atomicAdd(&counters[CT_MERGES], 1u)] = make_uint4(t, np, e, 0u);
+      for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
+    }
   }
 }
 // The records to their tiles' lists: position = first record of the tile + rank in the tile.
 constexpr uint32_t SCATTER_PER_THREAD = 4;
 __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                           const uint32_t* __restrict__ ranks, const uint32_t* __restrict__ count,
-                                                           uint32_t cap, const uint32_t* __restrict__ ts,
-                                                           uint32_t* __restrict__ vout) {
-  const uint32_t n = min(*count, cap);
+                                                           const uint32_t* __restrict__ ranks,
+                                                           const uint32_t* __restrict__ counters, uint32_t cap,
+                                                           const uint32_t* __restrict__ ts, uint32_t* __restrict__ vout,
+                                                           draw_mail* mail, uint32_t seq) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // every count is final; the host waits for seq
+    mail->total = counters[CT_TOTAL];
+    mail->merges = counters[CT_MERGES];
+    mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
+    __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  const uint32_t n = min(counters[CT_TOTAL], cap);
   const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
   if (b0 >= n) return;
   uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
@@ -1616,17 +1631,23 @@ __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restri
   }
 }
 
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, hipStream_t s) {
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t N = tile_slots(T), shift = tile_slot_shift(T);
   hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
-                     B.counters, order);
+                     B.counters, order, B.vis_part, B.vis_parts, B.vis_merges, cap);
+}
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, bool sorted, draw_mail* mail, uint32_t seq,
+                       hipStream_t s) {
+  const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
+  if (!T) return;
   const uint32_t per = 256 * SCATTER_PER_THREAD;
   hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max<uint32_t>(cap, 1) + per - 1) / per), dim3(256), 0, s, B.keys[0],
-                     B.vals[0], B.keys[1], B.counters + CT_TOTAL, cap, B.tstart, B.vals[1]);
-  if (sorted) hipLaunchKernelGGL(tile_sort_kernel, dim3(T), dim3(256), 0, s, B.tstart, B.tend, order,
-                                 B.counters, cap, B.vals[1], B.vals[0]);
+                     B.vals[0], B.keys[1], B.counters, cap, B.tstart, B.vals[1], mail, seq);
+  if (sorted)
+    hipLaunchKernelGGL(tile_sort_kernel, dim3(T), dim3(256), 0, s, B.tstart, B.tend, B.order, B.counters, cap, B.vals[1],
+                       B.vals[0]);
 }
 
 // Scheduling order of the GPU tiles, heaviest first so that the longest tiles start early.  Tiles

@@ -227,16 +227,16 @@ struct draw_scratch {
 static size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 // Bytes the record-sized buffers take for `records` binned records (keys, values and ranks as emitted,
-// values by tile, and the visibility work table), in take() order.
-static size_t record_scratch_bytes(uint32_t T, int samples, bool vis_tables, uint64_t records) {
+// values by tile, and the visibility pass's split tiles), in take() order.
+static size_t record_scratch_bytes(uint32_t prims, int samples, bool vis_tables, uint64_t records) {
   const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(records, 0xFFFFFFFFu));
   const size_t rn = std::max<uint32_t>(n, 1);
   size_t b = 4 * align256(rn * 4);
   if (vis_tables) {
-    uint32_t ne, nm, nsl;
-    vis_table_bounds(T, n, &ne, &nm, &nsl);
-    b += align256(static_cast<size_t>(ne) * 16) + align256(static_cast<size_t>(nm) * 16) + align256(16) +
-         align256(static_cast<size_t>(nsl) * 256 * samples * 8);
+    uint32_t np, nm;
+    vis_split_bounds(vis_part_size(prims, n), n, &np, &nm);
+    b += align256(static_cast<size_t>(np) * 16) + align256(static_cast<size_t>(nm) * 16) +
+         align256(static_cast<size_t>(np) * 256 * samples * 8);
   }
   return b + 256;
 }
@@ -322,9 +322,8 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   if (!fixed) {
     uint32_t recent = 0;
     for (uint32_t v : r->recent_records) recent = std::max(recent, v);
-    const uint64_t want = std::max<uint64_t>(std::max<uint64_t>(recent + static_cast<uint64_t>(recent) / 4, static_cast<uint64_t>(P3) + T),
-                                             1u << 16);
-    sized = static_cast<uint32_t>(std::min<uint64_t>(want, 0xFFFFFFF0u));
+    const uint64_t want = recent ? recent + static_cast<uint64_t>(recent) / 4 : static_cast<uint64_t>(P3) + T;
+    sized = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, 1u << 16), 0xFFFFFFF0u));
     RCHK(take_records(sized));
     const size_t held = std::min(std::min(r->keys0.cap, r->vals0.cap), std::min(r->keys1.cap, r->vals1.cap));
     capacity = static_cast<uint32_t>(std::min<size_t>(held, 0xFFFFFFF0u));
@@ -333,7 +332,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     uint64_t lo = 0, hi = 0xFFFFFFFEu;  // largest capacity whose buffers fit
     while (lo < hi) {
       const uint64_t mid = (lo + hi + 1) / 2;
-      if (record_scratch_bytes(T, samples, vis_tables, mid) <= room) lo = mid;
+      if (record_scratch_bytes(primcnt, samples, vis_tables, mid) <= room) lo = mid;
       else hi = mid - 1;
     }
     if (lo == 0) return fail(SRX_OUT_OF_MEMORY, "the draw's scratch exceeds the no-allocation region");
@@ -351,11 +350,15 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   auto mark = [&](int i) {
     if (prof) (void)hipEventRecord(de.ev[i], s);
   };
-  // sampler table: staged in pinned memory (the counter read-back below waits for the copy before the
-  // staging is reused); a renderer's own table is uploaded only when it changed
+  // A draw whose triangles cannot have more records than the lists are formed for (each lies on a tile at
+  // most once) nor split a tile need not be waited for.
+  const bool bounded = static_cast<uint64_t>(P3) * T <= sized && vis_part_size(primcnt, sized) == 0;
+  // sampler table: staged in pinned memory (reused once the last draw's mail shows that its copy has
+  // run); a renderer's own table is uploaded only when it changed
   const bool same_table = !fixed && r->samplers_valid && samplers_d == r->samplers_last_d &&
                           std::memcmp(&r->samplers_last, &SM, sizeof(ps_samplers)) == 0;
   if (!same_table) {
+    RCHK(wait_mail(r));
     *r->samplers_h = SM;
     HIPCHK(hipMemcpyAsync(samplers_d, r->samplers_h, sizeof(ps_samplers), hipMemcpyHostToDevice, s));
     r->samplers_last = SM;
@@ -366,6 +369,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   if (P.ps_id == PS_SASL) {
     const bool same_prog = !fixed && r->sasl_valid && std::memcmp(&r->sasl_last, &r->sasl_cur, sizeof(sasl_program)) == 0;
     if (!same_prog) {
+      RCHK(wait_mail(r));
       *r->sasl_h = r->sasl_cur;
       HIPCHK(hipMemcpyAsync(const_cast<sasl_program*>(P.sasl), r->sasl_h, sizeof(sasl_program), hipMemcpyHostToDevice, s));
       r->sasl_last = r->sasl_cur;
@@ -380,8 +384,6 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   launch_clip(P, B, capacity, s);
   mark(2);
   mark(3);
-  // the counters are final after the clip launch: their read-back overlaps the tiles' lists
-  HIPCHK(hipEventRecord(r->ev_counted, s));
   // A target's pending full clear is applied by the visibility or in-order pass as it writes the
   // target, when that pass covers the whole target (it then reads nothing back); the others run
   // here, while the record count travels to the host.
@@ -399,7 +401,6 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   for (auto& ct : r->st.color_targets)
     if (!(eat_color && ct.get() == ct0)) RCHK(run_pending_clear(ct.get(), s));
   if (!eat_ds) RCHK(run_pending_clear(dst, s));
-  RCHK(start_counter_read(r));
   const bool order_free = vis_tables && vis_applicable(P);  // tile lists need no primitive order
   if (eat_color) {
     P.clear_color = 1;
@@ -417,17 +418,20 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   bool fused = false;
   auto raster = [&]() -> int32_t {
     if (vis_tables) {
-      uint32_t ne, nm, nsl;
-      vis_table_bounds(T, sized, &ne, &nm, &nsl);
-      RCHK(X.take(r->vis_entries, ne, B.vis_entries));
-      RCHK(X.take(r->vis_merges, nm, B.vis_merges));
-      RCHK(X.take(r->vis_counts, 4, B.vis_counts));
-      RCHK(X.take(r->vis_partial, static_cast<size_t>(nsl) * 256 * samples, B.vis_partial));
+      uint32_t np, nm;
+      B.vis_part = vis_part_size(primcnt, sized);
+      vis_split_bounds(B.vis_part, sized, &np, &nm);
+      if (B.vis_part) {
+        RCHK(X.take(r->vis_parts, np, B.vis_parts));
+        RCHK(X.take(r->vis_merges, nm, B.vis_merges));
+        RCHK(X.take(r->vis_partial, static_cast<size_t>(np) * 256 * samples, B.vis_partial));
+      }
     }
     B.list_cap = sized;
-    launch_tile_lists(P, B, sized, order, !order_free, s);
+    launch_tile_ranges(P, B, sized, order, s);
+    launch_tile_lists(P, B, sized, !order_free, r->mail, T ? ++r->mail_seq : r->mail_seq, s);
     mark(4);
-    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, s);
+    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, s);
     if (!fused) {
       if (inorder_applicable(P)) launch_inorder(P, B, which, s);
       else launch_raster(P, B, which, s);
@@ -436,28 +440,34 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     return SRX_OK;
   };
   RCHK(raster());
-  uint32_t ctr[CT_COUNT];
-  RCHK(finish_counter_read(r, ctr));
-  if (ctr[CT_CLIP_OVERFLOW]) return fail(SRX_OUT_OF_MEMORY, "clip buffer overflow");
-  const uint32_t total = ctr[CT_TOTAL];
-  if (fixed && total > capacity)
-    return fail(SRX_OUT_OF_MEMORY, "the draw's binned records exceed the no-allocation region");
-  if (!fixed) r->recent_records[r->recent_next++ % 8] = total;
-  if (total > sized) {
-    if (total > capacity) {  // emit again into larger buffers, counting no statistics a second time
-      RCHK(take_records(total));
-      launch_fill_u32(B.counters, CT_COUNT, 0u, s);
-      launch_fill_u32(B.tile_count, tile_slots(T), 0u, s);
-      draw_params Pe = P;
-      draw_buffers Be = B;
-      Pe.count_stats = 0;
-      Be.stats = B.partial;
-      launch_setup(Pe, Be, total, s);
-      launch_clip(Pe, Be, total, s);
+  if (T && !bounded) {
+    RCHK(wait_mail(r));
+    if (r->mail->clip_overflow) return fail(SRX_OUT_OF_MEMORY, "clip buffer overflow");
+    const uint32_t total = r->mail->total;
+    if (fixed && total > capacity)
+      return fail(SRX_OUT_OF_MEMORY, "the draw's binned records exceed the no-allocation region");
+    if (!fixed) r->recent_records[r->recent_next++ % 8] = total;
+    if (total > sized) {
+      if (total > capacity) {  // emit again into larger buffers, counting no statistics a second time
+        RCHK(take_records(total));
+        launch_fill_u32(B.counters, CT_COUNT, 0u, s);
+        launch_fill_u32(B.tile_count, tile_slots(T), 0u, s);
+        draw_params Pe = P;
+        draw_buffers Be = B;
+        Pe.count_stats = 0;
+        Be.stats = B.partial;
+        launch_setup(Pe, Be, total, s);
+        launch_clip(Pe, Be, total, s);
+      }
+      sized = total;
+      launch_fill_u32(B.counters + CT_CURSOR, CT_COUNT - CT_CURSOR, 0u, s);
+      RCHK(raster());
+      RCHK(wait_mail(r));
     }
-    sized = total;
-    launch_fill_u32(B.counters + CT_CURSOR, CT_COUNT - CT_CURSOR, 0u, s);
-    RCHK(raster());
+    if (fused && r->mail->merges) {
+      launch_vis(P, B, which, needs_shading(P), sized, r->mail->merges, s);
+      mark(5);
+    }
   }
   if (eat_color) RCHK(run_pending_clear(ct0, s, true));
   if (eat_ds) RCHK(run_pending_clear(dst, s, true));
@@ -478,7 +488,6 @@ renderer_obj::~renderer_obj() {
   drop_recording(this);
   if (stream) (void)run_pending_clears(this);
   if (stream) (void)hipStreamSynchronize(stream);
-  if (side) (void)hipStreamSynchronize(side);
 
   auto fr = [](auto& a) {
     if (a.p) (void)hipFree(a.p);
@@ -488,18 +497,15 @@ renderer_obj::~renderer_obj() {
   if (sasl_h) (void)hipHostFree(sasl_h);
   if (sasl_d) (void)hipFree(sasl_d);
   fr(keys0); fr(keys1); fr(vals0); fr(vals1);
-  fr(tstart); fr(tend); fr(clip_hdr); fr(counters); fr(clip_flag); fr(clip_slot); fr(partial); fr(order); fr(tile_count); fr(wide); fr(vis_entries); fr(vis_merges); fr(vis_counts); fr(vis_partial);
+  fr(tstart); fr(tend); fr(clip_hdr); fr(counters); fr(clip_flag); fr(clip_slot); fr(partial); fr(order); fr(tile_count); fr(wide); fr(vis_parts); fr(vis_merges); fr(vis_partial);
   if (stats_d) (void)hipFree(stats_d);
-  if (pinned) (void)hipHostFree(pinned);
+  if (mail) (void)hipHostFree(mail);
   if (map_host) (void)hipHostFree(map_host);
   for (auto& d : pending_prof)
     for (auto e : d.ev)
       if (e) (void)hipEventDestroy(e);
   for (auto e : event_pool) (void)hipEventDestroy(e);
   if (stream) (void)hipStreamDestroy(stream);
-  if (side) (void)hipStreamDestroy(side);
-  if (ev_counted) (void)hipEventDestroy(ev_counted);
-  if (ev_read) (void)hipEventDestroy(ev_read);
 }
 
 
@@ -627,14 +633,12 @@ int32_t srx_create_renderer(uint32_t kind, srx_renderer* out) {
   }
   hipError_t e = hipGetDevice(&r->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&r->stream, hipStreamDefault);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&r->ev_counted, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&r->ev_read, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&r->counters.p, CT_COUNT * sizeof(uint32_t));
   if (e == hipSuccess) r->counters.cap = CT_COUNT;
   if (e == hipSuccess) e = hipMalloc(&r->stats_d, ST_COUNT * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(r->stats_d, 0, ST_COUNT * sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipHostMalloc(&r->pinned, CT_COUNT * sizeof(uint32_t), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc(&r->mail, sizeof(draw_mail), hipHostMallocCoherent);
+  if (e == hipSuccess) *r->mail = draw_mail{};
   if (e == hipSuccess) e = hipHostMalloc(&r->samplers_h, sizeof(ps_samplers), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc(&r->sasl_h, sizeof(sasl_program), hipHostMallocDefault);
   if (e != hipSuccess) {

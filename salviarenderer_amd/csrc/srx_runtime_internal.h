@@ -386,18 +386,16 @@ struct renderer_obj : object {
   dev_array<uint32_t> order;  // GPU tile scheduling order
   dev_array<uint32_t> tile_count;  // records per tile
   dev_array<uint32_t> wide;   // triangles whose records the clip launch emits
-  dev_array<uint4> vis_entries, vis_merges;  // visibility work table
-  dev_array<uint32_t> vis_counts;
+  dev_array<uint4> vis_parts, vis_merges;  // split tiles of the visibility pass
   dev_array<unsigned long long> vis_partial;
   dev_array<uint8_t> clip_flag;
   dev_array<int32_t> clip_slot;
   dev_array<unsigned long long> partial;
   unsigned long long* stats_d = nullptr;
-  uint32_t* pinned = nullptr;  // host staging for counter read-back (CT_COUNT words)
   std::vector<ref<surface_obj>> pending;  // surfaces holding a pending clear issued here
-  // the counters are read back on `side` (default priority) while the main stream forms the tile lists
-  hipStream_t side = nullptr;
-  hipEvent_t ev_counted = nullptr, ev_read = nullptr;
+  // the record count and split tiles of the last draw, written by its list launch (wait_mail)
+  draw_mail* mail = nullptr;  // pinned
+  uint32_t mail_seq = 0;      // sequence number of the last draw that writes it
   // binned records of the last draws; their maximum sizes the next draw's record buffer, so that
   // frames whose draws differ in size do not overflow it in turn
   uint32_t recent_records[8] = {};
@@ -460,18 +458,21 @@ inline int gpu_tile_size() {
   return g;
 }
 
-// Starts the read-back of the draw's device counters as they stood at ev_counted (recorded on the
-// main stream), on the side stream, so that work queued after ev_counted overlaps it.
-inline int32_t start_counter_read(renderer_obj* r) {
-  HIPCHK(hipStreamWaitEvent(r->side, r->ev_counted, 0));
-  HIPCHK(hipMemcpyAsync(r->pinned, r->counters.p, CT_COUNT * sizeof(uint32_t), hipMemcpyDeviceToHost, r->side));
-  HIPCHK(hipEventRecord(r->ev_read, r->side));
-  return SRX_OK;
-}
-inline int32_t finish_counter_read(renderer_obj* r, uint32_t* out) {
-  HIPCHK(hipEventSynchronize(r->ev_read));
-  for (int i = 0; i < CT_COUNT; ++i) out[i] = r->pinned[i];
-  return SRX_OK;
+// Waits until the draw with the renderer's last sequence number has written its mail (and with it every
+// earlier command of the stream has run).  The kernel's store reaches the pinned word within a
+// microsecond or two; a copy, an event and its wait took the host 15-25 us of every draw.
+inline int32_t wait_mail(renderer_obj* r) {
+  for (uint32_t spin = 1;; ++spin) {
+    if (__atomic_load_n(&r->mail->seq, __ATOMIC_ACQUIRE) == r->mail_seq) return SRX_OK;
+    __builtin_ia32_pause();
+    if (spin % 8192 == 0) {  // a stream that has ended (or failed) without the store never makes it
+      const hipError_t e = hipStreamQuery(r->stream);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return hip_fail(e, "hipStreamQuery");
+      if (__atomic_load_n(&r->mail->seq, __ATOMIC_ACQUIRE) == r->mail_seq) return SRX_OK;
+      return fail(SRX_E_HIP, "the draw ended without its record count");
+    }
+  }
 }
 
 #define RCHK(expr)                     \

@@ -10,67 +10,6 @@ hipError_t upload_ewa_table_vis(const float* table256, hipStream_t s) {
   return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_ewa), table256, 256 * sizeof(float), 0, hipMemcpyHostToDevice, s);
 }
 
-// records per workgroup beyond which a tile of a depth-only draw is split
-constexpr uint32_t VIS_PART = 256;
-
-// Work table of the order-independent visibility kernel for draws without shading (depth-only
-// passes), whose time is the longest tile's: a GPU tile with more than VIS_PART records is split
-// into parts of at most VIS_PART records, each a workgroup of the first launch that leaves its
-// partial per-sample keys in `partial`; the second launch merges a split tile's parts (a minimum,
-// so the order of the parts is immaterial) and finishes it.  (Draws that shade keep whole tiles:
-// their shading fills the GPU while the long tiles run.)  Entries follow `order`, heaviest first.
-//   entries[i] = (tile, part, parts, first partial slot)   i < counts[0]
-//   merges[i]  = (tile, parts, first partial slot, 0)      i < counts[1]
-__global__ void __launch_bounds__(1024) vis_table_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
-                                                         const uint32_t* __restrict__ order, uint32_t T,
-                                                         uint4* __restrict__ entries, uint4* __restrict__ merges,
-                                                         uint32_t* __restrict__ counts, const uint32_t* __restrict__ counters,
-                                                         uint32_t cap) {
-  if (counters[CT_TOTAL] > cap) {  // records were dropped: the draw is emitted again
-    if (threadIdx.x < 3) counts[threadIdx.x] = 0;
-    return;
-  }
-  __shared__ uint32_t wtot[3][16];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t per = (T + 1023) / 1024, p0 = tid * per, p1 = min(T, p0 + per);
-  uint32_t c[3] = {0, 0, 0};  // blocks, partial slots, merges in this thread's segment of `order`
-  for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = scheduled_tile(order, counters + CT_CLASS, T, p), n = te[t] - ts[t];
-    const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
-    c[0] += parts;
-    if (parts > 1) { c[1] += parts; c[2] += 1; }
-  }
-  uint32_t incl[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    incl[k] = wave_incl_scan(c[k]);
-    if (lane == 63) wtot[k][wave] = incl[k];
-  }
-  __syncthreads();
-  uint32_t base[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    uint32_t before = 0, total = 0;
-    for (uint32_t w = 0; w < 16; ++w) {
-      if (w < wave) before += wtot[k][w];
-      total += wtot[k][w];
-    }
-    base[k] = before + incl[k] - c[k];
-    if (tid == 0) counts[k == 0 ? 0 : (k == 1 ? 2 : 1)] = total;
-  }
-  uint32_t b = base[0], sl = base[1], m = base[2];
-  for (uint32_t p = p0; p < p1; ++p) {
-    const uint32_t t = scheduled_tile(order, counters + CT_CLASS, T, p), n = te[t] - ts[t];
-    const uint32_t parts = n > VIS_PART ? (n + VIS_PART - 1) / VIS_PART : 1u;
-    for (uint32_t k = 0; k < parts; ++k) entries[b + k] = make_uint4(t, k, parts, sl);
-    b += parts;
-    if (parts > 1) {
-      merges[m++] = make_uint4(t, parts, sl, 0u);
-      sl += parts;
-    }
-  }
-}
-
 // ---------------------------------------------------------------- order-independent visibility
 // For an opaque early-Z draw with blending off, the reference's sequential early-Z test (depth written
 // at test time, framebuffer.cpp:522-614) leaves in every sample the result of a running reduction:
@@ -306,27 +245,154 @@ __device__ __forceinline__ void vis_items(const draw_params& P, int mode, const 
 #ifndef SRX_VIS_THREADS
 #define SRX_VIS_THREADS 256
 #endif
-// LDS shared by phase 1 (a chunk of NT records + their (record, block) work list) and phase 3
-// (shading items), for GT x GT GPU tiles
+// LDS shared by phase 1 (a chunk of NT records, their (record, block) work list, and up to 2 NT records
+// that depth culling has let through) and phase 3 (shading items), for GT x GT GPU tiles
 __host__ __device__ constexpr int vis_union_bytes(int nt, int s, bool shade, int gt = 16) {
-  return (nt * 64 + nt * (gt / 4) * (gt / 4) * 2) > (shade ? gt * gt * s * 8 : 0) ? (nt * 64 + nt * (gt / 4) * (gt / 4) * 2)
-                                                                                   : gt * gt * s * 8;
+  const int chunk = nt * 64 + nt * (gt / 4) * (gt / 4) * 2 + nt * 8;
+  return chunk > (shade ? gt * gt * s * 8 : 0) ? chunk : gt * gt * s * 8;
+}
+// Records of a tile taken before depth culling begins: few for draws whose triangles lie on VIS_LARGE or
+// more GPU tiles on average, whose lists are deep (of the 323 records a tile of the 2,000-triangle
+// plain scene has, 50 of the last 259 survive: 60 -> 35 us); a whole chunk for draws of smaller ones,
+// which seldom cover a tile before its list ends (64 there: 161 -> 186 us for the mesh that fills the
+// target).
+constexpr uint32_t VIS_FIRST = 64, VIS_LARGE = 4;
+__host__ __device__ inline bool vis_large(uint64_t records, uint32_t prims) {
+  return records >= static_cast<uint64_t>(VIS_LARGE) * prims;
+}
+// A tile's time is its list's length, so lists much longer than an even share of the records over the
+// workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame at the
+// oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
+// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where every tile's list is near
+// the even share a split only adds work.  Draws of large triangles, whose lists depth culling
+// shortens as it goes, are split later.
+constexpr uint32_t VIS_PART_SMALL = 1024, VIS_PART_LARGE = 2048, VIS_SLOTS = 640;
+
+// S (depth, stencil) pairs of a pixel as wide stores (surfaces are allocated at 256-byte alignment, so a
+// pixel's samples start at a multiple of their size).
+template <int S>
+__device__ __forceinline__ void store_ds_pixel(uint8_t* p, const float (&d)[S], uint32_t stencil) {
+  const float f = __uint_as_float(stencil);
+  if constexpr (S == 1) {
+    *reinterpret_cast<float2*>(p) = make_float2(d[0], f);
+  } else {
+#pragma unroll
+    for (int s = 0; s < S; s += 2) *reinterpret_cast<float4*>(p + s * 8) = make_float4(d[s], f, d[s + 1], f);
+  }
+}
+template <int S>
+__device__ __forceinline__ void fill_color_pixel(const draw_params& P, int px, int py) {
+  const float4 c = make_float4(P.clear_rgba[0], P.clear_rgba[1], P.clear_rgba[2], P.clear_rgba[3]);
+  if (P.color.pf == PF_RGBA8 && S > 1) {
+    const uint32_t u = unorm8(c.x) | (unorm8(c.y) << 8) | (unorm8(c.z) << 16) | (unorm8(c.w) << 24);
+    uint8_t* p = sample_addr(P.color, px, py, 0);
+    if constexpr (S == 4) *reinterpret_cast<uint4*>(p) = make_uint4(u, u, u, u);
+    else *reinterpret_cast<uint2*>(p) = make_uint2(u, u);
+  } else {
+#pragma unroll
+    for (int s = 0; s < S; ++s) store_texel(P.color.pf, sample_addr(P.color, px, py, s), c);
+  }
 }
 // Static LDS of vis_body besides the union (keys, initial depths).
 __host__ __device__ constexpr int vis_static_bytes(int s, int gt) { return gt * gt * s * 12 + 256; }
+// Phases 2 and 3 of a tile whose keys are final (*nitems is zero).
+template <int NA, int S, bool SHADE, int GT>
+__device__ __forceinline__ void vis_finish(const draw_params& P, int mode, const unsigned long long* keys, uint2* items,
+                                           uint32_t* nitems, int ox, int oy, int NT, const float4* __restrict__ tri_rec,
+                                           const float4* __restrict__ tri_attr, const ps_samplers* __restrict__ SM,
+                                           uint32_t* __restrict__ wout) {
+  constexpr int PX = GT * GT;
+  const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
+  const int tid = threadIdx.x;
+  const bool has_ds = P.ds.data != nullptr;
+  // phase 2: winners -> depth, shading items
+  for (int p = tid; p < PX; p += NT) {
+    const int px = ox + (p % GT), py = oy + (p / GT);
+    if (px >= tw || py >= th) continue;
+    uint32_t w[S];
+    float d[S];
+    uint32_t left = 0;
+#pragma unroll
+    for (int smp = 0; smp < S; ++smp) {
+      const unsigned long long key = keys[p * S + smp];
+      w[smp] = key_winner(mode, key);
+      const bool won = w[smp] != NO_WINNER;
+      if (won) left |= 1u << smp;
+      d[smp] = P.clear_depth;
+      if (won && has_ds && P.write_depth) {
+        d[smp] = winner_depth<S>(P, mode, key, w[smp], tri_rec, px, py, smp);
+        if (!P.clear_ds) *reinterpret_cast<float*>(sample_addr(P.ds, px, py, smp)) = d[smp];
+      }
+      // winners for a separate shading pass (SASL pixel shaders), laid out like the colour samples
+      if (!SHADE && wout) wout[(static_cast<size_t>(py) * tw + px) * S + smp] = w[smp];
+    }
+    // a cleared target: every sample is written, the stencil keeps its clear value
+    if (has_ds && P.clear_ds) store_ds_pixel<S>(sample_addr(P.ds, px, py, 0), d, P.clear_stencil);
+    if (SHADE && P.clear_color) {
+      if (left == 0) {
+        fill_color_pixel<S>(P, px, py);
+      } else {
+#pragma unroll
+        for (int smp = 0; smp < S; ++smp)
+          if (!((left >> smp) & 1u))
+            store_texel(P.color.pf, sample_addr(P.color, px, py, smp),
+                        make_float4(P.clear_rgba[0], P.clear_rgba[1], P.clear_rgba[2], P.clear_rgba[3]));
+      }
+    }
+    if (SHADE) {
+#pragma unroll
+      for (int it = 0; it < S; ++it) {
+        if (!left) break;
+        const int s0 = __builtin_ctz(left);
+        uint32_t cur = w[0];
+#pragma unroll
+        for (int smp = 1; smp < S; ++smp)
+          if (smp == s0) cur = w[smp];
+        uint32_t m = 0;
+#pragma unroll
+        for (int smp = 0; smp < S; ++smp)
+          if (w[smp] == cur) m |= 1u << smp;
+        left &= ~m;
+        items[atomicAdd(nitems, 1u)] = make_uint2(cur, static_cast<uint32_t>(p) | (m << 12));
+      }
+    }
+  }
+  if (!SHADE) return;
+  __syncthreads();
+  // phase 3: shading items
+  const uint32_t n = *nitems;
+  for (uint32_t j = tid; j < n; j += NT) {
+    const uint2 item = items[j];
+    const uint32_t cur = item.x, p = item.y & 4095u, m = item.y >> 12;
+    if (cur >= 3u * P.prim_count) continue;  // every winner id is below 3 * prim_count
+    const int px = ox + static_cast<int>(p % GT), py = oy + static_cast<int>(p / GT);
+    const int pi = (px & 1) | ((py & 1) << 1);
+    attr_setup<NA> at;
+    load_attr<NA>(P, tri_attr, cur, at);
+    const quad_lazy<NA> q(at, P, px & ~1, py & ~1);
+    const float4 c = run_ps_pixel<NA>(P, SM, q, pi);
+#pragma unroll
+    for (int smp = 0; smp < S; ++smp)
+      if (m & (1u << smp)) store_texel(P.color.pf, sample_addr(P.color, px, py, smp), c);
+  }
+}
 // NTC > 0: NTC lanes per workgroup, static LDS.  NTC == 0: blockDim.x lanes (64, 128 or 256) with
 // the phase-1/3 union in dynamic LDS of vis_union_bytes(blockDim.x, S, SHADE, GT) bytes.
 // GT: GPU tile side, 8, 16 or 32 pixels: a quarter of a 16x16 stage-16 region, one region, or 2x2
 // regions of the reference's 64x64 tile; the 4x4 blocks are the reference's stage-4 blocks either way.
+// The tile's records are those of `ws`: a whole tile, or one part of a split tile.
+struct vis_span {
+  int tile;
+  uint32_t t0, t1;    // records
+  uint32_t parts;     // parts the tile is split into
+  uint32_t slot;      // this part's keys in vis_partial
+};
 template <int NA, int S, bool SHADE, int NTC, int GT>
-__device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pass, const uint32_t* __restrict__ order,
-                                         const uint4* __restrict__ entries, const uint4* __restrict__ merges,
-                                         const uint32_t* __restrict__ counts, unsigned long long* __restrict__ partial,
-                                         const uint32_t* __restrict__ vals, const uint32_t* __restrict__ tstart,
-                                         const uint32_t* __restrict__ tend, const float4* __restrict__ tri_rec,
-                                         const float4* __restrict__ tri_attr, const ps_samplers* __restrict__ SM,
-                                         uint32_t bx, uint32_t* __restrict__ wout = nullptr,
-                                         const uint32_t* __restrict__ classes = nullptr) {
+__device__ __forceinline__ void vis_body(const draw_params& P, int mode, const vis_span& ws,
+                                         unsigned long long* __restrict__ partial, const uint32_t* __restrict__ vals,
+                                         const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
+                                         const ps_samplers* __restrict__ SM, uint32_t first,
+                                         uint32_t* __restrict__ wout = nullptr) {
   static_assert(GT == 8 || GT == 16 || GT == 32, "GPU tile side");
   constexpr int PX = GT * GT;       // pixels per GPU tile
   constexpr int NBS = GT / 4;       // 4x4 blocks per side
@@ -341,49 +407,45 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
   unsigned char* const lds_union = NTC > 0 ? lds_static : lds_dynamic;
   __shared__ uint32_t wsum[4];
   __shared__ uint32_t hiz[NBS * NBS];
-  __shared__ uint32_t nitems;
+  __shared__ uint32_t nitems, nlist, far_now, far_start;
   float4* recs = reinterpret_cast<float4*>(lds_union);                           // [NT][4]
   uint16_t* work = reinterpret_cast<uint16_t*>(lds_union + NT * 64);             // [NT * NBS^2]
+  uint32_t* list = reinterpret_cast<uint32_t*>(lds_union + NT * 64 + NT * NBS * NBS * 2);  // [2 * NT]
   uint2* items = reinterpret_cast<uint2*>(lds_union);                            // [PX * S]
-  // pass 0: one tile, or one part of a split tile; pass 1: merge and finish a split tile
-  int gtile;
-  uint32_t part = 0, parts = 1, slot = 0;
-  if (entries == nullptr) {  // whole tiles in `order`
-    gtile = static_cast<int>(classes ? scheduled_tile(order, classes, static_cast<uint32_t>(P.gtiles_x * P.gtiles_y), bx)
-                                     : order[bx]);
-  } else if (pass == 0) {
-    if (bx >= counts[0]) return;
-    const uint4 en = entries[bx];
-    gtile = static_cast<int>(en.x);
-    part = en.y;
-    parts = en.z;
-    slot = en.w + en.y;
-  } else {
-    if (bx >= counts[1]) return;
-    const uint4 mg = merges[bx];
-    gtile = static_cast<int>(mg.x);
-    parts = mg.y;
-    slot = mg.z;
-  }
+  const int gtile = ws.tile;
+  const uint32_t t0 = ws.t0, t1 = ws.t1;
   const int gx = gtile % P.gtiles_x, gy = gtile / P.gtiles_x;
   const int ox = gx * GT, oy = gy * GT;
   const int t64x = ox & ~(TILE - 1), t64y = oy & ~(TILE - 1);
   const int tw = static_cast<int>(P.target_w), th = static_cast<int>(P.target_h);
   const int tid = threadIdx.x;
   const bool has_ds = P.ds.data != nullptr;
-  if (tid == 0) nitems = 0;
-  if (pass == 1) {
-    // the parts' keys, each started from the target's depth: their minimum is the tile's result
-    const unsigned long long* src = partial + static_cast<size_t>(slot) * (PX * S);
-    for (int i = tid; i < PX * S; i += NT) {
-      unsigned long long k = src[i];
-      for (uint32_t q = 1; q < parts; ++q) {
-        const unsigned long long kq = src[static_cast<size_t>(q) * (PX * S) + i];
-        k = kq < k ? kq : k;
+  // A tile without records takes the pending clears (88% of the textured mesh frame's tiles at the
+  // oblique camera, whose empty passes through the phases below were 40% of its instructions).
+  if (t0 == t1) {
+    for (int p = tid; p < PX; p += NT) {
+      const int px = ox + (p % GT), py = oy + (p / GT);
+      if (px >= tw || py >= th) continue;
+      if (has_ds && P.clear_ds) {
+        float d[S];
+#pragma unroll
+        for (int smp = 0; smp < S; ++smp) d[smp] = P.clear_depth;
+        store_ds_pixel<S>(sample_addr(P.ds, px, py, 0), d, P.clear_stencil);
       }
-      keys[i] = k;
+      if (SHADE && P.clear_color) fill_color_pixel<S>(P, px, py);
+      if (!SHADE && wout) {
+#pragma unroll
+        for (int smp = 0; smp < S; ++smp) wout[(static_cast<size_t>(py) * tw + px) * S + smp] = NO_WINNER;
+      }
     }
-  } else {
+    return;
+  }
+  if (tid == 0) {
+    nitems = 0;
+    far_start = 0;
+  }
+  {
+    uint32_t far = 0;
     for (int i = tid; i < PX * S; i += NT) {
       int px = ox + ((i / S) % GT), py = oy + ((i / S) / GT), smp = i % S;
       float d0 = 0.0f;
@@ -402,46 +464,105 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
       d0s[i] = d0;
       // a blocked sample's key is below every candidate's and decodes as no winner
       keys[i] = blocked ? ((mode == VIS_LEQUAL || mode == VIS_GEQUAL) ? 0xFFFFFFFFull : 0ull) : initial_key(mode, d0);
+      if (px < tw && py < th) far = max(far, static_cast<uint32_t>(keys[i] >> 32));
     }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) far = max(far, static_cast<uint32_t>(__shfl_xor(static_cast<int>(far), off, 64)));
+    __syncthreads();  // far_start is zero
+    if ((tid & 63) == 0) atomicMax(&far_start, far);
   }
-  // this workgroup's records: the whole tile, or one part of it (none when merging)
-  const uint32_t tr0 = tstart[gtile], tr1 = tend[gtile];
-  const uint32_t t0 = pass == 1 ? tr1 : min(tr1, tr0 + part * VIS_PART);
-  const uint32_t t1 = (pass == 1 || entries == nullptr) ? tr1 : min(tr1, t0 + VIS_PART);
   const int jx0 = (ox - t64x) >> 4, jy0 = (oy - t64y) >> 4;  // first stage-16 region of the tile
   // an 8x8 tile covers blocks [qx, qx+2) x [qy, qy+2) of its region; larger tiles whole regions
   const int qx = GT < 16 ? ((ox - t64x) & 15) >> 2 : 0, qy = GT < 16 ? ((oy - t64y) & 15) >> 2 : 0;
   constexpr int CW = GT < 16 ? GT / 4 : 4;  // block columns (rows) of a region inside the tile
   const float tvx = static_cast<float>(t64x), tvy = static_cast<float>(t64y);
-  // Depth culling from the second chunk on: hiz[b] is the largest key depth word of 4x4 block b's
-  // samples after the previous chunks.  Keys only decrease, so a record whose smallest possible
-  // depth word over the block exceeds it cannot win any sample there and skips the block.
+  // Depth culling after the first records (vis_first): hiz[b] is the largest key depth word of 4x4 block b's
+  // samples inside the target after the previous chunks, far_now the largest of the tile.  Keys only
+  // decrease, so a record whose smallest possible depth word over the tile (or a block) exceeds it
+  // cannot win any sample there.  Once the tile's farthest depth has come nearer than at the start,
+  // every lane tests one record against it and the survivors are listed, so that chunks stay full of
+  // records that can still win: of the lists of ~150 layers that the plain scenes give a tile, 15-35%
+  // survive.
   const bool depth_keys = mode == VIS_LESS || mode == VIS_LEQUAL || mode == VIS_GREATER || mode == VIS_GEQUAL;
   const bool far_is_min = mode == VIS_GREATER || mode == VIS_GEQUAL;
-  for (uint32_t c0 = t0; c0 < t1; c0 += NT) {
+  // smallest possible key depth word of a record's samples in the size x size square at (x, y): the depth
+  // plane's extreme, widened by far more than the rounding of the per-sample evaluation; planes with
+  // inf or nan terms are never culled
+  auto nearest_key = [&](float4 d3, float4 d4, int x, int y, float size) -> uint32_t {
+    const float z0 = d3.w, zx = d3.y, zy = d3.z, dzx = d4.x, dzy = d4.y;
+    const float ax = static_cast<float>(x) - zx, ay = static_cast<float>(y) - zy;
+    const float tx0 = dzx * ax, tx1 = dzx * (ax + size), ty0 = dzy * ay, ty1 = dzy * (ay + size);
+    const float margin = (fabsf(z0) + fmaxf(fabsf(tx0), fabsf(tx1)) + fmaxf(fabsf(ty0), fabsf(ty1))) * 1.52587890625e-05f;
+    const float zext = far_is_min ? (z0 + fmaxf(tx0, tx1) + fmaxf(ty0, ty1)) + margin
+                                  : (z0 + fminf(tx0, tx1) + fminf(ty0, ty1)) - margin;
+    if (!(fabsf(zext) < 3.0e38f)) return 0u;
+    return far_is_min ? ~ord_depth(zext) : ord_depth(zext);
+  };
+  uint32_t next = t0, held = 0;  // records not yet looked at; survivors waiting in `list` (both uniform)
+  while (next < t1 || held) {
     __syncthreads();  // the previous chunk's work list is consumed (and the keys are initialised)
-    const bool hiz_on = depth_keys && c0 > t0;
+    const bool hiz_on = depth_keys && next > t0;
+    bool cull = false;
     if (hiz_on) {
+      if (tid == 0) far_now = 0;
       // 16 consecutive lanes take one block's 16 pixels
+      uint32_t far = 0;
       for (int u = tid; u < PX; u += NT) {
         const int b = u >> 4, q = u & 15;
-        const int pl = ((b / NBS) * 4 + (q >> 2)) * GT + (b % NBS) * 4 + (q & 3);
+        const int pr = (b / NBS) * 4 + (q >> 2), pc = (b % NBS) * 4 + (q & 3);
+        const int pl = pr * GT + pc;
         uint32_t m = 0;
 #pragma unroll
         for (int smp = 0; smp < S; ++smp) m = max(m, static_cast<uint32_t>(keys[pl * S + smp] >> 32));
+        if (ox + pc >= tw || oy + pr >= th) m = 0;
         m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 1, 64)));
         m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 2, 64)));
         m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 4, 64)));
         m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 8, 64)));
         if (q == 0) hiz[b] = m;
+        far = max(far, m);
       }
       __syncthreads();
+      far = max(far, static_cast<uint32_t>(__shfl_xor(static_cast<int>(far), 16, 64)));
+      far = max(far, static_cast<uint32_t>(__shfl_xor(static_cast<int>(far), 32, 64)));
+      if ((tid & 63) == 0) atomicMax(&far_now, far);
+      __syncthreads();
+      cull = far_now < far_start;
+    }
+    uint32_t rec = 0xFFFFFFFFu;  // this lane's record of the chunk
+    if (cull) {
+      const uint32_t far = far_now;
+      if (tid == 0) nlist = held;
+      __syncthreads();
+      while (next < t1 && held < static_cast<uint32_t>(NT)) {
+        const uint32_t ri = next + tid;
+        uint32_t v = 0;
+        bool keep = false;
+        if (ri < t1) {
+          v = vals[ri];
+          const float4* tr = tri_rec + tri_slot(P, v >> 1) * 5;
+          keep = nearest_key(tr[3], tr[4], ox, oy, static_cast<float>(GT)) <= far;
+        }
+        const uint64_t km = __ballot(keep);
+        uint32_t at = 0;
+        if ((tid & 63) == 0 && km) at = atomicAdd(&nlist, static_cast<uint32_t>(__popcll(km)));
+        at = static_cast<uint32_t>(__shfl(static_cast<int>(at), 0, 64));
+        if (keep) list[at + __popcll(km & ((1ull << (tid & 63)) - 1ull))] = v;
+        next = min(next + static_cast<uint32_t>(NT), t1);
+        __syncthreads();
+        held = nlist;
+        __syncthreads();  // read before the next step adds to it
+      }
+      if (static_cast<uint32_t>(tid) < held) rec = list[tid];
+      if (!held) break;  // nothing left that can win
+    } else {
+      const uint32_t take = min(min(t1 - next, static_cast<uint32_t>(NT)), depth_keys && next == t0 ? first : static_cast<uint32_t>(NT));
+      if (static_cast<uint32_t>(tid) < take) rec = vals[next + tid];
+      next += take;
     }
     // phase 1a: one record per lane -> the 4x4 blocks of this GPU tile it reaches (full or partial)
     bmask_t bm = 0, fm = 0;
-    const uint32_t ri = c0 + tid;
-    if (ri < t1) {
-      const uint32_t rec = vals[ri];
+    if (rec != 0xFFFFFFFFu) {
       const uint32_t id = rec >> 1;
       const float4* tr = tri_rec + tri_slot(P, id) * 5;
       float e[9], bb[4];
@@ -527,20 +648,7 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
           }
           // the block's index in this tile
           const int b = ((rr / RPS) * 4 + iy4 - qy) * NBS + (rr % RPS) * 4 + ix4 - qx;
-          if (hiz_on) {
-            // the depth plane's extreme over the block's sample positions [Bx, Bx+4) x [By, By+4),
-            // widened by far more than the rounding of the per-sample evaluation
-            const float z0 = d3.w, zx = d3.y, zy = d3.z, dzx = d4.x, dzy = d4.y;
-            const float ax = static_cast<float>(rox + ix4 * 4) - zx, ay = static_cast<float>(roy + iy4 * 4) - zy;
-            const float tx0 = dzx * ax, tx1 = dzx * (ax + 4.0f), ty0 = dzy * ay, ty1 = dzy * (ay + 4.0f);
-            const float margin = (fabsf(z0) + fmaxf(fabsf(tx0), fabsf(tx1)) + fmaxf(fabsf(ty0), fabsf(ty1))) * 1.52587890625e-05f;
-            const float zext = far_is_min ? (z0 + fmaxf(tx0, tx1) + fmaxf(ty0, ty1)) + margin
-                                          : (z0 + fminf(tx0, tx1) + fminf(ty0, ty1)) - margin;
-            if (fabsf(zext) < 3.0e38f) {  // finite: planes with inf/nan terms are never culled
-              const uint32_t zk = far_is_min ? ~ord_depth(zext) : ord_depth(zext);
-              if (zk > hiz[b]) continue;
-            }
-          }
+          if (hiz_on && nearest_key(d3, d4, rox + ix4 * 4, roy + iy4 * 4, 4.0f) > hiz[b]) continue;
           bm |= static_cast<bmask_t>(1) << b;
           if (block_full) fm |= static_cast<bmask_t>(1) << b;
         }
@@ -560,6 +668,11 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
     const uint32_t incl = wave_incl_scan(cnt);
     if ((tid & 63) == 63) wsum[tid >> 6] = incl;
     __syncthreads();
+    if (held) {  // survivors beyond this chunk move to the front
+      const uint32_t rest = held > static_cast<uint32_t>(NT) ? held - NT : 0u;
+      if (static_cast<uint32_t>(tid) < rest) list[tid] = list[NT + tid];
+      held = rest;
+    }
     uint32_t off = incl - cnt, total = 0;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -588,98 +701,86 @@ __device__ __forceinline__ void vis_body(const draw_params& P, int mode, int pas
       vis_items<S, GT, false>(P, mode, recs, work, total_p, total_all, keys, d0s, ox, oy, tw, th, tid, NT);
   }
   __syncthreads();
-  if (pass == 0 && parts > 1) {  // one part of a split tile: leave the partial keys for the merge
-    unsigned long long* dst = partial + static_cast<size_t>(slot) * (PX * S);
+  if (ws.parts > 1) {  // one part of a split tile: leave its keys for the merge
+    unsigned long long* dst = partial + static_cast<size_t>(ws.slot) * (PX * S);
     for (int i = tid; i < PX * S; i += NT) dst[i] = keys[i];
     return;
   }
-  // phase 2: winners -> depth, shading items
-  for (int p = tid; p < PX; p += NT) {
-    const int px = ox + (p % GT), py = oy + (p / GT);
-    if (px >= tw || py >= th) continue;
-    uint32_t w[S];
-    uint32_t left = 0;
-#pragma unroll
-    for (int smp = 0; smp < S; ++smp) {
-      const unsigned long long key = keys[p * S + smp];
-      w[smp] = key_winner(mode, key);
-      const bool won = w[smp] != NO_WINNER;
-      if (won) left |= 1u << smp;
-      if (has_ds && P.clear_ds) {
-        // a cleared target: every sample is written, the stencil keeps its clear value
-        const float d = (won && P.write_depth) ? winner_depth<S>(P, mode, key, w[smp], tri_rec, px, py, smp) : P.clear_depth;
-        *reinterpret_cast<float2*>(sample_addr(P.ds, px, py, smp)) = make_float2(d, __uint_as_float(P.clear_stencil));
-      } else if (won && has_ds && P.write_depth) {
-        *reinterpret_cast<float*>(sample_addr(P.ds, px, py, smp)) =
-            winner_depth<S>(P, mode, key, w[smp], tri_rec, px, py, smp);
-      }
-      if (SHADE && !won && P.clear_color) {
-        const float4 cc = make_float4(P.clear_rgba[0], P.clear_rgba[1], P.clear_rgba[2], P.clear_rgba[3]);
-        store_texel(P.color.pf, sample_addr(P.color, px, py, smp), cc);
-      }
-      // winners for a separate shading pass (SASL pixel shaders), laid out like the colour samples
-      if (!SHADE && wout) wout[(static_cast<size_t>(py) * tw + px) * S + smp] = w[smp];
-    }
-    if (SHADE) {
-#pragma unroll
-      for (int it = 0; it < S; ++it) {
-        if (!left) break;
-        const int s0 = __builtin_ctz(left);
-        uint32_t cur = w[0];
-#pragma unroll
-        for (int smp = 1; smp < S; ++smp)
-          if (smp == s0) cur = w[smp];
-        uint32_t m = 0;
-#pragma unroll
-        for (int smp = 0; smp < S; ++smp)
-          if (w[smp] == cur) m |= 1u << smp;
-        left &= ~m;
-        items[atomicAdd(&nitems, 1u)] = make_uint2(cur, static_cast<uint32_t>(p) | (m << 12));
-      }
-    }
-  }
-  if (!SHADE) return;
-  __syncthreads();
-  // phase 3: shading items
-  const uint32_t n = nitems;
-  for (uint32_t j = tid; j < n; j += NT) {
-    const uint2 item = items[j];
-    const uint32_t cur = item.x, p = item.y & 4095u, m = item.y >> 12;
-    if (cur >= 3u * P.prim_count) continue;  // every winner id is below 3 * prim_count
-    const int px = ox + static_cast<int>(p % GT), py = oy + static_cast<int>(p / GT);
-    const int pi = (px & 1) | ((py & 1) << 1);
-    attr_setup<NA> at;
-    load_attr<NA>(P, tri_attr, cur, at);
-    const quad_lazy<NA> q(at, P, px & ~1, py & ~1);
-    const float4 c = run_ps_pixel<NA>(P, SM, q, pi);
-#pragma unroll
-    for (int smp = 0; smp < S; ++smp)
-      if (m & (1u << smp)) store_texel(P.color.pf, sample_addr(P.color, px, py, smp), c);
-  }
+  vis_finish<NA, S, SHADE, GT>(P, mode, keys, items, &nitems, ox, oy, NT, tri_rec, tri_attr, SM, wout);
 }
+// Single draws.  The first `max_parts` workgroups take the parts of split tiles, the others the tiles in
+// scheduling order; vis_merge_kernel then finishes the split tiles.
+struct vis_lists {
+  const uint32_t *order, *vals, *tstart, *tend, *counters;
+  const uint4 *parts, *merges;
+  unsigned long long* partial;
+  uint32_t cap, part, max_parts, first;
+};
 template <int NA, int S, bool SHADE>
-__global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, int pass,
-                                                   const uint32_t* __restrict__ order,
-                                                   const uint4* __restrict__ entries, const uint4* __restrict__ merges,
-                                                   const uint32_t* __restrict__ counts,
-                                                   unsigned long long* __restrict__ partial,
-                                                   const uint32_t* __restrict__ vals,
-                                                   const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
+__global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, vis_lists V,
                                                    const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
-                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout,
-                                                   const uint32_t* __restrict__ counters, uint32_t cap) {
-  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
-  vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, pass, order, entries, merges, counts, partial, vals, tstart, tend,
-                                              tri_rec, tri_attr, SM, blockIdx.x, wout, counters + CT_CLASS);
+                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
+  if (V.counters[CT_TOTAL] > V.cap) return;  // records were dropped: the draw is emitted again
+  vis_span ws;
+  ws.parts = 1;
+  ws.slot = 0;
+  const uint32_t b = blockIdx.x;
+  if (b < V.max_parts) {
+    if (b >= V.counters[CT_PARTS]) return;
+    const uint4 e = V.parts[b];
+    ws.tile = static_cast<int>(e.x);
+    ws.parts = e.z;
+    ws.slot = b;
+    ws.t0 = V.tstart[e.x] + e.y * V.part;
+    ws.t1 = min(V.tend[e.x], ws.t0 + V.part);
+  } else {
+    const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
+    const uint32_t t = scheduled_tile(V.order, V.counters + CT_CLASS, T, b - V.max_parts);
+    ws.tile = static_cast<int>(t);
+    ws.t0 = V.tstart[t];
+    ws.t1 = V.tend[t];
+    if (V.part && ws.t1 - ws.t0 > V.part) return;  // its parts take it
+  }
+  vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, ws, V.partial, V.vals, tri_rec, tri_attr, SM, V.first, wout);
 }
 
+// One split tile per workgroup: its keys are the minimum of the parts' keys (each started from the
+// target's depth), so the parts' order is immaterial.  512 lanes, as the tiles are few and full: 400 split
+// tiles of the textured mesh frame took 84 us with 256, 46 us with 512.
+constexpr int VIS_MERGE_THREADS = 512;
+template <int NA, int S, bool SHADE>
+__global__ void __launch_bounds__(VIS_MERGE_THREADS, 2) vis_merge_kernel(draw_params P, int mode, vis_lists V,
+                                                   const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
+                                                   const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
+  constexpr int PX = 256;
+  __shared__ unsigned long long keys[PX * S];
+  __shared__ uint2 items[SHADE ? PX * S : 1];
+  __shared__ uint32_t nitems;
+  const uint4 m = V.merges[blockIdx.x];
+  const unsigned long long* src = V.partial + static_cast<size_t>(m.z) * (PX * S);
+  for (int i = threadIdx.x; i < PX * S; i += VIS_MERGE_THREADS) {
+    unsigned long long k = src[i];
+    for (uint32_t q = 1; q < m.y; ++q) {
+      const unsigned long long kq = src[static_cast<size_t>(q) * (PX * S) + i];
+      k = kq < k ? kq : k;
+    }
+    keys[i] = k;
+  }
+  if (threadIdx.x == 0) nitems = 0;
+  __syncthreads();
+  const int ox = static_cast<int>(m.x) % P.gtiles_x * 16, oy = static_cast<int>(m.x) / P.gtiles_x * 16;
+  vis_finish<NA, S, SHADE, 16>(P, mode, keys, items, &nitems, ox, oy, VIS_MERGE_THREADS, tri_rec, tri_attr, SM, wout);
+}
 
 template <int NA, int S, bool SHADE, int GT>
 __global__ void __launch_bounds__(256, 4) vis_batch_kernel(const batch_job* __restrict__ jobs, stage_map m) {
   uint32_t lb, nb;
   const batch_job& J = jobs[stage_job(m, lb, nb)];
-  vis_body<NA, S, SHADE, 0, GT>(J.P, J.vis_mode, 0, J.B.order, nullptr, nullptr, nullptr, nullptr, J.B.vals[1], J.B.tstart,
-                            J.B.tend, J.B.tri_rec, J.B.tri_attr, J.B.samplers, lb);
+  const uint32_t t = J.B.order[lb];
+  const vis_span ws{static_cast<int>(t), J.B.tstart[t], J.B.tend[t], 1u, 0u};
+  const uint32_t records = J.B.cnt[3 * J.P.prim_count] - J.B.cnt[0];
+  vis_body<NA, S, SHADE, 0, GT>(J.P, J.vis_mode, ws, nullptr, J.B.vals[1], J.B.tri_rec, J.B.tri_attr, J.B.samplers,
+                                vis_large(records, J.P.prim_count) ? min(VIS_FIRST, blockDim.x) : blockDim.x);
 }
 
 // ============================================================== host launchers
@@ -703,14 +804,17 @@ int vis_mode(const draw_params& P) {
   }
 }
 
-void vis_table_bounds(uint32_t T, uint32_t records, uint32_t* entries, uint32_t* merges, uint32_t* slots) {
-  const uint32_t chunks = (records + VIS_PART - 1) / VIS_PART;
-  *entries = T + chunks;            // sum over tiles of max(1, ceil(n / VIS_PART))
-  *merges = records / (VIS_PART + 1) + 1;  // tiles with more than VIS_PART records
-  *slots = 2 * chunks + 1;          // parts of split tiles: ceil(n / VIS_PART) <= 2n / VIS_PART
+uint32_t vis_part_size(uint32_t prims, uint32_t records) {
+  const uint32_t part = std::max(vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL, records / VIS_SLOTS);
+  return 3ull * prims > part ? part : 0u;  // a primitive gives at most three triangles, each once on a tile
+}
+void vis_split_bounds(uint32_t part, uint32_t records, uint32_t* parts, uint32_t* merges) {
+  *parts = part ? 2 * (records / part + 1) : 0;  // ceil(n / part) < 2 n / part for n > part
+  *merges = part ? records / (part + 1) + 1 : 0;
 }
 
-bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, hipStream_t s) {
+bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
+                hipStream_t s) {
   int mode = vis_mode(P);
   // a SASL pixel shader runs in its own pass (launch_shade) over the winners this pass writes
   uint32_t* const wout = sasl_shades(P) ? B.vis : nullptr;
@@ -718,18 +822,18 @@ bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool sha
   uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (mode < 0 || P.gt != 16) return false;
   if (!T) return true;
-  uint32_t ne = T, nm = 0, nsl;
-  if (!shade) {
-    vis_table_bounds(T, records, &ne, &nm, &nsl);
-    hipLaunchKernelGGL(vis_table_kernel, dim3(1), dim3(1024), 0, s, B.tstart, B.tend, B.order, T, B.vis_entries,
-                       B.vis_merges, B.vis_counts, B.counters, B.list_cap);
-  }
-  const uint4* entries = shade ? nullptr : B.vis_entries;
-#define SRX_VIS_LAUNCH(NA, S, SH)                                                                                 \
-  for (int pass = 0; pass < (SH ? 1 : 2); ++pass)                                                                 \
-    hipLaunchKernelGGL((vis_kernel<NA, S, SH>), dim3(pass == 0 ? ne : nm), dim3(SRX_VIS_THREADS), 0, s, P, mode, pass, \
-                       B.order, entries, B.vis_merges, B.vis_counts, B.vis_partial, B.vals[which], B.tstart,      \
-                       B.tend, B.tri_rec, B.tri_attr, B.samplers, wout, B.counters, B.list_cap)
+  uint32_t np, nm;
+  vis_split_bounds(B.vis_part, records, &np, &nm);
+  const vis_lists V{B.order, B.vals[which], B.tstart, B.tend, B.counters, B.vis_parts, B.vis_merges, B.vis_partial,
+                    B.list_cap, B.vis_part, np,
+                    vis_large(records, P.prim_count) ? std::min<uint32_t>(VIS_FIRST, SRX_VIS_THREADS) : SRX_VIS_THREADS};
+#define SRX_VIS_LAUNCH(NA, S, SH)                                                                                       \
+  if (merges)                                                                                                           \
+    hipLaunchKernelGGL((vis_merge_kernel<NA, S, SH>), dim3(merges), dim3(VIS_MERGE_THREADS), 0, s, P, mode, V, B.tri_rec, \
+                       B.tri_attr, B.samplers, wout);                                                                   \
+  else                                                                                                                  \
+    hipLaunchKernelGGL((vis_kernel<NA, S, SH>), dim3(np + T), dim3(SRX_VIS_THREADS), 0, s, P, mode, V, B.tri_rec,       \
+                       B.tri_attr, B.samplers, wout)
 #define SRX_VIS_SHADE(NA)                   \
   switch (P.samples) {                      \
   case 1: SRX_VIS_LAUNCH(NA, 1, true); break; \

@@ -63,3 +63,30 @@ def test_records_outgrow_the_buffers(hip_lib, cpu_lib, blend):
     pos = np.concatenate([rng.uniform(-1, 1, (3 * n, 2)), rng.uniform(0.05, 0.95, (3 * n, 1)), np.ones((3 * n, 1))], 1)
     for draws in (1, 2):
         same(hip_lib, cpu_lib, (pos, rng.uniform(0, 1, (3 * n, 4))), 512, 512, 1, blend, draws=draws)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("samples", [1, 4])
+@pytest.mark.parametrize("n", [63, 64, 65, 1023, 1025, 2049, 5000])
+def test_split_and_culled_tiles(hip_lib, cpu_lib, n, samples):
+    """Opaque lists around the lengths where a tile is split and where depth culling begins, of triangles over
+    several tiles and of triangles inside one, for every depth order and for a depth-only pass."""
+    rng = np.random.default_rng(n)
+    w, h = 40, 24
+    for size in (2.0, 0.05):
+        c = rng.uniform(-0.7, 0.7, (n, 1, 2)) if size > 1 else rng.uniform(0.05, 0.55, (n, 1, 2)) * (1, -1)
+        xy = c + rng.uniform(-1, 1, (n, 3, 2)) * size
+        pos = np.concatenate([xy, rng.uniform(0.02, 0.98, (n, 3, 1)), np.ones((n, 3, 1))], -1).reshape(-1, 4)
+        col = rng.uniform(0, 1, (3 * n, 4))
+        for func, depth in ((A.CMP_LESS, 1.0), (A.CMP_GREATER_EQUAL, 0.0), (A.CMP_LESS_EQUAL, 0.5)):
+            out = []
+            for lib in (hip_lib, cpu_lib):
+                r = lib.renderer()
+                t = Target(r, w, h, samples)
+                t.clear((0.1, 0.2, 0.3, 0.4), depth)
+                keep = [draw_colored(r, pos, col, depth_func=func)]
+                r.set_render_targets([], t.ds)  # the same triangles nearer: depth only
+                keep.append(draw_colored(r, pos * (1, 1, 0.9, 1), col, depth_func=func))
+                out.append((t.color.read().copy(), t.ds.read().copy()))
+                del keep
+            assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][0], out[1][0]), (size, func)
