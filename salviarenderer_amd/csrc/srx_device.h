@@ -41,6 +41,8 @@ struct sampler_desc_dev {
   // 1: anisotropic mip filter (max_aniso > 1), linear min/mag, wrap/wrap, every level single-sample
   // RGBA8 -- the sampler's common case, which has a compact inline path
   int32_t fast_aniso;
+  // 1: linear min/mag and mip filters otherwise as above (trilinear)
+  int32_t fast_linear;
   surface_desc levels[MAX_LEVELS];
 };
 

@@ -127,6 +127,7 @@ __device__ __forceinline__ float4 tex2d_cpp(const sampler_desc_dev& sp, const qu
   const float lod = (sp.mip_filter == FILTER_ANISO && sp.max_aniso > 1) ? calc_aniso(sp, dxu, dxv, dyu, dyv, 0.0f).lod
                                                                         : calc_lod(sp, dxu, dxv, dyu, dyv, 0.0f);
   const float4 uv = q.reg(reg, pi, q.inv_w(pi), 2);
+  if (sp.fast_linear) return sample_linear_fast(sp, uv.x, uv.y, lod);
   return sample_impl(sp, uv.x, uv.y, lod, nullptr);
 }
 // eflib vector helpers on .xyz (vector_generic.h:110-118, math.cpp:39-41,85-87)
@@ -280,11 +281,7 @@ __device__ __forceinline__ float4 run_ps_pixel(const draw_params& P, const ps_sa
       const float dyu = c1.x - c0.x, dyv = c1.y - c0.y;
       const float4 nrm = q.reg(1, pi, iw, 3);
       float4 t = make_float4(0, 0, 0, 0);
-      if (P.has_sampler[0]) {
-        const sampler_desc_dev& sp = SM->s[0];
-        t = sp.fast_aniso ? sample_2d_grad_fast(sp, uv.x, uv.y, dxu, dxv, dyu, dyv, 0.0f)
-                          : sample_2d_grad(sp, uv.x, uv.y, dxu, dxv, dyu, dyv, 0.0f);
-      }
+      if (P.has_sampler[0]) t = sample_grad(SM->s[0], uv.x, uv.y, dxu, dxv, dyu, dyv);
       float nx, ny, nz;
       normalize3(nrm.x, nrm.y, nrm.z, nx, ny, nz);
       float d = nx * P.ps_consts[0] + ny * P.ps_consts[1] + nz * P.ps_consts[2];

@@ -56,8 +56,7 @@ __device__ __forceinline__ void shade_store(const draw_params& P, const ps_sampl
     sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
       if (!P.has_sampler[slot]) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       const sampler_desc_dev& sp = SM->s[slot];
-      return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                           : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
+      return sample_grad(sp, u, v, dxu, dxv, dyu, dyv);
     });
     for (int i = 0; i < 4; ++i) {
       const uint32_t m = (pm >> (4 * i)) & 15u;
@@ -478,8 +477,7 @@ __global__ void __launch_bounds__(64) sasl_shade_kernel(draw_params P, const ps_
     sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
       if (!P.has_sampler[slot]) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       const sampler_desc_dev& sp = SM->s[slot];
-      return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                           : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
+      return sample_grad(sp, u, v, dxu, dxv, dyu, dyv);
     });
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -555,8 +553,7 @@ __global__ void __launch_bounds__(64) sasl_quads_kernel(const sasl_program* __re
   sasl_exec(prog, R, [&](int slot, int, float u, float v, float dxu, float dxv, float dyu, float dyv) -> float4 {
     if (!((has_mask >> slot) & 1u)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const sampler_desc_dev& sp = SM->s[slot];
-    return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)
-                         : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);
+    return sample_grad(sp, u, v, dxu, dxv, dyu, dyv);
   });
   for (int px = 0; px < 4; ++px)
     for (uint32_t o = 0; o < nout; ++o) {

@@ -43,9 +43,10 @@ int32_t fill_sampler(renderer_obj* r, sampler_obj* so, sampler_desc_dev& sd) {
   }
   bool rgba8 = sd.nlevels > 0;
   for (int l = 0; l < sd.nlevels; ++l) rgba8 &= sd.levels[l].pf == SRX_PF_RGBA8 && sd.levels[l].samples == 1;
-  sd.fast_aniso = rgba8 && sd.mip_filter == SRX_FILTER_ANISOTROPIC && sd.max_aniso > 1 &&
-                  sd.min_filter == SRX_FILTER_LINEAR && sd.mag_filter == SRX_FILTER_LINEAR &&
-                  sd.addr_u == SRX_ADDRESS_WRAP && sd.addr_v == SRX_ADDRESS_WRAP;
+  const bool fast = rgba8 && sd.min_filter == SRX_FILTER_LINEAR && sd.mag_filter == SRX_FILTER_LINEAR &&
+                    sd.addr_u == SRX_ADDRESS_WRAP && sd.addr_v == SRX_ADDRESS_WRAP;
+  sd.fast_aniso = fast && sd.mip_filter == SRX_FILTER_ANISOTROPIC && sd.max_aniso > 1;
+  sd.fast_linear = fast && sd.mip_filter == SRX_FILTER_LINEAR;
   return SRX_OK;
 }
 

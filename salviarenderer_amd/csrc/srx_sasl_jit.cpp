@@ -51,8 +51,7 @@ std::string translate(const sasl_program& p, int NA, int S) {
        "    float v, float dxu, float dxv, float dyu, float dyv) {\n"
        "  if (!P.has_sampler[slot]) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);\n"
        "  const sampler_desc_dev& sp = SM->s[slot];\n"
-       "  return sp.fast_aniso ? sample_2d_grad_fast(sp, u, v, dxu, dxv, dyu, dyv, 0.0f)\n"
-       "                       : sample_2d_grad(sp, u, v, dxu, dxv, dyu, dyv, 0.0f);\n"
+       "  return sample_grad(sp, u, v, dxu, dxv, dyu, dyv);\n"
        "}\n"
        "// the quad's mask of lanes whose bit b is set\n"
        "__device__ __forceinline__ uint32_t quad_bits(uint32_t b) {\n"
