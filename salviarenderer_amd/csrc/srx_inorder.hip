@@ -50,9 +50,9 @@ __device__ __forceinline__ void store_words(uint8_t* p, const uint32_t (&w)[S]) 
 //     stencil and (8-bit colour formats) colour in registers, tests each against them, and shades and
 //     blends those that pass.  Lanes of a wave are at different records at the same time.
 // Measured (32k blended, trilinearly textured triangles over most of 1280x720, 4 samples): this kernel
-// 0.1 ms, the whole frame 0.20-0.26 ms; a wave walking the records together, with only the lanes of
+// 0.14 ms, the whole frame 0.14-0.24 ms (among others, alone); a wave walking the records together, with only the lanes of
 // the current record's quads shading and every blend a round trip to the target, 4.2 ms (frame 4.0-4.2).
-// It is bound by the pixel shader's latency at the 2 waves per SIMD its registers leave (221 for two
+// It is bound by the pixel shader's latency at the 2 waves per SIMD its registers leave (229 for two
 // attributes and 4 samples; capping them for 3 or 4 waves cost the textured frame 8 and 33% and gained
 // the nine-tap shadow frame 1 and 2%) and by the deepest pixel of each wave.
 constexpr int IO_CHUNK = 64;

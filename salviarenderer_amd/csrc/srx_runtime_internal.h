@@ -181,8 +181,9 @@ enum { PROF_GATHER = 0, PROF_VTX, PROF_CLIP, PROF_COMPACT, PROF_VP, PROF_DISPATC
        PROF_RAS_VIS, PROF_RAS_SHADE, PROF_COUNT };
 
 // HIP events bracketing the stages of one profiled draw, on the renderer's stream:
-// [0,1) vertex shader, [1,2) setup + clipping (viewport transform fused), [2,3) compaction scan,
-// [3,4) record emission + tile sort, [4,5) visibility or in-order raster, [5,6) deferred shading.
+// [0,1) vertex shader, [1,2) setup + clipping (viewport transform and record emission fused),
+// [2,3) empty (the profile's compaction slot), [3,4) tile ranges, scatter and sort, [4,5) visibility
+// (with the merge of split tiles) or in-order raster, [5,6) deferred shading.
 struct draw_events {
   hipEvent_t ev[7];
 };
