@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(256) inorder_kernel(draw_params P, const ps_sa
                                                       const uint32_t* __restrict__ tstart, const uint32_t* __restrict__ tend,
                                                       const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
                                                       const uint32_t* __restrict__ counters, uint32_t cap) {
-  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
+  if (record_total(counters) > cap) return;  // records were dropped: the draw is emitted again
   __shared__ float4 recs[IO_CHUNK * 4];            // edges, depth plane, id << 1 | front
   __shared__ unsigned long long cov[IO_CHUNK][16];  // covered samples of a record's block, 4 bits a pixel
   __shared__ unsigned long long pmask[256];         // records with a covered sample in the pixel (partial blocks)

@@ -16,13 +16,20 @@ enum stat_slot {
 };
 // Setup counters
 // CT_TOTAL: records emitted (single draws); CT_WIDE: primitives on wide_list, left to the clip launch.
-// The two are added to as one 64-bit word.
+// The two are added to as one 64-bit word.  CT_OVERRUN: the clip launch's additions carried CT_TOTAL past 32
+// bits (setup alone cannot: at most four records a primitive, whose buffers take over 600 bytes); read the
+// count with record_total.
 // CT_CURSOR: records given to the tiles' lists; CT_PARTS, CT_MERGES: parts of split tiles and split tiles;
 // CT_CLASS: GPU tiles per record-count class.
 constexpr int TILE_CLASSES = 16;
 enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_PARTS, CT_MERGES,
-                    CT_CLASS,
+                    CT_OVERRUN, CT_CLASS,
                     CT_COUNT = CT_CLASS + TILE_CLASSES };
+// Records of a single draw, 0xFFFFFFFF when the count does not fit (above every capacity).
+__host__ __device__ inline uint32_t record_total(const uint32_t* counters) {
+  return counters[CT_OVERRUN] ? 0xFFFFFFFFu : counters[CT_TOTAL];
+}
+constexpr uint32_t MAX_RECORDS = 0xFFFFFFF0u;  // a draw with more is refused
 static_assert(CT_TOTAL % 2 == 0 && CT_WIDE == CT_TOTAL + 1, "one aligned 64-bit word");
 
 // Where a tile's record count lies in tile_count: atomics to words of one cache line are served one after
@@ -160,7 +167,7 @@ void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity,
 // The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, the tiles by
 // record-count class in B.order (TILE_CLASSES * tiles words), and with B.vis_part the parts of split
 // tiles (when the count is within `cap`).  Lists: vals[1], or in primitive order vals[0] (`sorted`),
-// sized for `cap` records; the count is read from B.counters[CT_TOTAL] on the device.  The lists' launch
+// sized for `cap` records; the count is read from B.counters on the device.  The lists' launch
 // writes the draw's mail with sequence number `seq` (targets without GPU tiles: nothing is launched).
 void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s);
 void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, bool sorted, draw_mail* mail, uint32_t seq,

@@ -1074,7 +1074,10 @@ __device__ __forceinline__ void emit_wide(const draw_params& P, const draw_buffe
       if (w < wave) pos += L.wsum[w];
       all += L.wsum[w];
     }
-    if (tid == 0 && all) L.base = atomicAdd(&B.counters[CT_TOTAL], all);
+    if (tid == 0 && all) {
+      L.base = atomicAdd(&B.counters[CT_TOTAL], all);
+      if (L.base > ~all) B.counters[CT_OVERRUN] = 1;
+    }
     __syncthreads();
     const uint32_t base = L.base;
     for (uint32_t w0 = 0; w0 < all; w0 += WIDE_LIST) {
@@ -1509,7 +1512,7 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     ts[t] = base + incl - n;
     te[t] = base + incl;
     order[static_cast<size_t>(c) * T + at] = t;
-    if (part && n > part && counters[CT_TOTAL] <= cap) {  // with more records the tables' bounds do not hold
+    if (part && n > part && record_total(counters) <= cap) {  // with more records the tables' bounds do not hold
       const uint32_t np = (n + part - 1) / part;
       const uint32_t e = atomicAdd(&counters[CT_PARTS], np);
       merges[atomicAdd(&counters[CT_MERGES], 1u)] = make_uint4(t, np, e, 0u);
@@ -1525,12 +1528,12 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
                                                            const uint32_t* __restrict__ ts, uint32_t* __restrict__ vout,
                                                            draw_mail* mail, uint32_t seq) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {  // every count is final; the host waits for seq
-    mail->total = counters[CT_TOTAL];
+    mail->total = record_total(counters);
     mail->merges = counters[CT_MERGES];
     mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
     __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  const uint32_t n = min(counters[CT_TOTAL], cap);
+  const uint32_t n = min(record_total(counters), cap);
   const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
   if (b0 >= n) return;
   uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
@@ -1580,7 +1583,7 @@ __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restri
   __shared__ uint32_t a[SORT_LDS];
   __shared__ uint32_t hist[256];
   __shared__ uint32_t s_n, s_below, s_k;
-  if (counters[CT_TOTAL] > cap) return;  // records were dropped: the draw is emitted again
+  if (record_total(counters) > cap) return;  // records were dropped: the draw is emitted again
   const uint32_t t = scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x), t0 = ts[t], n = te[t] - t0, tid = threadIdx.x;
   if (n <= SORT_LDS) {
     if (n == 0) return;

@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(256) raster_kernel(draw_params P, const ps_sam
                                                       const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
                                                       uint32_t* __restrict__ vis, unsigned long long* __restrict__ partial,
                                                       const uint32_t* __restrict__ counters, uint32_t cap) {
-  if (counters[CT_TOTAL] > cap) {  // records were dropped: the draw is emitted again
+  if (record_total(counters) > cap) {  // records were dropped: the draw is emitted again
     if (P.count_stats) block_partial(partial, 0ull);
     return;
   }

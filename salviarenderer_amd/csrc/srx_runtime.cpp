@@ -324,13 +324,13 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     uint32_t recent = 0;
     for (uint32_t v : r->recent_records) recent = std::max(recent, v);
     const uint64_t want = recent ? recent + static_cast<uint64_t>(recent) / 4 : static_cast<uint64_t>(P3) + T;
-    sized = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, 1u << 16), 0xFFFFFFF0u));
+    sized = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, 1u << 16), MAX_RECORDS));
     RCHK(take_records(sized));
     const size_t held = std::min(std::min(r->keys0.cap, r->vals0.cap), std::min(r->keys1.cap, r->vals1.cap));
-    capacity = static_cast<uint32_t>(std::min<size_t>(held, 0xFFFFFFF0u));
+    capacity = static_cast<uint32_t>(std::min<size_t>(held, MAX_RECORDS));
   } else {
     const size_t room = fixed->bytes - std::min(fixed->bytes, align256(X.used));
-    uint64_t lo = 0, hi = 0xFFFFFFFEu;  // largest capacity whose buffers fit
+    uint64_t lo = 0, hi = MAX_RECORDS;  // largest capacity whose buffers fit
     while (lo < hi) {
       const uint64_t mid = (lo + hi + 1) / 2;
       if (record_scratch_bytes(primcnt, samples, vis_tables, mid) <= room) lo = mid;
@@ -447,6 +447,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
     const uint32_t total = r->mail->total;
     if (fixed && total > capacity)
       return fail(SRX_OUT_OF_MEMORY, "the draw's binned records exceed the no-allocation region");
+    if (total > MAX_RECORDS) return fail(SRX_OUT_OF_MEMORY, "more than 4,294,967,280 binned records in one draw");
     if (!fixed) r->recent_records[r->recent_next++ % 8] = total;
     if (total > sized) {
       if (total > capacity) {  // emit again into larger buffers, counting no statistics a second time

@@ -766,7 +766,7 @@ template <int NA, int S, bool SHADE>
 __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, vis_lists V,
                                                    const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
                                                    const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
-  if (V.counters[CT_TOTAL] > V.cap) return;  // records were dropped: the draw is emitted again
+  if (record_total(V.counters) > V.cap) return;  // records were dropped: the draw is emitted again
   vis_span ws;
   ws.parts = 1;
   ws.slot = 0;

@@ -90,3 +90,25 @@ def test_split_and_culled_tiles(hip_lib, cpu_lib, n, samples):
                 out.append((t.color.read().copy(), t.ds.read().copy()))
                 del keep
             assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][0], out[1][0]), (size, func)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
+def test_more_records_than_32_bits_count(hip_lib, blend):
+    """16,400 triangles over each of 262,144 GPU tiles are 4,299,161,600 records: the draw is refused, its targets
+    keep what they held, and the renderer draws on."""
+    n, side = 16400, 8191
+    r = hip_lib.renderer()
+    t = Target(r, side, side)
+    t.clear((0.2, 0.4, 0.6, 0.8))
+    pos = np.tile(np.array([[-1, -1, 0.5, 1], [3, -1, 0.5, 1], [-1, 3, 0.5, 1]], np.float32), (n, 1))
+    col = np.ones((3 * n, 4), np.float32)
+    with pytest.raises(A.SrxError) as e:
+        draw_colored(r, pos, col, blend=blend)
+    assert e.value.code == A.OUT_OF_MEMORY
+    assert (t.color.read().reshape(-1, 4) == (51, 102, 153, 204)).all()
+    small = [Target(r, 40, 30)]
+    small[0].clear()
+    keep = draw_colored(r, pos[:3], col[:3], blend=blend)
+    assert (small[0].color.read() == 255).all()
+    del keep
