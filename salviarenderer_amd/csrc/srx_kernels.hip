@@ -1551,13 +1551,22 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
   }
 }
 
-// Each tile's list in ascending order (primitive order: a triangle is on a tile once), from `in` to
-// `out`, one workgroup per tile.  Lists of up to SORT_LDS records are sorted in LDS; a longer one is
-// taken in windows of consecutive values that hold at most SORT_LDS records each, found by a histogram
-// of its values that is narrowed until its first bucket fits.  Sorting the lists costs in-order draws a
-// pass over their records; two stable radix passes over all records (by tile) took 50 us of a
-// 32k-triangle draw at 1280x720.
-constexpr uint32_t SORT_LDS = 2048;
+// Each tile's list in ascending order (primitive order: a triangle is on a tile once), from `in` to `out`, one
+// workgroup per tile.  Lists of up to SORT_LDS records are sorted in LDS.  A longer one is partitioned by the
+// leading 8 bits of its values (a histogram, then every record to its bucket in the other buffer, in any
+// order: the values are distinct), runs of buckets that fit are sorted in LDS, and a bucket that does not fit
+// is partitioned by its next 8 bits, back into the first buffer.  Every level reads its records twice, and
+// three levels leave buckets of at most 256 values, so the time grows with the list's length (blended
+// triangles on the same 16 tiles: 100,000 of them 9.7 ms a frame, 300,000 29, a million small ones 19; with
+// windows of SORT_LDS records, each found by reading the whole list, 14.6, 72 and 93).  Sorting the lists costs in-order draws a pass over their records; two stable radix
+// passes over all records (by tile) took 50 us of a 32k-triangle draw at 1280x720.
+constexpr uint32_t SORT_LDS = 2048, SORT_LEVELS = 3, SORT_FLIGHT = 8;
+struct sort_space {
+  uint32_t a[SORT_LDS];
+  uint32_t hist[256];
+  uint32_t start[SORT_LEVELS][257];  // the buckets of a level's partition
+  uint32_t wsum[4];
+};
 __device__ __forceinline__ void sort_lds(uint32_t* a, uint32_t n) {
   uint32_t m = 2;
   while (m < n) m <<= 1;  // uniform
@@ -1576,62 +1585,82 @@ __device__ __forceinline__ void sort_lds(uint32_t* a, uint32_t n) {
     }
   __syncthreads();
 }
+// f(x[i]) for i < n, SORT_FLIGHT loads of a lane in flight.
+template <class F>
+__device__ __forceinline__ void sort_each(const uint32_t* x, uint32_t n, F&& f) {
+  for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 256 * SORT_FLIGHT) {
+    uint32_t v[SORT_FLIGHT];
+#pragma unroll
+    for (uint32_t j = 0; j < SORT_FLIGHT; ++j) v[j] = x[min(i0 + j * 256, n - 1)];
+#pragma unroll
+    for (uint32_t j = 0; j < SORT_FLIGHT; ++j)
+      if (i0 + j * 256 < n) f(v[j]);
+  }
+}
+// Sorts x[0, n), n > SORT_LDS, whose values agree above bit shift + 8, into o, the buffer that holds x on odd
+// levels and y on even ones.
+template <uint32_t LEVEL>
+__device__ __forceinline__ void sort_long(uint32_t* x, uint32_t* y, uint32_t* o, uint32_t n, uint32_t shift, sort_space& L) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t* start = L.start[LEVEL];
+  while (true) {
+    L.hist[tid] = 0;
+    __syncthreads();
+    sort_each(x, n, [&](uint32_t v) { atomicAdd(&L.hist[(v >> shift) & 255u], 1u); });
+    __syncthreads();
+    const uint32_t c = L.hist[tid];
+    if (!__syncthreads_or(c == n) || shift == 0) break;
+    shift = shift > 8 ? shift - 8 : 0;  // all in one bucket: by the next bits
+  }
+  const uint32_t c = L.hist[tid], incl = wave_incl_scan(c);
+  if (lane == 63) L.wsum[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w)
+    if (w < wave) before += L.wsum[w];
+  start[tid + 1] = before + incl;
+  if (tid == 0) start[0] = 0;
+  L.hist[tid] = before + incl - c;
+  __syncthreads();
+  sort_each(x, n, [&](uint32_t v) { y[atomicAdd(&L.hist[(v >> shift) & 255u], 1u)] = v; });
+  __syncthreads();  // the buckets are written
+  uint32_t b = 0;
+  while (b < 256) {
+    const uint32_t s = start[b];
+    uint32_t e = b;
+    while (e < 256 && start[e + 1] - s <= SORT_LDS) ++e;  // uniform
+    if (e > b) {
+      const uint32_t m = start[e] - s;
+      if (m) {
+        for (uint32_t i = tid; i < m; i += 256) L.a[i] = y[s + i];
+        sort_lds(L.a, m);
+        for (uint32_t i = tid; i < m; i += 256) o[s + i] = L.a[i];
+        __syncthreads();
+      }
+      b = e;
+    } else {
+      if constexpr (LEVEL + 1 < SORT_LEVELS)
+        sort_long<LEVEL + 1>(y + s, x + s, o + s, start[b + 1] - s, shift > 8 ? shift - 8 : 0, L);
+      ++b;
+    }
+  }
+}
+// bits: the values lie below 1 << bits.
 __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
                                                         const uint32_t* __restrict__ order, const uint32_t* __restrict__ counters,
-                                                        uint32_t cap, const uint32_t* __restrict__ in,
-                                                        uint32_t* __restrict__ out) {
-  __shared__ uint32_t a[SORT_LDS];
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t s_n, s_below, s_k;
+                                                        uint32_t cap, uint32_t bits, uint32_t* in, uint32_t* out) {
+  __shared__ sort_space L;
   if (record_total(counters) > cap) return;  // records were dropped: the draw is emitted again
   const uint32_t t = scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x), t0 = ts[t], n = te[t] - t0, tid = threadIdx.x;
-  if (n <= SORT_LDS) {
-    if (n == 0) return;
-    for (uint32_t i = tid; i < n; i += 256) a[i] = in[t0 + i];
-    if (n > 1) sort_lds(a, n);
-    for (uint32_t i = tid; i < n; i += 256) out[t0 + i] = a[i];
+  if (n > SORT_LDS) {
+    sort_long<0>(in + t0, out + t0, out + t0, n, bits > 8 ? bits - 8 : 0, L);
     return;
   }
-  uint64_t lo = 0, hi = 1ull << 32;  // values in [lo, hi) are looked at; those below lo are written
-  uint32_t done = 0;
-  while (done < n) {
-    uint32_t shift = 0;  // at most 256 buckets of 1 << shift values
-    while (((hi - lo - 1) >> shift) > 255) ++shift;
-    hist[tid] = 0;
-    if (tid == 0) s_n = 0;
-    __syncthreads();
-    for (uint32_t i = tid; i < n; i += 256) {
-      const uint64_t v = in[t0 + i];
-      if (v >= lo && v < hi) atomicAdd(&hist[(v - lo) >> shift], 1u);
-    }
-    __syncthreads();
-    if (tid == 0) {  // the leading buckets that fit together
-      uint32_t k = 0, sum = 0;
-      while (k < 256 && sum + hist[k] <= SORT_LDS) sum += hist[k++];
-      s_k = k;
-      s_below = sum;
-    }
-    __syncthreads();
-    const uint32_t k = s_k, m = s_below;
-    if (k == 0) {  // the first bucket alone is too long: look into it
-      if (shift == 0) return;  // not reached: a value is in a list once
-      hi = lo + (1ull << shift);
-      __syncthreads();
-      continue;
-    }
-    const uint64_t end = min(hi, lo + (static_cast<uint64_t>(k) << shift));
-    for (uint32_t i = tid; i < n; i += 256) {
-      const uint64_t v = in[t0 + i];
-      if (v >= lo && v < end) a[atomicAdd(&s_n, 1u)] = static_cast<uint32_t>(v);
-    }
-    __syncthreads();
-    if (m > 1) sort_lds(a, m);
-    for (uint32_t i = tid; i < m; i += 256) out[t0 + done + i] = a[i];
-    __syncthreads();
-    done += m;
-    lo = end;
-    hi = 1ull << 32;
-  }
+  if (n == 0) return;
+  for (uint32_t i = tid; i < n; i += 256) L.a[i] = in[t0 + i];
+  if (n > 1) sort_lds(L.a, n);
+  for (uint32_t i = tid; i < n; i += 256) out[t0 + i] = L.a[i];
 }
 
 void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s) {
@@ -1648,9 +1677,12 @@ void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap
   const uint32_t per = 256 * SCATTER_PER_THREAD;
   hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max<uint32_t>(cap, 1) + per - 1) / per), dim3(256), 0, s, B.keys[0],
                      B.vals[0], B.keys[1], B.counters, cap, B.tstart, B.vals[1], mail, seq);
-  if (sorted)
-    hipLaunchKernelGGL(tile_sort_kernel, dim3(T), dim3(256), 0, s, B.tstart, B.tend, B.order, B.counters, cap, B.vals[1],
+  if (sorted) {
+    uint32_t bits = 1;  // the values are below 6 * prim_count
+    while (bits < 32 && (6ull * P.prim_count) >> bits) ++bits;
+    hipLaunchKernelGGL(tile_sort_kernel, dim3(T), dim3(256), 0, s, B.tstart, B.tend, B.order, B.counters, cap, bits, B.vals[1],
                        B.vals[0]);
+  }
 }
 
 // Scheduling order of the GPU tiles, heaviest first so that the longest tiles start early.  Tiles

@@ -55,6 +55,37 @@ def test_long_lists(hip_lib, cpu_lib, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ids", ["dense", "clusters", "sparse", "few_high"])
+def test_long_lists_in_primitive_order(hip_lib, cpu_lib, ids):
+    """Blended lists of 2,100 to 30,000 records on the same four tiles, their primitives consecutive, in clusters far
+    apart, spread over many that draw nothing, or all near the end (their leading bits agree)."""
+    n = {"dense": 30000, "clusters": 400000, "sparse": 400000, "few_high": 300001}[ids]
+    on = np.zeros(n, bool)
+    if ids == "dense":
+        on[:] = True
+    elif ids == "clusters":
+        on[:3000] = on[131072 - 1500: 131072 + 1500] = on[-2500:] = True
+    elif ids == "sparse":
+        on[::37] = True
+    else:
+        on[-2100:] = True
+    rng = np.random.default_rng(n)
+    pos = np.zeros((n, 3, 4), np.float32)  # off: no area
+    pos[..., 3] = 1
+    pos[on, :, :2] = rng.uniform(-1.5, 1.5, (on.sum(), 3, 2))
+    pos[on, :, 2] = rng.uniform(0.05, 0.95, (on.sum(), 3))
+    col = rng.uniform(0, 1, (3 * n, 4)).astype(np.float32) * (1, 1, 1, 1e-3)  # so faint that every layer tells
+    out = []
+    for lib in (hip_lib, cpu_lib):
+        r = lib.renderer()
+        t = Target(r, 20, 18, 1, A.PF_RGBA32F)
+        t.clear((0.1, 0.2, 0.3, 0.4))
+        keep = draw_colored(r, pos.reshape(-1, 4), col, blend=A.BLEND_ON, depth_func=A.CMP_ALWAYS)
+        out.append(t.color.read().copy())
+        del keep
+    assert np.array_equal(*out)
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
 def test_records_outgrow_the_buffers(hip_lib, cpu_lib, blend):
     """The first draw of a renderer emits more records than its buffers hold and is repeated; the second fits."""
