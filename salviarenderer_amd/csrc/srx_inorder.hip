@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(256) inorder_kernel(draw_params P, const ps_sa
   __shared__ unsigned long long fmask[16];          // records that cover the block whole
   __shared__ uint16_t work[IO_CHUNK * 16];
   __shared__ uint32_t nwork;
-  const int gtile = static_cast<int>(scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x));
+  const int gtile = static_cast<int>(order[blockIdx.x]);
   const uint32_t t0 = tstart[gtile], t1 = tend[gtile];
   if (t0 == t1 && !P.clear_ds && !P.clear_color) return;
   const int tid = threadIdx.x;

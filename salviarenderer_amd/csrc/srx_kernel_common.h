@@ -40,21 +40,6 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
   return v;
 }
 
-// The GPU tile of workgroup b of a single draw's raster pass (every class of tiles in turn, see
-// draw_buffers::order).
-__device__ __forceinline__ uint32_t scheduled_tile(const uint32_t* __restrict__ order, const uint32_t* __restrict__ classes,
-                                                   uint32_t T, uint32_t b) {
-  uint32_t at = b, k = 0;
-#pragma unroll
-  for (int c = 0; c < TILE_CLASSES - 1; ++c) {
-    const uint32_t n = classes[c];
-    const bool past = k == static_cast<uint32_t>(c) && at >= n;
-    at = past ? at - n : at;
-    k = past ? k + 1 : k;
-  }
-  return order[static_cast<size_t>(k) * T + at];
-}
-
 // Sums v over the workgroup and stores the total in partial[blockIdx.x] (no global atomics: many
 // same-address device-scope atomics from every XCD serialise badly).  All threads must call it.
 __device__ __forceinline__ void block_partial(unsigned long long* __restrict__ partial, unsigned long long v) {

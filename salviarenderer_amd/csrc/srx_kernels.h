@@ -74,9 +74,7 @@ struct draw_buffers {
   uint32_t* vals[2];   // records: triangle id << 1 | tile-level accept; [0] as emitted, [1] by tile
                        // (single draws that need primitive order: sorted back into [0])
   uint32_t list_cap;      // records the tiles' lists are formed for; with more the raster passes return at once
-  const uint32_t* order;  // workgroup launch order of the GPU tiles, heaviest record-count class first: single
-                          // draws, the tiles of class k at order[k * tiles], counters[CT_CLASS + k] of them
-                          // (scheduled_tile); batches, the tiles one after another
+  const uint32_t* order;  // workgroup launch order of the GPU tiles, heaviest record-count class first
   // Tiles of more than vis_part records are split into parts, each a workgroup of the visibility pass whose
   // per-sample keys a second launch merges: parts (tile, part, parts, 0) at their slot of vis_partial,
   // and (tile, parts, first slot, 0) per split tile (vis_split_bounds; vis_part 0: no tile is split)
@@ -164,14 +162,15 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
 // dropped) and count them per tile.
 void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
-// The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, the tiles by
-// record-count class in B.order (TILE_CLASSES * tiles words), and with B.vis_part the parts of split
-// tiles (when the count is within `cap`).  Lists: vals[1], or in primitive order vals[0] (`sorted`),
-// sized for `cap` records; the count is read from B.counters on the device.  The lists' launch
-// writes the draw's mail with sequence number `seq` (targets without GPU tiles: nothing is launched).
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s);
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, bool sorted, draw_mail* mail, uint32_t seq,
-                       hipStream_t s);
+// The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, each tile's
+// record-count class and rank in it (kept in B.partial until the lists' launch), and with B.vis_part the
+// parts of split tiles (when the count is within `cap`).  Lists: `order` (tiles words), and vals[1], or in
+// primitive order vals[0] (`sorted`), sized for `cap` records; the count is read from B.counters on the
+// device.  The lists' launch writes the draw's mail with sequence number `seq` (targets without GPU tiles:
+// nothing is launched).
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, hipStream_t s);
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
+                       uint32_t seq, hipStream_t s);
 // In-place exclusive scan of n u32; writes the total to *total_dev.  tmp holds >= scan_tmp_size(n).
 size_t scan_tmp_size(uint32_t n);
 void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* total_dev, hipStream_t s);

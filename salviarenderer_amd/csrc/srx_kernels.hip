@@ -1476,12 +1476,14 @@ __device__ __forceinline__ void bucket_range_body(const uint32_t* __restrict__ h
 }
 
 // ---------------------------------------------------------------- tile ranges of single draws
-// Each tile's range of the lists and its place in the scheduling order, both from cursors a wave takes
+// Each tile's range of the lists and its place in its record-count class, both from cursors a wave takes
 // its share of at once: neither the ranges nor the tiles of a class need an order, so no workgroup
-// waits for another's counts.  (A scan over all counts took 12 us whatever the number of tiles.)
+// waits for another's counts.  The lists' launch, which knows every class's count, makes the scheduling
+// order of the places.  (A scan over all counts took 12 us whatever the number of tiles.)
+constexpr uint32_t PLACE_BITS = 28;  // a place: class << PLACE_BITS | rank (targets have at most 2^18 GPU tiles)
 __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __restrict__ tile_count, uint32_t T, uint32_t N,
                                                           uint32_t shift, uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
-                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ order,
+                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ place,
                                                           uint32_t part, uint4* __restrict__ parts, uint4* __restrict__ merges,
                                                           uint32_t cap) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -1511,7 +1513,7 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
   if (valid) {
     ts[t] = base + incl - n;
     te[t] = base + incl;
-    order[static_cast<size_t>(c) * T + at] = t;
+    place[t] = (c << PLACE_BITS) | at;
     if (part && n > part && record_total(counters) <= cap) {  // with more records the tables' bounds do not hold
       const uint32_t np = (n + part - 1) / part;
       const uint32_t e = atomicAdd(&counters[CT_PARTS], np);
@@ -1520,18 +1522,26 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     }
   }
 }
-// The records to their tiles' lists: position = first record of the tile + rank in the tile.
+// The scheduling order, and the records to their tiles' lists: position = first record of the tile + rank in it.
 constexpr uint32_t SCATTER_PER_THREAD = 4;
 __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
                                                            const uint32_t* __restrict__ ranks,
                                                            const uint32_t* __restrict__ counters, uint32_t cap,
                                                            const uint32_t* __restrict__ ts, uint32_t* __restrict__ vout,
-                                                           draw_mail* mail, uint32_t seq) {
+                                                           uint32_t T, const uint32_t* __restrict__ place,
+                                                           uint32_t* __restrict__ order, draw_mail* mail, uint32_t seq) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {  // every count is final; the host waits for seq
     mail->total = record_total(counters);
     mail->merges = counters[CT_MERGES];
     mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
     __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < T; t += gridDim.x * 256) {
+    const uint32_t c = place[t] >> PLACE_BITS;
+    uint32_t at = place[t] & ((1u << PLACE_BITS) - 1u);
+#pragma unroll
+    for (uint32_t k = 0; k + 1 < TILE_CLASSES; ++k) at += k < c ? counters[CT_CLASS + k] : 0u;
+    order[at] = t;
   }
   const uint32_t n = min(record_total(counters), cap);
   const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
@@ -1652,7 +1662,7 @@ __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restri
                                                         uint32_t cap, uint32_t bits, uint32_t* in, uint32_t* out) {
   __shared__ sort_space L;
   if (record_total(counters) > cap) return;  // records were dropped: the draw is emitted again
-  const uint32_t t = scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x), t0 = ts[t], n = te[t] - t0, tid = threadIdx.x;
+  const uint32_t t = order[blockIdx.x], t0 = ts[t], n = te[t] - t0, tid = threadIdx.x;
   if (n > SORT_LDS) {
     sort_long<0>(in + t0, out + t0, out + t0, n, bits > 8 ? bits - 8 : 0, L);
     return;
@@ -1663,20 +1673,21 @@ __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restri
   for (uint32_t i = tid; i < n; i += 256) out[t0 + i] = L.a[i];
 }
 
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, hipStream_t s) {
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t N = tile_slots(T), shift = tile_slot_shift(T);
   hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
-                     B.counters, order, B.vis_part, B.vis_parts, B.vis_merges, cap);
+                     B.counters, reinterpret_cast<uint32_t*>(B.partial), B.vis_part, B.vis_parts, B.vis_merges, cap);
 }
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, bool sorted, draw_mail* mail, uint32_t seq,
-                       hipStream_t s) {
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
+                       uint32_t seq, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t per = 256 * SCATTER_PER_THREAD;
-  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max<uint32_t>(cap, 1) + per - 1) / per), dim3(256), 0, s, B.keys[0],
-                     B.vals[0], B.keys[1], B.counters, cap, B.tstart, B.vals[1], mail, seq);
+  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max(cap, T) + per - 1) / per), dim3(256), 0, s, B.keys[0], B.vals[0],
+                     B.keys[1], B.counters, cap, B.tstart, B.vals[1], T, reinterpret_cast<const uint32_t*>(B.partial), order,
+                     mail, seq);
   if (sorted) {
     uint32_t bits = 1;  // the values are below 6 * prim_count
     while (bits < 32 && (6ull * P.prim_count) >> bits) ++bits;

@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(256) raster_kernel(draw_params P, const ps_sam
   }
   extern __shared__ prim_lds lds[];
   const int G = P.gt, QW = G / 2;
-  const int gtile = static_cast<int>(scheduled_tile(order, counters + CT_CLASS, gridDim.x, blockIdx.x));
+  const int gtile = static_cast<int>(order[blockIdx.x]);
   const int gx = gtile % P.gtiles_x, gy = gtile / P.gtiles_x;
   const int tid = threadIdx.x, nthreads = blockDim.x;
   const int qx = tid % QW, qy = tid / QW;

@@ -297,7 +297,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   RCHK(X.take(r->tend, std::max<uint32_t>(T, 1), B.tend));
   RCHK(X.take(r->tile_count, std::max<uint32_t>(tile_slots(T), 1), B.tile_count));
   uint32_t* order = nullptr;
-  RCHK(X.take(r->order, static_cast<size_t>(TILE_CLASSES) * std::max<uint32_t>(T, 1), order));
+  RCHK(X.take(r->order, std::max<uint32_t>(T, 1), order));
   B.order = order;
   // clipping capacity for every primitive, so no read-back decides whether clipping runs
   RCHK(X.take(r->clip_verts, static_cast<size_t>(primcnt) * 5 * (nout + 1), B.clip_verts));
@@ -429,8 +429,8 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
       }
     }
     B.list_cap = sized;
-    launch_tile_ranges(P, B, sized, order, s);
-    launch_tile_lists(P, B, sized, !order_free, r->mail, T ? ++r->mail_seq : r->mail_seq, s);
+    launch_tile_ranges(P, B, sized, s);
+    launch_tile_lists(P, B, sized, order, !order_free, r->mail, T ? ++r->mail_seq : r->mail_seq, s);
     mark(4);
     fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, s);
     if (!fused) {

@@ -780,8 +780,7 @@ __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, 
     ws.t0 = V.tstart[e.x] + e.y * V.part;
     ws.t1 = min(V.tend[e.x], ws.t0 + V.part);
   } else {
-    const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
-    const uint32_t t = scheduled_tile(V.order, V.counters + CT_CLASS, T, b - V.max_parts);
+    const uint32_t t = V.order[b - V.max_parts];
     ws.tile = static_cast<int>(t);
     ws.t0 = V.tstart[t];
     ws.t1 = V.tend[t];

@@ -7,6 +7,8 @@ import pytest
 from salviarenderer_amd import api as A
 from salviarenderer_amd import scenes as S
 
+from helpers import Target, draw_colored
+
 pytestmark = pytest.mark.gpu
 
 
@@ -70,3 +72,24 @@ def test_noalloc_refuses_what_does_not_fit(hip_lib):
     small.render()
     r.flush()
     assert np.array_equal(got, small.color.read())
+
+
+def test_noalloc_blends_on_a_large_target(hip_lib):
+    """60,000 blended triangles on 262,144 GPU tiles take 52 of the region's 64 MiB: what a tile takes besides
+    the triangles' 800 bytes has to stay below 40."""
+    n, side = 60_000, 8191
+    rng = np.random.default_rng(2)
+    pos = np.concatenate([rng.uniform(-1, 1, (n, 1, 2)) + rng.uniform(-1e-3, 1e-3, (n, 3, 2)), rng.uniform(0.1, 0.9, (n, 3, 1)),
+                          np.ones((n, 3, 1))], -1)
+    col = rng.uniform(0.2, 1, (3 * n, 4))
+    out = []
+    for noalloc in (True, False):
+        r = hip_lib.renderer()
+        if noalloc:
+            r.draw = r.draw_noalloc
+        t = Target(r, side, side)
+        t.clear((0.1, 0.2, 0.3, 0.4))
+        keep = draw_colored(r, pos.reshape(-1, 4), col, blend=A.BLEND_ON)
+        out.append(t.color.read().copy())
+        del keep
+    assert np.array_equal(*out) and len(np.unique(out[0][::7, ::7].reshape(-1, 4), axis=0)) > 1
