@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "srx_device.h"
+#include "srx_vis_rules.h"
 
 namespace srx {
 
@@ -75,13 +76,13 @@ struct draw_buffers {
                        // (single draws that need primitive order: sorted back into [0])
   uint32_t list_cap;      // records the tiles' lists are formed for; with more the raster passes return at once
   const uint32_t* order;  // workgroup launch order of the GPU tiles, heaviest record-count class first
-  // Tiles of more than vis_part records are split into parts, each a workgroup of the visibility pass whose
+  // With vis_split, tiles of more than vis_part() records are split into parts, each a workgroup of the pass whose
   // per-sample keys a second launch merges: parts (tile, part, parts, 0) at their slot of vis_partial,
-  // and (tile, parts, first slot, 0) per split tile (vis_split_bounds; vis_part 0: no tile is split)
+  // and (tile, parts, first slot, 0) per split tile (vis_split_bounds)
   uint4* vis_parts;
   uint4* vis_merges;
   unsigned long long* vis_partial;  // the parts' keys
-  uint32_t vis_part;
+  bool vis_split;
   uint32_t* tstart;    // GPU tiles
   uint32_t* tile_count;  // tile_slots(T) words: records per tile, at tile_slot (zero before the setup launch)
   uint32_t* tend;
@@ -163,7 +164,7 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
 void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 // The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, each tile's
-// record-count class and rank in it (kept in B.partial until the lists' launch), and with B.vis_part the
+// record-count class and rank in it (kept in B.partial until the lists' launch), and with B.vis_split the
 // parts of split tiles (when the count is within `cap`).  Lists: `order` (tiles words), and vals[1], or in
 // primitive order vals[0] (`sorted`), sized for `cap` records; the count is read from B.counters on the
 // device.  The lists' launch writes the draw's mail with sequence number `seq` (targets without GPU tiles:
@@ -188,11 +189,6 @@ void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipS
 // that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles.
 bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
                 hipStream_t s);
-// Records per part of a split tile for a visibility pass over `prims` primitives and `records` expected
-// records (0: no tile can be split), and upper bounds of the parts and split tiles for at most `records`
-// records (a part takes 256 * samples keys of vis_partial).
-uint32_t vis_part_size(uint32_t prims, uint32_t records);
-void vis_split_bounds(uint32_t part, uint32_t records, uint32_t* parts, uint32_t* merges);
 bool needs_shading(const draw_params& P);
 // A SASL pixel shader whose colour is written: such draws run the in-order raster kernel.
 bool sasl_shades(const draw_params& P);

@@ -1484,7 +1484,7 @@ constexpr uint32_t PLACE_BITS = 28;  // a place: class << PLACE_BITS | rank (tar
 __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __restrict__ tile_count, uint32_t T, uint32_t N,
                                                           uint32_t shift, uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
                                                           uint32_t* __restrict__ counters, uint32_t* __restrict__ place,
-                                                          uint32_t part, uint4* __restrict__ parts, uint4* __restrict__ merges,
+                                                          bool split, uint32_t prims, uint4* __restrict__ parts, uint4* __restrict__ merges,
                                                           uint32_t cap) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   const int lane = __lane_id();
@@ -1514,7 +1514,8 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     ts[t] = base + incl - n;
     te[t] = base + incl;
     place[t] = (c << PLACE_BITS) | at;
-    if (part && n > part && record_total(counters) <= cap) {  // with more records the tables' bounds do not hold
+    const uint32_t total = record_total(counters), part = vis_part(prims, total);
+    if (split && n > part && total <= cap) {  // with more records the tables' bounds do not hold
       const uint32_t np = (n + part - 1) / part;
       const uint32_t e = atomicAdd(&counters[CT_PARTS], np);
       merges[atomicAdd(&counters[CT_MERGES], 1u)] = make_uint4(t, np, e, 0u);
@@ -1678,7 +1679,7 @@ void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t ca
   if (!T) return;
   const uint32_t N = tile_slots(T), shift = tile_slot_shift(T);
   hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
-                     B.counters, reinterpret_cast<uint32_t*>(B.partial), B.vis_part, B.vis_parts, B.vis_merges, cap);
+                     B.counters, reinterpret_cast<uint32_t*>(B.partial), B.vis_split, P.prim_count, B.vis_parts, B.vis_merges, cap);
 }
 void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
                        uint32_t seq, hipStream_t s) {

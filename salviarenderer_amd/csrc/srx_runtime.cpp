@@ -235,7 +235,7 @@ static size_t record_scratch_bytes(uint32_t prims, int samples, bool vis_tables,
   size_t b = 4 * align256(rn * 4);
   if (vis_tables) {
     uint32_t np, nm;
-    vis_split_bounds(vis_part_size(prims, n), n, &np, &nm);
+    vis_split_bounds(prims, n, &np, &nm);
     b += align256(static_cast<size_t>(np) * 16) + align256(static_cast<size_t>(nm) * 16) +
          align256(static_cast<size_t>(np) * 256 * samples * 8);
   }
@@ -353,7 +353,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   };
   // A draw whose triangles cannot have more records than the lists are formed for (each lies on a tile at
   // most once) nor split a tile need not be waited for.
-  const bool bounded = static_cast<uint64_t>(P3) * T <= sized && vis_part_size(primcnt, sized) == 0;
+  const bool bounded = static_cast<uint64_t>(P3) * T <= sized && !vis_can_split(primcnt);
   // sampler table: staged in pinned memory (reused once the last draw's mail shows that its copy has
   // run); a renderer's own table is uploaded only when it changed
   const bool same_table = !fixed && r->samplers_valid && samplers_d == r->samplers_last_d &&
@@ -420,9 +420,9 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   auto raster = [&]() -> int32_t {
     if (vis_tables) {
       uint32_t np, nm;
-      B.vis_part = vis_part_size(primcnt, sized);
-      vis_split_bounds(B.vis_part, sized, &np, &nm);
-      if (B.vis_part) {
+      B.vis_split = vis_can_split(primcnt);
+      vis_split_bounds(primcnt, sized, &np, &nm);
+      if (B.vis_split) {
         RCHK(X.take(r->vis_parts, np, B.vis_parts));
         RCHK(X.take(r->vis_merges, nm, B.vis_merges));
         RCHK(X.take(r->vis_partial, static_cast<size_t>(np) * 256 * samples, B.vis_partial));

@@ -297,23 +297,6 @@ __host__ __device__ constexpr int vis_union_bytes(int nt, int s, bool shade, int
   const int chunk = nt * 64 + nt * (gt / 4) * (gt / 4) * 2 + nt * 8;
   return chunk > (shade ? gt * gt * s * 8 : 0) ? chunk : gt * gt * s * 8;
 }
-// Records of a tile taken before depth culling begins: few for draws whose triangles lie on VIS_LARGE or
-// more GPU tiles on average, whose lists are deep (of the 323 records a tile of the 2,000-triangle
-// plain scene has, 50 of the last 259 survive: 60 -> 35 us); a whole chunk for draws of smaller ones,
-// which seldom cover a tile before its list ends (64 there: 161 -> 186 us for the mesh that fills the
-// target).
-constexpr uint32_t VIS_FIRST = 64, VIS_LARGE = 4;
-__host__ __device__ inline bool vis_large(uint64_t records, uint32_t prims) {
-  return records >= static_cast<uint64_t>(VIS_LARGE) * prims;
-}
-// A tile's time is its list's length, so lists much longer than an even share of the records over the
-// workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame at the
-// oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
-// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where every tile's list is near
-// the even share a split only adds work.  Draws of large triangles, whose lists depth culling
-// shortens as it goes, are split later.
-constexpr uint32_t VIS_PART_SMALL = 1024, VIS_PART_LARGE = 2048, VIS_SLOTS = 640;
-
 // S (depth, stencil) pairs of a pixel as wide stores (surfaces are allocated at 256-byte alignment, so a
 // pixel's samples start at a multiple of their size).
 template <int S>
@@ -760,13 +743,15 @@ struct vis_lists {
   const uint32_t *order, *vals, *tstart, *tend, *counters;
   const uint4 *parts, *merges;
   unsigned long long* partial;
-  uint32_t cap, part, max_parts, first;
+  uint32_t cap, max_parts;
 };
 template <int NA, int S, bool SHADE>
 __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, vis_lists V,
                                                    const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
                                                    const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
-  if (record_total(V.counters) > V.cap) return;  // records were dropped: the draw is emitted again
+  const uint32_t records = record_total(V.counters);
+  if (records > V.cap) return;  // records were dropped: the draw is emitted again
+  const uint32_t part = vis_part(P.prim_count, records);
   vis_span ws;
   ws.parts = 1;
   ws.slot = 0;
@@ -777,16 +762,17 @@ __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, 
     ws.tile = static_cast<int>(e.x);
     ws.parts = e.z;
     ws.slot = b;
-    ws.t0 = V.tstart[e.x] + e.y * V.part;
-    ws.t1 = min(V.tend[e.x], ws.t0 + V.part);
+    ws.t0 = V.tstart[e.x] + e.y * part;
+    ws.t1 = min(V.tend[e.x], ws.t0 + part);
   } else {
     const uint32_t t = V.order[b - V.max_parts];
     ws.tile = static_cast<int>(t);
     ws.t0 = V.tstart[t];
     ws.t1 = V.tend[t];
-    if (V.part && ws.t1 - ws.t0 > V.part) return;  // its parts take it
+    if (V.max_parts && ws.t1 - ws.t0 > part) return;  // its parts take it
   }
-  vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, ws, V.partial, V.vals, tri_rec, tri_attr, SM, V.first, wout);
+  vis_body<NA, S, SHADE, SRX_VIS_THREADS, 16>(P, mode, ws, V.partial, V.vals, tri_rec, tri_attr, SM,
+                                              vis_large(records, P.prim_count) ? VIS_FIRST : SRX_VIS_THREADS, wout);
 }
 
 // One split tile per workgroup: its keys are the minimum of the parts' keys (each started from the
@@ -849,15 +835,6 @@ int vis_mode(const draw_params& P) {
   }
 }
 
-uint32_t vis_part_size(uint32_t prims, uint32_t records) {
-  const uint32_t part = std::max(vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL, records / VIS_SLOTS);
-  return 3ull * prims > part ? part : 0u;  // a primitive gives at most three triangles, each once on a tile
-}
-void vis_split_bounds(uint32_t part, uint32_t records, uint32_t* parts, uint32_t* merges) {
-  *parts = part ? 2 * (records / part + 1) : 0;  // ceil(n / part) < 2 n / part for n > part
-  *merges = part ? records / (part + 1) + 1 : 0;
-}
-
 bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
                 hipStream_t s) {
   int mode = vis_mode(P);
@@ -868,10 +845,9 @@ bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool sha
   if (mode < 0 || P.gt != 16) return false;
   if (!T) return true;
   uint32_t np, nm;
-  vis_split_bounds(B.vis_part, records, &np, &nm);
+  vis_split_bounds(P.prim_count, records, &np, &nm);
   const vis_lists V{B.order, B.vals[which], B.tstart, B.tend, B.counters, B.vis_parts, B.vis_merges, B.vis_partial,
-                    B.list_cap, B.vis_part, np,
-                    vis_large(records, P.prim_count) ? std::min<uint32_t>(VIS_FIRST, SRX_VIS_THREADS) : SRX_VIS_THREADS};
+                    B.list_cap, B.vis_split ? np : 0u};
 #define SRX_VIS_LAUNCH(NA, S, SH)                                                                                       \
   if (merges)                                                                                                           \
     hipLaunchKernelGGL((vis_merge_kernel<NA, S, SH>), dim3(merges), dim3(VIS_MERGE_THREADS), 0, s, P, mode, V, B.tri_rec, \

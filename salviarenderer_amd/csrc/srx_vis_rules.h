@@ -1,0 +1,49 @@
+// Rules of the visibility pass that depend on a draw's record count, for host and device code: when depth
+// culling begins and which tiles are split.  The device applies them to the draw's own count; the host, which
+// does not know it yet, sizes the tables for every count up to the lists' capacity.
+#pragma once
+
+#include <stdint.h>
+
+#ifdef __HIPCC__
+#define SRX_HD __host__ __device__
+#else
+#define SRX_HD
+#endif
+
+namespace srx {
+
+// Records of a tile taken before depth culling begins: few for draws whose triangles lie on VIS_LARGE or
+// more GPU tiles on average, whose lists are deep (of the 323 records a tile of the 2,000-triangle
+// plain scene has, 50 of the last 259 survive: 60 -> 35 us); a whole chunk for draws of smaller ones,
+// which seldom cover a tile before its list ends (64 there: 161 -> 186 us for the mesh that fills the
+// target).
+constexpr uint32_t VIS_FIRST = 64, VIS_LARGE = 4;
+SRX_HD inline bool vis_large(uint64_t records, uint32_t prims) {
+  return records >= static_cast<uint64_t>(VIS_LARGE) * prims;
+}
+
+// A tile's time is its list's length, so lists much longer than an even share of the records over the
+// workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame at the
+// oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
+// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where every tile's list is near
+// the even share a split only adds work.  Draws of large triangles, whose lists depth culling
+// shortens as it goes, are split later.
+constexpr uint32_t VIS_PART_SMALL = 1024, VIS_PART_LARGE = 2048, VIS_SLOTS = 640;
+// Records per part of a draw with `records` records: a tile with more is split.
+SRX_HD inline uint32_t vis_part(uint32_t prims, uint32_t records) {
+  const uint32_t least = vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL, share = records / VIS_SLOTS;
+  return least > share ? least : share;
+}
+// Draws of which no tile is split: a primitive gives at most three triangles, each once on a tile.
+SRX_HD inline bool vis_can_split(uint32_t prims) { return 3ull * prims > VIS_PART_LARGE; }
+// Upper bounds of the parts and split tiles of a draw with at most `records` records: a tile of n > part
+// records has ceil(n / part) < 2 n / part parts, and records / part is at most records / VIS_PART_SMALL and
+// VIS_SLOTS.  A part takes 256 * samples keys.
+SRX_HD inline void vis_split_bounds(uint32_t prims, uint32_t records, uint32_t* parts, uint32_t* tiles) {
+  const uint32_t most = records / VIS_PART_SMALL < VIS_SLOTS ? records / VIS_PART_SMALL : VIS_SLOTS;
+  *parts = vis_can_split(prims) ? 2 * (most + 1) : 0;
+  *tiles = vis_can_split(prims) ? most + 1 : 0;
+}
+
+}  // namespace srx

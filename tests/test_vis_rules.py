@@ -1,0 +1,51 @@
+"""The visibility pass's rules on record counts (csrc/srx_vis_rules.h), compiled for the host: the tables sized for a
+capacity hold the parts and split tiles of every draw within it."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <cstdio>
+#include <random>
+#include <vector>
+#include "srx_vis_rules.h"
+using namespace srx;
+int main() {
+  std::mt19937_64 rng(1);
+  int bad = 0;
+  auto below = [&](uint64_t n) { return rng() % n; };
+  for (int it = 0; it < 20000; ++it) {
+    const uint32_t cap = uint32_t(1) << (8 + below(24)), total = uint32_t(below(uint64_t(cap) + 1));
+    const uint32_t prims = uint32_t(1 + below(it % 2 ? 100000 : 1u << 30));
+    uint32_t np, nt, parts = 0, tiles = 0;
+    vis_split_bounds(prims, cap, &np, &nt);
+    const uint32_t part = vis_part(prims, total);
+    if (vis_can_split(prims)) {
+      for (uint64_t left = total; left;) {  // lists just above a multiple of the part, or of any length
+        uint64_t n = it % 3 ? part + 1 + part * below(3) : 1 + below(left);
+        n = n < left ? n : left;
+        left -= n;
+        if (n > part) parts += uint32_t((n + part - 1) / part), ++tiles;
+        if (!(it % 3) && left < total / 64) break;
+      }
+    }
+    if (parts > np || tiles > nt) ++bad, std::printf("cap %u total %u prims %u: %u parts of %u, %u tiles of %u\n", cap, total, prims, parts, np, tiles, nt);
+  }
+  // a mesh of small triangles, and its neighbours on either side of the rule
+  if (vis_large(24000, 16384) || vis_part(16384, 24000) != VIS_PART_SMALL) ++bad;
+  if (vis_large(4 * 16384 - 1, 16384) || !vis_large(4 * 16384, 16384)) ++bad;
+  if (vis_part(2000, 330000) != VIS_PART_LARGE || vis_part(1u << 22, 6400000) != 10000) ++bad;
+  if (vis_can_split(682) || !vis_can_split(683)) ++bad;
+  return bad != 0;
+}
+"""
+
+
+def test_rules_on_the_host(tmp_path):
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "salviarenderer_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert res.returncode == 0, res.stdout
