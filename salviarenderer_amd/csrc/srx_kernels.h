@@ -21,7 +21,7 @@ enum stat_slot {
 // bits (setup alone cannot: at most four records a primitive, whose buffers take over 600 bytes); read the
 // count with record_total.
 // CT_CURSOR: records given to the tiles' lists; CT_PARTS, CT_MERGES: parts of split tiles and split tiles;
-// CT_CLASS: GPU tiles per record-count class.
+// CT_CLASS: GPU tiles per record-count class (the last class: without records).
 constexpr int TILE_CLASSES = 16;
 enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_PARTS, CT_MERGES,
                     CT_OVERRUN, CT_CLASS,
@@ -29,6 +29,10 @@ enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP
 // Records of a single draw, 0xFFFFFFFF when the count does not fit (above every capacity).
 __host__ __device__ inline uint32_t record_total(const uint32_t* counters) {
   return counters[CT_OVERRUN] ? 0xFFFFFFFFu : counters[CT_TOTAL];
+}
+// GPU tiles with records, of T (once the ranges' launch has run).
+__host__ __device__ inline uint32_t busy_tiles(const uint32_t* counters, uint32_t T) {
+  return T - counters[CT_CLASS + TILE_CLASSES - 1];
 }
 constexpr uint32_t MAX_RECORDS = 0xFFFFFFF0u;  // a draw with more is refused
 static_assert(CT_TOTAL % 2 == 0 && CT_WIDE == CT_TOTAL + 1, "one aligned 64-bit word");
@@ -55,6 +59,10 @@ __host__ __device__ inline uint32_t tile_slots(uint32_t T) {
 // What the host needs to know of a single draw, written by the device into pinned host memory: seq last.
 struct draw_mail {
   uint32_t seq, total, merges, clip_overflow;
+};
+struct mail_slot {
+  draw_mail* mail;  // null: another launch of the draw writes it
+  uint32_t seq;
 };
 
 // Per-draw device buffers (owned by the renderer, grown on demand).
@@ -83,6 +91,7 @@ struct draw_buffers {
   uint4* vis_merges;
   unsigned long long* vis_partial;  // the parts' keys
   bool vis_split;
+  uint32_t tile_cost;  // vis_tile_cost of the draw
   uint32_t* tstart;    // GPU tiles
   uint32_t* tile_count;  // tile_slots(T) words: records per tile, at tile_slot (zero before the setup launch)
   uint32_t* tend;
@@ -164,14 +173,14 @@ void launch_vs(const draw_params& P, float4* vbuf, uint32_t* counters, uint32_t*
 void launch_setup(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity, hipStream_t s);
 // The tiles' record lists from the emitted records, in two steps.  Ranges: tstart/tend, each tile's
-// record-count class and rank in it (kept in B.partial until the lists' launch), and with B.vis_split the
-// parts of split tiles (when the count is within `cap`).  Lists: `order` (tiles words), and vals[1], or in
+// record-count class and rank in it (kept in B.partial until the lists' launch).  Lists: `order` (tiles
+// words), with B.vis_split the parts of split tiles (when the count is within `cap`), and vals[1], or in
 // primitive order vals[0] (`sorted`), sized for `cap` records; the count is read from B.counters on the
-// device.  The lists' launch writes the draw's mail with sequence number `seq` (targets without GPU tiles:
-// nothing is launched).
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, hipStream_t s);
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
-                       uint32_t seq, hipStream_t s);
+// device.  The lists' launch writes the draw's mail, if it is given (targets without GPU tiles: nothing is
+// launched).
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, hipStream_t s);
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, mail_slot mail,
+                       hipStream_t s);
 // In-place exclusive scan of n u32; writes the total to *total_dev.  tmp holds >= scan_tmp_size(n).
 size_t scan_tmp_size(uint32_t n);
 void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* total_dev, hipStream_t s);
@@ -186,9 +195,10 @@ bool inorder_takes_color_clear(const draw_params& P);
 void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
 // Order-independent visibility (and, with shade, the deferred pixel shader) of an opaque early-Z draw,
 // laid out for `records` records; false when the draw needs the in-order kernel.  merges > 0: finishes
-// that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles.
+// that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles and written the
+// draw's mail, if it is given.
 bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
-                hipStream_t s);
+                mail_slot mail, hipStream_t s);
 bool needs_shading(const draw_params& P);
 // A SASL pixel shader whose colour is written: such draws run the in-order raster kernel.
 bool sasl_shades(const draw_params& P);

@@ -1483,9 +1483,7 @@ __device__ __forceinline__ void bucket_range_body(const uint32_t* __restrict__ h
 constexpr uint32_t PLACE_BITS = 28;  // a place: class << PLACE_BITS | rank (targets have at most 2^18 GPU tiles)
 __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __restrict__ tile_count, uint32_t T, uint32_t N,
                                                           uint32_t shift, uint32_t* __restrict__ ts, uint32_t* __restrict__ te,
-                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ place,
-                                                          bool split, uint32_t prims, uint4* __restrict__ parts, uint4* __restrict__ merges,
-                                                          uint32_t cap) {
+                                                          uint32_t* __restrict__ counters, uint32_t* __restrict__ place) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   const int lane = __lane_id();
   const uint32_t t = slot_tile(i, shift);
@@ -1514,37 +1512,39 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     ts[t] = base + incl - n;
     te[t] = base + incl;
     place[t] = (c << PLACE_BITS) | at;
-    const uint32_t total = record_total(counters), part = vis_part(prims, total);
-    if (split && n > part && total <= cap) {  // with more records the tables' bounds do not hold
-      const uint32_t np = (n + part - 1) / part;
-      const uint32_t e = atomicAdd(&counters[CT_PARTS], np);
-      merges[atomicAdd(&counters[CT_MERGES], 1u)] = make_uint4(t, np, e, 0u);
-      for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
-    }
   }
 }
-// The scheduling order, and the records to their tiles' lists: position = first record of the tile + rank in it.
+// The scheduling order, the parts of split tiles, and the records to their tiles' lists: position = first record of the tile + rank in it.
 constexpr uint32_t SCATTER_PER_THREAD = 4;
 __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
                                                            const uint32_t* __restrict__ ranks,
                                                            const uint32_t* __restrict__ counters, uint32_t cap,
-                                                           const uint32_t* __restrict__ ts, uint32_t* __restrict__ vout,
+                                                           const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
+                                                           uint32_t* __restrict__ vout,
                                                            uint32_t T, const uint32_t* __restrict__ place,
-                                                           uint32_t* __restrict__ order, draw_mail* mail, uint32_t seq) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {  // every count is final; the host waits for seq
-    mail->total = record_total(counters);
-    mail->merges = counters[CT_MERGES];
-    mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
-    __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+                                                           uint32_t* __restrict__ order, bool split, uint32_t prims,
+                                                           uint32_t tile_cost, uint32_t* __restrict__ ct_parts,
+                                                           uint32_t* __restrict__ ct_merges, uint4* __restrict__ parts,
+                                                           uint4* __restrict__ merges, mail_slot mail) {
+  if (mail.mail && blockIdx.x == 0 && threadIdx.x == 0) send_mail(mail, counters);
+  const uint32_t total = record_total(counters);
   for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < T; t += gridDim.x * 256) {
     const uint32_t c = place[t] >> PLACE_BITS;
     uint32_t at = place[t] & ((1u << PLACE_BITS) - 1u);
 #pragma unroll
     for (uint32_t k = 0; k + 1 < TILE_CLASSES; ++k) at += k < c ? counters[CT_CLASS + k] : 0u;
     order[at] = t;
+    if (split && total <= cap) {  // with more records the tables' bounds do not hold
+      const uint32_t len = te[t] - ts[t], part = vis_part(prims, total, busy_tiles(counters, T), tile_cost);
+      if (len > part) {
+        const uint32_t np = (len + part - 1) / part;
+        const uint32_t e = atomicAdd(ct_parts, np);
+        merges[atomicAdd(ct_merges, 1u)] = make_uint4(t, np, e, 0u);
+        for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
+      }
+    }
   }
-  const uint32_t n = min(record_total(counters), cap);
+  const uint32_t n = min(total, cap);
   const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
   if (b0 >= n) return;
   uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
@@ -1674,21 +1674,22 @@ __global__ void __launch_bounds__(256) tile_sort_kernel(const uint32_t* __restri
   for (uint32_t i = tid; i < n; i += 256) out[t0 + i] = L.a[i];
 }
 
-void launch_tile_ranges(const draw_params& P, const draw_buffers& B, uint32_t cap, hipStream_t s) {
+void launch_tile_ranges(const draw_params& P, const draw_buffers& B, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t N = tile_slots(T), shift = tile_slot_shift(T);
   hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
-                     B.counters, reinterpret_cast<uint32_t*>(B.partial), B.vis_split, P.prim_count, B.vis_parts, B.vis_merges, cap);
+                     B.counters, reinterpret_cast<uint32_t*>(B.partial));
 }
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
-                       uint32_t seq, hipStream_t s) {
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, mail_slot mail,
+                       hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t per = 256 * SCATTER_PER_THREAD;
   hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max(cap, T) + per - 1) / per), dim3(256), 0, s, B.keys[0], B.vals[0],
-                     B.keys[1], B.counters, cap, B.tstart, B.vals[1], T, reinterpret_cast<const uint32_t*>(B.partial), order,
-                     mail, seq);
+                     B.keys[1], B.counters, cap, B.tstart, B.tend, B.vals[1], T, reinterpret_cast<const uint32_t*>(B.partial),
+                     order, B.vis_split, P.prim_count, B.tile_cost, B.counters + CT_PARTS,
+                     B.counters + CT_MERGES, B.vis_parts, B.vis_merges, mail);
   if (sorted) {
     uint32_t bits = 1;  // the values are below 6 * prim_count
     while (bits < 32 && (6ull * P.prim_count) >> bits) ++bits;

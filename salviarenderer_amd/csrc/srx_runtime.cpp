@@ -420,7 +420,8 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   auto raster = [&]() -> int32_t {
     if (vis_tables) {
       uint32_t np, nm;
-      B.vis_split = vis_can_split(primcnt);
+      B.vis_split = will_vis && vis_can_split(primcnt);
+      B.tile_cost = vis_tile_cost(samples, needs_shading(P) && !sasl_shades(P));
       vis_split_bounds(primcnt, sized, &np, &nm);
       if (B.vis_split) {
         RCHK(X.take(r->vis_parts, np, B.vis_parts));
@@ -429,10 +430,12 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
       }
     }
     B.list_cap = sized;
-    launch_tile_ranges(P, B, sized, s);
-    launch_tile_lists(P, B, sized, order, !order_free, r->mail, T ? ++r->mail_seq : r->mail_seq, s);
+    const mail_slot mail{r->mail, T ? ++r->mail_seq : r->mail_seq}, none{nullptr, 0};
+    const bool late = B.vis_split;  // split tiles are counted by the lists' launch itself
+    launch_tile_ranges(P, B, s);
+    launch_tile_lists(P, B, sized, order, !order_free, late ? none : mail, s);
     mark(4);
-    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, s);
+    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, late ? mail : none, s);
     if (!fused) {
       if (inorder_applicable(P)) launch_inorder(P, B, which, s);
       else launch_raster(P, B, which, s);
@@ -467,7 +470,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
       RCHK(wait_mail(r));
     }
     if (fused && r->mail->merges) {
-      launch_vis(P, B, which, needs_shading(P), sized, r->mail->merges, s);
+      launch_vis(P, B, which, needs_shading(P), sized, r->mail->merges, mail_slot{nullptr, 0}, s);
       mark(5);
     }
   }

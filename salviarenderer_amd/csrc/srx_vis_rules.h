@@ -23,16 +23,21 @@ SRX_HD inline bool vis_large(uint64_t records, uint32_t prims) {
   return records >= static_cast<uint64_t>(VIS_LARGE) * prims;
 }
 
-// A tile's time is its list's length, so lists much longer than an even share of the records over the
-// workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame at the
-// oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
-// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where every tile's list is near
-// the even share a split only adds work.  Draws of large triangles, whose lists depth culling
-// shortens as it goes, are split later.
+// A tile's time is its list's length and what finishing it costs, so lists much longer than an even share of
+// both over the workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame
+// at the oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
+// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where the pass outlasts its longest tile
+// a split only adds work: the same mesh over most of the target takes 282 us a frame without splits and 311
+// with every tile of more than an even share of the records alone split (4 samples; 1 sample 173 and 192).
+// Draws of large triangles, whose lists depth culling shortens as it goes, are split later.
 constexpr uint32_t VIS_PART_SMALL = 1024, VIS_PART_LARGE = 2048, VIS_SLOTS = 640;
-// Records per part of a draw with `records` records: a tile with more is split.
-SRX_HD inline uint32_t vis_part(uint32_t prims, uint32_t records) {
-  const uint32_t least = vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL, share = records / VIS_SLOTS;
+// What finishing a tile costs, in records (depth, shading and stores): half as much splits tiles of the latter
+// view, twice as much leaves long tiles of the former whole (188 -> 206 us a frame).
+SRX_HD inline uint32_t vis_tile_cost(int samples, bool shade) { return shade ? 64u + 24u * static_cast<uint32_t>(samples) : 32u; }
+// Records per part of a draw with `records` records on `tiles` tiles: a tile with more is split.
+SRX_HD inline uint32_t vis_part(uint32_t prims, uint32_t records, uint32_t tiles, uint32_t tile_cost) {
+  const uint32_t least = vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL;
+  const uint32_t share = records / VIS_SLOTS + tiles * tile_cost / VIS_SLOTS;
   return least > share ? least : share;
 }
 // Draws of which no tile is split: a primitive gives at most three triangles, each once on a tile.

@@ -20,7 +20,7 @@ int main() {
     const uint32_t prims = uint32_t(1 + below(it % 2 ? 100000 : 1u << 30));
     uint32_t np, nt, parts = 0, tiles = 0;
     vis_split_bounds(prims, cap, &np, &nt);
-    const uint32_t part = vis_part(prims, total);
+    const uint32_t busy = uint32_t(below((1u << 18) + 1)), part = vis_part(prims, total, busy, vis_tile_cost(4, true));
     if (vis_can_split(prims)) {
       for (uint64_t left = total; left;) {  // lists just above a multiple of the part, or of any length
         uint64_t n = it % 3 ? part + 1 + part * below(3) : 1 + below(left);
@@ -33,9 +33,11 @@ int main() {
     if (parts > np || tiles > nt) ++bad, std::printf("cap %u total %u prims %u: %u parts of %u, %u tiles of %u\n", cap, total, prims, parts, np, tiles, nt);
   }
   // a mesh of small triangles, and its neighbours on either side of the rule
-  if (vis_large(24000, 16384) || vis_part(16384, 24000) != VIS_PART_SMALL) ++bad;
+  if (vis_large(24000, 16384) || vis_part(16384, 24000, 4096, 88) != VIS_PART_SMALL) ++bad;
   if (vis_large(4 * 16384 - 1, 16384) || !vis_large(4 * 16384, 16384)) ++bad;
-  if (vis_part(2000, 330000) != VIS_PART_LARGE || vis_part(1u << 22, 6400000) != 10000) ++bad;
+  if (vis_part(2000, 330000, 1024, 88) != VIS_PART_LARGE || vis_part(1u << 22, 6400000, 0, 160) != 10000) ++bad;
+  // lists that keep the pass waiting are split, lists of a pass that is busy for longer are not
+  if (vis_part(522242, 560000, 1008, vis_tile_cost(4, true)) > 1500 || vis_part(522242, 910000, 6500, vis_tile_cost(4, true)) < 2800) ++bad;
   if (vis_can_split(682) || !vis_can_split(683)) ++bad;
   return bad != 0;
 }
