@@ -110,9 +110,16 @@ __device__ __forceinline__ float4 shadow_pcf(const draw_params& P, const ps_samp
   return make_float4(a.x * k, a.y * k, a.z * k, a.w);
 }
 
+// Whether the shaders that any draw may use (PS_LAMBERT_TEX, PS_TEX_CPP, PS_BOX) sample by the inline paths.  With
+// three attributes and more their registers are spilled around every shader of the kernel, the ones in use
+// included: there only PS_CUP and PS_SSM, made for such draws, inline theirs (130k triangles at 1920x1080,
+// 4 samples: PS_CUP 274 -> 250 us a frame, PS_COLORIZED 240 -> 229, PS_MESH 230 -> 217).
+template <int NA>
+constexpr bool INLINE_TAPS = NA < 3;
+
 // cpp_pixel_shader::tex2d(s, reg) (cpp_pixel_shader.cpp:13-31): one LOD per quad from the register's
 // p1 - p0 and p2 - p0 (calc_lod_2d, sampler.cpp:834-852), then sample_2d_lod at pixel pi
-template <int NA>
+template <int NA, bool FAST = INLINE_TAPS<NA>>
 __device__ __forceinline__ float4 tex2d_cpp(const sampler_desc_dev& sp, const quad_lazy<NA>& q, int reg, int pi) {
   const float4 u0 = q.reg(reg, 0, q.inv_w(0), 2), u1 = q.reg(reg, 1, q.inv_w(1), 2), u2 = q.reg(reg, 2, q.inv_w(2), 2);
   const float dxu = u1.x - u0.x, dxv = u1.y - u0.y;
@@ -120,7 +127,7 @@ __device__ __forceinline__ float4 tex2d_cpp(const sampler_desc_dev& sp, const qu
   const float lod = (sp.mip_filter == FILTER_ANISO && sp.max_aniso > 1) ? calc_aniso(sp, dxu, dxv, dyu, dyv, 0.0f).lod
                                                                         : calc_lod(sp, dxu, dxv, dyu, dyv, 0.0f);
   const float4 uv = q.reg(reg, pi, q.inv_w(pi), 2);
-  if (sp.fast_linear) return sample_linear_fast(sp, uv.x, uv.y, lod);
+  if (FAST && sp.fast_linear) return sample_linear_fast(sp, uv.x, uv.y, lod);
   return sample_impl(sp, uv.x, uv.y, lod, nullptr);
 }
 // eflib vector helpers on .xyz (vector_generic.h:110-118, math.cpp:39-41,85-87)
@@ -209,7 +216,7 @@ __device__ __forceinline__ float4 ps_ssm(const draw_params& P, const ps_samplers
     occlusion = std_clamp(expf(occ - esm * lz), 0.0f, 1.0f);
   }
   float4 tex = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-  if (P.has_sampler[1]) tex = tex2d_cpp(SM->s[1], q, 1, pi);
+  if (P.has_sampler[1]) tex = tex2d_cpp<NA, true>(SM->s[1], q, 1, pi);
   const float4 n = normalize3v(q.reg(2, pi, iw, 3)), ld = normalize3v(q.reg(3, pi, iw, 3)), ed = normalize3v(q.reg(4, pi, iw, 3));
   const float idiff = std_clamp(dot3(ld, n), 0.0f, 1.0f);
   const float4 r = reflect3(ld, n);
@@ -233,7 +240,7 @@ __device__ __forceinline__ float4 ps_cup(const draw_params& P, const ps_samplers
                                          int pi) {
   const float iw = q.inv_w(pi);
   float4 tex = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-  if (P.has_sampler[0]) tex = tex2d_cpp(SM->s[0], q, 1, pi);
+  if (P.has_sampler[0]) tex = tex2d_cpp<NA, true>(SM->s[0], q, 1, pi);
   const float4 n = normalize3v(q.reg(2, pi, iw, 3)), ld = normalize3v(q.reg(3, pi, iw, 3)), ed = normalize3v(q.reg(4, pi, iw, 3));
   const float idiff = std_clamp(dot3(ld, n), 0.0f, 1.0f);
   const float ispec = std_clamp(dot3(reflect3(ld, n), ed), 0.0f, 1.0f);
@@ -274,7 +281,7 @@ __device__ __forceinline__ float4 run_ps_pixel(const draw_params& P, const ps_sa
       const float dyu = c1.x - c0.x, dyv = c1.y - c0.y;
       const float4 nrm = q.reg(1, pi, iw, 3);
       float4 t = make_float4(0, 0, 0, 0);
-      if (P.has_sampler[0]) t = sample_grad(SM->s[0], uv.x, uv.y, dxu, dxv, dyu, dyv);
+      if (P.has_sampler[0]) t = sample_grad<INLINE_TAPS<NA>>(SM->s[0], uv.x, uv.y, dxu, dxv, dyu, dyv);
       float nx, ny, nz;
       normalize3(nrm.x, nrm.y, nrm.z, nx, ny, nz);
       float d = nx * P.ps_consts[0] + ny * P.ps_consts[1] + nz * P.ps_consts[2];

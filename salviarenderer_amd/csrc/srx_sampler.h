@@ -612,7 +612,9 @@ __device__ __forceinline__ float4 sample_linear_fast(const sampler_desc_dev& p, 
   return lerp4(c0, c1, miplevel - static_cast<float>(lo));
 }
 
-// sample_2d_grad (sampler.cpp:854-873)
+// sample_2d_grad (sampler.cpp:854-873); LINEAR: trilinear samples take sample_linear_fast, for shaders that have
+// the registers (see sample_grad)
+template <bool LINEAR>
 __device__ __noinline__ float4 sample_2d_grad(const sampler_desc_dev& p, float u, float v, float dxu, float dxv, float dyu,
                                         float dyv, float bias) {
   if (p.mip_filter == FILTER_ANISO && p.max_aniso > 1) {
@@ -620,18 +622,19 @@ __device__ __noinline__ float4 sample_2d_grad(const sampler_desc_dev& p, float u
     return sample_impl(p, u, v, af.lod, &af);
   }
   float lod = calc_lod(p, dxu, dxv, dyu, dyv, bias);
-  if (p.fast_linear) return sample_linear_fast(p, u, v, lod);
+  if (LINEAR && p.fast_linear) return sample_linear_fast(p, u, v, lod);
   aniso_info dummy{};
   return sample_impl(p, u, v, lod, &dummy);
 }
 
-// sample_2d_grad (bias 0) by the inline path where it applies: the shaders' texture sample.  One call of
-// the general function, so that what lives across it is spilled once.
+// sample_2d_grad (bias 0): the shaders' texture sample.  FAST: by the inline path where it applies, with one call
+// of the general function, so that what lives across it is spilled once.
+template <bool FAST = true>
 __device__ __forceinline__ float4 sample_grad(const sampler_desc_dev& p, float u, float v, float dxu, float dxv, float dyu,
                                               float dyv) {
   float4 c;
-  if (p.fast_aniso && sample_aniso_fast(p, u, v, dxu, dxv, dyu, dyv, c)) return c;
-  return sample_2d_grad(p, u, v, dxu, dxv, dyu, dyv, 0.0f);
+  if (FAST && p.fast_aniso && sample_aniso_fast(p, u, v, dxu, dxv, dyu, dyv, c)) return c;
+  return sample_2d_grad<FAST>(p, u, v, dxu, dxv, dyu, dyv, 0.0f);
 }
 
 }  // namespace srx

@@ -10,7 +10,12 @@ from salviarenderer_amd import api as A
 from helpers import Target
 
 
-def render(lib, tw, th, mip, aniso, offset, scale, blend, samples):
+LAMBERT = (A.VS_WVP_NORMAL_UV, np.eye(4, dtype=np.float32).ravel(),
+           A.PS_LAMBERT_TEX, np.array([0.0, 0.3, 0.9, 0.0], np.float32))
+
+
+def render(lib, tw, th, mip, aniso, offset, scale, blend, samples, shaders=LAMBERT):
+    vs, vs_consts, ps, ps_consts = shaders
     r = lib.renderer()
     t = Target(r, 150, 90, samples)
     t.clear((0.1, 0.2, 0.3, 0.4))
@@ -24,12 +29,12 @@ def render(lib, tw, th, mip, aniso, offset, scale, blend, samples):
     vb = r.create_buffer_from(v)
     layout = r.create_input_layout([("POSITION", 0, A.FMT_R32G32B32_FLOAT, 0, 0),
                                     ("NORMAL", 0, A.FMT_R32G32B32_FLOAT, 0, 12),
-                                    ("TEXCOORD", 0, A.FMT_R32G32_FLOAT, 0, 24)], A.VS_WVP_NORMAL_UV)
+                                    ("TEXCOORD", 0, A.FMT_R32G32_FLOAT, 0, 24)], vs)
     r.set_input_layout(layout)
     r.set_vertex_buffers(0, [vb], [32])
     r.set_primitive_topology(A.TOPOLOGY_TRIANGLE_LIST)
-    r.set_vertex_shader(A.VS_WVP_NORMAL_UV, np.eye(4, dtype=np.float32).ravel())
-    r.set_pixel_shader(A.PS_LAMBERT_TEX, np.array([0.0, 0.3, 0.9, 0.0], np.float32))
+    r.set_vertex_shader(vs, vs_consts)
+    r.set_pixel_shader(ps, ps_consts)
     tex = r.create_tex2d(tw, th, 1, A.PF_RGBA8)
     tex.surface(0).write(rng.integers(0, 256, (th, tw, 4), dtype=np.uint8))
     tex.gen_mipmap(A.FILTER_LINEAR, True)
@@ -60,3 +65,16 @@ def test_taps(hip_lib, cpu_lib, tw, th, mip, aniso, blend):
     for offset, scale, samples in ((0, 0.02, 1), (0, 1.0, 4), (-3, 40.0, 2), (65535.5, 4.0, 1), (-65536, 6.0, 4), (1e9, 1e9, 1)):
         args = tw, th, mip, aniso, offset, scale, blend, samples
         assert np.array_equal(render(hip_lib, *args), render(cpu_lib, *args)), args
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
+@pytest.mark.parametrize("ps", [A.PS_LAMBERT_TEX, A.PS_TEX_CPP, A.PS_BOX, A.PS_CUP], ids=["lambert", "tex", "box", "cup"])
+def test_taps_of_four_attributes(hip_lib, cpu_lib, ps, blend):
+    """The shaders' samples behind a vertex shader of four attributes, where only PS_CUP's are inline."""
+    vs_consts = np.concatenate([np.eye(4).ravel(), (0, 0, -1, 1), (1, 1, -1, 1)]).astype(np.float32)
+    ps_consts = {A.PS_LAMBERT_TEX: LAMBERT[3], A.PS_CUP: np.linspace(0.1, 0.9, 12, dtype=np.float32)}.get(ps)
+    for (mip, aniso), (tw, th), samples in (((A.FILTER_LINEAR, 1), (64, 32), 1), ((A.FILTER_ANISOTROPIC, 8), (64, 64), 4),
+                                            ((A.FILTER_LINEAR, 1), (48, 20), 2), ((A.FILTER_ANISOTROPIC, 8), (61, 37), 1)):
+        args = tw, th, mip, aniso, 0, 1.0, blend, samples, (A.VS_CUP, vs_consts, ps, ps_consts)
+        assert np.array_equal(render(hip_lib, *args), render(cpu_lib, *args)), args[:4]
