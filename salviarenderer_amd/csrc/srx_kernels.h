@@ -5,7 +5,7 @@
 #include <stdint.h>
 
 #include "srx_device.h"
-#include "srx_vis_rules.h"
+#include "srx_record_rules.h"
 
 namespace srx {
 
@@ -34,7 +34,6 @@ __host__ __device__ inline uint32_t record_total(const uint32_t* counters) {
 __host__ __device__ inline uint32_t busy_tiles(const uint32_t* counters, uint32_t T) {
   return T - counters[CT_CLASS + TILE_CLASSES - 1];
 }
-constexpr uint32_t MAX_RECORDS = 0xFFFFFFF0u;  // a draw with more is refused
 static_assert(CT_TOTAL % 2 == 0 && CT_WIDE == CT_TOTAL + 1, "one aligned 64-bit word");
 
 // Where a tile's record count lies in tile_count: atomics to words of one cache line are served one after

@@ -1,6 +1,7 @@
-// Rules of the visibility pass that depend on a draw's record count, for host and device code: when depth
-// culling begins and which tiles are split.  The device applies them to the draw's own count; the host, which
-// does not know it yet, sizes the tables for every count up to the lists' capacity.
+// Rules on a draw's record count, for host and device code: the count its lists are first formed for, and in
+// the visibility pass when depth culling begins and which tiles are split.  The device applies the latter to
+// the draw's own count; the host, which does not know it yet, sizes the tables for every count up to the lists'
+// capacity.
 #pragma once
 
 #include <stdint.h>
@@ -12,6 +13,17 @@
 #endif
 
 namespace srx {
+
+// Records that the lists of a draw of `prims` primitives on T tiles are formed for before its count is known:
+// 5/4 of the most that recent draws had, and at least one for every triangle that clipping can leave, so that
+// a large mesh among small draws seldom outgrows its lists however many of those came in between (a frame of
+// one 522k-triangle mesh and ten draws of 20,000 triangles 720 -> 697 us, as nothing is queued twice).
+constexpr uint32_t MAX_RECORDS = 0xFFFFFFF0u;  // a draw with more is refused
+SRX_HD inline uint32_t record_estimate(uint32_t recent, uint32_t prims, uint32_t T) {
+  const uint64_t grown = recent + static_cast<uint64_t>(recent) / 4, own = 3ull * prims + T, least = 1u << 16;
+  const uint64_t want = grown > own ? grown : own;
+  return want < least ? static_cast<uint32_t>(least) : want < MAX_RECORDS ? static_cast<uint32_t>(want) : MAX_RECORDS;
+}
 
 // Records of a tile taken before depth culling begins: few for draws whose triangles lie on VIS_LARGE or
 // more GPU tiles on average, whose lists are deep (of the 323 records a tile of the 2,000-triangle

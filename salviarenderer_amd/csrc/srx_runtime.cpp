@@ -323,8 +323,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
   if (!fixed) {
     uint32_t recent = 0;
     for (uint32_t v : r->recent_records) recent = std::max(recent, v);
-    const uint64_t want = recent ? recent + static_cast<uint64_t>(recent) / 4 : static_cast<uint64_t>(P3) + T;
-    sized = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, 1u << 16), MAX_RECORDS));
+    sized = record_estimate(recent, primcnt, T);
     RCHK(take_records(sized));
     const size_t held = std::min(std::min(r->keys0.cap, r->vals0.cap), std::min(r->keys1.cap, r->vals1.cap));
     capacity = static_cast<uint32_t>(std::min<size_t>(held, MAX_RECORDS));

@@ -1,5 +1,6 @@
-"""The visibility pass's rules on record counts (csrc/srx_vis_rules.h), compiled for the host: the tables sized for a
-capacity hold the parts and split tiles of every draw within it."""
+"""The rules on record counts (csrc/srx_record_rules.h), compiled for the host: the estimate that a draw's lists are
+first formed for has the draw's own size in it, and the tables sized for a capacity hold the parts and split tiles
+of every draw within it."""
 import os
 import subprocess
 
@@ -9,7 +10,7 @@ PROGRAM = r"""
 #include <cstdio>
 #include <random>
 #include <vector>
-#include "srx_vis_rules.h"
+#include "srx_record_rules.h"
 using namespace srx;
 int main() {
   std::mt19937_64 rng(1);
@@ -36,6 +37,10 @@ int main() {
   if (vis_large(24000, 16384) || vis_part(16384, 24000, 4096, 88) != VIS_PART_SMALL) ++bad;
   if (vis_large(4 * 16384 - 1, 16384) || !vis_large(4 * 16384, 16384)) ++bad;
   if (vis_part(2000, 330000, 1024, 88) != VIS_PART_LARGE || vis_part(1u << 22, 6400000, 0, 160) != 10000) ++bad;
+  // a mesh keeps room for its own triangles after any number of small draws; deep draws are remembered
+  if (record_estimate(20000, 522242, 8160) != 3 * 522242 + 8160 || record_estimate(0, 522242, 8160) != 3 * 522242 + 8160) ++bad;
+  if (record_estimate(330000, 2000, 1024) != 412500 || record_estimate(0, 12, 64) != 65536) ++bad;
+  if (record_estimate(0xFFFFFFF0u, 1, 1) != MAX_RECORDS || record_estimate(0, 0x55554000u, 1 << 18) != MAX_RECORDS) ++bad;
   // lists that keep the pass waiting are split, lists of a pass that is busy for longer are not
   if (vis_part(522242, 560000, 1008, vis_tile_cost(4, true)) > 1500 || vis_part(522242, 910000, 6500, vis_tile_cost(4, true)) < 2800) ++bad;
   if (vis_can_split(682) || !vis_can_split(683)) ++bad;
