@@ -88,7 +88,7 @@ struct draw_params {
   int32_t samples;
   float sp[4][2];
   int32_t tiles_x, tiles_y;   // 64-pixel reference tiles
-  int32_t gt, gtiles_x, gtiles_y;  // GPU tile size (16/32/64) and counts
+  int32_t gt, gtiles_x, gtiles_y;  // GPU tile side (16 or 32, in batches 8 too) and counts
   // framebuffer
   surface_desc color;  // colour target 0 (data == nullptr: none)
   surface_desc ds;     // RG32F (data == nullptr: none)

@@ -1,4 +1,6 @@
-// Host-side launchers of the pipeline kernels (implemented in srx_kernels.hip).
+// Host-side launchers of the pipeline kernels: geometry, binning, clears and resolves (srx_kernels.hip), in-order
+// rasterisation under queries and with SASL shaders and deferred shading (srx_raster.hip), in-order
+// rasterisation otherwise (srx_inorder.hip), visibility (srx_vis.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -8,14 +8,17 @@
 //                   triangles on few tiles                                  (clipper.cpp, rasterizer.cpp:864-945)
 //   clip_kernel     Sutherland-Hodgman near/far clipping for the few primitives that need it; emits the
 //                   records of the clipped triangles and of those on many tiles
-//   tile_ranges     tile ranges and scheduling order from the record counts per tile
-//   tile_scatter    records to their tiles' lists; in-order draws then sort each list (tile_sort), so it
-//                   is in primitive order (the reference's per-tile std::sort, rasterizer.cpp:947-994)
-//   raster_kernel   (srx_raster.hip) one workgroup per GPU tile, one thread per 2x2 quad; walks its tile's list in
-//                   order and evaluates the reference's 64->16->4->sample decision chain per quad
-//                   (rasterizer.cpp:298-773), early/late depth-stencil, pixel shader and blending
-//                   (framebuffer.cpp).  Opaque early-Z draws defer the pixel shader to one pass over
-//                   the final per-sample winners.
+//   tile_ranges     tile ranges and classes from the record counts per tile
+//   tile_scatter    scheduling order, parts of split tiles, records to their tiles' lists; in-order draws then
+//                   sort each list (tile_sort), so it is in primitive order (the reference's per-tile
+//                   std::sort, rasterizer.cpp:947-994)
+//   inorder_kernel  (srx_inorder.hip) one workgroup per GPU tile, one thread per pixel; evaluates the
+//                   reference's 64->16->4->sample decision chain (rasterizer.cpp:298-773) for the records of
+//                   the tile's list, then every pixel's own in order: depth-stencil tests, pixel shader and
+//                   blending (framebuffer.cpp)
+//   raster_kernel   (srx_raster.hip) the same with one thread per 2x2 quad, for statistics queries, SASL
+//                   pixel shaders, 32-pixel tiles and NOT_EQUAL depth.  Opaque early-Z draws defer the
+//                   pixel shader to one pass over the final per-sample winners.
 //   vis_kernel      (srx_vis.hip) the same decisions for opaque early-Z draws, whose result does not
 //                   depend on primitive order, fused with their shading
 #include "srx_kernel_common.h"
@@ -537,8 +540,8 @@ __device__ __forceinline__ int bin_span(const draw_params& P, const float* bb) {
   const int ey = min(fast_ceili(std_max(0.0f, bb[3]) / TILE) + 1, P.tiles_y);
   return (ex > sx && ey > sy) ? (ex - sx) * (ey - sy) : 0;
 }
-// Triangles over more than this many 64x64 tiles are counted by a whole wave (clip launch), not by
-// setup's one lane.
+// Batches: triangles over more than this many 64x64 tiles are counted by a whole wave (clip launch), not by
+// setup's one lane, and emitted by a whole wave.  (Single draws emit as they set up; their rule is SMALL_SPAN.)
 constexpr int COUNT_WIDE = 32;
 
 // count_gtiles by a whole wave (every lane calls it with the same triangle): lanes take the 64x64
@@ -628,20 +631,6 @@ __device__ __forceinline__ void write_tri_attr(float4* a, const tri_setup<NA>& t
   tri_attr_words<NA>(t, w);
 #pragma unroll
   for (int k = 0; k < 3 * (NA + 1); ++k) a[k] = w[k];
-}
-
-// Sum of v over the workgroup, returned to thread 0.  All threads must call it.
-__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v) {
-  __shared__ uint32_t wsum[16];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, 64));
-  const int wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if ((threadIdx.x & 63) == 0) wsum[wave] = v;
-  __syncthreads();
-  uint32_t t = 0;
-  if (threadIdx.x == 0)
-    for (int w = 0; w < nw; ++w) t += wsum[w];
-  return t;
 }
 
 // stats[slot] += sum(partial[0..n))
@@ -1698,7 +1687,7 @@ void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap
   }
 }
 
-// Scheduling order of the GPU tiles, heaviest first so that the longest tiles start early.  Tiles
+// Batches: scheduling order of the GPU tiles, heaviest first so that the longest tiles start early.  Tiles
 // are independent, so the order never changes a pixel.  One workgroup buckets the tiles by record
 // count / 8 (heaviest bucket first) with LDS counters.
 __device__ __forceinline__ uint32_t tile_bucket(const uint32_t* ts, const uint32_t* te, uint32_t t) {
@@ -1729,11 +1718,6 @@ __device__ __forceinline__ void tile_order_body(const uint32_t* __restrict__ ts,
   __syncthreads();
   for (uint32_t t = tid; t < T; t += blockDim.x) order[wave_counted_add(cnt, tile_bucket(ts, te, t))] = t;
 }
-__global__ void __launch_bounds__(1024) tile_order_kernel(const uint32_t* __restrict__ ts, const uint32_t* __restrict__ te,
-                                                          uint32_t T, uint32_t* __restrict__ order) {
-  tile_order_body(ts, te, T, order);
-}
-
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s) {
   if (n) hipLaunchKernelGGL(fill_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
 }

@@ -1,8 +1,8 @@
 // srx_draw_noalloc: srx_draw for callers that cannot allocate device memory (code under HIP graph
 // capture, serving loops and harnesses that forbid hipMalloc).  Every buffer the draw needs beyond
-// its inputs and outputs -- vertex-shader outputs, triangle setup, per-triangle record counts and
-// their scan space, binned records, sort histograms, tile ranges and order, the visibility work
-// table and per-sample winners -- is carved from `scratch`, one fixed region per GPU that lives
+// its inputs and outputs -- vertex-shader outputs, triangle setup, clipped vertices, binned records
+// and the tiles' lists, tile counts, ranges and order, the visibility pass's split tiles and
+// per-sample winners -- is carved from `scratch`, one fixed region per GPU that lives
 // until the process ends.  The renderer's own small blocks (device counters, statistics, pinned
 // staging) were allocated when it was created.  No counterpart in the reference.
 #include "srx_runtime_internal.h"

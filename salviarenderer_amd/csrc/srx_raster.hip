@@ -1,6 +1,6 @@
-// In-order rasterisation and deferred shading: draws whose samples depend on primitive order
-// (blending, stencil that changes, statistics queries), and the pixel shader passes over the winners
-// of an opaque draw.
+// In-order rasterisation of the draws that inorder_kernel (srx_inorder.hip) does not take: statistics
+// queries, SASL pixel shaders, 32-pixel tiles, NOT_EQUAL depth; and the deferred pixel shader passes over
+// the winners of an opaque draw.
 #include "srx_kernel_common.h"
 #include "srx_sasl_exec.h"
 

@@ -1,6 +1,6 @@
-// Device helpers of the pixel-shading stage shared by the precompiled kernels (srx_kernels.hip)
-// and the SASL shading kernels compiled at run time (srx_sasl_jit.cpp): the per-triangle
-// interpolation data, the quad interpolation chain and the sample addressing of a surface.
+// Device helpers of the pixel-shading stage shared by the precompiled kernels (srx_raster.hip,
+// srx_inorder.hip, srx_vis.hip) and the SASL shading kernels compiled at run time (srx_sasl_jit.cpp): the
+// per-triangle interpolation data, the quad interpolation chain and the sample addressing of a surface.
 #pragma once
 
 #include "srx_device.h"
