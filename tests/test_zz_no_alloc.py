@@ -93,3 +93,25 @@ def test_noalloc_blends_on_a_large_target(hip_lib):
         out.append(t.color.read().copy())
         del keep
     assert np.array_equal(*out) and len(np.unique(out[0][::7, ::7].reshape(-1, 4), axis=0)) > 1
+
+
+@pytest.mark.parametrize("blend", [A.BLEND_OFF, A.BLEND_ON], ids=["opaque", "blend"])
+@pytest.mark.parametrize("n,side", [(5000, 40), (200, 300)], ids=["long_lists", "spread"])
+def test_noalloc_long_lists_and_blending(hip_lib, n, side, blend):
+    """Lists that are split (opaque) or sorted in several partitions (blended), and ordinary ones."""
+    rng = np.random.default_rng(n)
+    pos = np.concatenate([rng.uniform(-0.6, 0.6, (n, 1, 2)) + rng.uniform(-0.3, 0.3, (n, 3, 2)), rng.uniform(0.1, 0.9, (n, 3, 1)),
+                          np.ones((n, 3, 1))], -1).reshape(-1, 4)
+    col = rng.uniform(0.0, 1, (3 * n, 4))
+    for samples in (1, 4):
+        out = []
+        for noalloc in (True, False):
+            r = hip_lib.renderer()
+            if noalloc:
+                r.draw = r.draw_noalloc
+            t = Target(r, side, side, samples)
+            t.clear((0.1, 0.2, 0.3, 0.4))
+            keep = draw_colored(r, pos, col, blend=blend)
+            out.append({"color": t.color.read().copy(), "ds": t.ds.read().copy()})
+            del keep
+        same(*out)
