@@ -40,14 +40,6 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
   return v;
 }
 
-// Writes a single draw's mail, whose counts are final; the host waits for the sequence number.
-__device__ __forceinline__ void send_mail(mail_slot m, const uint32_t* __restrict__ counters) {
-  m.mail->total = record_total(counters);
-  m.mail->merges = counters[CT_MERGES];
-  m.mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
-  __hip_atomic_store(&m.mail->seq, m.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // Sums v over the workgroup and stores the total in partial[blockIdx.x] (no global atomics: many
 // same-address device-scope atomics from every XCD serialise badly).  All threads must call it.
 __device__ __forceinline__ void block_partial(unsigned long long* __restrict__ partial, unsigned long long v) {

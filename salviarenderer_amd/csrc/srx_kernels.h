@@ -23,11 +23,12 @@ enum stat_slot {
 // bits (setup alone cannot: at most four records a primitive, whose buffers take over 600 bytes); read the
 // count with record_total.
 // CT_CURSOR: records given to the tiles' lists; CT_PARTS, CT_MERGES: parts of split tiles and split tiles;
-// CT_CLASS: GPU tiles per record-count class (the last class: without records).
+// CT_CLASS: GPU tiles per record-count class (the last class: without records); CT_STEP: per vis_step.
 constexpr int TILE_CLASSES = 16;
 enum counter_slot { CT_TOTAL = 0, CT_WIDE, CT_CLIP_PRIMS, CT_CLIP_SLOTS, CT_CLIP_OVERFLOW, CT_CURSOR, CT_PARTS, CT_MERGES,
                     CT_OVERRUN, CT_CLASS,
-                    CT_COUNT = CT_CLASS + TILE_CLASSES };
+                    CT_STEP = CT_CLASS + TILE_CLASSES,
+                    CT_COUNT = CT_STEP + VIS_STEPS };
 // Records of a single draw, 0xFFFFFFFF when the count does not fit (above every capacity).
 __host__ __device__ inline uint32_t record_total(const uint32_t* counters) {
   return counters[CT_OVERRUN] ? 0xFFFFFFFFu : counters[CT_TOTAL];
@@ -60,10 +61,6 @@ __host__ __device__ inline uint32_t tile_slots(uint32_t T) {
 // What the host needs to know of a single draw, written by the device into pinned host memory: seq last.
 struct draw_mail {
   uint32_t seq, total, merges, clip_overflow;
-};
-struct mail_slot {
-  draw_mail* mail;  // null: another launch of the draw writes it
-  uint32_t seq;
 };
 
 // Per-draw device buffers (owned by the renderer, grown on demand).
@@ -177,11 +174,10 @@ void launch_clip(const draw_params& P, const draw_buffers& B, uint32_t capacity,
 // record-count class and rank in it (kept in B.partial until the lists' launch).  Lists: `order` (tiles
 // words), with B.vis_split the parts of split tiles (when the count is within `cap`), and vals[1], or in
 // primitive order vals[0] (`sorted`), sized for `cap` records; the count is read from B.counters on the
-// device.  The lists' launch writes the draw's mail, if it is given (targets without GPU tiles: nothing is
-// launched).
+// device.  The lists' launch writes the draw's mail (targets without GPU tiles: nothing is launched).
 void launch_tile_ranges(const draw_params& P, const draw_buffers& B, hipStream_t s);
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, mail_slot mail,
-                       hipStream_t s);
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
+                       uint32_t seq, hipStream_t s);
 // In-place exclusive scan of n u32; writes the total to *total_dev.  tmp holds >= scan_tmp_size(n).
 size_t scan_tmp_size(uint32_t n);
 void launch_exclusive_scan(uint32_t* data, uint32_t n, uint32_t* tmp, uint32_t* total_dev, hipStream_t s);
@@ -196,10 +192,9 @@ bool inorder_takes_color_clear(const draw_params& P);
 void launch_inorder(const draw_params& P, const draw_buffers& B, int which, hipStream_t s);
 // Order-independent visibility (and, with shade, the deferred pixel shader) of an opaque early-Z draw,
 // laid out for `records` records; false when the draw needs the in-order kernel.  merges > 0: finishes
-// that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles and written the
-// draw's mail, if it is given.
+// that many split tiles (counters[CT_MERGES]) after a call with 0 has rasterised the tiles.
 bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
-                mail_slot mail, hipStream_t s);
+                hipStream_t s);
 bool needs_shading(const draw_params& P);
 // A SASL pixel shader whose colour is written: such draws run the in-order raster kernel.
 bool sasl_shades(const draw_params& P);

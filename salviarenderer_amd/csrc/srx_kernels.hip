@@ -1501,6 +1501,7 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     ts[t] = base + incl - n;
     te[t] = base + incl;
     place[t] = (c << PLACE_BITS) | at;
+    if (n >= VIS_PART_SMALL) atomicAdd(&counters[CT_STEP + vis_step(n)], 1u);
   }
 }
 // The scheduling order, the parts of split tiles, and the records to their tiles' lists: position = first record of the tile + rank in it.
@@ -1514,28 +1515,41 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
                                                            uint32_t* __restrict__ order, bool split, uint32_t prims,
                                                            uint32_t tile_cost, uint32_t* __restrict__ ct_parts,
                                                            uint32_t* __restrict__ ct_merges, uint4* __restrict__ parts,
-                                                           uint4* __restrict__ merges, mail_slot mail) {
-  if (mail.mail && blockIdx.x == 0 && threadIdx.x == 0) send_mail(mail, counters);
+                                                           uint4* __restrict__ merges, draw_mail* mail, uint32_t seq) {
   const uint32_t total = record_total(counters);
+  const bool may_split = split && total <= cap;  // with more records the tables' bounds do not hold
+  const uint32_t part = may_split ? vis_part(prims, total, busy_tiles(counters, T), tile_cost) : 0u;
+  if (blockIdx.x == 0 && threadIdx.x < 64) {  // the counts are final; the host waits for seq
+    uint32_t split_tiles = 0;
+    if (may_split)
+      for (uint32_t k = vis_step(part + 1) + threadIdx.x; k < VIS_STEPS; k += 64) split_tiles += counters[CT_STEP + k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) split_tiles += static_cast<uint32_t>(__shfl_xor(static_cast<int>(split_tiles), off, 64));
+    if (threadIdx.x == 0) {
+      mail->total = total;
+      mail->merges = split_tiles;
+      mail->clip_overflow = counters[CT_CLIP_OVERFLOW];
+      __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
   for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < T; t += gridDim.x * 256) {
     const uint32_t c = place[t] >> PLACE_BITS;
     uint32_t at = place[t] & ((1u << PLACE_BITS) - 1u);
 #pragma unroll
     for (uint32_t k = 0; k + 1 < TILE_CLASSES; ++k) at += k < c ? counters[CT_CLASS + k] : 0u;
     order[at] = t;
-    if (split && total <= cap) {  // with more records the tables' bounds do not hold
-      const uint32_t len = te[t] - ts[t], part = vis_part(prims, total, busy_tiles(counters, T), tile_cost);
-      if (len > part) {
-        const uint32_t np = (len + part - 1) / part;
-        const uint32_t e = atomicAdd(ct_parts, np);
-        merges[atomicAdd(ct_merges, 1u)] = make_uint4(t, np, e, 0u);
-        for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
-      }
+    const uint32_t len = may_split ? te[t] - ts[t] : 0u;
+    if (may_split && len > part) {
+      const uint32_t np = (len + part - 1) / part;
+      const uint32_t e = atomicAdd(ct_parts, np);
+      merges[atomicAdd(ct_merges, 1u)] = make_uint4(t, np, e, 0u);
+      for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
     }
   }
+  // the first workgroup, which writes the mail, has no records
   const uint32_t n = min(total, cap);
-  const uint32_t b0 = blockIdx.x * (256 * SCATTER_PER_THREAD);
-  if (b0 >= n) return;
+  const uint32_t b0 = (blockIdx.x - 1) * (256 * SCATTER_PER_THREAD);
+  if (blockIdx.x == 0 || b0 >= n) return;
   uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
 #pragma unroll
   for (uint32_t j = 0; j < SCATTER_PER_THREAD; ++j) {  // clamped indices: no branch per load
@@ -1670,15 +1684,15 @@ void launch_tile_ranges(const draw_params& P, const draw_buffers& B, hipStream_t
   hipLaunchKernelGGL(tile_ranges_kernel, dim3((N + 255) / 256), dim3(256), 0, s, B.tile_count, T, N, shift, B.tstart, B.tend,
                      B.counters, reinterpret_cast<uint32_t*>(B.partial));
 }
-void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, mail_slot mail,
-                       hipStream_t s) {
+void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap, uint32_t* order, bool sorted, draw_mail* mail,
+                       uint32_t seq, hipStream_t s) {
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t per = 256 * SCATTER_PER_THREAD;
-  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max(cap, T) + per - 1) / per), dim3(256), 0, s, B.keys[0], B.vals[0],
+  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max(cap, T) + per - 1) / per + 1), dim3(256), 0, s, B.keys[0], B.vals[0],
                      B.keys[1], B.counters, cap, B.tstart, B.tend, B.vals[1], T, reinterpret_cast<const uint32_t*>(B.partial),
                      order, B.vis_split, P.prim_count, B.tile_cost, B.counters + CT_PARTS,
-                     B.counters + CT_MERGES, B.vis_parts, B.vis_merges, mail);
+                     B.counters + CT_MERGES, B.vis_parts, B.vis_merges, mail, seq);
   if (sorted) {
     uint32_t bits = 1;  // the values are below 6 * prim_count
     while (bits < 32 && (6ull * P.prim_count) >> bits) ++bits;

@@ -46,19 +46,32 @@ constexpr uint32_t VIS_PART_SMALL = 1024, VIS_PART_LARGE = 2048, VIS_SLOTS = 640
 // What finishing a tile costs, in records (depth, shading and stores): half as much splits tiles of the latter
 // view, twice as much leaves long tiles of the former whole (188 -> 206 us a frame).
 SRX_HD inline uint32_t vis_tile_cost(int samples, bool shade) { return shade ? 64u + 24u * static_cast<uint32_t>(samples) : 32u; }
-// Records per part of a draw with `records` records on `tiles` tiles: a tile with more is split.
+// Part sizes go by quarters of a power of two: lists of VIS_PART_SMALL and more records are counted by step as
+// the tiles' ranges are formed, so the next launch knows how many tiles a part size splits before it has
+// looked at any, and the host hears of it no later than of the record count (a launch later: 4 to 6 us a frame
+// of 50 to 100 us).
+constexpr uint32_t VIS_STEPS = 88;
+SRX_HD inline uint32_t vis_step_size(uint32_t k) { return (4u + (k & 3u)) << (8u + (k >> 2)); }
+SRX_HD inline uint32_t vis_step(uint32_t records) {  // the largest step of at most `records` >= VIS_PART_SMALL
+  const uint32_t lg = 31u - static_cast<uint32_t>(__builtin_clz(records));
+  return 4u * (lg - 10u) + ((records >> (lg - 2u)) & 3u);
+}
+static_assert(VIS_PART_SMALL == 1u << 10 && VIS_PART_LARGE >= VIS_PART_SMALL, "step 0");
+// Records per part of a draw with `records` records on `tiles` tiles: a tile with more is split, that is one
+// whose step is vis_step(part + 1) or above.
 SRX_HD inline uint32_t vis_part(uint32_t prims, uint32_t records, uint32_t tiles, uint32_t tile_cost) {
   const uint32_t least = vis_large(records, prims) ? VIS_PART_LARGE : VIS_PART_SMALL;
-  const uint32_t share = records / VIS_SLOTS + tiles * tile_cost / VIS_SLOTS;
-  return least > share ? least : share;
+  const uint32_t share = records / VIS_SLOTS + tiles * tile_cost / VIS_SLOTS, want = least > share ? least : share;
+  const uint32_t k = vis_step(want);
+  return vis_step_size(vis_step_size(k) < want ? k + 1 : k) - 1;
 }
 // Draws of which no tile is split: a primitive gives at most three triangles, each once on a tile.
 SRX_HD inline bool vis_can_split(uint32_t prims) { return 3ull * prims > VIS_PART_LARGE; }
 // Upper bounds of the parts and split tiles of a draw with at most `records` records: a tile of n > part
-// records has ceil(n / part) < 2 n / part parts, and records / part is at most records / VIS_PART_SMALL and
-// VIS_SLOTS.  A part takes 256 * samples keys.
+// records has ceil(n / part) < 2 n / part parts, and part, at least VIS_PART_SMALL - 1 and records / VIS_SLOTS - 1,
+// goes at most VIS_SLOTS + 2 times into them.  A part takes 256 * samples keys.
 SRX_HD inline void vis_split_bounds(uint32_t prims, uint32_t records, uint32_t* parts, uint32_t* tiles) {
-  const uint32_t most = records / VIS_PART_SMALL < VIS_SLOTS ? records / VIS_PART_SMALL : VIS_SLOTS;
+  const uint32_t n = records / (VIS_PART_SMALL - 1), most = n < VIS_SLOTS + 2 ? n : VIS_SLOTS + 2;
   *parts = vis_can_split(prims) ? 2 * (most + 1) : 0;
   *tiles = vis_can_split(prims) ? most + 1 : 0;
 }

@@ -429,12 +429,10 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
       }
     }
     B.list_cap = sized;
-    const mail_slot mail{r->mail, T ? ++r->mail_seq : r->mail_seq}, none{nullptr, 0};
-    const bool late = B.vis_split;  // split tiles are counted by the lists' launch itself
     launch_tile_ranges(P, B, s);
-    launch_tile_lists(P, B, sized, order, !order_free, late ? none : mail, s);
+    launch_tile_lists(P, B, sized, order, !order_free, r->mail, T ? ++r->mail_seq : r->mail_seq, s);
     mark(4);
-    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, late ? mail : none, s);
+    fused = vis_tables && launch_vis(P, B, which, needs_shading(P), sized, 0, s);
     if (!fused) {
       if (inorder_applicable(P)) launch_inorder(P, B, which, s);
       else launch_raster(P, B, which, s);
@@ -469,7 +467,7 @@ int32_t execute_draw(renderer_obj* r, bool indexed, uint32_t start, uint32_t pri
       RCHK(wait_mail(r));
     }
     if (fused && r->mail->merges) {
-      launch_vis(P, B, which, needs_shading(P), sized, r->mail->merges, mail_slot{nullptr, 0}, s);
+      launch_vis(P, B, which, needs_shading(P), sized, r->mail->merges, s);
       mark(5);
     }
   }

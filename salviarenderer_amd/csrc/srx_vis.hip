@@ -744,14 +744,12 @@ struct vis_lists {
   const uint4 *parts, *merges;
   unsigned long long* partial;
   uint32_t cap, max_parts, tile_cost;
-  mail_slot mail;
 };
 template <int NA, int S, bool SHADE>
 __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, int mode, vis_lists V,
                                                    const float4* __restrict__ tri_rec, const float4* __restrict__ tri_attr,
                                                    const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
   const uint32_t records = record_total(V.counters);
-  if (V.mail.mail && blockIdx.x == 0 && threadIdx.x == 0) send_mail(V.mail, V.counters);
   if (records > V.cap) return;  // records were dropped: the draw is emitted again
   const uint32_t part = vis_part(P.prim_count, records, busy_tiles(V.counters, static_cast<uint32_t>(P.gtiles_x * P.gtiles_y)),
                                  V.tile_cost);
@@ -839,7 +837,7 @@ int vis_mode(const draw_params& P) {
 }
 
 bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool shade, uint32_t records, uint32_t merges,
-                mail_slot mail, hipStream_t s) {
+                hipStream_t s) {
   int mode = vis_mode(P);
   // a SASL pixel shader runs in its own pass (launch_shade) over the winners this pass writes
   uint32_t* const wout = sasl_shades(P) ? B.vis : nullptr;
@@ -850,7 +848,7 @@ bool launch_vis(const draw_params& P, const draw_buffers& B, int which, bool sha
   uint32_t np, nm;
   vis_split_bounds(P.prim_count, records, &np, &nm);
   const vis_lists V{B.order, B.vals[which], B.tstart, B.tend, B.counters, B.vis_parts, B.vis_merges, B.vis_partial,
-                    B.list_cap, B.vis_split ? np : 0u, B.tile_cost, mail};
+                    B.list_cap, B.vis_split ? np : 0u, B.tile_cost};
 #define SRX_VIS_LAUNCH(NA, S, SH)                                                                                       \
   if (merges)                                                                                                           \
     hipLaunchKernelGGL((vis_merge_kernel<NA, S, SH>), dim3(merges), dim3(VIS_MERGE_THREADS), 0, s, P, mode, V, B.tri_rec, \

@@ -34,13 +34,23 @@ int main() {
     if (parts > np || tiles > nt) ++bad, std::printf("cap %u total %u prims %u: %u parts of %u, %u tiles of %u\n", cap, total, prims, parts, np, tiles, nt);
   }
   // a mesh of small triangles, and its neighbours on either side of the rule
-  if (vis_large(24000, 16384) || vis_part(16384, 24000, 4096, 88) != VIS_PART_SMALL) ++bad;
+  if (vis_large(24000, 16384) || vis_part(16384, 24000, 1024, 88) != VIS_PART_SMALL - 1) ++bad;
   if (vis_large(4 * 16384 - 1, 16384) || !vis_large(4 * 16384, 16384)) ++bad;
-  if (vis_part(2000, 330000, 1024, 88) != VIS_PART_LARGE || vis_part(1u << 22, 6400000, 0, 160) != 10000) ++bad;
+  if (vis_part(2000, 330000, 1024, 88) != VIS_PART_LARGE - 1 || vis_part(1u << 22, 6400000, 0, 160) != 10239) ++bad;
   // a mesh keeps room for its own triangles after any number of small draws; deep draws are remembered
   if (record_estimate(20000, 522242, 8160) != 3 * 522242 + 8160 || record_estimate(0, 522242, 8160) != 3 * 522242 + 8160) ++bad;
   if (record_estimate(330000, 2000, 1024) != 412500 || record_estimate(0, 12, 64) != 65536) ++bad;
   if (record_estimate(0xFFFFFFF0u, 1, 1) != MAX_RECORDS || record_estimate(0, 0x55554000u, 1 << 18) != MAX_RECORDS) ++bad;
+  // the steps are in order, and a list is in the step that holds it
+  for (uint32_t k = 0; k < VIS_STEPS; ++k) {
+    const uint32_t a = vis_step_size(k), last = k + 1 < VIS_STEPS ? vis_step_size(k + 1) - 1 : 0xFFFFFFFFu;
+    if (last <= a || vis_step(a) != k || vis_step(last) != k || vis_step(a + (last - a) / 2) != k) ++bad;
+  }
+  for (int it = 0; it < 100000; ++it) {  // the tiles that a part size splits are those of its step and above
+    const uint32_t part = vis_part(1 + uint32_t(below(1u << 30)), uint32_t(below(1ull << 32)), uint32_t(below(1u << 18)), 160);
+    const uint32_t n = it % 2 ? part + uint32_t(below(3)) : VIS_PART_SMALL + uint32_t(below(0xFFFFF000u));
+    if ((n > part) != (n >= VIS_PART_SMALL && vis_step(n) >= vis_step(part + 1))) ++bad;
+  }
   // lists that keep the pass waiting are split, lists of a pass that is busy for longer are not
   if (vis_part(522242, 560000, 1008, vis_tile_cost(4, true)) > 1500 || vis_part(522242, 910000, 6500, vis_tile_cost(4, true)) < 2800) ++bad;
   if (vis_can_split(682) || !vis_can_split(683)) ++bad;
