@@ -1504,7 +1504,8 @@ __global__ void __launch_bounds__(256) tile_ranges_kernel(const uint32_t* __rest
     if (n >= VIS_PART_SMALL) atomicAdd(&counters[CT_STEP + vis_step(n)], 1u);
   }
 }
-// The scheduling order, the parts of split tiles, and the records to their tiles' lists: position = first record of the tile + rank in it.
+// The scheduling order, the parts of split tiles and the mail (workgroups of the tiles), and the records to their
+// tiles' lists (the others): position = first record of the tile + rank in it.
 constexpr uint32_t SCATTER_PER_THREAD = 4;
 __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
                                                            const uint32_t* __restrict__ ranks,
@@ -1532,7 +1533,10 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
       __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
-  for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < T; t += gridDim.x * 256) {
+  const uint32_t tile_blocks = (T + 255) / 256;
+  if (blockIdx.x < tile_blocks) {
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= T) return;
     const uint32_t c = place[t] >> PLACE_BITS;
     uint32_t at = place[t] & ((1u << PLACE_BITS) - 1u);
 #pragma unroll
@@ -1545,11 +1549,11 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
       merges[atomicAdd(ct_merges, 1u)] = make_uint4(t, np, e, 0u);
       for (uint32_t k = 0; k < np; ++k) parts[e + k] = make_uint4(t, k, np, 0u);
     }
+    return;
   }
-  // the first workgroup, which writes the mail, has no records
   const uint32_t n = min(total, cap);
-  const uint32_t b0 = (blockIdx.x - 1) * (256 * SCATTER_PER_THREAD);
-  if (blockIdx.x == 0 || b0 >= n) return;
+  const uint32_t b0 = (blockIdx.x - tile_blocks) * (256 * SCATTER_PER_THREAD);
+  if (b0 >= n) return;
   uint32_t k[SCATTER_PER_THREAD], v[SCATTER_PER_THREAD], r[SCATTER_PER_THREAD];
 #pragma unroll
   for (uint32_t j = 0; j < SCATTER_PER_THREAD; ++j) {  // clamped indices: no branch per load
@@ -1689,7 +1693,7 @@ void launch_tile_lists(const draw_params& P, const draw_buffers& B, uint32_t cap
   const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
   if (!T) return;
   const uint32_t per = 256 * SCATTER_PER_THREAD;
-  hipLaunchKernelGGL(tile_scatter_kernel, dim3((std::max(cap, T) + per - 1) / per + 1), dim3(256), 0, s, B.keys[0], B.vals[0],
+  hipLaunchKernelGGL(tile_scatter_kernel, dim3((T + 255) / 256 + (std::max<uint32_t>(cap, 1) + per - 1) / per), dim3(256), 0, s, B.keys[0], B.vals[0],
                      B.keys[1], B.counters, cap, B.tstart, B.tend, B.vals[1], T, reinterpret_cast<const uint32_t*>(B.partial),
                      order, B.vis_split, P.prim_count, B.tile_cost, B.counters + CT_PARTS,
                      B.counters + CT_MERGES, B.vis_parts, B.vis_merges, mail, seq);

@@ -751,8 +751,8 @@ __global__ void __launch_bounds__(SRX_VIS_THREADS, 4) vis_kernel(draw_params P, 
                                                    const ps_samplers* __restrict__ SM, uint32_t* __restrict__ wout) {
   const uint32_t records = record_total(V.counters);
   if (records > V.cap) return;  // records were dropped: the draw is emitted again
-  const uint32_t part = vis_part(P.prim_count, records, busy_tiles(V.counters, static_cast<uint32_t>(P.gtiles_x * P.gtiles_y)),
-                                 V.tile_cost);
+  const uint32_t T = static_cast<uint32_t>(P.gtiles_x * P.gtiles_y);
+  const uint32_t part = V.max_parts ? vis_part(P.prim_count, records, busy_tiles(V.counters, T), V.tile_cost) : 0u;
   vis_span ws;
   ws.parts = 1;
   ws.slot = 0;
