@@ -38,7 +38,7 @@ SRX_HD inline bool vis_large(uint64_t records, uint32_t prims) {
 // A tile's time is its list's length and what finishing it costs, so lists much longer than an even share of
 // both over the workgroups the GPU holds at a time (VIS_SLOTS of them busy) are split: the textured mesh frame
 // at the oblique camera has 1,008 tiles with records, 433 in the median and 4,184 in the longest, which alone
-// kept the pass running for 170 us (split: 78 + 30 us for the merge).  Where the pass outlasts its longest tile
+// kept the pass running for 170 us (split: 88 + 29 us for the merge).  Where the pass outlasts its longest tile
 // a split only adds work: the same mesh over most of the target takes 282 us a frame without splits and 311
 // with every tile of more than an even share of the records alone split (4 samples; 1 sample 173 and 192).
 // Draws of large triangles, whose lists depth culling shortens as it goes, are split later.

@@ -308,8 +308,7 @@ __device__ __forceinline__ float4 bilinear_wrap_rgba8(const surface_desc& s, flo
 // instructions of wrap_linear_axis on each axis, and no multiplication or clamp for its addresses.
 // The shading is bound by instruction issue there: 32k blended triangles at 1280x720, trilinear, 178 -> 144 us
 // a pass; a 2-sample 1919x1079 mesh, 8x anisotropic, 235 -> 227; the compiled SASL shading of 522k triangles
-// at 1920x1080, 16x, 197 -> 169.  (The 4-sample fused kernel of that mesh spills five registers more for the
-// general call below: 157 -> 162.)
+// at 1920x1080, 16x, 197 -> 169.
 struct tap_level {
   const uint32_t* t;
   float sw, sh, bw, bh;  // sides, and sides * 8192
