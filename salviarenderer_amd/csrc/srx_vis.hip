@@ -788,6 +788,7 @@ __global__ void __launch_bounds__(VIS_MERGE_THREADS, 2) vis_merge_kernel(draw_pa
   __shared__ unsigned long long keys[PX * S];
   __shared__ uint2 items[SHADE ? PX * S : 1];
   __shared__ uint32_t nitems;
+  if (blockIdx.x >= V.counters[CT_MERGES]) return;  // the host's count, by steps, is the same
   const uint4 m = V.merges[blockIdx.x];
   const unsigned long long* src = V.partial + static_cast<size_t>(m.z) * (PX * S);
   for (int i = threadIdx.x; i < PX * S; i += VIS_MERGE_THREADS) {
