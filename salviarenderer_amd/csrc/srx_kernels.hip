@@ -1522,7 +1522,7 @@ __global__ void __launch_bounds__(256) tile_scatter_kernel(const uint32_t* __res
   const uint32_t part = may_split ? vis_part(prims, total, busy_tiles(counters, T), tile_cost) : 0u;
   if (blockIdx.x == 0 && threadIdx.x < 64) {  // the counts are final; the host waits for seq
     uint32_t split_tiles = 0;
-    if (may_split)
+    if (may_split && counters[CT_CLASS] + counters[CT_CLASS + 1])  // a tile of VIS_PART_SMALL records or more
       for (uint32_t k = vis_step(part + 1) + threadIdx.x; k < VIS_STEPS; k += 64) split_tiles += counters[CT_STEP + k];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) split_tiles += static_cast<uint32_t>(__shfl_xor(static_cast<int>(split_tiles), off, 64));

@@ -56,7 +56,7 @@ SRX_HD inline uint32_t vis_step(uint32_t records) {  // the largest step of at m
   const uint32_t lg = 31u - static_cast<uint32_t>(__builtin_clz(records));
   return 4u * (lg - 10u) + ((records >> (lg - 2u)) & 3u);
 }
-static_assert(VIS_PART_SMALL == 1u << 10 && VIS_PART_LARGE >= VIS_PART_SMALL, "step 0");
+static_assert(VIS_PART_SMALL == 1u << 10 && VIS_PART_LARGE >= VIS_PART_SMALL, "step 0, and the two heaviest classes of tiles");
 // Records per part of a draw with `records` records on `tiles` tiles: a tile with more is split, that is one
 // whose step is vis_step(part + 1) or above.
 SRX_HD inline uint32_t vis_part(uint32_t prims, uint32_t records, uint32_t tiles, uint32_t tile_cost) {
